@@ -148,7 +148,7 @@ int orb_match_bf(orb_context* ctx, const uint8_t* query, int nq, const uint8_t* 
  * of ORBmatcher::DescriptorDistance) -- over all nm map rows.
  * idx2/dist2: 2 ints per query (-1 / INT_MAX when fewer than two rows);
  * accept[i] = best < (float)second * ratio (may be NULL).
- * method 0: XOR + popcount kernel; 1: int8 +-1 MFMA kernel (dot = 256 - 2*d).
+ * method 0: XOR + popcount kernel; 1: FP4 MFMA kernel (exact sums of +-1).
  * Both give identical results.  nm < 2^31. */
 int orb_knn2(orb_context* ctx, const uint8_t* query, int nq, const uint8_t* map, int64_t nm, int method, float ratio,
              int32_t* idx2, int32_t* dist2, uint8_t* accept);

@@ -35,12 +35,12 @@ extern "C" hipError_t orb_launch_undistort(const OrbKeyPoint* in, int n, const i
 extern "C" hipError_t orb_launch_rgbd_depth(const OrbKeyPoint* kps, const OrbKeyPoint* kun, int n, const int* count,
                                             const float* depth, int w, int h, size_t pitch, float bf, float* uR,
                                             float* dep, hipStream_t st);
-extern "C" int orb_knn_chunks(long long nm);
+extern "C" int orb_knn_chunk_rows(int nq, long long nm, int method, size_t max_entries);
 extern "C" int orb_knn_scratch_setup(int device);
 extern "C" uint2* orb_knn_scratch(int device, size_t* entries);
 extern "C" hipError_t orb_launch_knn2(const uint8_t* q, int nq, const uint8_t* m, long long nm, int method,
-                                      float ratio, uint2* part, int* idx2, int* dist2, uint8_t* accept,
-                                      hipStream_t st, hipEvent_t* ev);
+                                      float ratio, uint2* part, int chunk_rows, int* idx2, int* dist2,
+                                      uint8_t* accept, hipStream_t st, hipEvent_t* ev);
 
 namespace orb_detail {
 

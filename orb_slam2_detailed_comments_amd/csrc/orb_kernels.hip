@@ -2172,18 +2172,23 @@ extern "C" hipError_t orb_launch_match_bf(const uint8_t* q, const int* nq, const
 // ============================================================ dense k=2
 // All-pairs Hamming search of nq queries against nm map rows, k = 2 nearest
 // by (distance, index), the order of ORBmatcher's best/second-best update
-// (ORBmatcher.cc:614-647).  The map is split into chunks of KNN_CHUNK rows;
-// each (chunk, query tile) workgroup keeps per query the two smallest keys
+// (ORBmatcher.cc:614-647).  The map is split into chunks of at most KNN_CHUNK
+// rows; each (chunk, query block) workgroup keeps two keys per query
 //   key = distance << 20 | row-in-chunk
-// (lexicographic (distance, index) is numeric key order, so the update is
-// k1 = med3(k0, k1, key); k0 = min(k0, key)), and a merge kernel reduces the
-// chunks.  Two kernels produce the same partial keys:
+// (lexicographic (distance, index) is numeric key order), and a merge kernel
+// reduces the chunks:
 //   knn_popc_kernel  XOR + v_bcnt popcount, one query per lane, map rows
-//                    broadcast from LDS
-//   knn_mfma_kernel  bits expanded to int8 +-1; v_mfma_i32_16x16x64_i8 gives
-//                    dot = 256 - 2*Hamming exactly (int32 accumulate)
+//                    broadcast from LDS; the keys are the chunk's two
+//                    smallest
+//   knn_mfma_kernel  bits expanded to FP4, the distance a sum of exact
+//                    products on the matrix cores; the keys are the two
+//                    smallest of the minima of groups of 16 rows, and the
+//                    merge looks at the best row's group
 #define KNN_CHUNK 8192
 #define KNN_NONE 0xFFFFFFFFu
+#ifndef KNN_NG
+#define KNN_NG 2                     // 32-query groups per wavefront (4: 1 % faster at 2000 x 1M, slower below)
+#endif
 
 // Median of three (the compiler emits v_med3_u32 / v_med3_i32).
 __device__ __forceinline__ unsigned med3u(unsigned a, unsigned b, unsigned c)
@@ -2198,7 +2203,7 @@ __device__ __forceinline__ int med3i(int a, int b, int c)
 
 __global__ __launch_bounds__(256) void knn_popc_kernel(const uint8_t* __restrict__ q, int nq,
                                                        const uint8_t* __restrict__ m, long long nm,
-                                                       uint2* __restrict__ part, int nchunks)
+                                                       uint2* __restrict__ part, int nchunks, int chunk_rows)
 {
     __shared__ uint4 rows[256][2];
     const int tid = threadIdx.x;
@@ -2209,8 +2214,8 @@ __global__ __launch_bounds__(256) void knn_popc_kernel(const uint8_t* __restrict
         a0 = *(const uint4*)(q + (size_t)qi * 32);
         a1 = *(const uint4*)(q + (size_t)qi * 32 + 16);
     }
-    const long long c0 = (long long)chunk * KNN_CHUNK;
-    const int len = (int)min((long long)KNN_CHUNK, nm - c0);
+    const long long c0 = (long long)chunk * chunk_rows;
+    const int len = (int)min((long long)chunk_rows, nm - c0);
     unsigned k0 = KNN_NONE, k1 = KNN_NONE;
     for (int t0 = 0; t0 < len; t0 += 256) {
         const int n = min(256, len - t0);
@@ -2239,228 +2244,213 @@ __global__ __launch_bounds__(256) void knn_popc_kernel(const uint8_t* __restrict
     if (qi < nq) part[(size_t)qi * nchunks + chunk] = make_uint2(k0, k1);
 }
 
-// Bit -> int8 expansion of the MFMA operands.  Flat dword F (0..63) of a
-// descriptor holds, in bytes 0..3, bits {i, i+8, i+16, i+24} of 32-bit word
-// u = F/8, with i = F%8.  Map side: a set bit becomes byte 0x80 (-128), a
-// clear bit 0 -- one shift and one mask.  Query side: a set bit becomes 0x40
-// (+64), a clear bit 0xC0 (-64) -- the same with an XOR.
-__device__ __forceinline__ unsigned expand_map_dword(unsigned w, int i)
+typedef int knn_v8i __attribute__((ext_vector_type(8)));
+typedef float knn_v16f __attribute__((ext_vector_type(16)));
+
+// Bit -> FP4 (E2M1) expansion of a descriptor word into the 32 nibbles of
+// one MFMA operand lane: nibble k of dword i holds bit 4k + i.  Map side: a
+// clear bit is 0 and a set bit 0.5, 1, 2 and 2 in dwords 0 .. 3 (the code's
+// bits 0, 1, 2 and 2, so that three of the four dwords are one mask each).
+// Query side: +-2, 1, 0.5 and 0.5, minus for a set bit, so every product is
+// 0 or +-1.  Both sides use the same order, so the hardware's own k order
+// cancels.
+__device__ __forceinline__ knn_v8i expand_map(unsigned w)
 {
-    return (w << (7 - i)) & 0x80808080u;
+    return (knn_v8i){(int)(w & 0x11111111u), (int)(w & 0x22222222u), (int)(w & 0x44444444u),
+                     (int)((w >> 1) & 0x44444444u), 0, 0, 0, 0};
 }
 
-__device__ __forceinline__ unsigned expand_query_dword(unsigned w, int i)
+__device__ __forceinline__ knn_v8i expand_query(unsigned w)
 {
-    return expand_map_dword(w, i) ^ 0xC0C0C0C0u;
+    return (knn_v8i){(int)(((w << 3) & 0x88888888u) | 0x44444444u), (int)(((w << 2) & 0x88888888u) | 0x22222222u),
+                     (int)(((w << 1) & 0x88888888u) | 0x11111111u), (int)((w & 0x88888888u) | 0x11111111u), 0, 0, 0, 0};
 }
 
-typedef int knn_v4i __attribute__((ext_vector_type(4)));
-
-// One 64-row tile into LDS: this thread's four map words (rows 16j + fl%16)
-// expanded to the operand dwords F0..F0+3 of lane fl, k-chunk fc.
-__device__ __forceinline__ void knn_fill_tile(uint4 (*A)[4][64], const unsigned* wn, int fc, int fl, int fi0)
-{
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        uint4 v;
-        v.x = expand_map_dword(wn[j], fi0 + 0);
-        v.y = expand_map_dword(wn[j], fi0 + 1);
-        v.z = expand_map_dword(wn[j], fi0 + 2);
-        v.w = expand_map_dword(wn[j], fi0 + 3);
-        A[j][fc][fl] = v;
-    }
-}
-
-// The 16 MFMAs of subtile s (16 map rows x 64 queries): acc[gq] = C + sum
-// over the four 64-wide k-chunks, C = `rows`.
-__device__ __forceinline__ void knn_subtile(const uint4 (*A)[4][64], int s, int lane, const knn_v4i (*B)[4],
-                                            knn_v4i rows, knn_v4i* acc)
-{
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const uint4 av = A[s][c][lane];
-        const knn_v4i a = (knn_v4i){(int)av.x, (int)av.y, (int)av.z, (int)av.w};
-#pragma unroll
-        for (int gq = 0; gq < 4; gq++)
-            acc[gq] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, B[gq][c], c == 0 ? rows : acc[gq], 0, 0, 0);
-    }
-}
-
-// Workgroup: 4 wavefronts x 64 queries, one map chunk.  Map rows are
-// expanded 64 at a time into LDS in operand order [subtile][k-chunk][lane];
-// each wavefront runs 4 (k-chunks) x 4 (query groups) MFMAs per 16 rows.
+// Workgroup: 4 wavefronts, the same 32 * NG queries, one map chunk; wavefront
+// w takes the 32-row tiles w, w + 4, ...  Bound: the MFMA pipe (a kernel of
+// the same instructions on registers alone reaches 7.5 of the 10 POP/s).
+// 2000 queries x 1M rows: search and merge 170 us (6.2 POP/s) where int8
+// MFMAs with every key kept took 404 us; 64 x 1M 15 us (171).
 //
-// The operands are scaled so that the accumulator is the search key itself.
-// With map bits m -> -128 m and query bits q -> 64 (2q - 1),
-//   sum -128 m 64 (2q - 1) = 8192 sum m (1 - 2q) = 8192 (Hamming - |q|)
-// since Hamming = |q| + sum m (1 - 2q); the MFMA's C input is the row's index
-// in the chunk.  |q| is constant per query, so
-//   key = 8192 (Hamming - |q|) + row          (|key| < 2^22)
-// orders (distance, row) exactly for rows under 8192 = KNN_CHUNK, and the
-// top-2 update is one v_med3_i32 and one v_min_i32 per map row and query.
-// 256 VGPRs would leave 3 wavefronts per SIMD and 768 of the 1024 workgroup
-// slots for the 984 workgroups of a 2000 x 1M search; the bound of 4 keeps
-// every workgroup resident.
-__global__ __launch_bounds__(256, 4) void knn_mfma_kernel(const uint8_t* __restrict__ q, int nq,
-                                                          const uint8_t* __restrict__ m, long long nm,
-                                                          uint2* __restrict__ part, int nchunks)
+// v_mfma_scale_f32_32x32x64_f8f6f4 on FP4 operands does 65536 multiply-adds
+// in 32 cycles, twice the int8 rate, and a descriptor word expands into one
+// operand lane with 5 VALU ops.  sum m (1 - 2q) = Hamming - |q|; the C input
+// adds 256 and the row / 8192, so every accumulator is a non-negative
+// multiple of 2^-13 of at most 22 bits, exact in float, and its bits order
+// as an integer:
+//   key = Hamming - |q| + 256 + row / 8192.
+// |q| is constant per query, so keys order (distance, row).
+//
+// The 16 accumulators of a lane are 16 rows of one tile for one query.  Only
+// the smallest is kept (8 v_min3 for 16 keys) and enters the lane's two
+// smallest: of all such groups of 16 rows, the best row is the minimum of
+// the group with the smallest minimum, and the second best is either the
+// next group's minimum or in the best row's own group, whose other 15 rows
+// the merge kernel looks at.  That is 11 VALU ops for 16 keys where keeping
+// the two smallest of all keys takes 32.
+template <int NG>
+__global__ __launch_bounds__(256) void knn_mfma_kernel(const uint8_t* __restrict__ q, int nq,
+                                                       const uint8_t* __restrict__ m, long long nm,
+                                                       uint2* __restrict__ part, int nchunks, int chunk_rows)
 {
-    __shared__ uint4 A[4][4][64];   // 16 KB: 64 rows of expanded bytes
-    __shared__ int popq[256];       // |q| of the workgroup's queries
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int g = lane >> 4, i16 = lane & 15;
-    const int chunk = blockIdx.x;
-    const int qbase = blockIdx.y * 256 + wv * 64;
-    {
-        const int qi = blockIdx.y * 256 + tid;
-        int pc = 0;
-        if (qi < nq) {
-#pragma unroll
-            for (int u = 0; u < 8; u++) pc += __popc(*(const unsigned*)(q + (size_t)qi * 32 + 4 * u));
-        }
-        popq[tid] = pc;   // read after the loop's first barrier
-    }
+    __shared__ int2 s_key[3][NG][64];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int hb = lane >> 5, i32 = lane & 31;
+    // XCD x (workgroups b with b % 8 == x) takes chunks x, x + 8, ..., all
+    // query blocks of a chunk one after another, so the chunk's rows come
+    // from memory once and from that XCD's L2 after that (2000 x 1M search
+    // 220 -> 197 us against chunks spread over the XCDs).
+    const int nqb = (nq + 32 * NG - 1) / (32 * NG);
+    const int slot = blockIdx.x / ORB_NUM_XCD;
+    const int chunk = slot / nqb * ORB_NUM_XCD + blockIdx.x % ORB_NUM_XCD;
+    const int qbase = slot % nqb * 32 * NG;
+    if (chunk >= nchunks) return;
 
-    // Query operands: group gq, k-chunk c -> this lane's 4 dwords F = 16c+4g+d.
-    knn_v4i B[4][4];
+    // Query operands: lane (query i32, half hb) holds words 4 hb + c.
+    knn_v8i B[NG][4];
+    int pop[NG];
 #pragma unroll
-    for (int gq = 0; gq < 4; gq++) {
-        const int qi = qbase + 16 * gq + i16;
-        unsigned w[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) w[u] = qi < nq ? *(const unsigned*)(q + (size_t)qi * 32 + 4 * u) : 0u;
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-#pragma unroll
-            for (int d = 0; d < 4; d++) {
-                const int F = 16 * c + 4 * g + d;
-                B[gq][c][d] = (int)expand_query_dword(w[F >> 3], F & 7);
-            }
-        }
+    for (int n = 0; n < NG; n++) {
+        const int qi = min(qbase + 32 * n + i32, nq - 1);
+        const uint4 w = gload16(q + (size_t)qi * 32 + 16 * hb);
+        B[n][0] = expand_query(w.x);
+        B[n][1] = expand_query(w.y);
+        B[n][2] = expand_query(w.z);
+        B[n][3] = expand_query(w.w);
+        pop[n] = __popc(w.x) + __popc(w.y) + __popc(w.z) + __popc(w.w);
+        pop[n] += __shfl_xor(pop[n], 32, 64);
     }
-    const long long c0 = (long long)chunk * KNN_CHUNK;
-    const int len = (int)min((long long)KNN_CHUNK, nm - c0);
-    int k0[4], k1[4];
+    const long long c0 = (long long)chunk * chunk_rows;
+    const int len = (int)min((long long)chunk_rows, nm - c0);
+    int k0[NG], k1[NG];
 #pragma unroll
-    for (int gq = 0; gq < 4; gq++) k0[gq] = k1[gq] = INT_MAX;
+    for (int n = 0; n < NG; n++) k0[n] = k1[n] = INT_MAX;
+    // Accumulator r of a lane is row 8 (r >> 2) + 4 hb + (r & 3) of the tile.
+    knn_v16f rows;
+#pragma unroll
+    for (int r = 0; r < 16; r++) rows[r] = 256.f + (float)(8 * (r >> 2) + 4 * hb + (r & 3)) * (1.f / KNN_CHUNK);
 
-    // Accumulator (lane, r) = (map row t0 + 16s + 4g + r, query 16gq + i16):
-    // `rows` is the C input of subtile s, advanced by 16 per subtile.
-    knn_v4i rows = (knn_v4i){4 * g, 4 * g + 1, 4 * g + 2, 4 * g + 3};
-    // Fill role of this thread: k-chunk fc = wavefront, operand lane fl, so
-    // that the wavefront's 16-byte LDS writes are consecutive (no bank
-    // conflicts): for subtile j, row 16j + (fl & 15), dwords F0..F0+3 with
-    // F0 = 16 fc + 4 (fl >> 4), i.e. bits 4 (fl >> 4 & 1) + 0..3 (+8k) of
-    // word 2 fc + (fl >> 5).  The next tile's words are loaded before the
-    // current tile's MFMAs run.  Full 64-row tiles run without bounds checks;
-    // the chunk's last, partial tile takes the checked form.
-    // Rows past the chunk's end read its last row instead (their keys are
-    // discarded in the checked form).
-    const int fc = wv, fl = lane;
-    const int fi0 = 4 * ((fl >> 4) & 1);
-    const uint8_t* mchunk = m + (size_t)c0 * 32;                 // uniform base
-    const unsigned fword = 4u * (unsigned)(2 * fc + (fl >> 5));  // + 32-bit lane offsets
-    const int nfull = len & ~63;
-    unsigned wn[4];
+    const uint8_t* mchunk = m + (size_t)c0 * 32;
+    // Rows past the chunk's end read its last row; their keys are discarded.
+    auto load = [&](int t0) {
+        return gload16(mchunk + ((unsigned)min(t0 + i32, len - 1) * 32u + 16u * (unsigned)hb));
+    };
+    uint4 wn = load(min(32 * wv, len - 1));
+    for (int t0 = 32 * wv; t0 < len; t0 += 128) {
+        const knn_v8i A[4] = {expand_map(wn.x), expand_map(wn.y), expand_map(wn.z), expand_map(wn.w)};
+        if (t0 + 128 < len) wn = load(t0 + 128);
+        knn_v16f acc[NG];
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-        wn[j] = *(const unsigned*)(mchunk + ((unsigned)min(16 * j + (fl & 15), len - 1) * 32u + fword));
-    for (int t0 = 0; t0 < nfull; t0 += 64) {
-        __syncthreads();
-        knn_fill_tile(A, wn, fc, fl, fi0);
-        __syncthreads();
-        if (t0 + 64 < len) {
+        for (int c = 0; c < 4; c++)
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                wn[j] = *(const unsigned*)(mchunk + ((unsigned)min(t0 + 64 + 16 * j + (fl & 15), len - 1) * 32u + fword));
-        }
+            for (int n = 0; n < NG; n++)
+                acc[n] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A[c], B[n][c], c == 0 ? rows : acc[n], 4, 4, 0, 0,
+                                                                        0, 0);
+        if (t0 + 32 > len) {                       // the chunk's last, partial tile
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-            knn_v4i acc[4];
-            knn_subtile(A, s, lane, B, rows, acc);
-            rows += 16;
+            for (int r = 0; r < 16; r++) {
+                const bool ok = t0 + 8 * (r >> 2) + 4 * hb + (r & 3) < len;
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-#pragma unroll
-                for (int gq = 0; gq < 4; gq++) {
-                    const int key = acc[gq][r];
-                    k1[gq] = med3i(k0[gq], k1[gq], key);
-                    k0[gq] = min(k0[gq], key);
-                }
+                for (int n = 0; n < NG; n++) acc[n][r] = ok ? acc[n][r] : __int_as_float(0x7F000000);
             }
         }
+        const float tile = (float)t0 * (1.f / KNN_CHUNK);
+#pragma unroll
+        for (int n = 0; n < NG; n++) {
+            int g = __float_as_int(acc[n][0]);
+#pragma unroll
+            for (int r = 1; r < 16; r++) g = min(g, __float_as_int(acc[n][r]));
+            const int key = __float_as_int(__int_as_float(g) + tile);
+            k1[n] = med3i(k0[n], k1[n], key);
+            k0[n] = min(k0[n], key);
+        }
     }
-    if (nfull < len) {
-        __syncthreads();
-        knn_fill_tile(A, wn, fc, fl, fi0);
-        __syncthreads();
-#pragma unroll 1
-        for (int s = 0; 16 * s < len - nfull; s++) {
-            knn_v4i acc[4];
-            knn_subtile(A, s, lane, B, rows, acc);
+    // Merge the two lanes that hold a query, then the four wavefronts.
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const bool ok = rows[r] < len;
+    for (int n = 0; n < NG; n++) {
+        const int b0 = __shfl_xor(k0[n], 32, 64), b1 = __shfl_xor(k1[n], 32, 64);
+        const int n0 = min(k0[n], b0);
+        k1[n] = min(max(k0[n], b0), min(k1[n], b1));
+        k0[n] = n0;
+        if (wv > 0) s_key[wv - 1][n][lane] = make_int2(k0[n], k1[n]);
+    }
+    __syncthreads();
+    if (wv == 0 && hb == 0) {
 #pragma unroll
-                for (int gq = 0; gq < 4; gq++) {
-                    const int key = ok ? acc[gq][r] : INT_MAX;
-                    k1[gq] = med3i(k0[gq], k1[gq], key);
-                    k0[gq] = min(k0[gq], key);
-                }
+        for (int n = 0; n < NG; n++) {
+#pragma unroll
+            for (int w = 0; w < 3; w++) {
+                const int2 o = s_key[w][n][lane];
+                const int n0 = min(k0[n], o.x);
+                k1[n] = min(max(k0[n], o.x), min(k1[n], o.y));
+                k0[n] = n0;
             }
-            rows += 16;
-        }
-    }
-    // Merge the four lanes that hold the same query (lanes i16 + 16g) and
-    // convert to the partial format distance << 20 | row.
+            const int qi = qbase + 32 * n + i32;
+            if (qi < nq) {
+                const int ks[2] = {k0[n], k1[n]};
+                unsigned out[2];
 #pragma unroll
-    for (int gq = 0; gq < 4; gq++) {
-#pragma unroll
-        for (int o = 16; o <= 32; o <<= 1) {
-            const int b0 = __shfl_xor(k0[gq], o, 64), b1 = __shfl_xor(k1[gq], o, 64);
-            const int n0 = min(k0[gq], b0);
-            const int n1 = min(max(k0[gq], b0), min(k1[gq], b1));
-            k0[gq] = n0;
-            k1[gq] = n1;
-        }
-        const int qi = qbase + 16 * gq + i16;
-        if (g == 0 && qi < nq) {
-            const int pc = popq[wv * 64 + 16 * gq + i16];
-            const int ks[2] = {k0[gq], k1[gq]};
-            unsigned out[2];
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-                out[t] = ks[t] == INT_MAX ? KNN_NONE
-                                          : ((unsigned)((ks[t] >> 13) + pc) << 20) | (unsigned)(ks[t] & (KNN_CHUNK - 1));
-            part[(size_t)qi * nchunks + chunk] = make_uint2(out[0], out[1]);
+                for (int t = 0; t < 2; t++) {
+                    // keys of rows past the end are at least 2^127
+                    const int v = ks[t] < 0x7F000000 ? (int)(__int_as_float(ks[t]) * KNN_CHUNK) : 0;
+                    out[t] = ks[t] >= 0x7F000000
+                                 ? KNN_NONE
+                                 : ((unsigned)((v >> 13) - 256 + pop[n]) << 20) | (unsigned)(v & (KNN_CHUNK - 1));
+                }
+                part[(size_t)qi * nchunks + chunk] = make_uint2(out[0], out[1]);
+            }
         }
     }
 }
 
 // Reduce the per-chunk keys of each query to the global two nearest and apply
-// the ratio test (best < ratio * second, in float).
+// the ratio test (best < ratio * second, in float).  A wavefront per query:
+// its lanes stride over the chunks, then 16 of them take a row each of the
+// best row's group (knn_mfma_kernel keeps one key per group of 16).  knn_popc_kernel's keys are
+// the two smallest already, and then the group holds none nearer.  Bound:
+// latency; 8 us for 2000 queries x 123 chunks, where one thread per query
+// took 47 us, a chain of scattered reads.
 __global__ __launch_bounds__(256) void knn_merge_kernel(const uint2* __restrict__ part, int nq, int nchunks,
-                                                        float ratio, int* __restrict__ idx2, int* __restrict__ dist2,
+                                                        int chunk_rows, const uint8_t* __restrict__ q,
+                                                        const uint8_t* __restrict__ m, long long nm, float ratio,
+                                                        int* __restrict__ idx2, int* __restrict__ dist2,
                                                         uint8_t* __restrict__ accept)
 {
-    const int qi = blockIdx.x * 256 + threadIdx.x;
-    if (qi >= nq) return;
-    unsigned long long b0 = ~0ull, b1 = ~0ull;
-    for (int c = 0; c < nchunks; c++) {
+    const int lane = threadIdx.x & 63, sub = lane & 15;
+    const int qi = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (qi >= nq) return;                          // the whole wavefront leaves
+    unsigned long long b0 = ~0ull, b1 = ~0ull;     // distance << 40 | row
+    auto take = [&](unsigned long long k) {
+        b1 = k < b0 ? b0 : (k < b1 ? k : b1);
+        b0 = k < b0 ? k : b0;
+    };
+    for (int c = lane; c < nchunks; c += 64) {
         const uint2 p = part[(size_t)qi * nchunks + c];
         const unsigned ks[2] = {p.x, p.y};
-        for (int t = 0; t < 2; t++) {
-            if (ks[t] == KNN_NONE) continue;
-            const unsigned long long k = ((unsigned long long)(ks[t] >> 20) << 40) |
-                                         (unsigned long long)((long long)c * KNN_CHUNK + (ks[t] & 0xFFFFF));
-            if (k < b0) {
-                b1 = b0;
-                b0 = k;
-            } else if (k < b1) {
-                b1 = k;
-            }
-        }
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+            if (ks[t] != KNN_NONE)
+                take(((unsigned long long)(ks[t] >> 20) << 40) |
+                     (unsigned long long)((long long)c * chunk_rows + (ks[t] & 0xFFFFF)));
     }
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned long long c0 = __shfl_xor(b0, o, 64), c1 = __shfl_xor(b1, o, 64);
+        const unsigned long long n0 = min(b0, c0);
+        b1 = min(max(b0, c0), min(b1, c1));
+        b0 = n0;
+    }
+    if (b0 != ~0ull) {
+        const long long best = (long long)(b0 & 0xFFFFFFFFFFull);
+        const long long row = (best & ~31ll) + 8 * (sub >> 2) + (best & 4) + (sub & 3);
+        unsigned long long k = ~0ull;
+        if (row < nm && row != best) {
+            const uint4 a0 = *(const uint4*)(q + (size_t)qi * 32), a1 = *(const uint4*)(q + (size_t)qi * 32 + 16);
+            k = ((unsigned long long)hamming32(a0, a1, m + (size_t)row * 32) << 40) | (unsigned long long)row;
+        }
+        for (int o = 1; o < 16; o <<= 1) k = min(k, __shfl_xor(k, o, 16));
+        b1 = min(b1, k);
+    }
+    if (lane != 0) return;
     const int d0 = b0 == ~0ull ? INT_MAX : (int)(b0 >> 40), d1 = b1 == ~0ull ? INT_MAX : (int)(b1 >> 40);
     idx2[2 * qi] = b0 == ~0ull ? -1 : (int)(b0 & 0xFFFFFFFFFFull);
     idx2[2 * qi + 1] = b1 == ~0ull ? -1 : (int)(b1 & 0xFFFFFFFFFFull);
@@ -2469,24 +2459,39 @@ __global__ __launch_bounds__(256) void knn_merge_kernel(const uint2* __restrict_
     if (accept) accept[qi] = (uint8_t)(b0 != ~0ull && b1 != ~0ull && (float)d0 < (float)d1 * ratio);
 }
 
-extern "C" int orb_knn_chunks(long long nm) { return (int)((nm + KNN_CHUNK - 1) / KNN_CHUNK); }
+// Rows per map chunk: KNN_CHUNK, halved while the grid has fewer than 1024
+// workgroups (the GPU holds that many), down to 512 rows, as long as the
+// partial keys (one entry per query and chunk) stay within max_entries.
+// Search of 500 x 100k: 13 us at 512 rows, 169 us before at 8192 (26
+// workgroups); 2000 x 1M: 197 us at 8192 rows, 201 at 4096, 211 at 2048, and
+// the merge grows with the chunks.
+extern "C" int orb_knn_chunk_rows(int nq, long long nm, int method, size_t max_entries)
+{
+    const long long tiles = method == 1 ? (nq + 32 * KNN_NG - 1) / (32 * KNN_NG) : (nq + 255) / 256;
+    int rows = KNN_CHUNK;
+    while (rows > 512 && tiles * ((nm + rows - 1) / rows) < 1024 &&
+           (unsigned long long)nq * (unsigned long long)((nm + rows / 2 - 1) / (rows / 2)) <= max_entries)
+        rows /= 2;
+    return rows;
+}
 
 extern "C" hipError_t orb_launch_knn2(const uint8_t* q, int nq, const uint8_t* m, long long nm, int method,
-                                      float ratio, uint2* part, int* idx2, int* dist2, uint8_t* accept,
-                                      hipStream_t st, hipEvent_t* ev)
+                                      float ratio, uint2* part, int chunk_rows, int* idx2, int* dist2,
+                                      uint8_t* accept, hipStream_t st, hipEvent_t* ev)
 {
-    const int nchunks = orb_knn_chunks(nm);
+    const int nchunks = (int)((nm + chunk_rows - 1) / chunk_rows);
     if (nq <= 0) return hipSuccess;
     if (ev) (void)hipEventRecord(ev[0], st);
     if (nchunks > 0) {
-        const dim3 grid(nchunks, (nq + 255) / 256);
         if (method == 1)
-            knn_mfma_kernel<<<grid, 256, 0, st>>>(q, nq, m, nm, part, nchunks);
+            knn_mfma_kernel<KNN_NG><<<(nchunks + ORB_NUM_XCD - 1) / ORB_NUM_XCD * ORB_NUM_XCD *
+                                          ((nq + 32 * KNN_NG - 1) / (32 * KNN_NG)),
+                                      256, 0, st>>>(q, nq, m, nm, part, nchunks, chunk_rows);
         else
-            knn_popc_kernel<<<grid, 256, 0, st>>>(q, nq, m, nm, part, nchunks);
+            knn_popc_kernel<<<dim3(nchunks, (nq + 255) / 256), 256, 0, st>>>(q, nq, m, nm, part, nchunks, chunk_rows);
     }
     if (ev) (void)hipEventRecord(ev[1], st);
-    knn_merge_kernel<<<(nq + 255) / 256, 256, 0, st>>>(part, nq, nchunks, ratio, idx2, dist2, accept);
+    knn_merge_kernel<<<(nq + 3) / 4, 256, 0, st>>>(part, nq, nchunks, chunk_rows, q, m, nm, ratio, idx2, dist2, accept);
     if (ev) (void)hipEventRecord(ev[2], st);
     return hipGetLastError();
 }

@@ -1295,10 +1295,11 @@ int orb_knn2_device(orb_context* ctx, const uint8_t* d_query, int nq, const uint
     if (nq == 0) return ORB_OK;
     if (!d_query || !d_idx2 || !d_dist2 || (nm && !d_map)) return ORB_E_ARG;
     HIP_TRY(hipSetDevice(ctx->device));
-    const size_t nchunks = (size_t)orb_knn_chunks(nm);
+    const int rows = orb_knn_chunk_rows(nq, nm, method, SIZE_MAX);
+    const size_t nchunks = (size_t)((nm + rows - 1) / rows);
     int rc = ctx->grow((void**)&ctx->d_part, &ctx->part_cap, std::max<size_t>(1, (size_t)nq * nchunks) * sizeof(uint2));
     if (rc) return rc;
-    HIP_TRY(orb_launch_knn2(d_query, nq, d_map, nm, method, ratio, ctx->d_part, d_idx2, d_dist2, d_accept,
+    HIP_TRY(orb_launch_knn2(d_query, nq, d_map, nm, method, ratio, ctx->d_part, rows, d_idx2, d_dist2, d_accept,
                             ctx->stream, nullptr));
     return ORB_OK;
 }
@@ -1312,9 +1313,10 @@ int orb_knn2_device_noalloc(orb_context* ctx, const uint8_t* d_query, int nq, co
     size_t entries = 0;
     uint2* part = orb_knn_scratch(ctx->device, &entries);
     if (!part) return ORB_E_DEVICE;
-    if ((size_t)nq * (size_t)orb_knn_chunks(nm) > entries) return ORB_E_CAPACITY;
+    const int rows = orb_knn_chunk_rows(nq, nm, method, entries);
+    if ((size_t)nq * (size_t)((nm + rows - 1) / rows) > entries) return ORB_E_CAPACITY;
     HIP_TRY(hipSetDevice(ctx->device));
-    HIP_TRY(orb_launch_knn2(d_query, nq, d_map, nm, method, ratio, part, d_idx2, d_dist2, d_accept, ctx->stream,
+    HIP_TRY(orb_launch_knn2(d_query, nq, d_map, nm, method, ratio, part, rows, d_idx2, d_dist2, d_accept, ctx->stream,
                             nullptr));
     return ORB_OK;
 }
@@ -1359,7 +1361,8 @@ int orb_knn2_time(orb_context* ctx, const uint8_t* query, int nq, const uint8_t*
         (method != 0 && method != 1))
         return ORB_E_ARG;
     HIP_TRY(hipSetDevice(ctx->device));
-    const size_t nchunks = (size_t)orb_knn_chunks(nm);
+    const int rows = orb_knn_chunk_rows(nq, nm, method, SIZE_MAX);
+    const size_t nchunks = (size_t)((nm + rows - 1) / rows);
     int rc = ctx->grow((void**)&ctx->d_part, &ctx->part_cap, (size_t)nq * nchunks * sizeof(uint2));
     if (!rc) rc = ctx->grow((void**)&ctx->d_kq, &ctx->kq_cap, (size_t)nq * 32);
     if (!rc) rc = ctx->grow((void**)&ctx->d_km, &ctx->km_cap, (size_t)nm * 32);
@@ -1374,7 +1377,7 @@ int orb_knn2_time(orb_context* ctx, const uint8_t* query, int nq, const uint8_t*
         rc = ORB_E_DEVICE;
     double a = 0, b = 0;
     for (int s = -3; s < steps && !rc; s++) {   // s < 0: untimed warm-up (clocks ramp over the first runs)
-        if (orb_launch_knn2(ctx->d_kq, nq, ctx->d_km, nm, method, ratio, ctx->d_part, d_out, d_out + 2 * (size_t)nq,
+        if (orb_launch_knn2(ctx->d_kq, nq, ctx->d_km, nm, method, ratio, ctx->d_part, rows, d_out, d_out + 2 * (size_t)nq,
                             (uint8_t*)(d_out + 4 * (size_t)nq), ctx->stream, ev) != hipSuccess ||
             hipEventSynchronize(ev[2]) != hipSuccess) {
             rc = ORB_E_DEVICE;
