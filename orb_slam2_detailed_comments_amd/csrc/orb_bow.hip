@@ -10,6 +10,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "orb_types.h"
 
 #define VOC_LANES 16                 // lanes per descriptor: one per child
@@ -70,48 +72,223 @@ __global__ __launch_bounds__(256) void voc_transform_kernel(VocDev V, const uint
     }
 }
 
-__device__ __forceinline__ void bitonic_sort_u64(unsigned long long* v, int npow)
+// The value of lane (lane ^ X) of a wavefront: DPP moves for X < 16, the LDS
+// crossbar beyond.
+template <int X>
+__device__ __forceinline__ unsigned lane_xor(unsigned v)
 {
-    for (int k = 2; k <= npow; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int a = threadIdx.x; a < npow; a += blockDim.x) {
-                const int b = a ^ j;
-                if (b > a) {
-                    const unsigned long long va = v[a], vb = v[b];
-                    const bool up = (a & k) == 0;
-                    if (up ? (va > vb) : (va < vb)) {
-                        v[a] = vb;
-                        v[b] = va;
-                    }
-                }
-            }
-            __syncthreads();
-        }
+    if constexpr (X == 1) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
+    else if constexpr (X == 2) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, false);   // [2,3,0,1]
+    else if constexpr (X == 4)                     // xor 7 (half mirror), then xor 3 (quad_perm [3,2,1,0])
+        return (unsigned)__builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, false), 0x1B, 0xF, 0xF,
+                                                  false);
+    else if constexpr (X == 8) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, false);  // row_ror:8
+    else return (unsigned)__shfl_xor((int)v, X, 64);
 }
 
-// One workgroup per image (1024 threads, thread t owns sorted positions
-// 4t..4t+3).  Rows with weight > 0 only (the reference's "not stopped" test).
-// BowVector: word-sorted; under TF / TF_IDF a word's value is its rows'
-// weights added in feature order (addWeight), under IDF / BINARY the weight
-// of its first row (addIfNotExist); TF / TF_IDF without normalisation then
-// divide by the number of words, and normalising scorings divide by the L1 or
-// L2 norm summed in word order (BowVector::normalize).  FeatureVector:
-// node-sorted, feature indices ascending within a node (addFeature in index
-// order).
-__device__ __forceinline__ int block_excl_scan_1024(int x, int* sc)
+// Ascending bitonic sort of npow (a power of two, <= 1024 E) keys held E per
+// thread, key i = E * tid + r, by a workgroup of 1024; keys past npow are
+// larger than all others and stay.  Steps over less than E keys stay in a
+// thread and steps over less than 64 E in a wavefront; only the longer ones
+// (10 of the 66 for 2048 keys) go through LDS, with two barriers each.
+template <int E>
+__device__ __forceinline__ void block_sort(unsigned long long (&v)[E], int npow, unsigned long long* lds)
 {
-    const int t = threadIdx.x;
-    sc[t] = x;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        const int y = t >= o ? sc[t - o] : 0;
-        __syncthreads();
-        sc[t] += y;
-        __syncthreads();
+    const int tid = threadIdx.x, i0 = E * tid;
+    // keeps the smaller key where key i is the pair's lower place of an
+    // ascending run, or the upper place of a descending one
+    auto pick = [](unsigned long long a, unsigned long long o, bool small) {
+        return (a < o) == small ? a : o;
+    };
+    auto lanes = [&](auto x, int k) {
+        constexpr int X = decltype(x)::value;
+        if (X * E >= k) return;
+#pragma unroll
+        for (int r = 0; r < E; r++) {
+            const unsigned long long o = ((unsigned long long)lane_xor<X>((unsigned)(v[r] >> 32)) << 32) |
+                                         lane_xor<X>((unsigned)v[r]);
+            v[r] = pick(v[r], o, ((i0 & (X * E)) == 0) == (((i0 + r) & k) == 0));
+        }
+    };
+    for (int k = 2; k <= npow; k <<= 1) {
+        for (int j = k >> 1; j >= 64 * E; j >>= 1) {
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < E; r++) lds[r * 1024 + tid] = v[r];
+            __syncthreads();
+            const int ot = tid ^ (j / E);
+#pragma unroll
+            for (int r = 0; r < E; r++) v[r] = pick(v[r], lds[r * 1024 + ot], ((i0 & j) == 0) == ((i0 & k) == 0));
+        }
+        lanes(std::integral_constant<int, 32>{}, k);
+        lanes(std::integral_constant<int, 16>{}, k);
+        lanes(std::integral_constant<int, 8>{}, k);
+        lanes(std::integral_constant<int, 4>{}, k);
+        lanes(std::integral_constant<int, 2>{}, k);
+        lanes(std::integral_constant<int, 1>{}, k);
+#pragma unroll
+        for (int j = E / 2; j > 0; j >>= 1) {
+            if (j >= k) continue;
+#pragma unroll
+            for (int r = 0; r < E; r++) {
+                if (r & j) continue;
+                const bool up = ((i0 + r) & k) == 0;
+                const unsigned long long a = v[r], b = v[r | j];
+                v[r] = pick(a, b, up);
+                v[r | j] = pick(b, a, !up);
+            }
+        }
     }
-    const int incl = sc[t];
     __syncthreads();
-    return incl - x;
+}
+
+// Exclusive scan over the 1024 threads, and the total.
+__device__ __forceinline__ int block_excl_scan_1024(int x, int* sc, int* total)
+{
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    int inc = x;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += y;
+    }
+    if (lane == 63) sc[wv] = inc;
+    __syncthreads();
+    int base = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < 16; w++) {
+        const int c = sc[w];
+        base += w < wv ? c : 0;
+        all += c;
+    }
+    *total = all;
+    return base + inc - x;
+}
+
+// Two workgroups per image (1024 threads): block 2i sorts image i's rows by
+// (word, feature) and writes its BowVector, block 2i + 1 sorts them by (node,
+// feature) and writes its FeatureVector.  Rows with weight > 0 only (the
+// reference's "not stopped" test).  BowVector: under TF / TF_IDF a word's
+// value is its rows' weights added in feature order (addWeight), under IDF /
+// BINARY the weight of its first row (addIfNotExist); TF / TF_IDF without
+// normalisation then divide by the number of words, and normalising scorings
+// divide by the L1 or L2 norm summed in word order (BowVector::normalize).
+// FeatureVector: node-sorted, feature indices ascending within a node
+// (addFeature in index order).
+// Bound: latency of the sort's steps and of the norm's chain of additions.
+// 16 images x 2000 rows: 31 us, 17 of them the norm (its terms as a chain of
+// 2000 dependent additions); one workgroup per image with the sorts through
+// LDS and the chain over strided reads took 85 us.
+template <int E>
+__device__ __forceinline__ void bow_image(const VocDev& V, const BowJob& J, int image, bool fv,
+                                          const int* __restrict__ word, const double* __restrict__ wgt,
+                                          const int* __restrict__ nidv, int* __restrict__ bow_word,
+                                          double* __restrict__ bow_value, int* __restrict__ n_bow,
+                                          int* __restrict__ fv_node, int* __restrict__ fv_feat,
+                                          int* __restrict__ n_fv, unsigned long long* key, int* sc,
+                                          double* s_norm)
+{
+    const int tid = threadIdx.x, n = min(J.n, BOW_CAP);
+    const int* id = fv ? nidv : word;
+    unsigned long long v[E];
+    int m = 0;
+#pragma unroll
+    for (int r = 0; r < E; r++) {
+        const int i = r * 1024 + tid;              // any order: the sort places them
+        const bool live = i < n && wgt[J.off + min(i, n - 1)] > 0;
+        v[r] = live ? ((unsigned long long)(unsigned)id[J.off + i] << 32) | (unsigned)i : ~0ull;
+        m += __syncthreads_count(live);
+    }
+    int npow = 2;
+    while (npow < n) npow <<= 1;
+    if (npow < 1024 * E) {                         // keys r * 1024 + tid to places E tid + r, so that a short
+        // list's keys lie in the first npow places
+#pragma unroll
+        for (int r = 0; r < E; r++) key[r * 1024 + tid] = v[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < E; r++) v[r] = key[E * tid + r];
+    }
+    block_sort<E>(v, npow, key);
+    if (fv) {
+#pragma unroll
+        for (int r = 0; r < E; r++) {
+            const int i = E * tid + r;
+            if (i < m) {
+                fv_node[J.off + i] = (int)(unsigned)(v[r] >> 32);
+                fv_feat[J.off + i] = (int)(unsigned)v[r];
+            }
+        }
+        if (tid == 0) n_fv[image] = m;
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < E; r++) key[E * tid + r] = v[r];
+    __syncthreads();
+    const bool tf = V.weighting == 0 || V.weighting == 1;
+    const bool must = V.scoring != 5;
+    const bool l2 = V.scoring == 1;
+    // heads of word runs among this thread's places, and their values
+    bool head[E];
+    double hv[E];
+    int nh = 0;
+#pragma unroll
+    for (int r = 0; r < E; r++) {
+        const int i = E * tid + r;
+        head[r] = i < m && (i == 0 || (unsigned)(key[max(i, 1) - 1] >> 32) != (unsigned)(v[r] >> 32));
+        hv[r] = head[r] ? wgt[J.off + (int)(unsigned)v[r]] : 0.0;
+        nh += head[r] ? 1 : 0;
+    }
+    if (tf) {
+#pragma unroll
+        for (int r = 0; r < E; r++)
+            if (head[r])
+                for (int i = E * tid + r + 1; i < m && (unsigned)(key[i] >> 32) == (unsigned)(v[r] >> 32); i++)
+                    hv[r] += wgt[J.off + (int)(unsigned)key[i]];
+    }
+    int nb;
+    int rank = block_excl_scan_1024(nh, sc, &nb);  // its barrier ends the reads of key above
+    // what each word adds to the norm, in word order
+    double* term = reinterpret_cast<double*>(key);
+    const int rank0 = rank;
+#pragma unroll
+    for (int r = 0; r < E; r++)
+        if (head[r]) term[rank++] = l2 ? hv[r] * hv[r] : fabs(hv[r]);
+    // zeros behind the last term: adding them leaves the norm as it is
+    if (tid < 16 && nb + tid < 1024 * E) term[nb + tid] = 0.0;
+    __syncthreads();
+    if (must && tid == 0) {
+        // one addition after another; the next eight terms are read while
+        // eight are added
+        double norm = 0.0, t[8], u[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) t[q] = term[q];
+        for (int i = 0; i < nb; i += 16) {         // nb <= 1024 E, a multiple of 16
+            const int next = min(i + 16, 1024 * E - 8);
+#pragma unroll
+            for (int q = 0; q < 8; q++) u[q] = term[i + 8 + q];
+#pragma unroll
+            for (int q = 0; q < 8; q++) norm += t[q];
+#pragma unroll
+            for (int q = 0; q < 8; q++) t[q] = term[next + q];
+#pragma unroll
+            for (int q = 0; q < 8; q++) norm += u[q];
+        }
+        *s_norm = l2 ? sqrt(norm) : norm;
+    }
+    if (tid == 0) n_bow[image] = nb;
+    __syncthreads();
+    const double norm = must ? *s_norm : 0.0;
+    rank = rank0;
+#pragma unroll
+    for (int r = 0; r < E; r++)
+        if (head[r]) {
+            double x = hv[r];
+            if (tf && !must) x = x / (double)nb;
+            if (must && norm > 0.0) x = x / norm;
+            bow_word[J.off + rank] = (int)(unsigned)(v[r] >> 32);
+            bow_value[J.off + rank++] = x;
+        }
 }
 
 __global__ __launch_bounds__(1024) void voc_bow_kernel(VocDev V, const BowJob* __restrict__ jobs,
@@ -121,98 +298,18 @@ __global__ __launch_bounds__(1024) void voc_bow_kernel(VocDev V, const BowJob* _
                                                        int* __restrict__ fv_node, int* __restrict__ fv_feat,
                                                        int* __restrict__ n_fv)
 {
-    __shared__ unsigned long long key[BOW_CAP];   // sort keys; later the word values (as double)
-    __shared__ int wordv[BOW_CAP];
-    __shared__ int sc[1024];
-    __shared__ int s_cnt;
+    __shared__ unsigned long long key[BOW_CAP];   // sort scratch; later the norm's terms (as double)
+    __shared__ int sc[16];
     __shared__ double s_norm;
-    const BowJob J = jobs[blockIdx.x];
-    const int n = min(J.n, BOW_CAP);
-    const int tid = threadIdx.x;
-    if (tid == 0) s_cnt = 0;
-    __syncthreads();
-    for (int i = tid; i < n; i += 1024)
-        if (wgt[J.off + i] > 0) key[atomicAdd(&s_cnt, 1)] = ((unsigned long long)(unsigned)word[J.off + i] << 32) | i;
-    __syncthreads();
-    const int m = s_cnt;
-    int npow = 1;
-    while (npow < m) npow <<= 1;
-    for (int i = m + tid; i < npow; i += 1024) key[i] = ~0ull;
-    __syncthreads();
-    bitonic_sort_u64(key, npow);
-    const bool tf = V.weighting == 0 || V.weighting == 1;
-    const bool must = V.scoring != 5;
-    const bool l2 = V.scoring == 1;
-    // heads of word runs among this thread's four positions, and their values
-    int hw[4];
-    double hv[4];
-    int nh = 0;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int i = 4 * tid + e;
-        hw[e] = -1;
-        hv[e] = 0.0;
-        if (i >= m) continue;
-        const unsigned w = (unsigned)(key[i] >> 32);
-        if (i > 0 && (unsigned)(key[i - 1] >> 32) == w) continue;
-        double v = wgt[J.off + (int)(unsigned)key[i]];
-        if (tf)
-            for (int r = i + 1; r < m && (unsigned)(key[r] >> 32) == w; r++) v += wgt[J.off + (int)(unsigned)key[r]];
-        hw[e] = (int)w;
-        hv[e] = v;
-        nh++;
-    }
-    const int rank0 = block_excl_scan_1024(nh, sc);
-    __syncthreads();                              // every key read above is done
-    double* val = reinterpret_cast<double*>(key);
-    int r = rank0;
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-        if (hw[e] >= 0) {
-            wordv[r] = hw[e];
-            val[r] = hv[e];
-            r++;
-        }
-    if (tid == 1023) sc[0] = r;                   // total heads (last thread's end rank)
-    __syncthreads();
-    const int nb = sc[0];
-    if (tid == 0) {
-        double norm = 0.0;
-        if (must) {
-            if (!l2) {
-                for (int i = 0; i < nb; i++) norm += fabs(val[i]);
-            } else {
-                for (int i = 0; i < nb; i++) norm += val[i] * val[i];
-                norm = sqrt(norm);
-            }
-        }
-        s_norm = norm;
-        n_bow[blockIdx.x] = nb;
-    }
-    __syncthreads();
-    const double norm = s_norm;
-    for (int i = tid; i < nb; i += 1024) {
-        double v = val[i];
-        if (tf && !must) v = v / (double)nb;
-        if (must && norm > 0.0) v = v / norm;
-        bow_word[J.off + i] = wordv[i];
-        bow_value[J.off + i] = v;
-    }
-    __syncthreads();
-    // FeatureVector: (node << 32 | feature) over the same kept rows
-    if (tid == 0) s_cnt = 0;
-    __syncthreads();
-    for (int i = tid; i < n; i += 1024)
-        if (wgt[J.off + i] > 0) key[atomicAdd(&s_cnt, 1)] = ((unsigned long long)(unsigned)nidv[J.off + i] << 32) | i;
-    __syncthreads();
-    for (int i = m + tid; i < npow; i += 1024) key[i] = ~0ull;
-    __syncthreads();
-    bitonic_sort_u64(key, npow);
-    for (int i = tid; i < m; i += 1024) {
-        fv_node[J.off + i] = (int)(unsigned)(key[i] >> 32);
-        fv_feat[J.off + i] = (int)(unsigned)key[i];
-    }
-    if (tid == 0) n_fv[blockIdx.x] = m;
+    const int image = blockIdx.x >> 1;
+    const bool fv = blockIdx.x & 1;
+    const BowJob J = jobs[image];
+#define ORB_BOW(E) \
+    bow_image<E>(V, J, image, fv, word, wgt, nidv, bow_word, bow_value, n_bow, fv_node, fv_feat, n_fv, key, sc, &s_norm)
+    if (J.n <= 1024) ORB_BOW(1);
+    else if (J.n <= 2048) ORB_BOW(2);
+    else ORB_BOW(4);
+#undef ORB_BOW
 }
 
 extern "C" hipError_t orb_launch_voc_transform(const VocDev* V, const uint8_t* desc, int n, int levelsup,
@@ -229,7 +326,7 @@ extern "C" hipError_t orb_launch_voc_bow(const VocDev* V, const BowJob* jobs, in
                                          int* n_bow, int* fv_node, int* fv_feat, int* n_fv, hipStream_t st)
 {
     if (n_images <= 0) return hipSuccess;
-    voc_bow_kernel<<<n_images, 1024, 0, st>>>(*V, jobs, word, weight, nid, bow_word, bow_value, n_bow, fv_node,
+    voc_bow_kernel<<<2 * n_images, 1024, 0, st>>>(*V, jobs, word, weight, nid, bow_word, bow_value, n_bow, fv_node,
                                               fv_feat, n_fv);
     return hipGetLastError();
 }
