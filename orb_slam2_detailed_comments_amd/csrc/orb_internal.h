@@ -26,8 +26,8 @@ extern "C" hipError_t orb_launch_match_bf(const uint8_t* q, const int* nq, const
 extern "C" hipError_t orb_launch_match_pairs(const MatchArgs* d_args, int npairs, int nwaves, hipStream_t st);
 extern "C" hipError_t orb_launch_gray(const uint8_t* src, size_t sstride, int scn, int bidx, int w, int h,
                                       uint8_t* dst, size_t dstride, hipStream_t st);
-extern "C" hipError_t orb_launch_distinctive(const uint8_t* desc, const int* offsets, int n_points, int* best,
-                                             uint8_t* out_desc, hipStream_t st);
+extern "C" hipError_t orb_launch_distinctive(const uint8_t* desc, const int* offsets, int n_points, int max_obs,
+                                             int* best, uint8_t* out_desc, hipStream_t st);
 extern "C" hipError_t orb_launch_hbm_copy(const void* src, void* dst, size_t bytes, hipStream_t st);
 extern "C" hipError_t orb_launch_copy_ops(const CopyOp* d_ops, int nops, int blocks_per_op, hipStream_t st);
 extern "C" hipError_t orb_launch_undistort(const OrbKeyPoint* in, int n, const int* count, const double* K4,

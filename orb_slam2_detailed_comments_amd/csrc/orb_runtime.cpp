@@ -1406,13 +1406,17 @@ int orb_knn2_time(orb_context* ctx, const uint8_t* query, int nq, const uint8_t*
 // MapPoint::ComputeDistinctiveDescriptors (src/MapPoint.cc:365-450) for
 // n_points points; point p's observations are rows offsets[p] ..
 // offsets[p+1]-1 of desc, in the order the reference would visit them.
-static int distinctive_stage(orb_context* ctx, int n_points, const uint8_t* desc, const int32_t* offsets)
+// max_obs receives the most rows of a point.
+static int distinctive_stage(orb_context* ctx, int n_points, const uint8_t* desc, const int32_t* offsets,
+                             int* max_obs)
 {
+    *max_obs = 0;
     const int rows = offsets[n_points];
     if (offsets[0] < 0 || rows < offsets[0]) return ORB_E_ARG;
     for (int p = 0; p < n_points; p++) {
         if (offsets[p + 1] < offsets[p]) return ORB_E_ARG;
         if (offsets[p + 1] - offsets[p] > 1024) return ORB_E_CAPACITY;
+        *max_obs = std::max(*max_obs, offsets[p + 1] - offsets[p]);
     }
     int rc = ctx->grow((void**)&ctx->d_mp, &ctx->mp_cap, (size_t)std::max(rows, 1) * 32);
     if (!rc) rc = ctx->grow((void**)&ctx->d_mpo, &ctx->mpo_cap, (size_t)(n_points + 1) * 4);
@@ -1541,10 +1545,12 @@ int orb_distinctive_descriptors(orb_context* ctx, int n_points, const uint8_t* d
     if (n_points == 0) return ORB_OK;
     if (offsets[n_points] > 0 && !desc) return ORB_E_ARG;
     HIP_TRY(hipSetDevice(ctx->device));
-    int rc = distinctive_stage(ctx, n_points, desc, offsets);
+    int max_obs = 0;
+    int rc = distinctive_stage(ctx, n_points, desc, offsets, &max_obs);
     if (rc) return rc;
     hipStream_t st = ctx->stream;
-    HIP_TRY(orb_launch_distinctive(ctx->d_mp, ctx->d_mpo, n_points, ctx->d_mpb, out_desc ? ctx->d_mpd : nullptr, st));
+    HIP_TRY(orb_launch_distinctive(ctx->d_mp, ctx->d_mpo, n_points, max_obs, ctx->d_mpb,
+                                   out_desc ? ctx->d_mpd : nullptr, st));
     HIP_TRY(hipMemcpyAsync(best, ctx->d_mpb, (size_t)n_points * 4, hipMemcpyDeviceToHost, st));
     if (out_desc) HIP_TRY(hipMemcpyAsync(out_desc, ctx->d_mpd, (size_t)n_points * 32, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
@@ -1556,16 +1562,17 @@ int orb_distinctive_descriptors_time(orb_context* ctx, int n_points, const uint8
 {
     if (!ctx || n_points <= 0 || !desc || !offsets || steps <= 0 || !ms) return ORB_E_ARG;
     HIP_TRY(hipSetDevice(ctx->device));
-    int rc = distinctive_stage(ctx, n_points, desc, offsets);
+    int max_obs = 0;
+    int rc = distinctive_stage(ctx, n_points, desc, offsets, &max_obs);
     if (rc) return rc;
     hipStream_t st = ctx->stream;
-    HIP_TRY(orb_launch_distinctive(ctx->d_mp, ctx->d_mpo, n_points, ctx->d_mpb, ctx->d_mpd, st));
+    HIP_TRY(orb_launch_distinctive(ctx->d_mp, ctx->d_mpo, n_points, max_obs, ctx->d_mpb, ctx->d_mpd, st));
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     (void)hipEventRecord(e0, st);
     for (int s = 0; s < steps; s++)
-        (void)orb_launch_distinctive(ctx->d_mp, ctx->d_mpo, n_points, ctx->d_mpb, ctx->d_mpd, st);
+        (void)orb_launch_distinctive(ctx->d_mp, ctx->d_mpo, n_points, max_obs, ctx->d_mpb, ctx->d_mpd, st);
     (void)hipEventRecord(e1, st);
     const hipError_t se = hipEventSynchronize(e1);
     float t = 0.f;
