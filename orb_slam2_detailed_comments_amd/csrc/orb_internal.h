@@ -157,6 +157,9 @@ struct orb_context {
     size_t win_cap = 0;
     void* d_wcand = nullptr;
     size_t wcand_cap = 0;
+    // pinned staging of the windowed searches' inputs and outputs
+    void* h_win = nullptr;
+    size_t hwin_cap = 0;
     // map-point scratch: observation descriptors, offsets, chosen rows
     uint8_t* d_mp = nullptr;
     int* d_mpo = nullptr;
@@ -166,6 +169,21 @@ struct orb_context {
     // Frame keypoint ops: keypoints in and out, the RGB-D depth image
     void* d_fr = nullptr;
     size_t fr_cap = 0;
+
+    // Pinned host memory, grown; the last call's copies have ended.
+    int grow_pinned(void** p, size_t* cap, size_t bytes)
+    {
+        if (bytes <= *cap) return ORB_OK;
+        if (*p) (void)hipHostFree(*p);
+        *p = nullptr;
+        *cap = 0;
+        if (hipHostMalloc(p, bytes) != hipSuccess) {
+            *p = nullptr;
+            return ORB_E_OOM;
+        }
+        *cap = bytes;
+        return ORB_OK;
+    }
 
     int grow(void** p, size_t* cap, size_t bytes)
     {

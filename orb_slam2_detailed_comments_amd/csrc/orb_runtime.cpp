@@ -54,6 +54,7 @@ void orb_context_release_ref(orb_context* ctx)
     void* mp[] = {ctx->d_mp, ctx->d_mpo, ctx->d_mpb, ctx->d_mpd, ctx->d_color, ctx->d_win, ctx->d_wcand, ctx->d_fr};
     for (void* q : mp)
         if (q) (void)hipFree(q);
+    if (ctx->h_win) (void)hipHostFree(ctx->h_win);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }

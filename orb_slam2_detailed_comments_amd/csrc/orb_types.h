@@ -170,7 +170,7 @@ struct BowJob {
 
 // One frame pair of ORBmatcher::SearchForInitialization: F1 / F2 keypoints
 // (mvKeysUn) and descriptors, the grid bounds (mnMinX .. mnMaxY), the search
-// positions (vbPrevMatched, updated in place), parameters, scratch and
+// positions (vbPrevMatched), parameters, scratch and
 // outputs.
 struct WinPair {
     const OrbKeyPoint* kp1;
@@ -179,16 +179,23 @@ struct WinPair {
     const uint8_t* d2;
     int n1, n2;
     float minX, maxX, minY, maxY;
-    float2* prev;
+    const float2* prev;
     int window;
     float nnratio;
     int check_orientation;
-    int* sorted;            // n2: F2 keypoints sorted by (cell, index)
+    // the grid's keypoints sorted by (cell, index): x, y, mvuRight,
+    // index | octave << 12; only keypoints a query can take (below)
+    float4* rec;
     int* cell_start;        // 64*48 + 1
+    const float* uright;    // SearchByProjection's frames: mvuRight and occupancy
+    const uint8_t* occupied;   // (occupied keypoints are left out); null: octave 0 only
     int* cnt;               // n1: candidates per query
-    int* off;               // n1 + 1: their offsets
+    unsigned* off;          // n1: where each query's list starts
     int2* cand;             // (i2, distance) lists
+    unsigned long long* total;   // list entries asked for (beyond cand_cap: lists are missing)
+    unsigned long long cand_cap;
     int* m12;               // n1: vnMatches12
+    float2* prev_out;       // n1: vbPrevMatched afterwards
     int* nmatch;            // nmatches
     // SearchForInitialization's in-order pass as parallel rounds (unused by
     // the grid kernels of SearchByProjection, which leave them null)
@@ -220,18 +227,18 @@ struct ProjQuery {
 struct ProjFrame {
     const OrbKeyPoint* kp;
     const uint8_t* desc;
-    const float* uright;
-    const uint8_t* occupied;    // mvpMapPoints[i] && Observations() > 0
     int n;
     float minX, maxX, minY, maxY;
-    const int* sorted;          // grid, as WinPair's
+    const float4* rec;          // grid, as WinPair's
     const int* cell_start;
     ProjQuery* q;
     const uint8_t* qdesc;
     int nq;
     int* cnt;                   // candidates per query
-    const int* off;             // their offsets (nq + 1)
+    unsigned* off;              // where each query's list starts
     unsigned* cand;             // i2 | distance << 12 | octave << 21, GetFeaturesInArea order
+    unsigned long long* total;  // as WinPair's
+    unsigned long long cand_cap;
     int* out[2];                // outcome per query by round parity: keypoint or -1
     int* claim[3];              // per keypoint: first claiming query (with observations), by round mod 3
     int* changed;               // [ORB_PROJ_MAXIT]: bit 0 round k changed some outcome, bit 2 not run

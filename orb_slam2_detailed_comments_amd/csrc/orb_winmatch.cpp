@@ -1,8 +1,10 @@
 // orb_winmatch.cpp -- C ABI of ORBmatcher::SearchForInitialization over the
 // Frame keypoint grid, for many frame pairs per call (kernels in
-// orb_winmatch.hip).  Two launches with one host read between them: the
-// candidate counts size the (i2, distance) lists exactly.  Device buffers
-// are the context's, grown on demand and kept between calls.
+// orb_winmatch.hip).  A call copies its inputs to the device once, launches
+// the grid, the candidate lists, four rounds and the finish, copies every
+// result back and waits once; it goes on only if some pair has not settled,
+// or if the lists did not fit their buffer (which then grows).  Device and
+// pinned buffers are the context's, grown on demand and kept between calls.
 #include <chrono>
 #include <cstring>
 #include <vector>
@@ -11,9 +13,7 @@
 
 using namespace orb_detail;
 
-extern "C" hipError_t orb_launch_win_count(const WinPair* d_pairs, int npairs, int max_n1, hipStream_t st);
-extern "C" hipError_t orb_launch_win_scan(const WinPair* d_pairs, int npairs, int* d_totals, hipStream_t st);
-extern "C" hipError_t orb_launch_win_fill(const WinPair* d_pairs, int npairs, int max_n1, hipStream_t st);
+extern "C" hipError_t orb_launch_win_lists(const WinPair* d_pairs, int npairs, int max_n1, hipStream_t st);
 extern "C" hipError_t orb_launch_win_rounds(const WinPair* d_pairs, int npairs, int max_n1, int k0, int k1,
                                             hipStream_t st);
 extern "C" hipError_t orb_launch_win_finish(const WinPair* d_pairs, int npairs, int sequential, hipStream_t st);
@@ -22,12 +22,47 @@ namespace {
 
 size_t up(size_t v) { return (v + 255) / 256 * 256; }
 
-}  // namespace
+// A call's device block: what is copied in, what is copied out, then scratch.
+// Inputs are packed in pinned memory at their device offsets, so that one
+// copy takes them; so are the outputs.
+struct Block {
+    size_t in = 0, out = 0, scratch = 0;
+    size_t add_in(size_t bytes) { return add(in, bytes); }
+    size_t add_out(size_t bytes) { return add(out, bytes); }
+    size_t add_scratch(size_t bytes) { return add(scratch, bytes); }
+    static size_t add(size_t& end, size_t bytes)
+    {
+        const size_t o = end;
+        end += up(bytes);
+        return o;
+    }
+};
 
-namespace {
+// Room per query for candidate lists when a call starts (entries); a call
+// whose windows hold more grows its lists to what they asked for, and the
+// buffer stays that large for the next.
+constexpr size_t kListStart = 64;
+
+// The lists' regions in a buffer of `have` entries: a pair's (or frame's)
+// nq[i] queries get kListStart entries each, or an even share of the buffer
+// if that is more, or what the pair asked for.  base[i] and cap[i] in
+// entries; returns the total.
+size_t list_regions(const std::vector<size_t>& nq, size_t have, const unsigned long long* asked,
+                    std::vector<size_t>& base, std::vector<unsigned long long>& cap)
+{
+    size_t all = 0, total = 0;
+    for (const size_t n : nq) all += n;
+    const size_t per = std::max(kListStart, all ? have / all : 0);
+    for (size_t i = 0; i < nq.size(); i++) {
+        cap[i] = asked ? std::max<unsigned long long>(nq[i] * kListStart, asked[i]) : nq[i] * per;
+        base[i] = total;
+        total += (size_t)cap[i];
+    }
+    return total;
+}
 
 // steps > 0: after the call's own run, `steps` more runs of the device work
-// with the inputs resident in HBM (vbPrevMatched restored before each), their
+// with the inputs resident in HBM, their
 // mean wall time in *ms; the results returned are the call's.
 int sfi_impl(orb_context* ctx, int n_pairs, const orb_keypoint* kp1, const uint8_t* desc1, const int32_t* off1,
              const orb_keypoint* kp2, const uint8_t* desc2, const int32_t* off2, const float* bounds,
@@ -49,149 +84,143 @@ int sfi_impl(orb_context* ctx, int n_pairs, const orb_keypoint* kp1, const uint8
     HIP_TRY(hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
     static_assert(sizeof(orb_keypoint) == sizeof(OrbKeyPoint), "keypoint layout");
-    // inputs and per-pair scratch in one allocation
-    const size_t s_kp1 = up((size_t)N1 * sizeof(OrbKeyPoint)), s_d1 = up((size_t)N1 * 32);
-    const size_t s_kp2 = up((size_t)N2 * sizeof(OrbKeyPoint)), s_d2 = up((size_t)N2 * 32);
-    const size_t s_prev = up((size_t)N1 * 8), s_sorted = up((size_t)N2 * 4);
-    const size_t s_cells = up((size_t)n_pairs * (64 * 48 + 1) * 4), s_cnt = up((size_t)N1 * 4);
-    const size_t s_off = up((size_t)(N1 + n_pairs) * 4), s_m12 = up((size_t)N1 * 4), s_nm = up((size_t)n_pairs * 4);
-    const size_t s_pairs = up((size_t)n_pairs * sizeof(WinPair)), s_tot = up((size_t)n_pairs * 4);
-    // round state: outcomes by parity, claims and claim counts by round mod 3, change flags
-    const size_t s_out = up((size_t)N1 * 4), s_claim = up((size_t)N2 * ORB_WIN_SLOTS * 4), s_ccnt = up((size_t)N2 * 4);
-    const size_t s_chg = up((size_t)n_pairs * ORB_WIN_MAXIT * 4);
-    const size_t total = s_kp1 + s_d1 + s_kp2 + s_d2 + 2 * s_prev + s_sorted + s_cells + s_cnt + s_off + s_m12 +
-                         s_nm + s_pairs + s_tot + 2 * s_out + 3 * s_claim + 3 * s_ccnt + s_chg;
-    int rc = ctx->grow(&ctx->d_win, &ctx->win_cap, total);     // kept by the context between calls
+    const size_t P = (size_t)n_pairs, n1 = (size_t)N1, n2 = (size_t)N2;
+    Block B;
+    const size_t i_kp1 = B.add_in(n1 * sizeof(OrbKeyPoint)), i_d1 = B.add_in(n1 * 32), i_prev = B.add_in(n1 * 8);
+    const size_t i_kp2 = B.add_in(n2 * sizeof(OrbKeyPoint)), i_d2 = B.add_in(n2 * 32);
+    const size_t i_pairs = B.add_in(P * sizeof(WinPair));
+    const size_t o_m12 = B.add_out(n1 * 4), o_prev = B.add_out(n1 * 8), o_nm = B.add_out(P * 4);
+    const size_t o_tot = B.add_out(P * 8), o_chg = B.add_out(P * ORB_WIN_MAXIT * 4);
+    const size_t s_rec = B.add_scratch(n2 * 16), s_cells = B.add_scratch(P * (64 * 48 + 1) * 4);
+    const size_t s_cnt = B.add_scratch(n1 * 4), s_off = B.add_scratch(n1 * 4);
+    // round state: outcomes by parity, claims and claim counts by round mod 3
+    const size_t s_out = B.add_scratch(2 * n1 * 4), s_claim = B.add_scratch(3 * n2 * ORB_WIN_SLOTS * 4);
+    const size_t s_ccnt = B.add_scratch(3 * n2 * 4);
+    int rc = ctx->grow(&ctx->d_win, &ctx->win_cap, B.in + B.out + B.scratch);
+    if (!rc) rc = ctx->grow_pinned(&ctx->h_win, &ctx->hwin_cap, B.in + B.out);
     if (rc) return rc;
-    char* m = (char*)ctx->d_win;
-    size_t o = 0;
-    auto take = [&](size_t s) {
-        char* q = m + o;
-        o += s;
-        return q;
-    };
-    OrbKeyPoint* d_kp1 = (OrbKeyPoint*)take(s_kp1);
-    uint8_t* d_d1 = (uint8_t*)take(s_d1);
-    OrbKeyPoint* d_kp2 = (OrbKeyPoint*)take(s_kp2);
-    uint8_t* d_d2 = (uint8_t*)take(s_d2);
-    float2* d_prev = (float2*)take(s_prev);
-    int* d_sorted = (int*)take(s_sorted);
-    int* d_cells = (int*)take(s_cells);
-    int* d_cnt = (int*)take(s_cnt);
-    int* d_off = (int*)take(s_off);
-    int* d_m12 = (int*)take(s_m12);
-    int* d_nm = (int*)take(s_nm);
-    WinPair* d_pairs = (WinPair*)take(s_pairs);
-    int* d_tot = (int*)take(s_tot);
-    int* d_out[2] = {(int*)take(s_out), (int*)take(s_out)};
-    unsigned* d_claim[3] = {(unsigned*)take(s_claim), (unsigned*)take(s_claim), (unsigned*)take(s_claim)};
-    int* d_ccnt[3] = {(int*)take(s_ccnt), (int*)take(s_ccnt), (int*)take(s_ccnt)};
-    int* d_chg = (int*)take(s_chg);
-    float2* d_prev0 = (float2*)take(s_prev);       // vbPrevMatched as passed, for timed repeats
+    char *d_in = (char*)ctx->d_win, *d_out = d_in + B.in, *d_s = d_out + B.out;
+    char *h_in = (char*)ctx->h_win, *h_out = h_in + B.in;
     if (N1) {
-        HIP_TRY(hipMemcpyAsync(d_kp1, kp1, (size_t)N1 * sizeof(OrbKeyPoint), hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemcpyAsync(d_d1, desc1, (size_t)N1 * 32, hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemcpyAsync(d_prev, prev_matched, (size_t)N1 * 8, hipMemcpyHostToDevice, st));
+        std::memcpy(h_in + i_kp1, kp1, n1 * sizeof(OrbKeyPoint));
+        std::memcpy(h_in + i_d1, desc1, n1 * 32);
+        std::memcpy(h_in + i_prev, prev_matched, n1 * 8);
     }
     if (N2) {
-        HIP_TRY(hipMemcpyAsync(d_kp2, kp2, (size_t)N2 * sizeof(OrbKeyPoint), hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemcpyAsync(d_d2, desc2, (size_t)N2 * 32, hipMemcpyHostToDevice, st));
+        std::memcpy(h_in + i_kp2, kp2, n2 * sizeof(OrbKeyPoint));
+        std::memcpy(h_in + i_d2, desc2, n2 * 32);
     }
-    std::vector<WinPair> pairs(n_pairs);
+    WinPair* pairs = (WinPair*)(h_in + i_pairs);
+    std::vector<size_t> nq(P), base(P);
+    std::vector<unsigned long long> cap(P);
     for (int p = 0; p < n_pairs; p++) {
         WinPair& w = pairs[p];
         std::memset(&w, 0, sizeof(w));
-        w.kp1 = d_kp1 + off1[p];
-        w.d1 = d_d1 + (size_t)off1[p] * 32;
-        w.kp2 = d_kp2 + off2[p];
-        w.d2 = d_d2 + (size_t)off2[p] * 32;
+        w.kp1 = (const OrbKeyPoint*)(d_in + i_kp1) + off1[p];
+        w.d1 = (const uint8_t*)(d_in + i_d1) + (size_t)off1[p] * 32;
+        w.kp2 = (const OrbKeyPoint*)(d_in + i_kp2) + off2[p];
+        w.d2 = (const uint8_t*)(d_in + i_d2) + (size_t)off2[p] * 32;
         w.n1 = off1[p + 1] - off1[p];
         w.n2 = off2[p + 1] - off2[p];
         w.minX = bounds[4 * p];
         w.maxX = bounds[4 * p + 1];
         w.minY = bounds[4 * p + 2];
         w.maxY = bounds[4 * p + 3];
-        w.prev = d_prev + off1[p];
+        w.prev = (const float2*)(d_in + i_prev) + off1[p];
         w.window = window_size;
         w.nnratio = nn_ratio;
         w.check_orientation = check_orientation ? 1 : 0;
-        w.sorted = d_sorted + off2[p];
-        w.cell_start = d_cells + (size_t)p * (64 * 48 + 1);
-        w.cnt = d_cnt + off1[p];
-        w.off = d_off + off1[p] + p;
-        w.m12 = d_m12 + off1[p];
-        w.nmatch = d_nm + p;
-        for (int b = 0; b < 2; b++) w.out[b] = d_out[b] + off1[p];
+        w.rec = (float4*)(d_s + s_rec) + off2[p];
+        w.cell_start = (int*)(d_s + s_cells) + (size_t)p * (64 * 48 + 1);
+        w.cnt = (int*)(d_s + s_cnt) + off1[p];
+        w.off = (unsigned*)(d_s + s_off) + off1[p];
+        w.total = (unsigned long long*)(d_out + o_tot) + p;
+        w.m12 = (int*)(d_out + o_m12) + off1[p];
+        w.prev_out = (float2*)(d_out + o_prev) + off1[p];
+        w.nmatch = (int*)(d_out + o_nm) + p;
+        for (int b = 0; b < 2; b++) w.out[b] = (int*)(d_s + s_out) + b * n1 + off1[p];
         for (int b = 0; b < 3; b++) {
-            w.claim[b] = d_claim[b] + (size_t)off2[p] * ORB_WIN_SLOTS;
-            w.ccnt[b] = d_ccnt[b] + off2[p];
+            w.claim[b] = (unsigned*)(d_s + s_claim) + (b * n2 + off2[p]) * ORB_WIN_SLOTS;
+            w.ccnt[b] = (int*)(d_s + s_ccnt) + b * n2 + off2[p];
         }
-        w.changed = d_chg + (size_t)p * ORB_WIN_MAXIT;
+        w.changed = (int*)(d_out + o_chg) + (size_t)p * ORB_WIN_MAXIT;
+        nq[p] = (size_t)w.n1;
     }
-    if (steps > 0 && N1) HIP_TRY(hipMemcpyAsync(d_prev0, d_prev, (size_t)N1 * 8, hipMemcpyDeviceToDevice, st));
+    const unsigned long long* tot = (const unsigned long long*)(h_out + o_tot);
+    const int* chg = (const int*)(h_out + o_chg);
+    // the lists' regions into the pairs, and all pairs to the device
+    auto place_lists = [&](const unsigned long long* asked) -> int {
+        const size_t n = list_regions(nq, ctx->wcand_cap / sizeof(int2), asked, base, cap);
+        const int rg = ctx->grow(&ctx->d_wcand, &ctx->wcand_cap, std::max<size_t>(n, 1) * sizeof(int2));
+        if (rg) return rg;
+        for (int p = 0; p < n_pairs; p++) {
+            pairs[p].cand = (int2*)ctx->d_wcand + base[p];
+            pairs[p].cand_cap = cap[p];
+        }
+        return ORB_OK;
+    };
+    rc = place_lists(nullptr);
+    if (rc) return rc;
+    HIP_TRY(hipMemcpyAsync(d_in, h_in, B.in, hipMemcpyHostToDevice, st));
+    const WinPair* d_pairs = (const WinPair*)(d_in + i_pairs);
     auto run_device = [&]() -> int {
-    HIP_TRY(hipMemcpyAsync(d_pairs, pairs.data(), n_pairs * sizeof(WinPair), hipMemcpyHostToDevice, st));
-    HIP_TRY(orb_launch_win_count(d_pairs, n_pairs, max_n1, st));
-    HIP_TRY(orb_launch_win_scan(d_pairs, n_pairs, d_tot, st));
-    std::vector<int> tot(n_pairs);
-    HIP_TRY(hipMemcpyAsync(tot.data(), d_tot, n_pairs * 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    size_t ncand = 0;
-    std::vector<size_t> base(n_pairs);
-    for (int p = 0; p < n_pairs; p++) {
-        base[p] = ncand;
-        ncand += (size_t)tot[p];
-    }
-    const int rg = ctx->grow(&ctx->d_wcand, &ctx->wcand_cap, std::max<size_t>(ncand, 1) * sizeof(int2));
-    if (rg) return rg;
-    for (int p = 0; p < n_pairs; p++) pairs[p].cand = (int2*)ctx->d_wcand + base[p];
-    HIP_TRY(hipMemcpyAsync(d_pairs, pairs.data(), n_pairs * sizeof(WinPair), hipMemcpyHostToDevice, st));
-    HIP_TRY(orb_launch_win_fill(d_pairs, n_pairs, max_n1, st));
-    // Rounds in chunks of 4 between reads of the change flags, until every
-    // pair has settled; pairs still changing after ORB_WIN_MAXIT rounds get
-    // the sequential pass.
-    std::vector<int> chg((size_t)n_pairs * ORB_WIN_MAXIT);
-    int k = 0;
-    bool settled = false;
-    const int limit = std::min(ctx->round_limit, ORB_WIN_MAXIT);
-    while (!settled && k < limit) {
-        const int k1 = std::min(limit, k + 4);
-        HIP_TRY(orb_launch_win_rounds(d_pairs, n_pairs, max_n1, k, k1, st));
-        k = k1;
-        HIP_TRY(hipMemcpyAsync(chg.data(), d_chg, chg.size() * 4, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
-        settled = true;
-        for (int p = 0; p < n_pairs && settled; p++) {
-            const int* c = chg.data() + (size_t)p * ORB_WIN_MAXIT;
-            bool sp = false;
-            for (int r = 1; r < k && !sp; r++) sp = c[r] == 0 && !(c[r - 1] & 2);
-            settled = sp;
+        const int limit = std::min(ctx->round_limit, ORB_WIN_MAXIT);
+        int k = 0;
+        bool settled = false;
+        HIP_TRY(orb_launch_win_lists(d_pairs, n_pairs, max_n1, st));
+        // Rounds in chunks of 4, each followed by the finish of the pairs
+        // that have settled; pairs still changing at the limit get the
+        // sequential pass.
+        for (;;) {
+            const int k1 = std::min(limit, k + 4);
+            HIP_TRY(orb_launch_win_rounds(d_pairs, n_pairs, max_n1, k, k1, st));
+            k = k1;
+            HIP_TRY(orb_launch_win_finish(d_pairs, n_pairs, 0, st));
+            HIP_TRY(hipMemcpyAsync(h_out, d_out, B.out, hipMemcpyDeviceToHost, st));
+            HIP_TRY(hipStreamSynchronize(st));
+            bool fits = true;
+            for (int p = 0; p < n_pairs; p++) fits = fits && tot[p] <= cap[p];
+            if (!fits) {                           // longer lists, from the start
+                const int rl = place_lists(tot);
+                if (rl) return rl;
+                HIP_TRY(hipMemcpyAsync(d_in + i_pairs, pairs, P * sizeof(WinPair), hipMemcpyHostToDevice, st));
+                HIP_TRY(orb_launch_win_lists(d_pairs, n_pairs, max_n1, st));
+                k = 0;
+                continue;
+            }
+            settled = true;
+            for (int p = 0; p < n_pairs && settled; p++) {
+                const int* c = chg + (size_t)p * ORB_WIN_MAXIT;
+                bool sp = false;
+                for (int r = 1; r < k && !sp; r++) sp = c[r] == 0 && !(c[r - 1] & 2);
+                settled = sp;
+            }
+            if (settled || k >= limit) break;
         }
-    }
-    ctx->last_rounds = k;
-    ctx->last_sequential = settled ? 0 : 1;
-    HIP_TRY(orb_launch_win_finish(d_pairs, n_pairs, settled ? 0 : 1, st));
-    return ORB_OK;
+        ctx->last_rounds = k;
+        ctx->last_sequential = settled ? 0 : 1;
+        if (!settled) {
+            HIP_TRY(orb_launch_win_finish(d_pairs, n_pairs, 1, st));
+            HIP_TRY(hipMemcpyAsync(h_out, d_out, B.out, hipMemcpyDeviceToHost, st));
+            HIP_TRY(hipStreamSynchronize(st));
+        }
+        return ORB_OK;
     };
     rc = run_device();
     if (rc) return rc;
     if (steps > 0) {
-        HIP_TRY(hipStreamSynchronize(st));
         const auto t0 = std::chrono::steady_clock::now();
         for (int i = 0; i < steps; i++) {
-            if (N1) HIP_TRY(hipMemcpyAsync(d_prev, d_prev0, (size_t)N1 * 8, hipMemcpyDeviceToDevice, st));
             rc = run_device();
             if (rc) return rc;
         }
-        HIP_TRY(hipStreamSynchronize(st));
         *ms = (float)(std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count() / steps);
     }
     if (N1) {
-        HIP_TRY(hipMemcpyAsync(matches12, d_m12, (size_t)N1 * 4, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipMemcpyAsync(prev_matched, d_prev, (size_t)N1 * 8, hipMemcpyDeviceToHost, st));
+        std::memcpy(matches12, h_out + o_m12, n1 * 4);
+        std::memcpy(prev_matched, h_out + o_prev, n1 * 8);
     }
-    HIP_TRY(hipMemcpyAsync(nmatches, d_nm, n_pairs * 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    std::memcpy(nmatches, h_out + o_nm, P * 4);
     return ORB_OK;
 }
 
@@ -225,9 +254,8 @@ int orb_search_for_initialization_time(orb_context* ctx, int n_pairs, const orb_
 extern "C" hipError_t orb_launch_proj_prep(ProjFrame* d_frames, int nframes, int max_nq, int rule, const float* d_pts,
                                            const int* d_pt_off, const float* d_scale, int nlevels, const float* d_cam,
                                            int mono, float th, hipStream_t st);
-extern "C" hipError_t orb_launch_proj_count(const WinPair* d_grid, ProjFrame* d_frames, int nframes, int max_nq,
-                                            int* d_totals, hipStream_t st);
-extern "C" hipError_t orb_launch_proj_fill(ProjFrame* d_frames, int nframes, int max_nq, hipStream_t st);
+extern "C" hipError_t orb_launch_proj_lists(const WinPair* d_grid, const ProjFrame* d_frames, int nframes, int max_nq,
+                                            hipStream_t st);
 extern "C" hipError_t orb_launch_proj_rounds(ProjFrame* d_frames, int nframes, int max_nq, int k0, int k1,
                                              hipStream_t st);
 extern "C" hipError_t orb_launch_proj_finish(ProjFrame* d_frames, int nframes, int sequential, hipStream_t st);
@@ -274,173 +302,164 @@ int proj_search(orb_context* ctx, int rule, int n_frames, const orb_keypoint* kp
     }
     HIP_TRY(hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    const int F = n_frames;
-    const size_t s_kp = up((size_t)N * sizeof(OrbKeyPoint)), s_desc = up((size_t)N * 32), s_ur = up((size_t)N * 4),
-                 s_occ = up((size_t)N), s_pts = up((size_t)Q * 24), s_pdesc = up((size_t)Q * 32),
-                 s_ptoff = up((size_t)(F + 1) * 4), s_scale = up(ORB_MAX_LEVELS * 4), s_cam = up((size_t)F * 7 * 4),
-                 s_sorted = up((size_t)N * 4), s_cells = up((size_t)F * (64 * 48 + 1) * 4),
-                 s_q = up((size_t)Q * sizeof(ProjQuery)), s_cnt = up((size_t)Q * 4), s_off = up((size_t)(Q + F) * 4),
-                 s_out = up((size_t)Q * 4), s_claim = up((size_t)N * 4), s_chg = up((size_t)F * ORB_PROJ_MAXIT * 4),
-                 s_nm = up((size_t)F * 4), s_grid = up((size_t)F * sizeof(WinPair)),
-                 s_frames = up((size_t)F * sizeof(ProjFrame)), s_tot = up((size_t)F * 4);
-    const size_t total = s_kp + s_desc + s_ur + s_occ + s_pts + s_pdesc + s_ptoff + s_scale + s_cam + s_sorted +
-                         s_cells + s_q + s_cnt + s_off + 3 * s_out + 4 * s_claim + s_chg + s_nm + s_grid + s_frames +
-                         s_tot;
-    int rc = ctx->grow(&ctx->d_win, &ctx->win_cap, total);
-    if (rc) return rc;
-    char* m = (char*)ctx->d_win;
-    size_t o = 0;
-    auto take = [&](size_t s) {
-        char* q = m + o;
-        o += s;
-        return q;
-    };
-    OrbKeyPoint* d_kp = (OrbKeyPoint*)take(s_kp);
-    uint8_t* d_desc = (uint8_t*)take(s_desc);
-    float* d_ur = (float*)take(s_ur);
-    uint8_t* d_occ = (uint8_t*)take(s_occ);
-    float* d_pts = (float*)take(s_pts);
-    uint8_t* d_pdesc = (uint8_t*)take(s_pdesc);
-    int* d_ptoff = (int*)take(s_ptoff);
-    float* d_scale = (float*)take(s_scale);
-    float* d_cam = (float*)take(s_cam);
-    int* d_sorted = (int*)take(s_sorted);
-    int* d_cells = (int*)take(s_cells);
-    ProjQuery* d_q = (ProjQuery*)take(s_q);
-    int* d_cnt = (int*)take(s_cnt);
-    int* d_off = (int*)take(s_off);
-    int* d_out0 = (int*)take(s_out);
-    int* d_out1 = (int*)take(s_out);
-    int* d_ptm = (int*)take(s_out);
-    int* d_claim0 = (int*)take(s_claim);
-    int* d_claim1 = (int*)take(s_claim);
-    int* d_claim2 = (int*)take(s_claim);
-    int* d_keyp = (int*)take(s_claim);
-    int* d_chg = (int*)take(s_chg);
-    int* d_nm = (int*)take(s_nm);
-    WinPair* d_grid = (WinPair*)take(s_grid);
-    ProjFrame* d_frames = (ProjFrame*)take(s_frames);
-    int* d_tot = (int*)take(s_tot);
     static_assert(sizeof(orb_keypoint) == sizeof(OrbKeyPoint), "keypoint layout");
+    const size_t F = (size_t)n_frames, nk = (size_t)N, np = (size_t)Q;
+    Block B;
+    const size_t i_kp = B.add_in(nk * sizeof(OrbKeyPoint)), i_desc = B.add_in(nk * 32), i_ur = B.add_in(nk * 4),
+                 i_occ = B.add_in(nk), i_pts = B.add_in(np * 24), i_pdesc = B.add_in(np * 32),
+                 i_ptoff = B.add_in((F + 1) * 4), i_scale = B.add_in(ORB_MAX_LEVELS * 4), i_cam = B.add_in(F * 7 * 4),
+                 i_grid = B.add_in(F * sizeof(WinPair)), i_frames = B.add_in(F * sizeof(ProjFrame));
+    const size_t o_ptm = B.add_out(np * 4), o_keyp = B.add_out(nk * 4), o_nm = B.add_out(F * 4),
+                 o_tot = B.add_out(F * 8), o_chg = B.add_out(F * ORB_PROJ_MAXIT * 4);
+    const size_t s_rec = B.add_scratch(nk * 16), s_cells = B.add_scratch(F * (64 * 48 + 1) * 4),
+                 s_q = B.add_scratch(np * sizeof(ProjQuery)), s_cnt = B.add_scratch(np * 4),
+                 s_off = B.add_scratch(np * 4), s_out = B.add_scratch(2 * np * 4), s_claim = B.add_scratch(3 * nk * 4);
+    int rc = ctx->grow(&ctx->d_win, &ctx->win_cap, B.in + B.out + B.scratch);
+    if (!rc) rc = ctx->grow_pinned(&ctx->h_win, &ctx->hwin_cap, B.in + B.out);
+    if (rc) return rc;
+    char *d_in = (char*)ctx->d_win, *d_out = d_in + B.in, *d_s = d_out + B.out;
+    char *h_in = (char*)ctx->h_win, *h_out = h_in + B.in;
     if (N) {
-        HIP_TRY(hipMemcpyAsync(d_kp, kp, (size_t)N * sizeof(OrbKeyPoint), hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemcpyAsync(d_desc, desc, (size_t)N * 32, hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemcpyAsync(d_ur, uright, (size_t)N * 4, hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemcpyAsync(d_occ, occupied, (size_t)N, hipMemcpyHostToDevice, st));
+        std::memcpy(h_in + i_kp, kp, nk * sizeof(OrbKeyPoint));
+        std::memcpy(h_in + i_desc, desc, nk * 32);
+        std::memcpy(h_in + i_ur, uright, nk * 4);
+        std::memcpy(h_in + i_occ, occupied, nk);
     }
     if (Q) {
-        HIP_TRY(hipMemcpyAsync(d_pts, pts, (size_t)Q * 24, hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemcpyAsync(d_pdesc, pdesc, (size_t)Q * 32, hipMemcpyHostToDevice, st));
+        std::memcpy(h_in + i_pts, pts, np * 24);
+        std::memcpy(h_in + i_pdesc, pdesc, np * 32);
     }
-    HIP_TRY(hipMemcpyAsync(d_ptoff, pt_off, (size_t)(F + 1) * 4, hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemcpyAsync(d_scale, scale, (size_t)nlevels * 4, hipMemcpyHostToDevice, st));
-    if (rule == 2) HIP_TRY(hipMemcpyAsync(d_cam, cam, (size_t)F * 7 * 4, hipMemcpyHostToDevice, st));
-    std::vector<WinPair> grid(F);
-    std::vector<ProjFrame> frames(F);
-    for (int f = 0; f < F; f++) {
+    std::memcpy(h_in + i_ptoff, pt_off, (F + 1) * 4);
+    std::memcpy(h_in + i_scale, scale, (size_t)nlevels * 4);
+    if (rule == 2) std::memcpy(h_in + i_cam, cam, F * 7 * 4);
+    WinPair* grid = (WinPair*)(h_in + i_grid);
+    ProjFrame* frames = (ProjFrame*)(h_in + i_frames);
+    std::vector<size_t> nq(F), base(F);
+    std::vector<unsigned long long> cap(F);
+    for (int f = 0; f < n_frames; f++) {
         const int k0 = key_off[f], q0 = pt_off[f];
         WinPair& w = grid[f];
         std::memset(&w, 0, sizeof(w));
-        w.kp2 = d_kp + k0;
+        w.kp2 = (const OrbKeyPoint*)(d_in + i_kp) + k0;
+        w.uright = (const float*)(d_in + i_ur) + k0;
+        w.occupied = (const uint8_t*)(d_in + i_occ) + k0;
         w.n2 = key_off[f + 1] - k0;
         w.minX = bounds[4 * f];
         w.maxX = bounds[4 * f + 1];
         w.minY = bounds[4 * f + 2];
         w.maxY = bounds[4 * f + 3];
-        w.sorted = d_sorted + k0;
-        w.cell_start = d_cells + (size_t)f * (64 * 48 + 1);
-        w.n1 = pt_off[f + 1] - q0;
-        w.cnt = d_cnt + q0;
-        w.off = d_off + q0 + f;
+        w.rec = (float4*)(d_s + s_rec) + k0;
+        w.cell_start = (int*)(d_s + s_cells) + (size_t)f * (64 * 48 + 1);
+        w.total = (unsigned long long*)(d_out + o_tot) + f;
         ProjFrame& P = frames[f];
         std::memset(&P, 0, sizeof(P));
-        P.kp = d_kp + k0;
-        P.desc = d_desc + (size_t)k0 * 32;
-        P.uright = d_ur + k0;
-        P.occupied = d_occ + k0;
+        P.kp = w.kp2;
+        P.desc = (const uint8_t*)(d_in + i_desc) + (size_t)k0 * 32;
         P.n = w.n2;
         P.minX = w.minX;
         P.maxX = w.maxX;
         P.minY = w.minY;
         P.maxY = w.maxY;
-        P.sorted = w.sorted;
+        P.rec = w.rec;
         P.cell_start = w.cell_start;
-        P.q = d_q + q0;
-        P.qdesc = d_pdesc + (size_t)q0 * 32;
-        P.nq = w.n1;
-        P.cnt = w.cnt;
-        P.off = w.off;
-        P.out[0] = d_out0 + q0;
-        P.out[1] = d_out1 + q0;
-        P.claim[0] = d_claim0 + k0;
-        P.claim[1] = d_claim1 + k0;
-        P.claim[2] = d_claim2 + k0;
-        P.changed = d_chg + (size_t)f * ORB_PROJ_MAXIT;
+        P.q = (ProjQuery*)(d_s + s_q) + q0;
+        P.qdesc = (const uint8_t*)(d_in + i_pdesc) + (size_t)q0 * 32;
+        P.nq = pt_off[f + 1] - q0;
+        P.cnt = (int*)(d_s + s_cnt) + q0;
+        P.off = (unsigned*)(d_s + s_off) + q0;
+        P.total = w.total;
+        for (int b = 0; b < 2; b++) P.out[b] = (int*)(d_s + s_out) + b * np + q0;
+        for (int b = 0; b < 3; b++) P.claim[b] = (int*)(d_s + s_claim) + b * nk + k0;
+        P.changed = (int*)(d_out + o_chg) + (size_t)f * ORB_PROJ_MAXIT;
         P.rule = rule;
         P.nnratio = nnratio;
         P.check_orientation = check_orientation ? 1 : 0;
-        P.pt_match = d_ptm + q0;
-        P.key_point = d_keyp + k0;
-        P.nmatch = d_nm + f;
+        P.pt_match = (int*)(d_out + o_ptm) + q0;
+        P.key_point = (int*)(d_out + o_keyp) + k0;
+        P.nmatch = (int*)(d_out + o_nm) + f;
+        nq[f] = (size_t)P.nq;
     }
-    auto run_device = [&]() -> int {
-    HIP_TRY(hipMemcpyAsync(d_grid, grid.data(), (size_t)F * sizeof(WinPair), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemcpyAsync(d_frames, frames.data(), (size_t)F * sizeof(ProjFrame), hipMemcpyHostToDevice, st));
-    HIP_TRY(orb_launch_proj_prep(d_frames, F, max_nq, rule, d_pts, d_ptoff, d_scale, nlevels, d_cam, mono, th, st));
-    HIP_TRY(orb_launch_proj_count(d_grid, d_frames, F, max_nq, d_tot, st));
-    std::vector<int> tot(F);
-    HIP_TRY(hipMemcpyAsync(tot.data(), d_tot, (size_t)F * 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    size_t ncand = 0;
-    for (int f = 0; f < F; f++) ncand += (size_t)tot[f];
-    const int rg = ctx->grow(&ctx->d_wcand, &ctx->wcand_cap, std::max<size_t>(ncand, 1) * sizeof(unsigned));
-    if (rg) return rg;
-    size_t base = 0;
-    for (int f = 0; f < F; f++) {
-        frames[f].cand = (unsigned*)ctx->d_wcand + base;
-        base += (size_t)tot[f];
-    }
-    HIP_TRY(hipMemcpyAsync(d_frames, frames.data(), (size_t)F * sizeof(ProjFrame), hipMemcpyHostToDevice, st));
-    HIP_TRY(orb_launch_proj_fill(d_frames, F, max_nq, st));
-    // claim-resolution rounds until every frame has a round that changed nothing
-    std::vector<int> chg((size_t)F * ORB_PROJ_MAXIT);
-    int k = 0;
-    bool settled = false;
-    const int limit = std::min(ctx->round_limit, ORB_PROJ_MAXIT);
-    while (!settled && k < limit) {
-        const int k1 = std::min(limit, k + 4);
-        HIP_TRY(orb_launch_proj_rounds(d_frames, F, max_nq, k, k1, st));
-        k = k1;
-        HIP_TRY(hipMemcpyAsync(chg.data(), d_chg, chg.size() * 4, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
-        settled = true;
-        for (int f = 0; f < F && settled; f++) {
-            bool s = false;
-            for (int r = 1; r < k && !s; r++) s = chg[(size_t)f * ORB_PROJ_MAXIT + r] == 0;
-            settled = s;
+    const unsigned long long* tot = (const unsigned long long*)(h_out + o_tot);
+    const int* chg = (const int*)(h_out + o_chg);
+    auto place_lists = [&](const unsigned long long* asked) -> int {
+        const size_t n = list_regions(nq, ctx->wcand_cap / sizeof(unsigned), asked, base, cap);
+        const int rg = ctx->grow(&ctx->d_wcand, &ctx->wcand_cap, std::max<size_t>(n, 1) * sizeof(unsigned));
+        if (rg) return rg;
+        for (int f = 0; f < n_frames; f++) {
+            frames[f].cand = (unsigned*)ctx->d_wcand + base[f];
+            frames[f].cand_cap = cap[f];
         }
-    }
-    ctx->last_rounds = k;
-    ctx->last_sequential = settled ? 0 : 1;
-    HIP_TRY(orb_launch_proj_finish(d_frames, F, settled ? 0 : 1, st));
-    return ORB_OK;
+        return ORB_OK;
+    };
+    rc = place_lists(nullptr);
+    if (rc) return rc;
+    HIP_TRY(hipMemcpyAsync(d_in, h_in, B.in, hipMemcpyHostToDevice, st));
+    const WinPair* d_grid = (const WinPair*)(d_in + i_grid);
+    ProjFrame* d_frames = (ProjFrame*)(d_in + i_frames);
+    auto lists = [&]() -> int {
+        HIP_TRY(orb_launch_proj_prep(d_frames, n_frames, max_nq, rule, (const float*)(d_in + i_pts),
+                                     (const int*)(d_in + i_ptoff), (const float*)(d_in + i_scale), nlevels,
+                                     (const float*)(d_in + i_cam), mono, th, st));
+        HIP_TRY(orb_launch_proj_lists(d_grid, d_frames, n_frames, max_nq, st));
+        return ORB_OK;
+    };
+    auto run_device = [&]() -> int {
+        const int limit = std::min(ctx->round_limit, ORB_PROJ_MAXIT);
+        int k = 0;
+        bool settled = false;
+        int rl = lists();
+        if (rl) return rl;
+        // claim-resolution rounds until every frame has a round that changed
+        // nothing, in chunks of 4, each followed by the finish of the frames
+        // that have settled
+        for (;;) {
+            const int k1 = std::min(limit, k + 4);
+            HIP_TRY(orb_launch_proj_rounds(d_frames, n_frames, max_nq, k, k1, st));
+            k = k1;
+            HIP_TRY(orb_launch_proj_finish(d_frames, n_frames, 0, st));
+            HIP_TRY(hipMemcpyAsync(h_out, d_out, B.out, hipMemcpyDeviceToHost, st));
+            HIP_TRY(hipStreamSynchronize(st));
+            bool fits = true;
+            for (int f = 0; f < n_frames; f++) fits = fits && tot[f] <= cap[f];
+            if (!fits) {                           // longer lists, from the start
+                rl = place_lists(tot);
+                if (rl) return rl;
+                HIP_TRY(hipMemcpyAsync(d_in + i_frames, frames, F * sizeof(ProjFrame), hipMemcpyHostToDevice, st));
+                rl = lists();
+                if (rl) return rl;
+                k = 0;
+                continue;
+            }
+            settled = true;
+            for (int f = 0; f < n_frames && settled; f++) {
+                bool s = false;
+                for (int r = 1; r < k && !s; r++) s = chg[(size_t)f * ORB_PROJ_MAXIT + r] == 0;
+                settled = s;
+            }
+            if (settled || k >= limit) break;
+        }
+        ctx->last_rounds = k;
+        ctx->last_sequential = settled ? 0 : 1;
+        if (!settled) {
+            HIP_TRY(orb_launch_proj_finish(d_frames, n_frames, 1, st));
+            HIP_TRY(hipMemcpyAsync(h_out, d_out, B.out, hipMemcpyDeviceToHost, st));
+            HIP_TRY(hipStreamSynchronize(st));
+        }
+        return ORB_OK;
     };
     rc = run_device();
     if (rc) return rc;
     if (steps > 0) {        // repeats with the inputs resident in HBM (they are not modified)
-        HIP_TRY(hipStreamSynchronize(st));
         const auto t0 = std::chrono::steady_clock::now();
         for (int i = 0; i < steps; i++) {
             rc = run_device();
             if (rc) return rc;
         }
-        HIP_TRY(hipStreamSynchronize(st));
         *ms = (float)(std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count() / steps);
     }
-    if (Q) HIP_TRY(hipMemcpyAsync(pt_match, d_ptm, (size_t)Q * 4, hipMemcpyDeviceToHost, st));
-    if (N) HIP_TRY(hipMemcpyAsync(key_point, d_keyp, (size_t)N * 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(nmatches, d_nm, (size_t)F * 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    if (Q) std::memcpy(pt_match, h_out + o_ptm, np * 4);
+    if (N) std::memcpy(key_point, h_out + o_keyp, nk * 4);
+    std::memcpy(nmatches, h_out + o_nm, F * 4);
     return ORB_OK;
 }
 

@@ -12,8 +12,6 @@
 //                      contiguous run, and GetFeaturesInArea's order (ix
 //                      outer, iy inner, index order within a cell) is the
 //                      sorted order over the window's columns
-//   win_count_kernel   per query (one wavefront): how many candidates
-//   win_scan_kernel    per pair: exclusive scan of the counts
 //   win_fill_kernel    per query: the ordered (i2, distance) candidate list
 //   win_round_kernel   one round of the in-order pass resolved in parallel
 //                      (below), 16 lanes per query
@@ -27,104 +25,160 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "orb_sort.h"
 #include "orb_types.h"
 
 #define WIN_COLS 64
 #define WIN_ROWS 48
 #define WIN_CELLS (WIN_COLS * WIN_ROWS)
 #define WIN_CAP 4096                 // keypoints per frame
+#define WIN_PER (WIN_CAP / 1024)     // of them per thread of a workgroup of 1024
 #define WIN_HISTO 30
 
-// Candidate enumeration of GetFeaturesInArea(x, y, r, 0, 0) over the sorted
-// grid; calls f(i2, position) for each candidate in the reference's order.
-// All lanes of the wavefront take part; positions are assigned by ballot.
-template <class F>
-__device__ __forceinline__ int win_enumerate(const WinPair& P, float x, float y, float r, F&& f)
+// The cells of GetFeaturesInArea(x, y, r): columns cx0 .. cx1, rows cy0 ..
+// cy1 of the grid; false if there are none.
+__device__ __forceinline__ bool grid_window(float minX, float maxX, float minY, float maxY, float x, float y, float r,
+                                            int* cx0, int* cx1, int* cy0, int* cy1)
 {
-    const int lane = threadIdx.x & 63;
-    const float minX = P.minX, minY = P.minY;
-    const float invW = static_cast<float>(WIN_COLS) / static_cast<float>(P.maxX - P.minX);
-    const float invH = static_cast<float>(WIN_ROWS) / static_cast<float>(P.maxY - P.minY);
-    const int nMinCellX = max(0, (int)floorf((x - minX - r) * invW));
-    if (nMinCellX >= WIN_COLS) return 0;
-    const int nMaxCellX = min(WIN_COLS - 1, (int)ceilf((x - minX + r) * invW));
-    if (nMaxCellX < 0) return 0;
-    const int nMinCellY = max(0, (int)floorf((y - minY - r) * invH));
-    if (nMinCellY >= WIN_ROWS) return 0;
-    const int nMaxCellY = min(WIN_ROWS - 1, (int)ceilf((y - minY + r) * invH));
-    if (nMaxCellY < 0) return 0;
-    const float rr = r * r;
+    const float invW = static_cast<float>(WIN_COLS) / static_cast<float>(maxX - minX);
+    const float invH = static_cast<float>(WIN_ROWS) / static_cast<float>(maxY - minY);
+    *cx0 = max(0, (int)floorf((x - minX - r) * invW));
+    *cx1 = min(WIN_COLS - 1, (int)ceilf((x - minX + r) * invW));
+    *cy0 = max(0, (int)floorf((y - minY - r) * invH));
+    *cy1 = min(WIN_ROWS - 1, (int)ceilf((y - minY + r) * invH));
+    return *cx0 < WIN_COLS && *cx1 >= 0 && *cy0 < WIN_ROWS && *cy1 >= 0;
+}
+
+// Keypoints in the window's cells, by a group of G lanes (all of them call).
+template <int G>
+__device__ __forceinline__ int grid_count(const int* __restrict__ cell_start, int cx0, int cx1, int cy0, int cy1)
+{
+    const int sub = threadIdx.x & (G - 1);
+    int n = 0;
+    for (int ix = cx0 + sub; ix <= cx1; ix += G)
+        n += cell_start[ix * WIN_ROWS + cy1 + 1] - cell_start[ix * WIN_ROWS + cy0];
+#pragma unroll
+    for (int o = 1; o < G; o <<= 1) n += __shfl_xor(n, o, G);
+    return n;
+}
+
+// The window's keypoints in the reference's order (column by column; a
+// column's cells are one run of rec) by a group of G lanes: a lane per column
+// reads its run, and the runs of G columns are walked as one list, G entries
+// at a time.  Calls f(record, position) for those that pass take(record);
+// returns their number.  Branches are uniform within a group.
+template <int G, class T, class F>
+__device__ __forceinline__ int grid_enumerate(const int* __restrict__ cell_start, const float4* __restrict__ rec,
+                                              int cx0, int cx1, int cy0, int cy1, T&& take, F&& f)
+{
+    const int sub = threadIdx.x & (G - 1), gbase = threadIdx.x & 63 & ~(G - 1);
     int pos = 0;
-    for (int ix = nMinCellX; ix <= nMaxCellX; ix++) {
-        const int a = P.cell_start[ix * WIN_ROWS + nMinCellY], b = P.cell_start[ix * WIN_ROWS + nMaxCellY + 1];
-        for (int j0 = a; j0 < b; j0 += 64) {
-            const int j = j0 + lane;
-            bool take = false;
-            int i2 = 0;
-            if (j < b) {
-                i2 = P.sorted[j];
-                const OrbKeyPoint k = P.kp2[i2];
-                if (k.octave == 0) {             // minLevel = maxLevel = level1 = 0
-                    const float distx = k.x - x, disty = k.y - y;
-                    take = distx * distx + disty * disty < rr;
-                }
+    for (int c0 = cx0; c0 <= cx1; c0 += G) {
+        const int ix = c0 + sub;
+        int a = 0, len = 0;
+        if (ix <= cx1) {
+            a = cell_start[ix * WIN_ROWS + cy0];
+            len = cell_start[ix * WIN_ROWS + cy1 + 1] - a;
+        }
+        int inc = len;                             // inclusive scan of the run lengths
+#pragma unroll
+        for (int o = 1; o < G; o <<= 1) {
+            const int y = __shfl_up(inc, o, G);
+            if (sub >= o) inc += y;
+        }
+        const int tot = __shfl(inc, G - 1, G);
+        const int start = a - (inc - len);         // rec index of list entry t of this column: start + t
+        for (int t0 = 0; t0 < tot; t0 += G) {
+            const int t = t0 + sub;
+            int col = 0;                           // first column whose scan exceeds t
+#pragma unroll
+            for (int o = G / 2; o > 0; o >>= 1)
+                if (__shfl(inc, col + o - 1, G) <= t) col += o;
+            const int j = __shfl(start, col, G) + t;
+            float4 k = make_float4(0.f, 0.f, 0.f, 0.f);
+            bool ok = false;
+            if (t < tot) {
+                k = rec[j];
+                ok = take(k);
             }
-            const unsigned long long bal = __ballot(take);
-            if (take) {
-                const int p = pos + __popcll(bal & ((1ull << lane) - 1ull));
-                f(i2, p);
-            }
+            const unsigned long long all = __ballot(ok) >> gbase;
+            const unsigned long long bal = G == 64 ? all : all & ((1ull << G) - 1ull);
+            if (ok) f(k, pos + __popcll(bal & ((1ull << sub) - 1ull)));
             pos += __popcll(bal);
         }
     }
     return pos;
 }
 
-// One workgroup per pair: cell of every F2 keypoint (PosInGrid: round() of
-// the float offset times the float inverse cell size; outside -> no cell),
-// bitonic sort of (cell << 20 | index), and the first sorted position of
-// every cell.
-__global__ __launch_bounds__(1024) void win_grid_kernel(const WinPair* __restrict__ pairs)
+// Room for n list entries of each group of a workgroup of 256 (n is the same
+// for a group's G lanes, 0 where there is no query): *off receives the
+// group's first entry; false where the lists do not fit.  One atomic per
+// workgroup.
+template <int G>
+__device__ __forceinline__ bool take_entries(int n, unsigned long long* total, unsigned long long cap, unsigned* off)
 {
-    __shared__ unsigned key[WIN_CAP];
-    const WinPair& P = pairs[blockIdx.x];
-    const int n = P.n2;
-    const float invW = static_cast<float>(WIN_COLS) / static_cast<float>(P.maxX - P.minX);
-    const float invH = static_cast<float>(WIN_ROWS) / static_cast<float>(P.maxY - P.minY);
-    int npow = 1;
-    while (npow < n) npow <<= 1;
-    for (int i = threadIdx.x; i < npow; i += 1024) {
-        unsigned k = 0xFFFFFFFFu;
-        if (i < n) {
-            const OrbKeyPoint kp = P.kp2[i];
-            const int px = (int)roundf((kp.x - P.minX) * invW), py = (int)roundf((kp.y - P.minY) * invH);
-            const bool in = px >= 0 && px < WIN_COLS && py >= 0 && py < WIN_ROWS;
-            k = ((unsigned)(in ? px * WIN_ROWS + py : 4095) << 20) | (unsigned)i;
-        }
-        key[i] = k;
+    __shared__ int s_n[256 / G];
+    __shared__ unsigned long long s_base;
+    const int g = threadIdx.x / G;
+    if ((threadIdx.x & (G - 1)) == 0) s_n[g] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int all = 0;
+        for (int i = 0; i < 256 / G; i++) all += s_n[i];
+        s_base = all > 0 ? atomicAdd(total, (unsigned long long)all) : 0;
     }
     __syncthreads();
-    for (int k = 2; k <= npow; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int a = threadIdx.x; a < npow; a += 1024) {
-                const int b = a ^ j;
-                if (b > a) {
-                    const unsigned va = key[a], vb = key[b];
-                    const bool up = (a & k) == 0;
-                    if (up ? (va > vb) : (va < vb)) {
-                        key[a] = vb;
-                        key[b] = va;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    for (int i = threadIdx.x; i < n; i += 1024) P.sorted[i] = (int)(key[i] & 0xFFFFFu);
-    if (P.changed) {   // SearchForInitialization's rounds: rounds 0 and 1 write claim buffers 1 and 2
-        for (int i = threadIdx.x; i < n; i += 1024) P.ccnt[0][i] = P.ccnt[1][i] = 0;
-        for (int k = threadIdx.x; k < ORB_WIN_MAXIT; k += 1024) P.changed[k] = k == 0 ? 1 : 4;   // bit 2: not run
+    unsigned long long o = s_base;
+    for (int i = 0; i < g; i++) o += (unsigned)s_n[i];
+    const bool fits = o + (unsigned)n <= cap;
+    *off = fits ? (unsigned)o : 0u;
+    return fits;
+}
+
+// Cell of keypoint (x, y) (PosInGrid: round() of the float offset times the
+// float inverse cell size), or -1 outside the grid and for keypoints that no
+// query can take: for SearchForInitialization those above level 0 (minLevel =
+// maxLevel = 0), for SearchByProjection those a map point with observations
+// holds.
+__device__ __forceinline__ int grid_cell(const WinPair& P, int i, float x, float y, int octave)
+{
+    const float invW = static_cast<float>(WIN_COLS) / static_cast<float>(P.maxX - P.minX);
+    const float invH = static_cast<float>(WIN_ROWS) / static_cast<float>(P.maxY - P.minY);
+    const int px = (int)roundf((x - P.minX) * invW), py = (int)roundf((y - P.minY) * invH);
+    const bool can = P.occupied ? P.occupied[i] == 0 : octave == 0;
+    return px >= 0 && px < WIN_COLS && py >= 0 && py < WIN_ROWS && can ? px * WIN_ROWS + py : -1;
+}
+
+// Place of every keypoint by sorting (cell << 20 | index); cells' first
+// places by bisection.  For frames with a crowded cell.
+template <int E>
+__device__ __forceinline__ void grid_by_sort(const WinPair& P, int n, const int (&cell)[WIN_PER], unsigned* key,
+                                             unsigned short* place)
+{
+    const int tid = threadIdx.x;
+    unsigned v[E];
+#pragma unroll
+    for (int r = 0; r < E; r++) {
+        const int i = r * 1024 + tid;
+        v[r] = i < n ? ((unsigned)(cell[r] < 0 ? 4095 : cell[r]) << 20) | (unsigned)i : 0xFFFFFFFFu;
     }
-    for (int c = threadIdx.x; c <= WIN_CELLS; c += 1024) {
+    int npow = 2;
+    while (npow < n) npow <<= 1;
+    if (npow < 1024 * E) {                         // keys to places E tid + r: the first npow hold all of them
+#pragma unroll
+        for (int r = 0; r < E; r++) key[r * 1024 + tid] = v[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < E; r++) v[r] = key[E * tid + r];
+    }
+    block_sort<E>(v, npow, key);
+#pragma unroll
+    for (int r = 0; r < E; r++) {
+        key[E * tid + r] = v[r];
+        if (v[r] != 0xFFFFFFFFu) place[v[r] & 0xFFFFFu] = (unsigned short)(E * tid + r);
+    }
+    __syncthreads();
+    for (int c = tid; c <= WIN_CELLS; c += 1024) {
         int lo = 0, hi = n;
         while (lo < hi) {
             const int mid = (lo + hi) >> 1;
@@ -135,70 +189,142 @@ __global__ __launch_bounds__(1024) void win_grid_kernel(const WinPair* __restric
     }
 }
 
-__device__ __forceinline__ bool win_query(const WinPair& P, int i1, float* x, float* y)
+// One workgroup per pair: the first place of every cell and the keypoints'
+// records in (cell, index) order.  A counting sort in LDS: cells counted with
+// atomics, scanned, keypoints scattered in arrival order and then ranked by
+// index among their cell's few; a frame with more than GRID_CROWD keypoints
+// in a cell, whose ranking would grow with the square, is sorted.  Bound:
+// latency of one workgroup.  2000 keypoints: 8 us (17 with the sort in
+// registers, 36 with a sort through LDS).
+#define GRID_CROWD 32
+__global__ __launch_bounds__(1024) void win_grid_kernel(const WinPair* __restrict__ pairs)
 {
-    if (P.kp1[i1].octave > 0) return false;
-    *x = P.prev[i1].x;
-    *y = P.prev[i1].y;
-    return true;
-}
-
-// grid (ceil(max n1 / 4), pairs): one wavefront per F1 keypoint
-__global__ __launch_bounds__(256) void win_count_kernel(const WinPair* __restrict__ pairs)
-{
-    const WinPair& P = pairs[blockIdx.y];
-    const int i1 = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i1 >= P.n1) return;
-    float x, y;
-    int c = 0;
-    if (win_query(P, i1, &x, &y)) c = win_enumerate(P, x, y, (float)P.window, [](int, int) {});
-    if ((threadIdx.x & 63) == 0) P.cnt[i1] = c;
-}
-
-// one workgroup per pair: off[i] = sum of cnt[0..i), total in off[n1]
-__global__ __launch_bounds__(1024) void win_scan_kernel(const WinPair* __restrict__ pairs, int* __restrict__ totals)
-{
-    __shared__ int part[1024];
+    static_assert(WIN_CELLS < 4 * 1024 && WIN_CAP == WIN_PER * 1024, "four cells and keypoints a thread");
+    __shared__ int start[4 * 1024];
+    __shared__ unsigned key[WIN_CAP];
+    __shared__ unsigned short place[WIN_CAP];
+    __shared__ int part[16];
     const WinPair& P = pairs[blockIdx.x];
-    const int n = P.n1, t = threadIdx.x;
-    const int per = (n + 1023) / 1024;
-    const int a = min(t * per, n), b = min(a + per, n);
-    int s = 0;
-    for (int i = a; i < b; i++) s += P.cnt[i];
-    part[t] = s;
+    const int n = P.n2, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+#pragma unroll
+    for (int r = 0; r < 4; r++) start[r * 1024 + tid] = 0;
+    if (P.changed) {   // SearchForInitialization's rounds: rounds 0 and 1 write claim buffers 1 and 2
+        for (int i = tid; i < n; i += 1024) P.ccnt[0][i] = P.ccnt[1][i] = 0;
+        for (int k = tid; k < ORB_WIN_MAXIT; k += 1024) P.changed[k] = k == 0 ? 1 : 4;   // bit 2: not run
+    }
+    if (tid == 0) *P.total = 0;
+    float4 rec[WIN_PER];
+    int cell[WIN_PER], at[WIN_PER];
+#pragma unroll
+    for (int r = 0; r < WIN_PER; r++) {
+        const int i = r * 1024 + tid;
+        cell[r] = -1;
+        if (i < n) {
+            const OrbKeyPoint* k = P.kp2 + i;
+            const float x = k->x, y = k->y;
+            const int octave = k->octave;
+            rec[r] = make_float4(x, y, P.uright ? P.uright[i] : 0.f, __int_as_float(i | (octave << 12)));
+            cell[r] = grid_cell(P, i, x, y, octave);
+        }
+    }
     __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        const int v = t >= o ? part[t - o] : 0;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
+#pragma unroll
+    for (int r = 0; r < WIN_PER; r++) at[r] = cell[r] >= 0 ? atomicAdd(&start[cell[r]], 1) : 0;
+    __syncthreads();
+    const int4 c4 = *(const int4*)&start[4 * tid];
+    const int sum = c4.x + c4.y + c4.z + c4.w;
+    int inc = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += y;
     }
-    int run = part[t] - s;
-    for (int i = a; i < b; i++) {
-        P.off[i] = run;
-        run += P.cnt[i];
+    if (lane == 63) part[wv] = inc;
+    const bool crowd = __syncthreads_or(max(max(c4.x, c4.y), max(c4.z, c4.w)) > GRID_CROWD);
+    if (crowd) {
+        if (n <= 1024) grid_by_sort<1>(P, n, cell, key, place);
+        else if (n <= 2048) grid_by_sort<2>(P, n, cell, key, place);
+        else grid_by_sort<4>(P, n, cell, key, place);
+#pragma unroll
+        for (int r = 0; r < WIN_PER; r++)
+            if (cell[r] >= 0) P.rec[place[r * 1024 + tid]] = rec[r];
+        return;
     }
-    if (t == 1023) {
-        P.off[n] = part[1023];
-        totals[blockIdx.x] = part[1023];
+    int base = inc - sum;
+#pragma unroll
+    for (int w = 0; w < 16; w++) base += w < wv ? part[w] : 0;
+    const int4 s4 = make_int4(base, base + c4.x, base + c4.x + c4.y, base + c4.x + c4.y + c4.z);
+    *(int4*)&start[4 * tid] = s4;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int c = 4 * tid + e;
+        if (c <= WIN_CELLS) P.cell_start[c] = e == 0 ? s4.x : (e == 1 ? s4.y : (e == 2 ? s4.z : s4.w));
     }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < WIN_PER; r++)
+        if (cell[r] >= 0) key[start[cell[r]] + at[r]] = (unsigned)(r * 1024 + tid);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < WIN_PER; r++)
+        if (cell[r] >= 0) {
+            const int a = start[cell[r]], b = start[cell[r] + 1];
+            int rank = 0;
+            for (int j = a; j < b; j++) rank += key[j] < (unsigned)(r * 1024 + tid) ? 1 : 0;
+            P.rec[a + rank] = rec[r];
+        }
 }
 
+__device__ __forceinline__ int row_distance(const uint4 a0, const uint4 a1, const uint8_t* b)
+{
+    const uint4 b0 = *(const uint4*)b, b1 = *(const uint4*)(b + 16);
+    return __popc(a0.x ^ b0.x) + __popc(a0.y ^ b0.y) + __popc(a0.z ^ b0.z) + __popc(a0.w ^ b0.w) +
+           __popc(a1.x ^ b1.x) + __popc(a1.y ^ b1.y) + __popc(a1.z ^ b1.z) + __popc(a1.w ^ b1.w);
+}
+
+// grid (ceil(max n1 / (256 / WIN_G)), pairs): WIN_G lanes per F1 keypoint.
+// Each level-0 query takes room for all its window's keypoints and stores the
+// (i2, distance) of those inside the circle, in the reference's order.
+// Bound: latency (a few dependent loads per query).  2000 queries, window 100:
+// 9.5 us; counting, scanning and filling in turn, a wavefront per query that
+// walked its window column by column, took 44 us.
+#define WIN_G 32
 __global__ __launch_bounds__(256) void win_fill_kernel(const WinPair* __restrict__ pairs)
 {
     const WinPair& P = pairs[blockIdx.y];
-    const int i1 = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i1 >= P.n1) return;
-    float x, y;
-    if (!win_query(P, i1, &x, &y) || P.cnt[i1] == 0) return;
-    const uint4 a0 = *(const uint4*)(P.d1 + (size_t)i1 * 32), a1 = *(const uint4*)(P.d1 + (size_t)i1 * 32 + 16);
-    int2* out = P.cand + P.off[i1];
-    win_enumerate(P, x, y, (float)P.window, [&](int i2, int p) {
-        const uint4 b0 = *(const uint4*)(P.d2 + (size_t)i2 * 32), b1 = *(const uint4*)(P.d2 + (size_t)i2 * 32 + 16);
-        const int d = __popc(a0.x ^ b0.x) + __popc(a0.y ^ b0.y) + __popc(a0.z ^ b0.z) + __popc(a0.w ^ b0.w) +
-                      __popc(a1.x ^ b1.x) + __popc(a1.y ^ b1.y) + __popc(a1.z ^ b1.z) + __popc(a1.w ^ b1.w);
-        out[p] = make_int2(i2, d);
-    });
+    const int q = blockIdx.x * (256 / WIN_G) + threadIdx.x / WIN_G;
+    const float r = (float)P.window;
+    int cx0 = 0, cx1 = -1, cy0 = 0, cy1 = -1, n = 0;
+    float x = 0.f, y = 0.f;
+    if (q < P.n1 && P.kp1[q].octave <= 0) {
+        x = P.prev[q].x;
+        y = P.prev[q].y;
+        if (grid_window(P.minX, P.maxX, P.minY, P.maxY, x, y, r, &cx0, &cx1, &cy0, &cy1))
+            n = grid_count<WIN_G>(P.cell_start, cx0, cx1, cy0, cy1);
+    }
+    unsigned off;
+    const bool fits = take_entries<WIN_G>(n, P.total, P.cand_cap, &off);
+    if (q >= P.n1) return;
+    int cnt = 0;
+    if (n > 0 && fits) {
+        const uint4 a0 = *(const uint4*)(P.d1 + (size_t)q * 32), a1 = *(const uint4*)(P.d1 + (size_t)q * 32 + 16);
+        const float rr = r * r;
+        int2* out = P.cand + off;
+        cnt = grid_enumerate<WIN_G>(
+            P.cell_start, P.rec, cx0, cx1, cy0, cy1,
+            [&](const float4& k) {
+                const float distx = k.x - x, disty = k.y - y;
+                return distx * distx + disty * disty < rr;
+            },
+            [&](const float4& k, int p) {
+                const int i2 = __float_as_int(k.w) & 0xFFF;
+                out[p] = make_int2(i2, row_distance(a0, a1, P.d2 + (size_t)i2 * 32));
+            });
+    }
+    if ((threadIdx.x & (WIN_G - 1)) == 0) {
+        P.cnt[q] = cnt;
+        P.off[q] = off;
+    }
 }
 
 // One wavefront per pair.  Query by query, in index order: lanes take the
@@ -211,11 +337,23 @@ __global__ __launch_bounds__(256) void win_fill_kernel(const WinPair* __restrict
 // The first round k >= 1 that ran, changed no outcome and read complete
 // claims (round k - 1 did not overflow its slots): its outcomes are the
 // in-order pass's.  0 if there is none.
+// (Every lane of the wavefront calls.)
 __device__ __forceinline__ int win_settled_round(const int* chg)
 {
-    for (int k = 1; k < ORB_WIN_MAXIT; k++)
-        if (chg[k] == 0 && !(chg[k - 1] & 2)) return k;
-    return 0;
+    static_assert(ORB_WIN_MAXIT <= 64 && ORB_PROJ_MAXIT <= 64, "one round per lane");
+    const int k = threadIdx.x & 63;
+    const bool ok = k >= 1 && k < ORB_WIN_MAXIT && chg[k] == 0 && !(chg[k - 1] & 2);
+    const unsigned long long b = __ballot(ok);
+    return b ? __ffsll((long long)b) - 1 : 0;
+}
+
+// The first round k >= 1 of a SearchByProjection frame that ran and changed
+// nothing, or 0.  (Every lane of the wavefront calls.)
+__device__ __forceinline__ int proj_settled_round(const int* chg)
+{
+    const int k = threadIdx.x & 63;
+    const unsigned long long b = __ballot(k >= 1 && k < ORB_PROJ_MAXIT && chg[k] == 0);
+    return b ? __ffsll((long long)b) - 1 : 0;
 }
 
 __global__ __launch_bounds__(64) void win_greedy_kernel(const WinPair* __restrict__ pairs, int skip_settled)
@@ -343,30 +481,17 @@ __global__ __launch_bounds__(64) void win_greedy_kernel(const WinPair* __restric
     for (int i = lane; i < n1; i += 64) {
         const int m = m12[i];
         P.m12[i] = m;
-        if (m >= 0) P.prev[i] = make_float2(P.kp2[m].x, P.kp2[m].y);
+        P.prev_out[i] = m >= 0 ? make_float2(P.kp2[m].x, P.kp2[m].y) : P.prev[i];
     }
     if (lane == 0) *P.nmatch = s_n;
 }
 
-extern "C" hipError_t orb_launch_win_count(const WinPair* d_pairs, int npairs, int max_n1, hipStream_t st)
+extern "C" hipError_t orb_launch_win_lists(const WinPair* d_pairs, int npairs, int max_n1, hipStream_t st)
 {
     if (npairs <= 0) return hipSuccess;
     win_grid_kernel<<<npairs, 1024, 0, st>>>(d_pairs);
-    if (max_n1 > 0) win_count_kernel<<<dim3((max_n1 + 3) / 4, npairs), 256, 0, st>>>(d_pairs);
-    return hipGetLastError();
-}
-
-extern "C" hipError_t orb_launch_win_scan(const WinPair* d_pairs, int npairs, int* d_totals, hipStream_t st)
-{
-    if (npairs <= 0) return hipSuccess;
-    win_scan_kernel<<<npairs, 1024, 0, st>>>(d_pairs, d_totals);
-    return hipGetLastError();
-}
-
-extern "C" hipError_t orb_launch_win_fill(const WinPair* d_pairs, int npairs, int max_n1, hipStream_t st)
-{
-    if (npairs <= 0 || max_n1 <= 0) return hipSuccess;
-    win_fill_kernel<<<dim3((max_n1 + 3) / 4, npairs), 256, 0, st>>>(d_pairs);
+    if (max_n1 > 0)
+        win_fill_kernel<<<dim3((max_n1 + 256 / WIN_G - 1) / (256 / WIN_G), npairs), 256, 0, st>>>(d_pairs);
     return hipGetLastError();
 }
 
@@ -386,69 +511,19 @@ extern "C" hipError_t orb_launch_win_fill(const WinPair* d_pairs, int npairs, in
 // not settled after ORB_PROJ_MAXIT rounds gets the sequential pass.
 //   proj_prep_*        the per-point arithmetic of each overload -> ProjQuery
 //   win_grid_kernel    the frame's keypoint grid (as for SearchForInitialization)
-//   proj_count_kernel  per query: candidates after the static filters (levels,
-//                      circle, occupied keys, mvuRight)
-//   win_scan_kernel    offsets
-//   proj_fill_kernel   per query: (keypoint, distance, octave) in GetFeaturesInArea order
+//   proj_fill_kernel   per query: (keypoint, distance, octave) of the candidates
+//                      that pass the static filters (levels, circle, occupied
+//                      keys, mvuRight), in GetFeaturesInArea order
 //   proj_round_kernel  one claim-resolution round, 16 lanes per query
 //   proj_seq_kernel    the sequential pass, for frames that did not settle
 //   proj_finish_kernel per frame: key_point, nmatches, the rotation check
 
-// GetFeaturesInArea(x, y, r, minLevel, maxLevel) over the sorted grid; calls
-// f(i2, position) in the reference's order for candidates that also pass
-// keep(i2).  All lanes of the wavefront take part.
-template <class K, class F>
-__device__ __forceinline__ int area_enumerate(const ProjFrame& P, const ProjQuery& Q, K&& keep, F&& f)
+// The frame's round state before round 0: no claims, no round run.
+__device__ __forceinline__ void proj_reset(const ProjFrame& P)
 {
-    const int lane = threadIdx.x & 63;
-    const float x = Q.x, y = Q.y, r = Q.r;
-    const float invW = static_cast<float>(WIN_COLS) / static_cast<float>(P.maxX - P.minX);
-    const float invH = static_cast<float>(WIN_ROWS) / static_cast<float>(P.maxY - P.minY);
-    const int nMinCellX = max(0, (int)floorf((x - P.minX - r) * invW));
-    if (nMinCellX >= WIN_COLS) return 0;
-    const int nMaxCellX = min(WIN_COLS - 1, (int)ceilf((x - P.minX + r) * invW));
-    if (nMaxCellX < 0) return 0;
-    const int nMinCellY = max(0, (int)floorf((y - P.minY - r) * invH));
-    if (nMinCellY >= WIN_ROWS) return 0;
-    const int nMaxCellY = min(WIN_ROWS - 1, (int)ceilf((y - P.minY + r) * invH));
-    if (nMaxCellY < 0) return 0;
-    const bool checkLevels = (Q.minL > 0) || (Q.maxL >= 0);
-    const float rr = r * r;
-    int pos = 0;
-    for (int ix = nMinCellX; ix <= nMaxCellX; ix++) {
-        const int a = P.cell_start[ix * WIN_ROWS + nMinCellY], b = P.cell_start[ix * WIN_ROWS + nMaxCellY + 1];
-        for (int j0 = a; j0 < b; j0 += 64) {
-            const int j = j0 + lane;
-            bool take = false;
-            int i2 = 0;
-            if (j < b) {
-                i2 = P.sorted[j];
-                const OrbKeyPoint k = P.kp[i2];
-                take = !checkLevels || (k.octave >= Q.minL && (Q.maxL < 0 || k.octave <= Q.maxL));
-                if (take) {
-                    const float distx = k.x - x, disty = k.y - y;
-                    take = distx * distx + disty * disty < rr && keep(i2);
-                }
-            }
-            const unsigned long long bal = __ballot(take);
-            if (take) f(i2, pos + __popcll(bal & ((1ull << lane) - 1ull)));
-            pos += __popcll(bal);
-        }
-    }
-    return pos;
-}
-
-// Static candidate filters: keypoints held by a map point with observations,
-// and mvuRight beyond the radius of the query's right-image u.
-__device__ __forceinline__ bool proj_keep(const ProjFrame& P, const ProjQuery& Q, int i2)
-{
-    if (P.occupied[i2]) return false;
-    const float ur = P.uright[i2];
-    if (ur > 0) {
-        const float er = fabsf(Q.su - ur);
-        if (er > Q.r) return false;
-    }
-    return true;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t < ORB_PROJ_MAXIT) P.changed[t] = t == 0 ? 1 : 4;   // bit 2: not run
+    for (int i = t; i < P.n; i += gridDim.x * 256) P.claim[0][i] = P.claim[1][i] = 0x7FFFFFFF;
 }
 
 // SearchByProjection(Frame&, vector<MapPoint*>, th) per point (:82-105):
@@ -459,8 +534,7 @@ __global__ __launch_bounds__(256) void proj_prep_local_kernel(ProjFrame* __restr
 {
     ProjFrame& P = frames[blockIdx.y];
     const int q = blockIdx.x * 256 + threadIdx.x;
-    if (blockIdx.x == 0)
-        for (int k = threadIdx.x; k < ORB_PROJ_MAXIT; k += 256) P.changed[k] = k == 0 ? 1 : 4;   // bit 2: not run
+    proj_reset(P);
     if (q >= P.nq) return;
     const float* src = pts + (size_t)(pt_off[blockIdx.y] + q) * 6;   // proj_x, proj_y, proj_xr, view_cos, level, flags
     const int level = __float_as_int(src[4]), fl = __float_as_int(src[5]);
@@ -490,8 +564,7 @@ __global__ __launch_bounds__(256) void proj_prep_last_kernel(ProjFrame* __restri
 {
     ProjFrame& P = frames[blockIdx.y];
     const int q = blockIdx.x * 256 + threadIdx.x;
-    if (blockIdx.x == 0)
-        for (int k = threadIdx.x; k < ORB_PROJ_MAXIT; k += 256) P.changed[k] = k == 0 ? 1 : 4;   // bit 2: not run
+    proj_reset(P);
     if (q >= P.nq) return;
     const float* c = cam + (size_t)blockIdx.y * 7;
     const float fx = c[0], fy = c[1], cx = c[2], cy = c[3], mbf = c[4], mb = c[5], tlc_z = c[6];
@@ -529,38 +602,50 @@ __global__ __launch_bounds__(256) void proj_prep_last_kernel(ProjFrame* __restri
     P.q[q] = Q;
 }
 
-// grid (ceil(max nq / 4), frames): one wavefront per query.  Also resets the
-// first two claim buffers of the frame (no claims before round 0).
-__global__ __launch_bounds__(256) void proj_count_kernel(ProjFrame* __restrict__ frames)
-{
-    ProjFrame& P = frames[blockIdx.y];
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < P.n; i += gridDim.x * 256) {
-        P.claim[0][i] = 0x7FFFFFFF;
-        P.claim[1][i] = 0x7FFFFFFF;
-    }
-    const int q = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (q >= P.nq) return;
-    const ProjQuery Q = P.q[q];
-    int c = 0;
-    if (Q.flags & ORB_PQ_VALID)
-        c = area_enumerate(P, Q, [&](int i2) { return proj_keep(P, Q, i2); }, [](int, int) {});
-    if ((threadIdx.x & 63) == 0) P.cnt[q] = c;
-}
-
+// grid (ceil(max nq / 16), frames): 16 lanes per query.  Each valid query
+// takes room for all its window's keypoints and stores those that pass
+// GetFeaturesInArea's level rule and circle and the mvuRight check (:111-118:
+// the right-image u within the radius), in the reference's order.
+// Bound: latency (a few dependent loads per query).  16 frames x 1800 points,
+// th 15: 27 us (counting, scanning and filling in turn 91 us); 1 frame, th 3:
+// 9 us (26).
 __global__ __launch_bounds__(256) void proj_fill_kernel(const ProjFrame* __restrict__ frames)
 {
     const ProjFrame& P = frames[blockIdx.y];
-    const int q = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (q >= P.nq || P.cnt[q] == 0) return;
-    const ProjQuery Q = P.q[q];
-    const uint4 a0 = *(const uint4*)(P.qdesc + (size_t)q * 32), a1 = *(const uint4*)(P.qdesc + (size_t)q * 32 + 16);
-    unsigned* out = P.cand + P.off[q];
-    area_enumerate(P, Q, [&](int i2) { return proj_keep(P, Q, i2); }, [&](int i2, int p) {
-        const uint4 b0 = *(const uint4*)(P.desc + (size_t)i2 * 32), b1 = *(const uint4*)(P.desc + (size_t)i2 * 32 + 16);
-        const int d = __popc(a0.x ^ b0.x) + __popc(a0.y ^ b0.y) + __popc(a0.z ^ b0.z) + __popc(a0.w ^ b0.w) +
-                      __popc(a1.x ^ b1.x) + __popc(a1.y ^ b1.y) + __popc(a1.z ^ b1.z) + __popc(a1.w ^ b1.w);
-        out[p] = (unsigned)i2 | ((unsigned)d << 12) | ((unsigned)P.kp[i2].octave << 21);
-    });
+    const int q = blockIdx.x * 16 + (threadIdx.x >> 4);
+    ProjQuery Q = {};
+    if (q < P.nq) Q = P.q[q];
+    int cx0 = 0, cx1 = -1, cy0 = 0, cy1 = -1, n = 0;
+    if ((Q.flags & ORB_PQ_VALID) &&
+        grid_window(P.minX, P.maxX, P.minY, P.maxY, Q.x, Q.y, Q.r, &cx0, &cx1, &cy0, &cy1))
+        n = grid_count<16>(P.cell_start, cx0, cx1, cy0, cy1);
+    unsigned off;
+    const bool fits = take_entries<16>(n, P.total, P.cand_cap, &off);
+    if (q >= P.nq) return;
+    int cnt = 0;
+    if (n > 0 && fits) {
+        const uint4 a0 = *(const uint4*)(P.qdesc + (size_t)q * 32), a1 = *(const uint4*)(P.qdesc + (size_t)q * 32 + 16);
+        const bool checkLevels = (Q.minL > 0) || (Q.maxL >= 0);
+        const float rr = Q.r * Q.r;
+        unsigned* out = P.cand + off;
+        cnt = grid_enumerate<16>(
+            P.cell_start, P.rec, cx0, cx1, cy0, cy1,
+            [&](const float4& k) {
+                const int octave = __float_as_int(k.w) >> 12;
+                if (checkLevels && !(octave >= Q.minL && (Q.maxL < 0 || octave <= Q.maxL))) return false;
+                const float distx = k.x - Q.x, disty = k.y - Q.y;
+                if (!(distx * distx + disty * disty < rr)) return false;
+                return !(k.z > 0 && fabsf(Q.su - k.z) > Q.r);
+            },
+            [&](const float4& k, int p) {
+                const unsigned w = (unsigned)__float_as_int(k.w), i2 = w & 0xFFFu;
+                out[p] = i2 | ((unsigned)row_distance(a0, a1, P.desc + (size_t)i2 * 32) << 12) | ((w >> 12) << 21);
+            });
+    }
+    if ((threadIdx.x & 15) == 0) {
+        P.cnt[q] = cnt;
+        P.off[q] = off;
+    }
 }
 
 // The per-point decision over its candidate list with blocked keypoints
@@ -615,8 +700,8 @@ __device__ __forceinline__ int proj_decide(const ProjFrame& P, int q, int sub, B
 __global__ __launch_bounds__(256) void proj_round_kernel(ProjFrame* __restrict__ frames, int k)
 {
     ProjFrame& P = frames[blockIdx.y];
-    for (int j = 1; j < k; j++)
-        if (P.changed[j] == 0) return;                 // settled at round j: later rounds are left alone
+    const int ks = proj_settled_round(P.changed);
+    if (ks > 0 && ks < k) return;                      // settled: later rounds are left alone
     if (k > 0 && blockIdx.x == 0 && threadIdx.x == 0) atomicAnd(&P.changed[k], ~4);
     const int* __restrict__ claimR = P.claim[k % 3];
     int* claimW = P.claim[(k + 1) % 3];
@@ -641,9 +726,7 @@ __global__ __launch_bounds__(64) void proj_seq_kernel(ProjFrame* __restrict__ fr
 {
     __shared__ int claimer[WIN_CAP];
     ProjFrame& P = frames[blockIdx.x];
-    bool settled = false;
-    for (int k = 1; k < ORB_PROJ_MAXIT; k++) settled |= P.changed[k] == 0;
-    if (settled) return;
+    if (proj_settled_round(P.changed) > 0) return;
     for (int i = threadIdx.x; i < P.n; i += 64) claimer[i] = 0;
     __syncthreads();
     for (int q = 0; q < P.nq; q++) {
@@ -705,8 +788,8 @@ __global__ __launch_bounds__(1024) void proj_finish_kernel(const ProjFrame* __re
     __shared__ int s_ind[3];
     __shared__ int s_count[2];
     const ProjFrame& P = frames[blockIdx.x];
-    int kc = 1;
-    while (kc < ORB_PROJ_MAXIT - 1 && P.changed[kc] != 0) kc++;
+    const int kc = proj_settled_round(P.changed);
+    if (kc == 0 || *P.total > P.cand_cap) return;      // more rounds, or longer lists, to come
     const int* out = P.out[kc & 1];
     for (int i = threadIdx.x; i < P.n; i += 1024) owner[i] = -1;
     if (threadIdx.x < WIN_HISTO) hist[threadIdx.x] = 0;
@@ -765,21 +848,13 @@ extern "C" hipError_t orb_launch_proj_prep(ProjFrame* d_frames, int nframes, int
 }
 
 // d_grid: one WinPair per frame carrying the grid fields (kp2, n2, bounds,
-// sorted, cell_start) and the scan fields (n1 = queries, cnt, off).
-extern "C" hipError_t orb_launch_proj_count(const WinPair* d_grid, ProjFrame* d_frames, int nframes, int max_nq,
-                                            int* d_totals, hipStream_t st)
+// uright, occupied, rec, cell_start) and the list total.
+extern "C" hipError_t orb_launch_proj_lists(const WinPair* d_grid, const ProjFrame* d_frames, int nframes, int max_nq,
+                                            hipStream_t st)
 {
     if (nframes <= 0) return hipSuccess;
     win_grid_kernel<<<nframes, 1024, 0, st>>>(d_grid);
-    proj_count_kernel<<<dim3((max(max_nq, 1) + 3) / 4, nframes), 256, 0, st>>>(d_frames);
-    win_scan_kernel<<<nframes, 1024, 0, st>>>(d_grid, d_totals);
-    return hipGetLastError();
-}
-
-extern "C" hipError_t orb_launch_proj_fill(ProjFrame* d_frames, int nframes, int max_nq, hipStream_t st)
-{
-    if (nframes <= 0 || max_nq <= 0) return hipSuccess;
-    proj_fill_kernel<<<dim3((max_nq + 3) / 4, nframes), 256, 0, st>>>(d_frames);
+    if (max_nq > 0) proj_fill_kernel<<<dim3((max_nq + 15) / 16, nframes), 256, 0, st>>>(d_frames);
     return hipGetLastError();
 }
 
@@ -889,68 +964,72 @@ __global__ __launch_bounds__(256) void win_round_kernel(const WinPair* __restric
 __global__ __launch_bounds__(1024) void win_finish_kernel(const WinPair* __restrict__ pairs)
 {
     __shared__ int owner[WIN_CAP];
-    __shared__ signed char bin[WIN_CAP];
     __shared__ int hist[WIN_HISTO];
     __shared__ int s_ind[3];
-    __shared__ int s_n[2];
+    __shared__ int s_n;
     const WinPair& P = pairs[blockIdx.x];
     const int ks = win_settled_round(P.changed);
-    if (ks == 0) return;                           // the sequential pass takes this pair
+    if (ks == 0 || *P.total > P.cand_cap) return;  // more rounds, the sequential pass or longer lists to come
     const int* out = P.out[ks & 1];
     const int n1 = P.n1, t = threadIdx.x;
+    constexpr int PER = WIN_PER;                   // queries t, t + 1024, ... of a thread, read together
+    int r[PER];
+    float2 pos[PER];
+    float a1[PER];
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+        const int q = t + 1024 * e;
+        r[e] = -1;
+        if (q < n1) {
+            r[e] = out[q];
+            pos[e] = P.prev[q];
+            a1[e] = P.kp1[q].angle;
+        }
+    }
     for (int i = t; i < P.n2; i += 1024) owner[i] = -1;
     if (t < WIN_HISTO) hist[t] = 0;
-    if (t < 2) s_n[t] = 0;
-    __syncthreads();
-    for (int q = t; q < n1; q += 1024) {
-        const int r = out[q];
-        if (r >= 0) atomicMax(&owner[r >> 9], q);
-    }
+    if (t == 0) s_n = 0;
     __syncthreads();
     const float factor = WIN_HISTO / 360.0f;
-    int kept = 0;
-    for (int q = t; q < n1; q += 1024) {
-        const int r = out[q];
-        int m = -1, b = -1;
-        if (r >= 0) {
-            const int tg = r >> 9;
-            if (owner[tg] == q) {
-                m = tg;
-                kept++;
-            }
+    int bin[PER];
+    float2 at[PER];
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+        bin[e] = -1;
+        if (r[e] >= 0) {
+            const int tg = r[e] >> 9;
+            atomicMax(&owner[tg], t + 1024 * e);
+            at[e] = make_float2(P.kp2[tg].x, P.kp2[tg].y);
             if (P.check_orientation) {
-                float rot = P.kp1[q].angle - P.kp2[tg].angle;
+                float rot = a1[e] - P.kp2[tg].angle;
                 if (rot < 0.0f) rot += 360.0f;
-                b = (int)roundf(rot * factor);
+                int b = (int)roundf(rot * factor);
                 if (b == WIN_HISTO) b = 0;
+                bin[e] = b;
                 atomicAdd(&hist[b], 1);
             }
         }
-        bin[q] = (signed char)b;
-        P.m12[q] = m;
     }
-    atomicAdd(&s_n[0], kept);
     __syncthreads();
     if (P.check_orientation) {
         if (t == 0) three_maxima(hist, s_ind);
         __syncthreads();
-        int dropped = 0;
-        for (int q = t; q < n1; q += 1024) {
-            const int b = bin[q];
-            if (b < 0 || b == s_ind[0] || b == s_ind[1] || b == s_ind[2]) continue;
-            if (P.m12[q] >= 0) {
-                P.m12[q] = -1;
-                dropped++;
-            }
-        }
-        atomicAdd(&s_n[1], dropped);
-        __syncthreads();
     }
-    for (int q = t; q < n1; q += 1024) {
-        const int m = P.m12[q];
-        if (m >= 0) P.prev[q] = make_float2(P.kp2[m].x, P.kp2[m].y);
+    int kept = 0;
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+        const int q = t + 1024 * e;
+        if (q >= n1) continue;
+        const int b = bin[e];
+        const bool drop = b >= 0 && b != s_ind[0] && b != s_ind[1] && b != s_ind[2];
+        const bool keep = r[e] >= 0 && owner[max(r[e], 0) >> 9] == q && !drop;
+        kept += keep ? 1 : 0;
+        P.m12[q] = keep ? r[e] >> 9 : -1;
+        P.prev_out[q] = keep ? at[e] : pos[e];
     }
-    if (t == 0) *P.nmatch = s_n[0] - s_n[1];
+    atomicAdd(&s_n, kept);
+    __syncthreads();
+    if (t == 0) *P.nmatch = s_n;
 }
 
 extern "C" hipError_t orb_launch_win_rounds(const WinPair* d_pairs, int npairs, int max_n1, int k0, int k1,
