@@ -408,6 +408,9 @@ struct orb_extractor {
             // change of tile heights never reallocates (the frames stay put)
             ntab += (size_t)p.lv[l].w + p.lv[l].h + p.lv[l].tiles_x + (p.lv[l].h + 15) / 16;
         const size_t o_tab = take(ntab * 8);
+        size_t noct = 0;
+        for (int l = 0; l < nlevels; l++) noct += (size_t)p.lv[l].w + p.lv[l].h;
+        const size_t o_oct = take(noct * 2);
         const size_t total = off;
         if (total > mem_bytes) {
             if (d_mem) (void)hipFree(d_mem);
@@ -470,12 +473,14 @@ struct orb_extractor {
             L.node = (int*)(d_mem + o_node) + P.key_off;
             L.ret = (unsigned long long*)(d_mem + o_ret) + P.ret_off;
         }
+        // resize taps and quadtree places, sent in one copy
+        std::vector<char> tables(o_oct - o_tab + noct * 2);
         // cv::resize INTER_LINEAR taps of every level from the level above
         // (ComputePyramid, ORBextractor.cc:1677): per destination column and
         // row, the source index and the two 11-bit weights, with the float
         // statements of OpenCV's generic path.
         {
-            std::vector<int2> tab(ntab);
+            int2* tab = (int2*)tables.data();
             size_t t = 0;
             for (int l = 1; l < nlevels; l++) {
                 const int w = p.lv[l].w, h = p.lv[l].h, sw = p.lv[l - 1].w, sh = p.lv[l - 1].h;
@@ -537,7 +542,54 @@ struct orb_extractor {
                     tab[t].y = hi;
                 }
             }
-            if (ntab) HIP_TRY(hipMemcpy(d_mem + o_tab, tab.data(), ntab * 8, hipMemcpyHostToDevice));
+        }
+        // Quadtree place at depth ORB_OCT_D, split into its x and y parts: the
+        // root (ORBextractor.cc:695-763, in float as there), then one bit per
+        // halving (DivideNode, :600-625).  The kernel's numbering turns every
+        // other depth's quadrant around (octree_kernel).
+        {
+            unsigned short* tab = (unsigned short*)(tables.data() + (o_oct - o_tab));
+            size_t t = 0;
+            // bits of the halvings of [lo, hi) that lead to v, the same up to *next
+            auto halve = [](int lo, int hi, int v, int bit0, int* next) {
+                unsigned bits = 0;
+                for (int d = 1; d <= ORB_OCT_D; d++) {
+                    const int mid = lo + ((hi - lo + 1) >> 1);
+                    if (v < mid) {
+                        hi = mid;
+                        *next = std::min(*next, mid);
+                    } else {
+                        lo = mid;
+                        bits |= 1u << (2 * (ORB_OCT_D - d) + bit0);
+                    }
+                }
+                return bits;
+            };
+            unsigned turn = 0;
+            for (int d = 2; d <= ORB_OCT_D; d += 2) turn |= 3u << (2 * (ORB_OCT_D - d));
+            for (int l = 0; l < nlevels; l++) {
+                const LevelPlan& P = p.lv[l];
+                J.lv[l].octx = (const unsigned short*)(d_mem + o_oct) + t;
+                for (int x = 0, r = 0, rend = 0; x < P.w;) {
+                    // roots by (int)(x / hX), the last one to the end
+                    if (x >= rend) {
+                        r = std::min((int)((float)x / P.hX), P.nIni - 1);
+                        rend = r == P.nIni - 1 ? P.w : std::max(x + 1, P.root_x[r + 1] - 1);
+                        while (rend < P.w && std::min((int)((float)rend / P.hX), P.nIni - 1) == r) rend++;
+                    }
+                    int next = rend;
+                    const unsigned v = ((unsigned)r << (2 * ORB_OCT_D)) ^ turn ^
+                                       halve(P.root_x[r], P.root_x[r + 1], x, 0, &next);
+                    for (; x < next; x++) tab[t++] = (unsigned short)v;
+                }
+                J.lv[l].octy = (const unsigned short*)(d_mem + o_oct) + t;
+                for (int y = 0; y < P.h;) {
+                    int next = P.h;
+                    const unsigned v = halve(0, P.maxBorderY - ORB_MIN_BORDER, y, 1, &next);
+                    for (; y < next; y++) tab[t++] = (unsigned short)v;
+                }
+            }
+            HIP_TRY(hipMemcpy(d_mem + o_tab, tables.data(), tables.size(), hipMemcpyHostToDevice));
         }
         d_uR = (float*)(d_mem + o_uR);
         d_depth = (float*)(d_mem + o_dep);

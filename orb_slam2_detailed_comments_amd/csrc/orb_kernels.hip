@@ -159,8 +159,8 @@ __device__ __forceinline__ int lanes_below(unsigned long long mask)
 //   4. per-cell non-max suppression at iniThFAST and at minThFAST: a neighbour
 //      counts only if it lies in the same 30-px cell's detection area, which is
 //      exactly cv::FAST run on that cell's window (ORBextractor.cc:1075-1142);
-//   5. candidates of both thresholds appended to the level's key list, and a
-//      per-cell flag set when the cell has an iniThFAST survivor.  The quadtree
+//   5. candidates of either threshold appended to the level's key list (one
+//      entry says which), and a per-cell flag set when the cell has an iniThFAST survivor.  The quadtree
 //      kernel keeps minThFAST candidates only for cells without that flag,
 //      which is the reference's per-cell retry.
 #define LT_W ORB_TILE_W
@@ -313,7 +313,7 @@ union LevelScratch {
     uint4 hs[TH + 6][LT_W / 4];
     struct {
         unsigned short queue[(TH + 2) * (LT_W + 2)];
-        unsigned kloc[LK_CAP];       // tile-local candidate: ly | lx | score | retry
+        unsigned kloc[LK_CAP];       // tile-local candidate: ly | lx | score | passes
     } f;
 };
 
@@ -842,26 +842,22 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
             loc = ((unsigned)ly << 6) | (unsigned)lx | ((unsigned)mc << 11);
             if (keepA) gstore1(L.cellflag + (rowv & 0xFFFF) * L.nCols + (colv & 0xFFFF), 1);
         }
-        // Append (A entry, then B entry, per lane): the wave's exclusive
-        // prefix from two ballots, one LDS atomic per wave.
-        const unsigned long long ba = __ballot(keepA), bb = __ballot(keepB);
-        const int tot = __popcll(ba) + __popcll(bb);
-        if (tot) {
+        // Append, one entry for both passes: the wave's prefix from a ballot,
+        // one LDS atomic per wave.
+        const bool keep = keepA || keepB;
+        const unsigned long long bal = __ballot(keep);
+        if (bal) {
             int base = 0;
-            if (lane == 0) base = atomicAdd(&s_kn, tot);
+            if (lane == 0) base = atomicAdd(&s_kn, __popcll(bal));
             base = __builtin_amdgcn_readfirstlane(base);     // every lane is active here
-            int pos = base + lanes_below(ba) + lanes_below(bb);
-            if (keepA) {
-                if (pos < LK_CAP) u.f.kloc[pos] = loc;
-                pos++;
-            }
-            if (keepB && pos < LK_CAP) u.f.kloc[pos] = loc | (1u << 19);
+            const int pos = base + lanes_below(bal);
+            if (keep && pos < LK_CAP) u.f.kloc[pos] = loc | (keepA ? 1u << 19 : 0u) | (keepB ? 1u << 20 : 0u);
         }
     }
     __syncthreads();
 
     // ---- 5. append the tile's candidates to the level list as
-    // (score << 32 | cell row, cell col, y, x in cell) [| retry]
+    // (score << 32 | cell row, cell col, y, x in cell) | passes
     const int kn = s_kn;
     if (kn == 0) return;
     if (tid == 0) {
@@ -880,7 +876,7 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
         const unsigned yl = (unsigned)(y - (ORB_MIN_BORDER + ci * L.hCell));
         const unsigned ok = ((unsigned)ci << 20) | ((unsigned)cj << 12) | (yl << 6) | xl;
         unsigned long long key = ((unsigned long long)(unsigned)(mc - 1) << 32) | ok;
-        if (loc & (1u << 19)) key |= ORB_KEY_RETRY;
+        key |= (unsigned long long)((loc >> 19) & 3u) << 40;         // ORB_KEY_INI, ORB_KEY_MIN
         gstore8(L.keys + base + i, key);
     }
 }
@@ -892,15 +888,23 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
 // splitting every node with more than one key and pushing its non-empty
 // children to the list front (n1..n4, so they read n4,n3,n2,n1); phase 2
 // sorts the expandable nodes by (size, address) and splits from the largest
-// until the quota is reached.  Here the list is an array in LDS that is
-// rebuilt each pass with prefix sums; each candidate carries the index of the
-// list node that holds it.  Node order, membership and retained keys are
-// exactly the list's.  Ties in the phase-2 sort are broken by creation order
+// until the quota is reached.  Here the list is an array in LDS; each candidate
+// carries the index of the list node that holds it.  octree_fast finds the
+// list at the end of phase 1 at once; octree_general, for the candidate sets
+// it does not reach, rebuilds the list each pass with prefix sums.  Node
+// order, membership and retained keys are exactly the list's.  Ties in the phase-2 sort are broken by creation order
 // (newer = larger), the oracle's fixed stand-in for the heap address.
 #define OCT_T 1024
-#define OCT_REG 4                    // candidates per thread held in registers
+#define OCT_REG 4                    // general form: candidates per thread held in registers
+#define OCT_D ORB_OCT_D
+#define OCT_KEYS 8192                // fast form: candidates held in LDS (the others in global memory)
+#define OCT_CELLS 2048               // fast form: cells of the depth that ends phase 1
+#define OCT_FLAGS 4096               // fast form: FAST cells whose flags are held in LDS
+// Words of the occupancy bitmaps of depths OCT_D .. 0 for n roots, one after
+// another: n * 4^d cells at depth d.
+#define OCT_WORDS(n) (170 * (n) + ((n) + 1) / 2 + ((n) + 7) / 8 + 1)
 
-struct OctShared {
+struct OctGeneral {
     int rx[2][ORB_LIST_CAP];     // x0 | x1 << 16
     int ry[2][ORB_LIST_CAP];     // y0 | y1 << 16
     int cnt[2][ORB_LIST_CAP];
@@ -910,37 +914,81 @@ struct OctShared {
     short keep[ORB_LIST_CAP];
     unsigned long long sortk[ORB_LIST_CAP];
     unsigned long long best[ORB_LIST_CAP];
-    int scan[OCT_T / 64 + 1];
+    int scan[2][OCT_T / 64];
     int vars[8];
 };
 
-__device__ __forceinline__ int block_scan(int v, int* sh, int* total)
+struct OctFast {
+    unsigned key[OCT_KEYS];      // place at depth OCT_D | list node << 16
+    union {
+        unsigned bm[2][OCT_WORDS(ORB_MAX_ROOTS)];   // occupied cells; cells of two or more keys
+        struct {
+            int4 cc[ORB_LIST_CAP];       // keys per quadrant of a node
+            unsigned at[ORB_LIST_CAP];   // where the round puts a node or its children
+        };
+    };
+    union {
+        int cell[OCT_CELLS];     // list node of each cell of the depth that ends phase 1
+        unsigned long long best[ORB_LIST_CAP];
+    };
+    union {
+        uint8_t flag[OCT_FLAGS];
+        unsigned sortk[ORB_LIST_CAP];
+    };
+    unsigned short order[ORB_LIST_CAP];
+    unsigned done[ORB_LIST_CAP / 32];   // nodes split in this round
+    int scan[2][OCT_T / 64];
+    int na[OCT_D + 1], nm[OCT_D + 1];   // set bits per depth
+    int nkeys, nexp, end, deep, p1, size, cp;
+};
+
+// First word of depth d's bitmap (n roots).
+__device__ __forceinline__ int oct_word0(int d, int n)
 {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    int x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) sh[wid] = x;
+    const int w = d == 6 ? 0 : (d == 5 ? 128 : (d == 4 ? 160 : (d == 3 ? 168 : 170)));
+    return w * n + (d < 2 ? (n + 1) / 2 : 0) + (d < 1 ? (n + 7) / 8 : 0);
+}
+
+// LDS written by this wavefront is read by its other lanes next.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Inclusive scan over the wavefront by DPP (rows of 16, then the row totals).
+__device__ __forceinline__ int wave_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);   // row_bcast:15 to rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);   // row_bcast:31 to rows 2 and 3
+    return v;
+}
+
+// Exclusive scan over the workgroup, and the total: one barrier.  Two scans
+// in a row use the two halves of sh in turn (`half`), so that a scan's writes
+// never meet the reads of the one before.
+__device__ __forceinline__ int block_scan(int v, int (*sh)[OCT_T / 64], int& half, int* total)
+{
+    static_assert(OCT_T / 64 == 16, "a row of 16 lanes scans the wavefronts' totals");
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x = wave_scan(v);
+    int* h = sh[half];
+    half ^= 1;
+    if (lane == 63) h[wid] = x;
     __syncthreads();
-    if (wid == 0) {
-        const int wsum = lane < OCT_T / 64 ? sh[lane] : 0;
-        int s = wsum;
-#pragma unroll
-        for (int o = 1; o < OCT_T / 64; o <<= 1) {
-            const int y = __shfl_up(s, o, 64);
-            if (lane >= o) s += y;
-        }
-        if (lane < OCT_T / 64) sh[lane] = s - wsum;
-        if (lane == OCT_T / 64 - 1) sh[OCT_T / 64] = s;
-    }
-    __syncthreads();
-    const int r = x - v + sh[wid];
-    *total = sh[OCT_T / 64];
-    __syncthreads();
-    return r;
+    int t = h[lane & 15];
+    t += __builtin_amdgcn_update_dpp(0, t, 0x111, 0xF, 0xF, false);
+    t += __builtin_amdgcn_update_dpp(0, t, 0x112, 0xF, 0xF, false);
+    t += __builtin_amdgcn_update_dpp(0, t, 0x114, 0xF, 0xF, false);
+    t += __builtin_amdgcn_update_dpp(0, t, 0x118, 0xF, 0xF, false);
+    *total = __builtin_amdgcn_readlane(t, 15);
+    const int below = wid > 0 ? __builtin_amdgcn_readlane(t, wid > 0 ? wid - 1 : 0) : 0;
+    return below + x - v;
 }
 
 __device__ __forceinline__ void key_xy(unsigned long long key, int wCell, int hCell, int* x, int* y)
@@ -968,20 +1016,328 @@ __device__ __forceinline__ void child_rect(int rx, int ry, int q, int* crx, int*
     *cry = cy0 | (cy1 << 16);
 }
 
-__global__ __launch_bounds__(OCT_T, 8) void octree_kernel(const ImageJob* __restrict__ jobs, int max_levels)
+// The fast form.  A key's path through the quadtree depends on its position
+// alone, so all of phase 1 can be found at once:
+//   - A cell's place among its depth's cells in list order is a number that
+//     follows from its path: a pass pushes the children of the nodes it
+//     visits in list order to the front, so with o_0 = root and M_d = roots *
+//     4^d, o_d = M_d - 1 - (4 o_{d-1} + quadrant): the quadrants' digits, every
+//     other one turned around.  A key's place at depth OCT_D comes from two
+//     tables (its x and its y); its places above are shifts of that.
+//   - Every key marks its depth-OCT_D cell in a bitmap, and in a second one
+//     if the cell was marked; the shallower depths' bitmaps follow by nibbles.
+//     The list after pass p has as many nodes as depth p has occupied cells,
+//     and as many to expand as cells of two or more keys: that decides the
+//     pass p1 that ends phase 1.
+//   - Its list is the depth-p1 cells by o_p1, then the single-key cells of
+//     depth p1 - 1 whose parent was split, by their o, and so on to the
+//     roots: marking every cell's node in that order and counting the marks
+//     below it numbers the nodes, per cell of depth p1, not per key.
+// Phase 2 then needs only the keys per quadrant of each node: the nodes it
+// may split are those of the last pass, all of one depth, and the reference's
+// (size, newest first) order among them is (size, list position).
+// Returns false where it does not reach: phase 1 beyond depth OCT_D - 1 or
+// OCT_CELLS cells, a split of a depth-OCT_D cell (candidates in small
+// clusters).
+// Bound: latency (barriers, LDS round trips, and 16 cycles an instruction
+// where all 16 wavefronts run it).  640x480 with 1000 features 14.5 us (27 pass
+// by pass), 1280x720 with 2000 25 us (55), 128 images of 1241x376 63 us (105),
+// 64 of four sizes 43 us (95).
+__device__ __forceinline__ bool octree_fast(OctFast& S, const LevelJob& L, int level, int* ctr)
 {
-    __shared__ OctShared S;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int K0 = min(ctr[ORB_CNT_KEYS + level], L.key_cap);
+    const int N = L.quota, n = L.nIni, nCols = L.nCols, ncells = L.ncells;
+    const int wC = L.wCell, hC = L.hCell;
+    const int nwords = OCT_WORDS(n);
+    int half = 0;
+    // A candidate's place | node << 16: in LDS, or in global memory past OCT_KEYS.
+    auto put = [&](int k, unsigned v) {
+        if (k < OCT_KEYS) S.key[k] = v;
+        else gstore4((uint8_t*)(L.node + k), v);
+    };
+    auto get = [&](int k) { return k < OCT_KEYS ? S.key[k] : gload4((const uint8_t*)(L.node + k)); };
+
+    // ---- the per-cell retry (ORBextractor.cc:1111-1124): a cell keeps its
+    // iniThFAST candidates when it has any, else its minThFAST candidates.
+    // The survivors' places go to LDS, the survivors to keys2 (in any order:
+    // the level kernels append them in none, and the result depends on the
+    // set alone).
+    unsigned long long key[4];
+#pragma unroll
+    for (int m = 0; m < 4; m++) key[m] = gload8u64(L.keys + min(tid + OCT_T * m, max(K0 - 1, 0)));
+    const bool lds_flags = ncells <= OCT_FLAGS;
+    if (lds_flags)
+        for (int i = tid; i < ncells; i += OCT_T) S.flag[i] = gload1(L.cellflag + i);
+    for (int i = tid; i < nwords; i += OCT_T) S.bm[0][i] = S.bm[1][i] = 0u;
+    if (tid <= OCT_D) S.na[tid] = S.nm[tid] = 0;
+    if (tid == 0) S.nkeys = S.deep = 0;
+    __syncthreads();
+    for (int c0 = 0; c0 < K0; c0 += 4 * OCT_T) {
+        unsigned o[4];
+        unsigned long long k[4];
+        int cnt = 0;
+        bool v[4];
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            k[m] = key[m];
+            const unsigned ok = (unsigned)k[m];
+            const unsigned xl = ok & 63, yl = (ok >> 6) & 63, j = (ok >> 12) & 255, i = (ok >> 20) & 255;
+            o[m] = (unsigned)(L.octx[__umul24(j, wC) + xl] ^ L.octy[__umul24(i, hC) + yl]);
+            const unsigned c = __umul24(i, nCols) + j;
+            const int f = lds_flags ? S.flag[c] : gload1(L.cellflag + c);
+            v[m] = c0 + tid + OCT_T * m < K0 && (k[m] & (f ? ORB_KEY_INI : ORB_KEY_MIN));
+            cnt += v[m] ? 1 : 0;
+        }
+        if (c0 + 4 * OCT_T < K0) {
+#pragma unroll
+            for (int m = 0; m < 4; m++) key[m] = gload8u64(L.keys + min(c0 + 4 * OCT_T + tid + OCT_T * m, K0 - 1));
+        }
+        const int inc = wave_scan(cnt);
+        int base = 0;
+        if (lane == 63 && inc) base = atomicAdd(&S.nkeys, inc);
+        int pos = __builtin_amdgcn_readlane(base, 63) + inc - cnt;
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+            if (v[m]) {
+                put(pos, o[m]);
+                gstore8(L.keys2 + pos++, k[m] & ORB_KEY_RANK);
+                const unsigned bit = 1u << (o[m] & 31);
+                if (atomicOr(&S.bm[0][o[m] >> 5], bit) & bit) atomicOr(&S.bm[1][o[m] >> 5], bit);
+            }
+    }
+    __syncthreads();
+    const int K = S.nkeys;
+
+    // ---- occupancy of the shallower depths: cell o's children are nibble
+    // M - 1 - o of the next depth
+    auto reduce = [&](int d, int o) {
+        const int M = n << (2 * d), w0 = oct_word0(d, n), wc = oct_word0(d + 1, n);
+        bool occ = false, multi = false;
+        if (o < M) {
+            const int c = M - 1 - o;
+            const unsigned ca = (S.bm[0][wc + (c >> 3)] >> (4 * (c & 7))) & 15u;
+            const unsigned cm = (S.bm[1][wc + (c >> 3)] >> (4 * (c & 7))) & 15u;
+            occ = ca != 0;
+            multi = cm != 0 || (ca & (ca - 1)) != 0;
+        }
+        const unsigned long long ba = __ballot(occ), bb = __ballot(multi);
+        const int w = (o >> 5) & ~1;             // the wavefront's two words
+        if (lane < 2 && 32 * (w + lane) < M) {
+            S.bm[0][w0 + w + lane] = (unsigned)(ba >> (32 * lane));
+            S.bm[1][w0 + w + lane] = (unsigned)(bb >> (32 * lane));
+        }
+        if (lane == 0 && ba) {
+            atomicAdd(&S.na[d], __popcll(ba));
+            atomicAdd(&S.nm[d], __popcll(bb));
+        }
+    };
+    for (int o = tid; o - lane < n << 10; o += OCT_T) reduce(5, o);
+    __syncthreads();
+    for (int o = tid; o - lane < n << 8; o += OCT_T) reduce(4, o);
+    __syncthreads();
+    if (wv == 0) {                               // the others wait at the barrier below
+        for (int d = 3; d >= 0; d--) {
+            for (int o = lane; o - lane < n << (2 * d); o += 64) reduce(d, o);
+            wave_lds_sync();
+        }
+        // the pass that ends phase 1 (ORBextractor.cc:779-893), lane p = pass p
+        const int p = min(lane, OCT_D), size = S.na[p], prev = S.na[max(p - 1, 0)], nexp = S.nm[p];
+        const bool last = size >= N || size == prev;
+        const unsigned long long ends = __ballot(lane >= 1 && lane < OCT_D &&
+                                                 (last || size + 3 * nexp > N || size > ORB_LIST_CAP));
+        const int p1 = ends ? __ffsll((long long)ends) - 1 : 0;
+        if (lane == p1) {
+            S.p1 = p1;
+            S.size = size;
+            S.end = last ? 1 : 0;
+        }
+    }
+    __syncthreads();
+    const int p1 = S.p1;
+    int size = S.size;
+    const int M = n << (2 * p1);
+    if (p1 == 0 || M > OCT_CELLS || size > ORB_LIST_CAP) return false;
+    bool more = !S.end;
+
+    // ---- the list after pass p1: every occupied depth-p1 cell's node, the
+    // shallowest cell of one key above it or the cell itself, as depth << 17 |
+    // place.  Cells are numbered as shifts of the depth-OCT_D place: the place
+    // at depth p1, turned around where OCT_D - p1 is odd.
+    const int sh = 2 * (OCT_D - p1);
+    const bool turn = p1 & 1;
+    const int wfirst = oct_word0(p1, n), nw = nwords - wfirst;
+    for (int c = tid; c < M; c += OCT_T) {
+        int o = turn ? M - 1 - c : c, nd = -1;
+        if ((S.bm[0][wfirst + (o >> 5)] >> (o & 31)) & 1u) {
+            nd = (p1 << 17) | o;
+            for (int d = p1 - 1; d >= 0; d--) {
+                o = ((n << (2 * (d + 1))) - 1 - o) >> 2;
+                if (!((S.bm[1][oct_word0(d, n) + (o >> 5)] >> (o & 31)) & 1u)) nd = (d << 17) | o;
+            }
+        }
+        S.cell[c] = nd;
+    }
+    __syncthreads();
+    for (int i = tid; i < nw; i += OCT_T) S.bm[0][wfirst + i] = 0u;
+    __syncthreads();
+    for (int c = tid; c < M; c += OCT_T) {
+        const int nd = S.cell[c], o = nd & 0x1FFFF;
+        if (nd >= 0) atomicOr(&S.bm[0][oct_word0(nd >> 17, n) + (o >> 5)], 1u << (o & 31));
+    }
+    __syncthreads();
+    if (wv == 0) {                               // marks below each word
+        int run = 0;
+        for (int i0 = 0; i0 < nw; i0 += 64) {
+            const int c = i0 + lane < nw ? __popc(S.bm[0][wfirst + i0 + lane]) : 0;
+            const int inc = wave_scan(c);
+            if (i0 + lane < nw) S.bm[1][wfirst + i0 + lane] = (unsigned)(run + inc - c);
+            run += __builtin_amdgcn_readlane(inc, 63);
+        }
+    }
+    __syncthreads();
+    for (int c = tid; c < M; c += OCT_T) {
+        const int nd = S.cell[c], o = nd & 0x1FFFF;
+        if (nd >= 0) {
+            const int w = oct_word0(nd >> 17, n) + (o >> 5);
+            S.cell[c] = (int)S.bm[1][w] + __popc(S.bm[0][w] & ((1u << (o & 31)) - 1u));
+        }
+    }
+    __syncthreads();
+    // each key's node, and (for phase 2) the keys per quadrant of the nodes
+    // the last pass made; the bitmaps make way for the counts
+    if (tid < size) S.cc[tid] = make_int4(0, 0, 0, 0);
+    __syncthreads();
+    // quadrant of a key's depth-d cell in its parent: its digit, turned around at even depths
+    auto quadrant = [](unsigned place, int d) {
+        return (int)((place >> (2 * (OCT_D - d))) & 3u) ^ (d & 1 ? 0 : 3);
+    };
+#pragma unroll 2
+    for (int k = tid; k < K; k += OCT_T) {
+        const unsigned place = get(k);
+        const int nd = S.cell[place >> sh];
+        put(k, place | ((unsigned)nd << 16));
+        if (more) atomicAdd((int*)&S.cc[nd] + quadrant(place, p1 + 1), 1);
+    }
+    __syncthreads();
+
+    // ---- phase 2 (:908-991): split the largest nodes until the quota.  At
+    // round r every node of two or more keys has depth p1 + r; every round
+    // that does not end the loop grows the list, which holds at most
+    // ORB_LIST_CAP nodes.
+    for (int depth = p1; more; depth++) {
+        // the nodes to expand, keyed by (keys, list position)
+        int4 c4 = make_int4(0, 0, 0, 0);
+        if (tid < size) c4 = S.cc[tid];
+        const int cnt = c4.x + c4.y + c4.z + c4.w;
+        if (tid == 0) S.nexp = 0;
+        if (tid < ORB_LIST_CAP / 32) S.done[tid] = 0u;
+        __syncthreads();
+        {
+            const unsigned long long b = __ballot(cnt >= 2);
+            int base = 0;
+            if (lane == 0 && b) base = atomicAdd(&S.nexp, __popcll(b));
+            base = __builtin_amdgcn_readfirstlane(base);
+            if (cnt >= 2) S.sortk[base + lanes_below(b)] = ((unsigned)cnt << 10) | (unsigned)(ORB_LIST_CAP - 1 - tid);
+        }
+        __syncthreads();
+        const int nE = S.nexp;
+        {
+            // a key's place in descending order is the number of larger keys;
+            // up to 16 lanes share its comparisons
+            int lg = 0;
+            while (lg < 4 && (nE << (lg + 1)) <= OCT_T) lg++;
+            const int i = tid >> lg, step = 1 << lg;
+            if (i - (lane >> lg) < nE) {
+                const unsigned mine = i < nE ? S.sortk[i] : 0u;
+                int rank = 0;
+                for (int j = tid & (step - 1); j < nE; j += step) rank += S.sortk[j] > mine ? 1 : 0;
+                for (int o = 1; o < step; o <<= 1) rank += __shfl_xor(rank, o, 64);
+                if (i < nE && (tid & (step - 1)) == 0)
+                    S.order[rank] = (unsigned short)(ORB_LIST_CAP - 1 - (mine & (ORB_LIST_CAP - 1)));
+            }
+        }
+        __syncthreads();
+        // gains in processing order, and the first split that reaches the quota
+        const int j = tid;
+        int nd = 0, nc = 0;
+        unsigned occ = 0;
+        int4 q4 = make_int4(0, 0, 0, 0);
+        if (j < nE) {
+            nd = S.order[j];
+            q4 = S.cc[nd];
+            occ = (q4.x > 0 ? 1u : 0u) | (q4.y > 0 ? 2u : 0u) | (q4.z > 0 ? 4u : 0u) | (q4.w > 0 ? 8u : 0u);
+            nc = __popc(occ);
+        }
+        int all;
+        const int ex = block_scan(j < nE ? nc - 1 : 0, S.scan, half, &all);
+        const int jstar = min(__syncthreads_count(j < nE && size + ex + nc - 1 < N), nE - 1);
+        const bool proc = j <= jstar;
+        if (proc) {
+            atomicOr(&S.done[nd >> 5], 1u << (nd & 31));
+            if (j == jstar) S.cp = ex + nc + j;  // children of the nodes 0 .. jstar
+        }
+        __syncthreads();
+        const int cp = nE > 0 ? S.cp : 0, nsize = cp + size - (jstar + 1);
+        if (nsize > ORB_LIST_CAP) return false;  // the general form reports it
+        more = nsize < N && nsize != size;
+        if (proc) {                              // children in front, the last quadrant first
+            S.at[nd] = (unsigned)(cp - (ex + j) - nc) | (occ << 16) | 0x80000000u;
+            if (depth + 1 == OCT_D && max(max(q4.x, q4.y), max(q4.z, q4.w)) >= 2) S.deep = 1;
+        }
+        {
+            // kept nodes follow in list order
+            const int w = lane < ORB_LIST_CAP / 32 ? (int)S.done[lane] : 0;
+            const int below = wave_scan(__popc(w)) - __popc(w);
+            const int mw = tid >> 5;
+            const int pre = __shfl(below, mw, 64), bits = __shfl(w, mw, 64);
+            if (tid < size && !((bits >> (tid & 31)) & 1))
+                S.at[tid] = (unsigned)(cp + tid - pre - __popc((unsigned)bits & ((1u << (tid & 31)) - 1u)));
+        }
+        __syncthreads();
+        if (more && S.deep) return false;
+        size = nsize;
+        if (more) {
+            if (tid < size) S.cc[tid] = make_int4(0, 0, 0, 0);
+            __syncthreads();
+        }
+        for (int k = tid; k < K; k += OCT_T) {
+            const unsigned v = get(k), place = v & 0xFFFFu, at = S.at[v >> 16];
+            const int pos = (int)(at & 0xFFFFu) +
+                            (at >> 31 ? __popc(((at >> 16) & 15u) >> (quadrant(place, depth + 1) + 1)) : 0);
+            put(k, place | ((unsigned)pos << 16));
+            if (more) atomicAdd((int*)&S.cc[pos] + quadrant(place, depth + 2), 1);
+        }
+        __syncthreads();
+    }
+
+    // ---- retain the best response per node; first in key order on ties
+    if (tid < size) S.best[tid] = 0ull;
+    __syncthreads();
+#pragma unroll 4
+    for (int k = tid; k < K; k += OCT_T) {
+        const unsigned long long kk = gload8u64(L.keys2 + k);
+        atomicMax(&S.best[get(k) >> 16], (kk & 0xFFFFFFFF00000000ull) | (0xFFFFFFFFull - (kk & 0xFFFFFFFFull)));
+    }
+    __syncthreads();
+    if (size > min(L.list_cap, ORB_LIST_CAP)) return false;   // the general form reports it
+    if (tid < size) {
+        const unsigned long long b = S.best[tid];
+        gstore8(L.ret + tid, (b & 0xFFFFFFFF00000000ull) | (0xFFFFFFFFull - (b & 0xFFFFFFFFull)));
+    }
+    if (tid == 0) ctr[ORB_CNT_RET + level] = size;
+    return true;
+}
+
+// The general form: any candidate set, pass by pass.
+__device__ __forceinline__ void octree_general(OctGeneral& S, const LevelJob& L, int level, int* ctr)
+{
     const int tid = threadIdx.x;
-    const int jb = blockIdx.x / max_levels, level = blockIdx.x % max_levels;
-    const ImageJob& J = jobs[jb];
-    if (level >= J.nlevels) return;
-    const LevelJob& L = J.lv[level];
-    int* ctr = J.counters;
     const int K0 = min(ctr[ORB_CNT_KEYS + level], L.key_cap);
     const int N = L.quota;
     const int wC = L.wCell, hC = L.hCell;
     int* node = L.node;
-    int total;
+    int total, half = 0;
 
     // ---- per-cell retry (ORBextractor.cc:1111-1124): a cell keeps its
     // iniThFAST candidates when it has any, else its minThFAST candidates.
@@ -1004,13 +1360,13 @@ __global__ __launch_bounds__(OCT_T, 8) void octree_kernel(const ImageJob* __rest
         bool v[OCT_REG];
 #pragma unroll
         for (int m = 0; m < OCT_REG; m++) {
-            v[m] = c0 + tid + OCT_T * m < K0 && ((key[m] & ORB_KEY_RETRY) ? flag[m] == 0 : flag[m] != 0);
+            v[m] = c0 + tid + OCT_T * m < K0 && (key[m] & (flag[m] ? ORB_KEY_INI : ORB_KEY_MIN));
             cnt += v[m] ? 1 : 0;
         }
-        int pos = block_scan(cnt, S.scan, &total);
+        int pos = block_scan(cnt, S.scan, half, &total);
 #pragma unroll
         for (int m = 0; m < OCT_REG; m++)
-            if (v[m]) gstore8(L.keys2 + K + pos++, key[m] & ~ORB_KEY_RETRY);
+            if (v[m]) gstore8(L.keys2 + K + pos++, key[m] & ORB_KEY_RANK);
         K += total;
     }
     __syncthreads();
@@ -1054,7 +1410,7 @@ __global__ __launch_bounds__(OCT_T, 8) void octree_kernel(const ImageJob* __rest
     __syncthreads();
     {
         const int c = tid < L.nIni ? S.cc[tid][0] : 0;
-        const int pos = block_scan(c > 0 ? 1 : 0, S.scan, &total);
+        const int pos = block_scan(c > 0 ? 1 : 0, S.scan, half, &total);
         if (tid < L.nIni && c > 0) {
             S.rx[0][pos] = L.root_x[tid] | (L.root_x[tid + 1] << 16);
             S.ry[0][pos] = 0 | ((L.maxBorderY - ORB_MIN_BORDER) << 16);
@@ -1093,8 +1449,8 @@ __global__ __launch_bounds__(OCT_T, 8) void octree_kernel(const ImageJob* __rest
         if (split) nc = (S.cc[i][0] > 0) + (S.cc[i][1] > 0) + (S.cc[i][2] > 0) + (S.cc[i][3] > 0);
         const int kp = (i < size && !split) ? 1 : 0;
         int C, nkeep;
-        const int ex_nc = block_scan(nc, S.scan, &C);
-        const int ex_kp = block_scan(kp, S.scan, &nkeep);
+        const int ex_nc = block_scan(nc, S.scan, half, &C);
+        const int ex_kp = block_scan(kp, S.scan, half, &nkeep);
         const int nsize = C + nkeep;
         int nexp = 0;
         if (nsize <= ORB_LIST_CAP) {
@@ -1128,7 +1484,7 @@ __global__ __launch_bounds__(OCT_T, 8) void octree_kernel(const ImageJob* __rest
             }
         }
         int nToExpand;
-        block_scan(nexp, S.scan, &nToExpand);
+        block_scan(nexp, S.scan, half, &nToExpand);
         if (nsize > ORB_LIST_CAP) {
             if (tid == 0) atomicOr(&ctr[ORB_CNT_ERR], ORB_ERR_LIST);
             size = 0;
@@ -1166,22 +1522,29 @@ __global__ __launch_bounds__(OCT_T, 8) void octree_kernel(const ImageJob* __rest
         // Expandable nodes, sorted by (size, creation order), largest first.
         const bool e = tid < size && S.cnt[cur][tid] >= 2;
         int nE;
-        const int ex_e = block_scan(e ? 1 : 0, S.scan, &nE);
+        const int ex_e = block_scan(e ? 1 : 0, S.scan, half, &nE);
         // The keys are distinct (they carry the node index), so a key's
-        // place in descending order is the number of larger keys; every
-        // thread reads the same key at a time (an LDS broadcast).  S.keep
+        // place in descending order is the number of larger keys.  S.keep
         // holds each node's place (32767: not expandable).
         if (e)
             S.sortk[ex_e] = ((unsigned long long)S.cnt[cur][tid] << 32) |
                             ((unsigned long long)(unsigned)S.seq[cur][tid] << 16) | (unsigned)tid;
         if (tid < size) S.keep[tid] = 32767;
         __syncthreads();
-        if (tid < nE) {
-            const unsigned long long mine = S.sortk[tid];
+        {
+            // up to 16 lanes share a key's comparisons
+            int lg = 0;
+            while (lg < 4 && (nE << (lg + 1)) <= OCT_T) lg++;
+            const int i = tid >> lg, step = 1 << lg;
+            const bool mine_ok = i < nE;
+            const unsigned long long mine = S.sortk[mine_ok ? i : 0];
             int rank = 0;
-            for (int j2 = 0; j2 < nE; j2++) rank += S.sortk[j2] > mine;
-            S.best[rank] = mine;                  // S.best is free until the retain step
-            S.keep[mine & 0xFFFF] = (short)rank;
+            for (int j2 = tid & (step - 1); j2 < nE; j2 += step) rank += S.sortk[j2] > mine;
+            for (int o2 = 1; o2 < step; o2 <<= 1) rank += __shfl_xor(rank, o2, 64);
+            if (mine_ok && (tid & (step - 1)) == 0) {
+                S.best[rank] = mine;             // S.best is free until the retain step
+                S.keep[mine & 0xFFFF] = (short)rank;
+            }
         }
         __syncthreads();
         // Gains in processing order and the first split reaching the quota.
@@ -1192,7 +1555,7 @@ __global__ __launch_bounds__(OCT_T, 8) void octree_kernel(const ImageJob* __rest
             nc = (S.cc[node_j][0] > 0) + (S.cc[node_j][1] > 0) + (S.cc[node_j][2] > 0) + (S.cc[node_j][3] > 0);
         }
         int gsum;
-        const int ex_g = block_scan(j < nE ? nc - 1 : 0, S.scan, &gsum);
+        const int ex_g = block_scan(j < nE ? nc - 1 : 0, S.scan, half, &gsum);
         if (tid == 0) S.vars[0] = nE - 1;
         __syncthreads();
         if (j < nE && size + ex_g + nc - 1 >= N) atomicMin(&S.vars[0], j);
@@ -1205,7 +1568,7 @@ __global__ __launch_bounds__(OCT_T, 8) void octree_kernel(const ImageJob* __rest
         static_assert(4 * ORB_LIST_CAP < (1 << 16) && ORB_LIST_CAP <= OCT_T, "octree list packing");
         const bool kp = tid < size && S.keep[tid] > jstar;
         int tot;
-        const int ex = block_scan((proc ? nc : 0) | ((kp ? 1 : 0) << 16), S.scan, &tot);
+        const int ex = block_scan((proc ? nc : 0) | ((kp ? 1 : 0) << 16), S.scan, half, &tot);
         const int ex_nc = ex & 0xFFFF, ex_kp = ex >> 16, Cp = tot & 0xFFFF, nkeep = tot >> 16;
         const int nsize = Cp + nkeep;
         if (nsize > ORB_LIST_CAP) {
@@ -1279,6 +1642,21 @@ __global__ __launch_bounds__(OCT_T, 8) void octree_kernel(const ImageJob* __rest
         gstore8(L.ret + i, (p & 0xFFFFFFFF00000000ull) | (0xFFFFFFFFull - (p & 0xFFFFFFFFull)));
     }
     if (tid == 0) ctr[ORB_CNT_RET + level] = size;
+}
+
+__global__ __launch_bounds__(OCT_T, 8) void octree_kernel(const ImageJob* __restrict__ jobs, int max_levels)
+{
+    __shared__ union {
+        OctFast f;
+        OctGeneral g;
+    } S;
+    const int jb = blockIdx.x / max_levels, level = blockIdx.x % max_levels;
+    const ImageJob& J = jobs[jb];
+    if (level >= J.nlevels) return;
+    const LevelJob& L = J.lv[level];
+    if (octree_fast(S.f, L, level, J.counters)) return;
+    __syncthreads();
+    octree_general(S.g, L, level, J.counters);
 }
 
 // ============================================================== describe

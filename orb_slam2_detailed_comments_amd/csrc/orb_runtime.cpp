@@ -451,7 +451,7 @@ int orb_extractor_debug_candidates(orb_extractor* ex, int level, int* xyr, int c
     for (unsigned long long key : all) {
         const unsigned ok = (unsigned)key;
         const bool flagged = flags[((ok >> 20) & 255) * L.nCols + ((ok >> 12) & 255)] != 0;
-        if ((key & ORB_KEY_RETRY) ? !flagged : flagged) keys.push_back(key & ~ORB_KEY_RETRY);
+        if (key & (flagged ? ORB_KEY_INI : ORB_KEY_MIN)) keys.push_back(key & ORB_KEY_RANK);
     }
     k = (int)keys.size();
     *n = k;

@@ -25,7 +25,10 @@
 #define ORB_CNT_MATCH (ORB_CNT_ERR + 1)      // stereo matches recorded
 #define ORB_CNT_SLOTS 64
 
-#define ORB_KEY_RETRY (1ull << 40)   // candidate from the minThFAST pass
+#define ORB_KEY_INI (1ull << 40)     // candidate of the iniThFAST pass
+#define ORB_KEY_MIN (1ull << 41)     // candidate of the minThFAST pass (mostly the same pixels and more)
+#define ORB_KEY_RANK ((1ull << 40) - 1)   // response and order key
+#define ORB_OCT_D 6                  // quadtree passes found at once
 
 #define ORB_ERR_KEYS 1        // candidate buffer overflow
 #define ORB_ERR_LIST 2        // quadtree list overflow
@@ -56,7 +59,7 @@ struct LevelJob {
     uint8_t* lvl;                    // level image
     uint8_t* blur;                   // 7x7 sigma-2 blur of the level
     uint8_t* cellflag;               // per FAST cell: has an iniThFAST survivor
-    unsigned long long* keys;        // candidates: response<<32 | order key
+    unsigned long long* keys;        // candidates: response<<32 | order key | passes
     unsigned long long* keys2;       // candidates after the per-cell retry
     int* node;                       // per-candidate quadtree node (scratch)
     unsigned long long* ret;         // kept keypoints in output order
@@ -64,6 +67,8 @@ struct LevelJob {
     const int2* ytab;                // resize from level-1; per row {sy, b0 | b1 << 16}
     const int2* xwin;                // levels >= 1: per tile column / row, the source
     const int2* ywin;                // columns / rows {first, last} the tile's taps read
+    const unsigned short* octx;      // quadtree place at depth ORB_OCT_D of a candidate at (x, y):
+    const unsigned short* octy;      // octx[x] ^ octy[y] (x, y relative to the border)
 };
 
 struct ImageJob {
