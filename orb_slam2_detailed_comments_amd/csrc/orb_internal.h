@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <new>
 #include <vector>
 
 #include "orb_gpu.h"
@@ -30,6 +31,7 @@ extern "C" hipError_t orb_launch_distinctive(const uint8_t* desc, const int* off
                                              int* best, uint8_t* out_desc, hipStream_t st);
 extern "C" hipError_t orb_launch_hbm_copy(const void* src, void* dst, size_t bytes, hipStream_t st);
 extern "C" hipError_t orb_launch_copy_ops(const CopyOp* d_ops, int nops, int blocks_per_op, hipStream_t st);
+extern "C" hipError_t orb_launch_copy_list(const CopyList* list, int blocks_per_op, hipStream_t st);
 extern "C" hipError_t orb_launch_undistort(const OrbKeyPoint* in, int n, const int* count, const double* K4,
                                            const double* k5, OrbKeyPoint* out, hipStream_t st);
 extern "C" hipError_t orb_launch_rgbd_depth(const OrbKeyPoint* kps, const OrbKeyPoint* kun, int n, const int* count,
@@ -247,8 +249,12 @@ struct orb_extractor {
     uint8_t* d_stage = nullptr;   // contiguous landing buffer for host frames
     ImageJob hjob{};
     ImageJob* d_job = nullptr;
-    RunTable* h_rt = nullptr;     // pinned
+    RunTable* h_rt = nullptr;
     RunTable* d_rt = nullptr;
+    // pinned landing buffer of a call's results, written by the device:
+    // counters, then six arrays of res_cap entries (res_at)
+    char* h_res = nullptr;
+    int res_cap = 0;
     // stereo state (this extractor as the left view)
     float* d_uR = nullptr;
     float* d_depth = nullptr;
@@ -600,7 +606,7 @@ struct orb_extractor {
         d_rows = (int2*)(d_mem + o_rows);
         if (!d_job && hipMalloc(&d_job, sizeof(ImageJob)) != hipSuccess) return ORB_E_OOM;
         if (!d_rt && hipMalloc(&d_rt, sizeof(RunTable)) != hipSuccess) return ORB_E_OOM;
-        if (!h_rt && hipHostMalloc(&h_rt, sizeof(RunTable)) != hipSuccess) return ORB_E_OOM;
+        if (!h_rt && !(h_rt = new (std::nothrow) RunTable())) return ORB_E_OOM;
         const orb_extractor* one[1] = {this};
         int rc_t = build_table(one, 1, *h_rt);
         if (rc_t) return rc_t;
@@ -683,24 +689,99 @@ struct orb_extractor {
         return c[ORB_CNT_ERR] ? ORB_E_OVERFLOW : ORB_OK;
     }
 
-    int read_results(orb_keypoint* kps, int cap, uint8_t* desc, int* n)
+    // The caller's arrays for a call's results (any may be null) and, for the
+    // outputs beside the extractor's own, where they are on the device.
+    struct Outputs {
+        orb_keypoint* kps = nullptr;
+        uint8_t* desc = nullptr;
+        orb_keypoint* kps_un = nullptr;
+        float* uRight = nullptr;
+        float* depth = nullptr;
+        const OrbKeyPoint* d_kun = nullptr;
+        const float* d_uR = nullptr;
+        const float* d_depth = nullptr;
+    };
+    struct OutArray {
+        void* to;
+        const void* from;
+        int words;                // per keypoint
+    };
+    static constexpr int kOutArrays = 5;
+    void out_arrays(const Outputs& o, OutArray (&a)[kOutArrays]) const
     {
-        int c[ORB_CNT_SLOTS];
-        HIP_TRY(hipMemcpyAsync(c, hjob.counters, sizeof(c), hipMemcpyDeviceToHost, ctx->stream));
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        const int kw = (int)(sizeof(OrbKeyPoint) / 4);
+        a[0] = {o.kps, hjob.kps, kw};
+        a[1] = {o.desc, hjob.desc, 8};
+        a[2] = {o.kps_un, o.d_kun, kw};
+        a[3] = {o.uRight, o.d_uR, 1};
+        a[4] = {o.depth, o.d_depth, 1};
+    }
+
+    // Adds the results to a copy list into the pinned buffer: the counters,
+    // and as many entries of each wanted array as the device counted.
+    int list_results(const Outputs& o, CopyList& l)
+    {
+        static_assert(2 * (1 + 2) + 2 <= ORB_COPY_LIST && 1 + kOutArrays <= ORB_COPY_LIST, "a stereo or an RGB-D frame");
+        if (hjob.out_cap > res_cap) {
+            const size_t cap = (size_t)(hjob.out_cap + 63) / 64 * 64;
+            if (h_res) (void)hipHostFree(h_res);          // its last copies have ended
+            h_res = nullptr;
+            res_cap = 0;
+            if (hipHostMalloc((void**)&h_res, res_at((int)cap, kOutArrays), hipHostMallocCoherent) != hipSuccess) {
+                h_res = nullptr;
+                return ORB_E_OOM;
+            }
+            res_cap = (int)cap;
+        }
+        OutArray a[kOutArrays];
+        out_arrays(o, a);
+        l.op[l.n++] = CopyOp{(const unsigned*)hjob.counters, (unsigned*)h_res, nullptr, ORB_CNT_SLOTS, 0};
+        for (int i = 0; i < kOutArrays; i++)
+            if (a[i].to)
+                l.op[l.n++] = CopyOp{(const unsigned*)a[i].from, (unsigned*)(h_res + res_at(res_cap, i)),
+                                     hjob.counters + ORB_CNT_NOUT, hjob.out_cap * a[i].words, a[i].words};
+        return ORB_OK;
+    }
+    // Offset of array i in the pinned buffer (of all: i = kOutArrays); cap is
+    // a multiple of 64, so every array starts 256-byte aligned.
+    static size_t res_at(int cap, int i)
+    {
+        constexpr int words[kOutArrays] = {(int)(sizeof(OrbKeyPoint) / 4), 8, (int)(sizeof(OrbKeyPoint) / 4), 1, 1};
+        size_t at = 256;
+        for (int k = 0; k < i; k++) at += (size_t)cap * words[k] * 4;
+        return at;
+    }
+    // After the copy list has run: the results into the caller's arrays.
+    int take_results(const Outputs& o, int cap, int* n) const
+    {
+        const int* c = (const int*)h_res;
         if (c[ORB_CNT_ERR]) return ORB_E_OVERFLOW;
         const int cnt = c[ORB_CNT_NOUT];
         *n = cnt;
         if (cnt > cap) return ORB_E_CAPACITY;
-        if (cnt > 0) {
-            if (kps)
-                HIP_TRY(hipMemcpyAsync(kps, hjob.kps, (size_t)cnt * sizeof(orb_keypoint), hipMemcpyDeviceToHost,
-                                       ctx->stream));
-            if (desc)
-                HIP_TRY(hipMemcpyAsync(desc, hjob.desc, (size_t)cnt * 32, hipMemcpyDeviceToHost, ctx->stream));
-            HIP_TRY(hipStreamSynchronize(ctx->stream));
-        }
+        OutArray a[kOutArrays];
+        out_arrays(o, a);
+        for (int i = 0; i < kOutArrays; i++)
+            if (a[i].to && cnt > 0) std::memcpy(a[i].to, h_res + res_at(res_cap, i), (size_t)cnt * a[i].words * 4);
         return ORB_OK;
+    }
+
+    int read_results(const Outputs& o, int cap, int* n)
+    {
+        CopyList l;
+        l.n = 0;
+        const int rc = list_results(o, l);
+        if (rc) return rc;
+        HIP_TRY(orb_launch_copy_list(&l, ORB_COPY_BLOCKS, ctx->stream));
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        return take_results(o, cap, n);
+    }
+    int read_results(orb_keypoint* kps, int cap, uint8_t* desc, int* n)
+    {
+        Outputs o;
+        o.kps = kps;
+        o.desc = desc;
+        return read_results(o, cap, n);
     }
 
     // Two-view run table (left = this, right = r) for the stereo frame.
@@ -709,7 +790,7 @@ struct orb_extractor {
         if (pair_right == r && pair_gen_l == gen && pair_gen_r == r->gen) return ORB_OK;
         if (!d_pair_jobs && hipMalloc(&d_pair_jobs, 2 * sizeof(ImageJob)) != hipSuccess) return ORB_E_OOM;
         if (!d_pair_rt && hipMalloc(&d_pair_rt, sizeof(RunTable)) != hipSuccess) return ORB_E_OOM;
-        if (!h_pair_rt && hipHostMalloc(&h_pair_rt, sizeof(RunTable)) != hipSuccess) return ORB_E_OOM;
+        if (!h_pair_rt && !(h_pair_rt = new (std::nothrow) RunTable())) return ORB_E_OOM;
         const orb_extractor* two[2] = {this, r};
         const int rc_t = build_table(two, 2, *h_pair_rt);
         if (rc_t) return rc_t;
@@ -764,12 +845,13 @@ struct orb_extractor {
         if (d_mem) (void)hipFree(d_mem);
         if (d_job) (void)hipFree(d_job);
         if (d_rt) (void)hipFree(d_rt);
-        if (h_rt) (void)hipHostFree(h_rt);
+        delete h_rt;
+        if (h_res) (void)hipHostFree(h_res);
         if (d_kin) (void)hipFree(d_kin);
         if (d_din) (void)hipFree(d_din);
         if (d_pair_jobs) (void)hipFree(d_pair_jobs);
         if (d_pair_rt) (void)hipFree(d_pair_rt);
-        if (h_pair_rt) (void)hipHostFree(h_pair_rt);
+        delete h_pair_rt;
         if (d_sargs) (void)hipFree(d_sargs);
     }
 };

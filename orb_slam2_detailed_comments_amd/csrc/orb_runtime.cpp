@@ -398,16 +398,25 @@ int orb_stereo_frame(orb_extractor* left, orb_extractor* right, const uint8_t* i
     rc = left->upload_stereo_args(0, a);
     if (rc) return rc;
     HIP_TRY(orb_launch_stereo(left->d_sargs, 1, a.cap_l, st, nullptr));
-    rc = left->read_results(kl, capacity, dl, nl);
+    orb_extractor::Outputs ol, orr;
+    ol.kps = kl;
+    ol.desc = dl;
+    ol.uRight = uRight;
+    ol.depth = depth;
+    ol.d_uR = left->d_uR;
+    ol.d_depth = left->d_depth;
+    orr.kps = kr;
+    orr.desc = dr;
+    CopyList l;
+    l.n = 0;
+    rc = left->list_results(ol, l);
+    if (!rc) rc = right->list_results(orr, l);
     if (rc) return rc;
-    rc = right->read_results(kr, capacity, dr, nr);
+    HIP_TRY(orb_launch_copy_list(&l, ORB_COPY_BLOCKS, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    rc = left->take_results(ol, capacity, nl);
     if (rc) return rc;
-    if (*nl > 0) {
-        if (uRight) HIP_TRY(hipMemcpyAsync(uRight, left->d_uR, (size_t)*nl * 4, hipMemcpyDeviceToHost, st));
-        if (depth) HIP_TRY(hipMemcpyAsync(depth, left->d_depth, (size_t)*nl * 4, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
-    }
-    return ORB_OK;
+    return right->take_results(orr, capacity, nr);
 }
 
 int orb_extractor_debug_image(orb_extractor* ex, int level, int kind, uint8_t* dst, size_t dst_stride)
@@ -620,10 +629,14 @@ struct orb_batch {
         drop_branches();
     }
 
-    // pinned staging of orb_batch_read_all
-    int* h_ctr = nullptr;
-    char* h_res = nullptr;
-    size_t h_res_cap = 0;
+    // orb_batch_read_all: the results' layout in pinned memory that the device
+    // writes, with the counters first and the slots in groups, so that the
+    // host copies one group out while the device writes the next
+    char* h_all = nullptr;
+    CopyOp* d_all_ops = nullptr;
+    std::vector<int> all_start;             // first operation of each group (0: the counters)
+    std::vector<hipEvent_t> all_ev;         // recorded after each group
+    int all_pairs = -1;                     // pair count the layout was built for
 
     // Pinned transfers (orb_batch_pinned_images / _upload_pinned /
     // _read_async).  Inputs: every slot's image at its device pitch in one
@@ -689,6 +702,7 @@ struct orb_batch {
     int refresh_pinned()
     {
         drop_pinned_out();
+        drop_read_all();
         return d_in_ops ? write_in_ops() : ORB_OK;
     }
 
@@ -706,17 +720,15 @@ struct orb_batch {
         out_ready = false;
     }
 
-    int setup_pinned_out()
+    // Offsets of every output in a results buffer.
+    void layout_out()
     {
-        if (h_out && out_pairs == (int)pl.size()) return ORB_OK;
-        drop_pinned_out();
         const int n = (int)ex.size(), np = (int)pl.size();
         out_ctr.assign(n, 0);
         out_kps.assign(n, 0);
         out_desc.assign(n, 0);
         out_ur.assign(np, 0);
         out_dep.assign(np, 0);
-        std::vector<CopyOp> ops;
         size_t o = 0;
         for (int s = 0; s < n; s++) {
             const ImageJob& J = ex[s]->hjob;
@@ -736,25 +748,91 @@ struct orb_batch {
             o += up256(cap * 4);
         }
         out_bytes = o;
+    }
+
+    // The copy list of the slots' counters into such a buffer at dst, and of
+    // the other outputs of slots s0 .. s1 - 1 and pairs p0 .. p1 - 1.
+    void list_counters(char* dst, std::vector<CopyOp>& ops) const
+    {
+        for (size_t s = 0; s < ex.size(); s++)
+            ops.push_back(CopyOp{(const unsigned*)ex[s]->hjob.counters, (unsigned*)(dst + out_ctr[s]), nullptr,
+                                 ORB_CNT_SLOTS, 0});
+    }
+    void list_outputs(char* dst, int s0, int s1, int p0, int p1, std::vector<CopyOp>& ops) const
+    {
+        for (int s = s0; s < s1; s++) {
+            const ImageJob& J = ex[s]->hjob;
+            const int* cnt = J.counters + ORB_CNT_NOUT;
+            ops.push_back(CopyOp{(const unsigned*)J.kps, (unsigned*)(dst + out_kps[s]), cnt,
+                                 J.out_cap * (int)(sizeof(OrbKeyPoint) / 4), (int)(sizeof(OrbKeyPoint) / 4)});
+            ops.push_back(CopyOp{(const unsigned*)J.desc, (unsigned*)(dst + out_desc[s]), cnt, J.out_cap * 8, 8});
+        }
+        for (int p = p0; p < p1; p++) {
+            const orb_extractor* L = ex[pl[p]];
+            const int* cnt = L->hjob.counters + ORB_CNT_NOUT;
+            ops.push_back(CopyOp{(const unsigned*)L->d_uR, (unsigned*)(dst + out_ur[p]), cnt, L->hjob.out_cap, 1});
+            ops.push_back(CopyOp{(const unsigned*)L->d_depth, (unsigned*)(dst + out_dep[p]), cnt, L->hjob.out_cap, 1});
+        }
+    }
+
+    // The read_all buffer, its copy list (counters, then all_groups() groups
+    // of slots and pairs) and an event a group.
+    int all_groups() const { return std::max(1, std::min(8, (int)ex.size() / 8)); }
+    int setup_read_all()
+    {
+        if (h_all && all_pairs == (int)pl.size()) return ORB_OK;
+        drop_read_all();
+        layout_out();
+        if (hipHostMalloc((void**)&h_all, out_bytes, hipHostMallocCoherent) != hipSuccess) {
+            h_all = nullptr;
+            return ORB_E_OOM;
+        }
+        const int n = (int)ex.size(), np = (int)pl.size(), ng = all_groups();
+        std::vector<CopyOp> ops;
+        all_start.assign(1, 0);
+        list_counters(h_all, ops);
+        for (int g = 0; g < ng; g++) {
+            all_start.push_back((int)ops.size());
+            list_outputs(h_all, n * g / ng, n * (g + 1) / ng, np * g / ng, np * (g + 1) / ng, ops);
+        }
+        all_start.push_back((int)ops.size());
+        if (hipMalloc(&d_all_ops, ops.size() * sizeof(CopyOp)) != hipSuccess) {
+            d_all_ops = nullptr;
+            drop_read_all();
+            return ORB_E_OOM;
+        }
+        HIP_TRY(hipMemcpy(d_all_ops, ops.data(), ops.size() * sizeof(CopyOp), hipMemcpyHostToDevice));
+        while ((int)all_ev.size() < ng + 1) {
+            hipEvent_t e = nullptr;
+            HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem));
+            all_ev.push_back(e);
+        }
+        all_pairs = np;
+        return ORB_OK;
+    }
+    void drop_read_all()
+    {
+        if (h_all) (void)hipHostFree(h_all);
+        if (d_all_ops) (void)hipFree(d_all_ops);
+        h_all = nullptr;
+        d_all_ops = nullptr;
+        all_pairs = -1;
+    }
+
+    int setup_pinned_out()
+    {
+        if (h_out && out_pairs == (int)pl.size()) return ORB_OK;
+        drop_pinned_out();
+        layout_out();
+        const int n = (int)ex.size(), np = (int)pl.size();
         if (hipHostMalloc((void**)&h_out, out_bytes) != hipSuccess) {
             h_out = nullptr;
             return ORB_E_OOM;
         }
         if (hipMalloc((void**)&d_out, out_bytes) != hipSuccess) return ORB_E_OOM;
-        for (int s = 0; s < n; s++) {
-            const ImageJob& J = ex[s]->hjob;
-            const int* cnt = J.counters + ORB_CNT_NOUT;
-            ops.push_back(CopyOp{(const unsigned*)J.counters, (unsigned*)(d_out + out_ctr[s]), nullptr, ORB_CNT_SLOTS, 0});
-            ops.push_back(CopyOp{(const unsigned*)J.kps, (unsigned*)(d_out + out_kps[s]), cnt,
-                                 J.out_cap * (int)(sizeof(OrbKeyPoint) / 4), (int)(sizeof(OrbKeyPoint) / 4)});
-            ops.push_back(CopyOp{(const unsigned*)J.desc, (unsigned*)(d_out + out_desc[s]), cnt, J.out_cap * 8, 8});
-        }
-        for (int p = 0; p < np; p++) {
-            const orb_extractor* L = ex[pl[p]];
-            const int* cnt = L->hjob.counters + ORB_CNT_NOUT;
-            ops.push_back(CopyOp{(const unsigned*)L->d_uR, (unsigned*)(d_out + out_ur[p]), cnt, L->hjob.out_cap, 1});
-            ops.push_back(CopyOp{(const unsigned*)L->d_depth, (unsigned*)(d_out + out_dep[p]), cnt, L->hjob.out_cap, 1});
-        }
+        std::vector<CopyOp> ops;
+        list_counters(d_out, ops);
+        list_outputs(d_out, 0, n, 0, np, ops);
         n_out_ops = (int)ops.size();
         if (hipMalloc(&d_out_ops, ops.size() * sizeof(CopyOp)) != hipSuccess) return ORB_E_OOM;
         HIP_TRY(hipMemcpy(d_out_ops, ops.data(), ops.size() * sizeof(CopyOp), hipMemcpyHostToDevice));
@@ -776,8 +854,8 @@ struct orb_batch {
 
     ~orb_batch()
     {
-        if (h_ctr) (void)hipHostFree(h_ctr);
-        if (h_res) (void)hipHostFree(h_res);
+        drop_read_all();
+        for (hipEvent_t e : all_ev) (void)hipEventDestroy(e);
         if (h_in) (void)hipHostFree(h_in);
         if (d_in) (void)hipFree(d_in);
         if (d_in_ops) (void)hipFree(d_in_ops);
@@ -892,63 +970,43 @@ int orb_batch_read_all(orb_batch* b, orb_keypoint* keypoints, uint8_t* descripto
     HIP_TRY(hipSetDevice(b->ctx->device));
     hipStream_t st = b->ctx->stream;
     const int n = (int)b->ex.size(), np = (int)b->pl.size();
-    if (!b->h_ctr && hipHostMalloc((void**)&b->h_ctr, (size_t)n * ORB_CNT_SLOTS * sizeof(int)) != hipSuccess) {
-        b->h_ctr = nullptr;
-        return ORB_E_OOM;
+    const int rc = b->setup_read_all();
+    if (rc) return rc;
+    // the counters, then the groups, all enqueued at once
+    const int ng = b->all_groups();
+    for (int g = 0; g <= ng; g++) {
+        const int o = b->all_start[g];
+        HIP_TRY(orb_launch_copy_ops(b->d_all_ops + o, b->all_start[g + 1] - o, g ? 8 : 1, st));
+        HIP_TRY(hipEventRecord(b->all_ev[g], st));
     }
-    for (int s = 0; s < n; s++)
-        HIP_TRY(hipMemcpyAsync(b->h_ctr + (size_t)s * ORB_CNT_SLOTS, b->ex[s]->hjob.counters,
-                               ORB_CNT_SLOTS * sizeof(int), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    size_t need = 0;
-    for (int s = 0; s < n; s++) {
-        const int* c = b->h_ctr + (size_t)s * ORB_CNT_SLOTS;
-        if (c[ORB_CNT_ERR]) return ORB_E_OVERFLOW;
-        counts[s] = c[ORB_CNT_NOUT];
-        if (counts[s] > capacity) return ORB_E_CAPACITY;
-        need += (size_t)counts[s] * (sizeof(orb_keypoint) + 32);
-    }
-    for (int p = 0; p < np; p++) need += (size_t)counts[b->pl[p]] * 8;
-    if (need > b->h_res_cap) {
-        if (b->h_res) (void)hipHostFree(b->h_res);
-        b->h_res = nullptr;
-        b->h_res_cap = 0;
-        if (hipHostMalloc((void**)&b->h_res, need) != hipSuccess) return ORB_E_OOM;
-        b->h_res_cap = need;
-    }
-    size_t o = 0;
-    std::vector<size_t> at(n + np);
-    for (int s = 0; s < n; s++) {
-        const size_t c = (size_t)counts[s];
-        at[s] = o;
-        if (c) {
-            HIP_TRY(hipMemcpyAsync(b->h_res + o, b->ex[s]->hjob.kps, c * sizeof(orb_keypoint), hipMemcpyDeviceToHost,
-                                   st));
-            HIP_TRY(hipMemcpyAsync(b->h_res + o + c * sizeof(orb_keypoint), b->ex[s]->hjob.desc, c * 32,
-                                   hipMemcpyDeviceToHost, st));
+    const int bad = [&] {
+        HIP_TRY(hipEventSynchronize(b->all_ev[0]));
+        for (int s = 0; s < n; s++) {
+            const int* c = (const int*)(b->h_all + b->out_ctr[s]);
+            if (c[ORB_CNT_ERR]) return ORB_E_OVERFLOW;
+            counts[s] = c[ORB_CNT_NOUT];
+            if (counts[s] > capacity) return ORB_E_CAPACITY;
         }
-        o += c * (sizeof(orb_keypoint) + 32);
+        return ORB_OK;
+    }();
+    if (bad) {
+        HIP_TRY(hipStreamSynchronize(st));                // the buffer is free again
+        return bad;
     }
-    for (int p = 0; p < np; p++) {
-        const orb_extractor* L = b->ex[b->pl[p]];
-        const size_t c = (size_t)counts[b->pl[p]];
-        at[n + p] = o;
-        if (c) {
-            HIP_TRY(hipMemcpyAsync(b->h_res + o, L->d_uR, c * 4, hipMemcpyDeviceToHost, st));
-            HIP_TRY(hipMemcpyAsync(b->h_res + o + c * 4, L->d_depth, c * 4, hipMemcpyDeviceToHost, st));
+    for (int g = 0; g < ng; g++) {
+        HIP_TRY(hipEventSynchronize(b->all_ev[g + 1]));
+        for (int s = n * g / ng; s < n * (g + 1) / ng; s++) {
+            const size_t c = (size_t)counts[s];
+            if (!c) continue;
+            std::memcpy(keypoints + (size_t)s * capacity, b->h_all + b->out_kps[s], c * sizeof(orb_keypoint));
+            std::memcpy(descriptors + (size_t)s * capacity * 32, b->h_all + b->out_desc[s], c * 32);
         }
-        o += c * 8;
-    }
-    HIP_TRY(hipStreamSynchronize(st));
-    for (int s = 0; s < n; s++) {
-        const size_t c = (size_t)counts[s];
-        std::memcpy(keypoints + (size_t)s * capacity, b->h_res + at[s], c * sizeof(orb_keypoint));
-        std::memcpy(descriptors + (size_t)s * capacity * 32, b->h_res + at[s] + c * sizeof(orb_keypoint), c * 32);
-    }
-    for (int p = 0; p < np; p++) {
-        const size_t c = (size_t)counts[b->pl[p]];
-        if (uRight) std::memcpy(uRight + (size_t)p * capacity, b->h_res + at[n + p], c * 4);
-        if (depth) std::memcpy(depth + (size_t)p * capacity, b->h_res + at[n + p] + c * 4, c * 4);
+        for (int p = np * g / ng; p < np * (g + 1) / ng; p++) {
+            const size_t c = (size_t)counts[b->pl[p]];
+            if (!c) continue;
+            if (uRight) std::memcpy(uRight + (size_t)p * capacity, b->h_all + b->out_ur[p], c * 4);
+            if (depth) std::memcpy(depth + (size_t)p * capacity, b->h_all + b->out_dep[p], c * 4);
+        }
     }
     return ORB_OK;
 }
@@ -1526,17 +1584,16 @@ int orb_rgbd_frame(orb_extractor* ex, const uint8_t* image, int width, int heigh
     if (depth)
         HIP_TRY(orb_launch_rgbd_depth(ex->hjob.kps, d_kun, cap, cnt, (const float*)m, width, height, depth_pitch, bf,
                                       d_uR, d_uR + cap, st));
-    rc = ex->read_results(keypoints, capacity, descriptors, n);
-    if (rc) return rc;
-    if (*n > 0) {
-        if (keypoints_un)
-            HIP_TRY(hipMemcpyAsync(keypoints_un, d_kun, (size_t)*n * sizeof(OrbKeyPoint), hipMemcpyDeviceToHost, st));
-        if (depth && uRight) HIP_TRY(hipMemcpyAsync(uRight, d_uR, (size_t)*n * 4, hipMemcpyDeviceToHost, st));
-        if (depth && depth_out)
-            HIP_TRY(hipMemcpyAsync(depth_out, d_uR + cap, (size_t)*n * 4, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
-    }
-    return ORB_OK;
+    orb_extractor::Outputs o;
+    o.kps = keypoints;
+    o.desc = descriptors;
+    o.kps_un = keypoints_un;
+    o.uRight = depth ? uRight : nullptr;
+    o.depth = depth ? depth_out : nullptr;
+    o.d_kun = d_kun;
+    o.d_uR = d_uR;
+    o.d_depth = d_uR + cap;
+    return ex->read_results(o, capacity, n);
 }
 
 int orb_distinctive_descriptors(orb_context* ctx, int n_points, const uint8_t* desc, const int32_t* offsets,

@@ -91,6 +91,10 @@ struct Lane {                    // one HIP stream with its staging
 
 size_t result_bytes(int cap) { return 256 + (size_t)cap * (sizeof(OrbKeyPoint) + 32 + 8); }
 
+// Most pinned memory a server takes when it is made; more is allocated frame
+// by frame.
+constexpr size_t kSlabBytes = (size_t)64 << 20;
+
 // Row pitch of a frame's pinned staging copy: that of the extractor's level 0.
 size_t img_pitch(int w) { return ((size_t)w + 63) / 64 * 64; }
 
@@ -110,10 +114,13 @@ struct orb_server {
     int max_cap = 0;
     std::vector<uint8_t*> img_pool;
     std::vector<char*> res_pool;
+    std::vector<void*> host_blocks;   // pinned allocations the pools' buffers lie in
 
     std::mutex mu;
     std::condition_variable cv;
     std::deque<Request*> pending;
+    std::deque<Request*> waiting;    // taken from pending by the loop, not admitted yet (its thread's alone)
+    int n_waiting = 0;
     std::vector<Request*> completed;
     std::map<uint64_t, Request*> done;
     uint64_t next_ticket = 1;
@@ -162,6 +169,7 @@ struct orb_server {
             return -1;
         }
         s.d_mdist = s.d_midx + e->plan.out_cap;
+        std::lock_guard<std::mutex> g(mu);   // stats() reads both
         used += s.bytes;
         slots.push_back(s);
         return (int)slots.size() - 1;
@@ -277,7 +285,7 @@ struct orb_server {
     void loop()
     {
         (void)hipSetDevice(ctx->device);
-        std::vector<Request*> batch;
+        std::vector<Request*> batch, refused;
         while (!stop.load()) {
             for (Lane& L : lanes)
                 if (L.busy && hipEventQuery(L.ev) == hipSuccess) finish(L);
@@ -288,56 +296,69 @@ struct orb_server {
                     break;
                 }
             batch.clear();
+            refused.clear();
+            if (free_lane) {
+                std::lock_guard<std::mutex> g(mu);
+                waiting.insert(waiting.end(), pending.begin(), pending.end());
+                pending.clear();
+                n_waiting = (int)waiting.size();
+            }
+            // Admission, without the lock: allocating a slot takes longer than
+            // a submission, which need not wait for it.
+            if (free_lane && !waiting.empty()) {
+                std::vector<char> blocked(cams.size(), 0);
+                const double t = clock_s();
+                for (auto it = waiting.begin(); it != waiting.end() && (int)batch.size() < max_batch;) {
+                    Request* r = *it;
+                    Camera& c = cams[r->stream];
+                    // one frame per stream per batch; at most one per lane in flight
+                    if (blocked[r->stream] || c.inflight >= (int)lanes.size()) {
+                        blocked[r->stream] = 1;
+                        ++it;
+                        continue;
+                    }
+                    const int s = slot_for(c);
+                    if (s == -2) {
+                        // refused: the budget cannot hold a slot of this size
+                        r->status = ORB_E_ADMISSION;
+                        r->t_admit = r->t_done = t;
+                        refused.push_back(r);
+                        it = waiting.erase(it);
+                        continue;
+                    }
+                    if (s < 0) {
+                        blocked[r->stream] = 1;
+                        ++it;
+                        continue;
+                    }
+                    slots[s].free = false;
+                    r->slot = s;
+                    r->t_admit = t;
+                    r->dep_lane = c.inflight > 0 ? c.last_lane : -1;
+                    c.inflight++;
+                    c.last_lane = (int)(free_lane - lanes.data());
+                    blocked[r->stream] = 1;
+                    batch.push_back(r);
+                    it = waiting.erase(it);
+                }
+            }
             {
                 std::unique_lock<std::mutex> lk(mu);
-                if (free_lane && !pending.empty()) {
-                    std::vector<char> blocked(cams.size(), 0);
-                    const double t = clock_s();
-                    for (auto it = pending.begin(); it != pending.end() && (int)batch.size() < max_batch;) {
-                        Request* r = *it;
-                        Camera& c = cams[r->stream];
-                        // one frame per stream per batch; at most one per lane in flight
-                        if (blocked[r->stream] || c.inflight >= (int)lanes.size()) {
-                            blocked[r->stream] = 1;
-                            ++it;
-                            continue;
-                        }
-                        const int s = slot_for(c);
-                        if (s == -2) {
-                            // refused: the budget cannot hold a slot of this size
-                            r->status = ORB_E_ADMISSION;
-                            r->t_admit = r->t_done = t;
-                            img_pool.push_back(r->h_img);
-                            r->h_img = nullptr;
-                            completed.push_back(r);
-                            it = pending.erase(it);
-                            continue;
-                        }
-                        if (s < 0) {
-                            blocked[r->stream] = 1;
-                            ++it;
-                            continue;
-                        }
-                        slots[s].free = false;
-                        r->slot = s;
-                        r->t_admit = t;
-                        r->dep_lane = c.inflight > 0 ? c.last_lane : -1;
-                        c.inflight++;
-                        c.last_lane = (int)(free_lane - lanes.data());
-                        blocked[r->stream] = 1;
-                        batch.push_back(r);
-                        it = pending.erase(it);
-                    }
+                for (Request* r : refused) {
+                    img_pool.push_back(r->h_img);
+                    r->h_img = nullptr;
+                    completed.push_back(r);
                 }
-                if (batch.empty()) {
-                    if (inflight == 0) cv.wait_for(lk, std::chrono::milliseconds(1));
-                } else {
-                    // The batch counts as in flight from the moment it leaves
-                    // `pending`, so drain() never sees it in neither place.
+                // The batch counts as in flight from the moment it stops
+                // waiting, so drain() never sees it in neither place.
+                n_waiting = (int)waiting.size();
+                if (!batch.empty()) {
                     free_lane->busy = true;
                     inflight++;
                     n_batches++;
                     n_requests += (int64_t)batch.size();
+                } else if (inflight == 0 && pending.empty()) {
+                    cv.wait_for(lk, std::chrono::milliseconds(1));
                 }
             }
             if (!batch.empty()) {
@@ -368,16 +389,11 @@ struct orb_server {
         }
         for (Camera& c : cams)
             if (c.d_prev) (void)hipFree(c.d_prev);
-        auto drop = [&](Request* r) {
-            if (r->h_img) img_pool.push_back(r->h_img);
-            if (r->h_res) res_pool.push_back(r->h_res);
-            delete r;
-        };
-        for (Request* r : pending) drop(r);
-        for (Request* r : completed) drop(r);
-        for (auto& kv : done) drop(kv.second);
-        for (uint8_t* p : img_pool) (void)hipHostFree(p);
-        for (char* p : res_pool) (void)hipHostFree(p);
+        for (Request* r : pending) delete r;
+        for (Request* r : waiting) delete r;
+        for (Request* r : completed) delete r;
+        for (auto& kv : done) delete kv.second;
+        for (void* p : host_blocks) (void)hipHostFree(p);
     }
 };
 
@@ -448,6 +464,21 @@ int orb_server_create(orb_context* ctx, int nstreams, const int* widths, const i
             return ORB_E_OOM;
         }
     }
+    // Pinned buffers of a frame per stream (as many as kSlabBytes hold) in one
+    // allocation: one of a megabyte costs 250 us, more than a frame's service,
+    // and a first frame of every stream paid for two.
+    const size_t ib = (s->max_img + 255) / 256 * 256, rb = (result_bytes(s->max_cap) + 255) / 256 * 256;
+    const size_t frames = std::min((size_t)nstreams, kSlabBytes / (ib + rb));
+    char* slab = nullptr;
+    if (frames && hipHostMalloc((void**)&slab, frames * (ib + rb), hipHostMallocCoherent) == hipSuccess) {
+        s->host_blocks.push_back(slab);
+        for (size_t i = 0; i < frames; i++) {
+            s->img_pool.push_back((uint8_t*)(slab + i * ib));
+            s->res_pool.push_back(slab + frames * ib + i * rb);
+        }
+    } else {
+        (void)hipGetLastError();       // each frame allocates its own
+    }
     s->th = std::thread([s] { s->loop(); });
     *out = s;
     return ORB_OK;
@@ -466,7 +497,7 @@ int orb_server_submit(orb_server* s, int stream, const uint8_t* image, size_t st
     {
         std::lock_guard<std::mutex> g(s->mu);
         if (s->error.load()) return s->error.load();
-        if (s->pending.size() >= 4096) return ORB_E_ADMISSION;
+        if (s->pending.size() + s->n_waiting >= 4096) return ORB_E_ADMISSION;
         if (!s->img_pool.empty()) {
             img = s->img_pool.back();
             s->img_pool.pop_back();
@@ -479,8 +510,19 @@ int orb_server_submit(orb_server* s, int stream, const uint8_t* image, size_t st
     // Coherent (fine-grained) pinned memory: the device reads the frame and
     // writes the results over PCIe with no copy engine in between, so neither
     // side may keep them in a cache.
-    if (!img && hipHostMalloc(&img, s->max_img, hipHostMallocCoherent) != hipSuccess) return ORB_E_OOM;
-    if (!res && hipHostMalloc(&res, result_bytes(s->max_cap), hipHostMallocCoherent) != hipSuccess) return ORB_E_OOM;
+    const bool own_img = !img, own_res = !res;
+    if (own_img && hipHostMalloc((void**)&img, s->max_img, hipHostMallocCoherent) != hipSuccess) img = nullptr;
+    if (own_res && hipHostMalloc((void**)&res, result_bytes(s->max_cap), hipHostMallocCoherent) != hipSuccess) res = nullptr;
+    if ((own_img && img) || (own_res && res) || !img || !res) {
+        std::lock_guard<std::mutex> g(s->mu);
+        if (own_img && img) s->host_blocks.push_back(img);
+        if (own_res && res) s->host_blocks.push_back(res);
+        if (!img || !res) {
+            if (img) s->img_pool.push_back(img);
+            if (res) s->res_pool.push_back(res);
+            return ORB_E_OOM;
+        }
+    }
     const size_t pitch = img_pitch(c.w);
     for (int y = 0; y < c.h; y++) std::memcpy(img + (size_t)y * pitch, image + (size_t)y * stride, c.w);
     Request* r = new Request();
@@ -568,7 +610,7 @@ int orb_server_drain(orb_server* s, double timeout_s)
     if (!s) return ORB_E_ARG;
     const double t_end = clock_s() + timeout_s;
     std::unique_lock<std::mutex> lk(s->mu);
-    while (!s->pending.empty() || s->inflight > 0) {
+    while (!s->pending.empty() || s->n_waiting > 0 || s->inflight > 0) {
         if (clock_s() > t_end) return ORB_E_DEVICE;
         s->cv.wait_for(lk, std::chrono::milliseconds(1));
     }

@@ -153,6 +153,14 @@ struct CopyOp {
     int unit_words;
 };
 
+// A copy list short enough to be a kernel argument.
+#define ORB_COPY_LIST 8
+#define ORB_COPY_BLOCKS 16            // workgroups an operation of a single call's list
+struct CopyList {
+    CopyOp op[ORB_COPY_LIST];
+    int n;
+};
+
 // A DBoW2 vocabulary tree on the device, nodes renumbered breadth-first so
 // that every node's children are contiguous (in their file order).
 struct VocDev {
