@@ -409,14 +409,19 @@ struct orb_extractor {
         const size_t o_srec = take((size_t)p.out_cap * 16), o_sdesc = take((size_t)p.out_cap * 32);
         const size_t o_rows = take((size_t)nlevels * ((size_t)H + 2) * 8);
         size_t ntab = 0;
-        for (int l = 1; l < nlevels; l++)
-            // tile-row windows sized for the smallest tile height, so that a
-            // change of tile heights never reallocates (the frames stay put)
-            ntab += (size_t)p.lv[l].w + p.lv[l].h + p.lv[l].tiles_x + (p.lv[l].h + 15) / 16;
+        for (int l = 1; l < nlevels; l++) ntab += (size_t)p.lv[l].w + p.lv[l].h;
         const size_t o_tab = take(ntab * 8);
         size_t noct = 0;
         for (int l = 0; l < nlevels; l++) noct += (size_t)p.lv[l].w + p.lv[l].h;
         const size_t o_oct = take(noct * 2);
+        // the chains' windows: of every level, at most that and all below per
+        // tile column and row
+        size_t nchain = 0;
+        for (int v = 0; v < ORB_CH_VARIANTS; v++)
+            for (int l = 1; l < nlevels; l++)
+                nchain += (size_t)(l + 1) * ((p.lv[l].w + ORB_CH_W(v) - 1) / ORB_CH_W(v) +
+                                             (p.lv[l].h + ORB_CH_H(v) - 1) / ORB_CH_H(v));
+        const size_t o_chain = take(nchain * sizeof(ChainWin));
         const size_t total = off;
         if (total > mem_bytes) {
             if (d_mem) (void)hipFree(d_mem);
@@ -479,8 +484,8 @@ struct orb_extractor {
             L.node = (int*)(d_mem + o_node) + P.key_off;
             L.ret = (unsigned long long*)(d_mem + o_ret) + P.ret_off;
         }
-        // resize taps and quadtree places, sent in one copy
-        std::vector<char> tables(o_oct - o_tab + noct * 2);
+        // resize taps, quadtree places and chain windows, sent in one copy
+        std::vector<char> tables(o_chain - o_tab + nchain * sizeof(ChainWin));
         // cv::resize INTER_LINEAR taps of every level from the level above
         // (ComputePyramid, ORBextractor.cc:1677): per destination column and
         // row, the source index and the two 11-bit weights, with the float
@@ -508,8 +513,6 @@ struct orb_extractor {
                     tab[t].x = sx | ((x < rs_end ? 1 : 0) << 30);
                     tab[t].y = (int)std::nearbyint((1.f - fx) * 2048.f) | ((int)std::nearbyint(fx * 2048.f) << 16);
                 }
-                const size_t tx = t - w;
-                // ytab == xtab + w: the level kernel reads both through xtab.
                 J.lv[l].ytab = (const int2*)(d_mem + o_tab) + t;
                 const double scale_y = 1. / ((double)h / sh);
                 for (int y = 0; y < h; y++, t++) {
@@ -522,31 +525,6 @@ struct orb_extractor {
                     tab[t].y = (int)std::nearbyint((1.f - fy) * 2048.f) | ((int)std::nearbyint(fy * 2048.f) << 16);
                 }
                 const size_t ty = t - h;
-                // Per tile column and row: the source range its taps read,
-                // halo (REFLECT_101) included, as the level kernel stages it.
-                J.lv[l].xwin = (const int2*)(d_mem + o_tab) + t;
-                for (int c = 0; c < p.lv[l].tiles_x; c++, t++) {
-                    int lo = INT_MAX, hi = -1;
-                    for (int i = 0; i < ORB_TILE_W + 8; i++) {
-                        const int sx = tab[tx + reflect101(c * ORB_TILE_W - 4 + i, w)].x & 0x3FFFFFFF;
-                        lo = std::min(lo, sx);
-                        hi = std::max(hi, sx + 1 < sw ? sx + 1 : sx);
-                    }
-                    tab[t].x = lo;
-                    tab[t].y = hi;
-                }
-                J.lv[l].ywin = (const int2*)(d_mem + o_tab) + t;
-                for (int r = 0; r < p.lv[l].tiles_y; r++, t++) {
-                    int lo = INT_MAX, hi = -1;
-                    const int th = p.lv[l].tile_h;
-                    for (int i = 0; i < th + 8; i++) {
-                        const int sy01 = tab[ty + reflect101(r * th - 4 + i, h)].x;
-                        lo = std::min(lo, sy01 & 0xFFFF);
-                        hi = std::max(hi, sy01 >> 16);
-                    }
-                    tab[t].x = lo;
-                    tab[t].y = hi;
-                }
             }
         }
         // Quadtree place at depth ORB_OCT_D, split into its x and y parts: the
@@ -595,8 +573,11 @@ struct orb_extractor {
                     for (; y < next; y++) tab[t++] = (unsigned short)v;
                 }
             }
-            HIP_TRY(hipMemcpy(d_mem + o_tab, tables.data(), tables.size(), hipMemcpyHostToDevice));
         }
+        rc = plan_chains(J, (const int2*)tables.data(), (const int2*)(d_mem + o_tab), (ChainWin*)(tables.data() + (o_chain - o_tab)),
+                         (const ChainWin*)(d_mem + o_chain), nchain);
+        if (rc) return rc;
+        HIP_TRY(hipMemcpy(d_mem + o_tab, tables.data(), tables.size(), hipMemcpyHostToDevice));
         d_uR = (float*)(d_mem + o_uR);
         d_depth = (float*)(d_mem + o_dep);
         d_msad = (int*)(d_mem + o_msad);
@@ -612,6 +593,93 @@ struct orb_extractor {
         if (rc_t) return rc_t;
         HIP_TRY(hipMemcpy(d_job, &hjob, sizeof(ImageJob), hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(d_rt, h_rt, sizeof(RunTable), hipMemcpyHostToDevice));
+        return ORB_OK;
+    }
+
+    // The pyramid's chains: from each base as many levels in one launch as
+    // have windows (for a tile of the last) that fit the kernel's LDS.  taps:
+    // the levels' tap tables on the host, as d_taps on the device; tab
+    // receives the windows (d_tab on the device; room for cap entries).
+    int plan_chains(ImageJob& J, const int2* taps, const int2* d_taps, ChainWin* tab, const ChainWin* d_tab, size_t cap) const
+    {
+        // source range of columns / rows a .. b of level l
+        auto xsrc = [&](int l, int x) { return taps[(J.lv[l].xtab - d_taps) + x].x & 0x3FFFFFFF; };
+        auto ysrc = [&](int l, int y, int tap) {
+            const int v = taps[(J.lv[l].ytab - d_taps) + y].x;
+            return tap ? v >> 16 : v & 0xFFFF;
+        };
+        size_t t = 0;
+        // windows of a chain base .. base + m into tab + t; false if one does not fit
+        auto windows = [&](int variant, int base, int m, ChainWin* out, int tx, int ty) {
+            int maxd[ORB_MAX_LEVELS] = {}, maxr[ORB_MAX_LEVELS] = {};
+            for (int dir = 0; dir < 2; dir++) {
+                const int n = dir ? ty : tx, step = dir ? ORB_CH_H(variant) : ORB_CH_W(variant);
+                std::vector<int> start((size_t)(m + 1) * (n + 1));
+                for (int i = 0; i <= n; i++)
+                    for (int k = m; k >= 0; k--) {
+                        const LevelJob& L = J.lv[base + k];
+                        const int len = dir ? L.h : L.w;
+                        int v;
+                        if (i == n) v = len;
+                        else if (i == 0) v = 0;
+                        else if (k == m) v = i * step;
+                        else {
+                            const int up = start[(size_t)(k + 1) * (n + 1) + i];
+                            v = dir ? ysrc(base + k + 1, up, 0) : xsrc(base + k + 1, up) & ~3;
+                        }
+                        start[(size_t)k * (n + 1) + i] = v;
+                    }
+                for (int i = 0; i < n; i++) {
+                    int lo = 0, hi = -1;
+                    for (int k = m; k >= 0; k--) {
+                        const LevelJob& L = J.lv[base + k];
+                        const int len = dir ? L.h : L.w;
+                        const int o0 = start[(size_t)k * (n + 1) + i], o1 = start[(size_t)k * (n + 1) + i + 1];
+                        int a = o0, b = o1 - 1;
+                        if (k < m) {
+                            const int sa = dir ? ysrc(base + k + 1, lo, 0) : xsrc(base + k + 1, lo);
+                            const int sb = dir ? ysrc(base + k + 1, hi, 1) : std::min(xsrc(base + k + 1, hi) + 1, len - 1);
+                            a = (k == 0 || o0 >= o1) ? sa : std::min(a, sa);
+                            b = (k == 0 || o0 >= o1) ? sb : std::max(b, sb);
+                        }
+                        if (!dir) {
+                            a &= ~3;
+                            b = std::min(b | 3, len - 1);
+                        }
+                        lo = a;
+                        hi = b;
+                        const unsigned nd = (unsigned)((b >> 2) - (a >> 2) + 1);
+                        out[(dir ? (size_t)tx * (m + 1) : 0) + (size_t)i * (m + 1) + k] =
+                            ChainWin{a, b, o0, o1, (int)nd, ((1u << 20) + nd - 1) / nd, {0, 0}};
+                        if (dir) maxr[k] = std::max(maxr[k], b - a + 1);
+                        else maxd[k] = std::max(maxd[k], (b >> 2) - (a >> 2) + 1);
+                    }
+                }
+            }
+            bool fits = maxr[m] <= ORB_CH_ROWS && maxd[m] <= ORB_CH_COLS;
+            for (int k = 0; k < m; k++)
+                fits = fits && maxr[k] <= ORB_CH_ROWS && maxd[k] <= ORB_CH_COLS && maxr[k] * maxd[k] <= ORB_CH_DWORDS;
+            return fits;
+        };
+        for (int v = 0; v < ORB_CH_VARIANTS; v++) {
+            J.nchains[v] = 0;
+            for (int base = 0; base + 1 < nlevels;) {
+                ChainJob& ch = J.ch[v][J.nchains[v]++];
+                ch.base = base;
+                for (ch.m = nlevels - 1 - base;; ch.m--) {
+                    const LevelJob& T = J.lv[base + ch.m];
+                    ch.tiles_x = (T.w + ORB_CH_W(v) - 1) / ORB_CH_W(v);
+                    ch.tiles_y = (T.h + ORB_CH_H(v) - 1) / ORB_CH_H(v);
+                    if (t + (size_t)(ch.m + 1) * (ch.tiles_x + ch.tiles_y) > cap) return ORB_E_ARG;   // cannot happen
+                    ch.staged = windows(v, base, ch.m, tab + t, ch.tiles_x, ch.tiles_y) ? 1 : 0;
+                    if (ch.staged || ch.m == 1) break;
+                }
+                ch.xr = d_tab + t;
+                ch.yr = d_tab + t + (size_t)(ch.m + 1) * ch.tiles_x;
+                t += (size_t)(ch.m + 1) * (ch.tiles_x + ch.tiles_y);
+                base += ch.m;
+            }
+        }
         return ORB_OK;
     }
 
@@ -645,6 +713,36 @@ struct orb_extractor {
             for (int j = 0; j < n; j++)
                 eq = eq && rt.tile_start[l][j + 1] - rt.tile_start[l][j] == rt.tile_start[l][1] - rt.tile_start[l][0];
             rt.tiles_per_job[l] = eq ? rt.tile_start[l][1] - rt.tile_start[l][0] : 0;
+        }
+        for (int g = 0; g < 2; g++) {
+            int all = 0;
+            for (int l = 0; l <= maxl; l++) {
+                rt.all_start[g][l] = all;
+                if (l < maxl && rt.tile_h[l] == (g ? 16 : 32)) all += rt.tile_start[l][n];
+            }
+        }
+        // pyramid launches: small tiles while they leave the GPU room
+        int small = 0;
+        for (int j = 0; j < n; j++)
+            if (exs[j]->hjob.nchains[0] > 0) small += exs[j]->hjob.ch[0][0].tiles_x * exs[j]->hjob.ch[0][0].tiles_y;
+        const int cv = rt.chain_variant = small > ORB_CH_FEW ? 1 : 0;
+        rt.chain_zeroes = n > 0;
+        for (int j = 0; j < n; j++) {
+            rt.nchains = std::max(rt.nchains, exs[j]->hjob.nchains[cv]);
+            rt.chain_zeroes = rt.chain_zeroes && exs[j]->hjob.nchains[cv] > 0;
+        }
+        for (int c = 0; c < rt.nchains; c++) {
+            int blocks = 0;
+            for (int j = 0; j < n; j++) {
+                const ImageJob& J = exs[j]->hjob;
+                rt.chain_start[c][j] = blocks;
+                blocks += c < J.nchains[cv] ? J.ch[cv][c].tiles_x * J.ch[cv][c].tiles_y : 0;
+            }
+            rt.chain_start[c][n] = blocks;
+            bool same = blocks > 0;
+            for (int j = 0; j < n; j++)
+                same = same && rt.chain_start[c][j + 1] - rt.chain_start[c][j] == rt.chain_start[c][1];
+            rt.chain_per_job[c] = same ? rt.chain_start[c][1] : 0;
         }
         int acc = 0;
         for (int j = 0; j < n; j++)

@@ -1,11 +1,11 @@
 // orb_kernels.hip -- gfx950 kernels of the ORB front end.
 //
 // Pipeline per image (one launch per stage covers every job of a run):
-//   level_kernel   (x nlevels) pyramid level l from level l-1 (8-bit fixed
-//                  point bilinear, ORBextractor.cc:1677), its 7x7 sigma-2
-//                  blur (ORBextractor.cc:1607-1615), FAST-9 with per-cell
-//                  non-max suppression at both thresholds
-//                  (ORBextractor.cc:1075-1142), from one LDS tile
+//   pyramid_kernel levels 1 .. from level 0 (8-bit fixed point bilinear,
+//                  ORBextractor.cc:1677), several levels per launch
+//   level_kernel   every level's 7x7 sigma-2 blur (ORBextractor.cc:1607-1615)
+//                  and FAST-9 with per-cell non-max suppression at both
+//                  thresholds (ORBextractor.cc:1075-1142), from one LDS tile
 //   octree_kernel  the per-cell iniThFAST/minThFAST retry, then
 //                  DistributeOctTree as a per-level workgroup quadtree
 //                  (ORBextractor.cc:688-1033)
@@ -149,11 +149,11 @@ __device__ __forceinline__ int lanes_below(unsigned long long mask)
 }
 
 // ================================================================ level
-// One workgroup per 64x32 output tile of pyramid level l:
+// One workgroup per 64x32 (or 64x16) output tile of pyramid level l, the tiles
+// of all levels in one launch:
 //   1. level pixels for the tile plus a 4-px halo (REFLECT_101 at the level
-//      edges) into LDS: copied for level 0, else cv::resize INTER_LINEAR 8U
-//      from level l-1 (ComputePyramid, ORBextractor.cc:1677);
-//   2. the level and its 7x7 sigma-2 blur (ORBextractor.cc:1607-1615);
+//      edges) into LDS;
+//   2. its 7x7 sigma-2 blur (ORBextractor.cc:1607-1615);
 //   3. FAST-9 arc strength for the tile plus a 1-px ring, computed exactly only
 //      for pixels that pass a necessary cardinal-point test, after compaction;
 //   4. per-cell non-max suppression at iniThFAST and at minThFAST: a neighbour
@@ -302,14 +302,247 @@ __device__ __forceinline__ unsigned resize4(BytePtr base, unsigned o0, unsigned 
     return d;
 }
 
-// LDS that the phases use one after another: the resize source window
-// (phase 1), the horizontal blur sums (phase 2), then the FAST queue and the
-// tile's candidate list (phases 3-5).
-#define LW_MAX 2656                  // source window dwords: scale <= ~1.9
-#define LS_K 6                       // window dwords per thread read before the first wait
+// Four output pixels from the source rows at q0, q1 (dword pointers to the
+// dword that holds byte b0 of the four pixels' span, shb = b0 & 3): a source
+// row is three aligned dword reads realigned by two v_alignbyte, each pixel's
+// tap pair (p[sx], p[nx]) one v_perm into 16-bit lanes (sel), and S one
+// v_dot2_u32_u16 with the packed taps (a0 | a1 << 16).
+template <int MODE>
+__device__ __forceinline__ unsigned resize_dword(const unsigned* q0, const unsigned* q1, unsigned shb, const unsigned* sel,
+                                                 const int* tap, unsigned ybv, const unsigned* sse)
+{
+    const unsigned w00 = __builtin_amdgcn_alignbyte(q0[1], q0[0], shb);
+    const unsigned w01 = __builtin_amdgcn_alignbyte(q0[2], q0[1], shb);
+    const unsigned w10 = __builtin_amdgcn_alignbyte(q1[1], q1[0], shb);
+    const unsigned w11 = __builtin_amdgcn_alignbyte(q1[2], q1[1], shb);
+    if constexpr (MODE == 1) {
+        // SSE2 rounding with the horizontal taps scaled by 16: S16 = 16 S, so
+        // S16 & 0xFFFF00 = (S >> 4) << 8 (S16 < 2^23), and the high word of
+        // its product with b << 8 is ((S >> 4) * b) >> 16 in one
+        // v_mul_hi_u32_u24.  t = h0 + h1 + 2 <= 1023 fits a 16-bit lane: the
+        // >> 2 is done two pixels at a time and the four bytes gathered by
+        // one v_perm.
+        const unsigned bs0 = (ybv << 8) & 0xFFFF00u, bs1 = (ybv >> 8) & 0xFFFF00u;
+        unsigned t[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const orb_u16x2 tk = __builtin_bit_cast(orb_u16x2, (unsigned)tap[k] << 4);
+            const unsigned S0 = __builtin_amdgcn_udot2(
+                __builtin_bit_cast(orb_u16x2, __builtin_amdgcn_perm(w01, w00, sel[k])), tk, 0u, false);
+            const unsigned S1 = __builtin_amdgcn_udot2(
+                __builtin_bit_cast(orb_u16x2, __builtin_amdgcn_perm(w11, w10, sel[k])), tk, 0u, false);
+            t[k] = mulhi_u24(S0 & 0xFFFF00u, bs0) + mulhi_u24(S1 & 0xFFFF00u, bs1) + 2u;
+        }
+        const orb_u16x2 two = {2, 2};
+        const unsigned u01 = __builtin_bit_cast(unsigned, __builtin_bit_cast(orb_u16x2, t[0] | (t[1] << 16)) >> two);
+        const unsigned u23 = __builtin_bit_cast(unsigned, __builtin_bit_cast(orb_u16x2, t[2] | (t[3] << 16)) >> two);
+        return __builtin_amdgcn_perm(u23, u01, 0x06040200u);
+    } else {
+        const unsigned bv0 = ybv & 0xFFFFu, bv1 = ybv >> 16;
+        unsigned d = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const orb_u16x2 tk = __builtin_bit_cast(orb_u16x2, (unsigned)tap[k]);
+            const unsigned S0 = __builtin_amdgcn_udot2(
+                __builtin_bit_cast(orb_u16x2, __builtin_amdgcn_perm(w01, w00, sel[k])), tk, 0u, false);
+            const unsigned S1 = __builtin_amdgcn_udot2(
+                __builtin_bit_cast(orb_u16x2, __builtin_amdgcn_perm(w11, w10, sel[k])), tk, 0u, false);
+            d |= vresize<MODE>(S0, S1, bv0, bv1, sse[k]) << (8 * k);
+        }
+        return d;
+    }
+}
+
+// ============================================================== pyramid
+// cv::resize INTER_LINEAR 8U of levels base + 1 .. base + m, each from the
+// level before (ComputePyramid, ORBextractor.cc:1677).  A workgroup takes one
+// tile of the last level and computes, level by level in LDS, what that tile
+// needs of each; the levels' tiles overlap by a few pixels, and each pixel is
+// written by the one workgroup that owns it (windows and ownership come from
+// the host, by tile column and row).  At scale factor 1.2 all seven levels
+// are one launch, with 1.4 times the pixels computed.  Bound: latency (one
+// LDS round trip and barrier per level) in a single call, VALU in a batch.
+// One image of 640 x 480 14.9 us and every level's tiles after it 12.2, where a
+// launch per level that resized its own tile took 82; 128 images of 1241 x 376
+// 151 + 566 us (725).
+// The source index and 11-bit taps of each column and row come from the
+// level's tables (computed on the host with OpenCV's double/float
+// statements).
+__device__ __forceinline__ void zero_job(const ImageJob& J)
+{
+    if (threadIdx.x < ORB_CNT_SLOTS) gstore4((uint8_t*)(J.counters + threadIdx.x), 0u);
+    // 32 threads per level, the levels side by side
+    for (int l = threadIdx.x >> 5; l < J.nlevels; l += blockDim.x >> 5) {
+        uint8_t* f = J.lv[l].cellflag;
+        const int n = J.lv[l].ncells;
+        for (int i = threadIdx.x & 31; i < n; i += 32) gstore1(f + i, 0);
+    }
+}
+
+template <int V>
+__global__ __launch_bounds__(ORB_CH_T) void pyramid_kernel(const ImageJob* __restrict__ jobs,
+                                                             const RunTable* __restrict__ rt, int chain, int zero)
+{
+    constexpr int T = ORB_CH_T;
+    __shared__ unsigned buf[2][ORB_CH_DWORDS + 4];
+    __shared__ int2 s_row[2][ORB_CH_ROWS];
+    const int tid = threadIdx.x;
+    const int blk = xcd_block(blockIdx.x, gridDim.x);
+    const int tpj = rt->chain_per_job[chain];
+    const int job = tpj > 0 ? blk / tpj : find_segment(rt->chain_start[chain], rt->njobs, blk);
+    const int t = blk - rt->chain_start[chain][job];
+    const ImageJob& J = jobs[job];
+    const ChainJob& C = J.ch[V][chain];
+    const int m = C.m, base = C.base;
+    const ChainWin* xr = C.xr + (size_t)(t % C.tiles_x) * (m + 1);
+    const ChainWin* yr = C.yr + (size_t)(t / C.tiles_x) * (m + 1);
+    if (zero && t == 0) zero_job(J);
+
+    if (!C.staged) {
+        // a window too large for LDS (m = 1): taps read from memory
+        const LevelJob& L = J.lv[base + 1];
+        const LevelJob& P = J.lv[base];
+        const ChainWin cx = xr[1], cy = yr[1];
+        const int nd = ((cx.o1 - 1) >> 2) - (cx.o0 >> 2) + 1;
+        for (int e = tid; e < nd * (cy.o1 - cy.o0); e += T) {
+            const int y = cy.o0 + e / nd, x = cx.o0 + 4 * (e % nd);
+            int sxk[4], nxk[4], tap[4];
+            unsigned sse[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint2 v = gload8((const uint8_t*)(L.xtab + min(x + k, L.w - 1)));
+                sxk[k] = (int)v.x & 0x3FFFFFFF;
+                nxk[k] = min(sxk[k] + 1, P.w - 1);
+                sse[k] = v.x >> 30;
+                tap[k] = (int)v.y;
+            }
+            const uint2 r = gload8((const uint8_t*)(L.ytab + y));
+            gstore4(L.lvl + (unsigned)(y * L.pitch + x),
+                    resize4((const __attribute__((address_space(1))) uint8_t*)P.lvl, __umul24(r.x & 0xFFFFu, P.pitch),
+                            __umul24(r.x >> 16, P.pitch), sxk, nxk, tap, (int)r.y, sse));
+        }
+        return;
+    }
+
+    // Of level base + k: this thread's 4-column group's taps (thread tid
+    // takes group tid % nd, rows tid / nd, + T / nd, ...), and one row entry.
+    uint2 xt[4], yt;
+    auto load_taps = [&](int k) {
+        const LevelJob& L = J.lv[base + k];
+        const int nd = xr[k].nd, c = tid - (int)(__umul24((unsigned)tid, xr[k].rcp) >> 20) * nd, x = xr[k].a + 4 * c;
+#pragma unroll
+        for (int q = 0; q < 4; q++) xt[q] = gload8((const uint8_t*)(L.xtab + min(x + q, L.w - 1)));
+        yt = gload8((const uint8_t*)(L.ytab + min(yr[k].a + min(tid, ORB_CH_ROWS - 1), L.h - 1)));
+    };
+    {
+        // the base window, in whole aligned dwords (level rows start 64-byte
+        // aligned, so no read leaves its row's pitch); the input when it is not
+        // level 0 itself
+        const uint8_t* src = base == 0 ? J.src : J.lv[base].lvl;
+        const int sp = base == 0 ? J.src_pitch : J.lv[base].pitch;
+        const int nd = xr[0].nd, n = nd * (yr[0].b - yr[0].a + 1);
+        const unsigned rcp = xr[0].rcp;            // e / nd, exact for e * nd < 2^20
+        const uint8_t* s0 = src + (size_t)yr[0].a * sp + xr[0].a;
+        load_taps(1);
+        constexpr int Q = 6;
+        for (int e0 = tid; e0 < n; e0 += Q * T) {
+            unsigned d[Q];
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                const int e = min(e0 + T * q, n - 1);
+                const int r = (int)(__umul24((unsigned)e, rcp) >> 20);
+                const unsigned off = (unsigned)(r * sp + 4 * (e - r * nd));
+                d[q] = (sp & 3) == 0 ? gload4(s0 + off) : gload4u(s0 + off);
+            }
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+                if (e0 + T * q < n) buf[0][e0 + T * q] = d[q];
+        }
+        if (tid < ORB_CH_ROWS) s_row[1][tid] = make_int2((int)yt.x, (int)yt.y);
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int k = 1; k <= m; k++) {
+        const LevelJob& L = J.lv[base + k];
+        const int sw = J.lv[base + k - 1].w;
+        const ChainWin cx = xr[k], cy = yr[k];
+        const int nd = cx.nd, nrows = cy.b - cy.a + 1;
+        const int wx0 = xr[k - 1].a, wy0 = yr[k - 1].a, ws = xr[k - 1].nd;
+        const int r0 = (int)(__umul24((unsigned)tid, cx.rcp) >> 20), rstep = (int)(((unsigned)T * cx.rcp) >> 20);
+        const int c = tid - r0 * nd;
+        const unsigned* src = buf[(k - 1) & 1];
+        unsigned* dst = buf[k & 1];
+        int sxk[4], nxk[4], tap[4];
+        unsigned sse[4];                           // SSE2 rounding for the column (xtab bit 30)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int sx = (int)xt[q].x & 0x3FFFFFFF;
+            sse[q] = xt[q].x >> 30;
+            sxk[q] = sx - wx0;
+            nxk[q] = min(sx + 1, sw - 1) - wx0;
+            tap[q] = (int)xt[q].y;
+        }
+        if (k < m) load_taps(k + 1);               // in flight under this level's rows
+        // Rounding of the window's columns: all scalar, all SSE2, or per
+        // column where it reaches the last columns the SSE2 kernel leaves to
+        // the scalar pass.
+        const int rmode = L.rs_end == 0 ? 0 : (cx.b < L.rs_end ? 1 : 2);
+        const int x = cx.a + 4 * c;
+        const bool xin = x >= cx.o0 && x < cx.o1;
+        const int pitch = L.pitch;
+        uint8_t* out = L.lvl + (unsigned)(cy.a * pitch + x);
+        auto emit = [&](int ey, unsigned d) {
+            if (k < m) dst[ey * nd + c] = d;
+            if (xin && cy.a + ey >= cy.o0 && cy.a + ey < cy.o1) gstore4(out + (unsigned)(ey * pitch), d);
+        };
+        if (r0 < rstep) {
+            // The four pixels' source bytes usually lie within 8 bytes (scale
+            // factors up to ~2.3).
+            if (nxk[3] - sxk[0] <= 7) {
+                const unsigned* wd = src + (sxk[0] >> 2);
+                const unsigned shb = (unsigned)(sxk[0] & 3);
+                unsigned sel[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    sel[q] = 0x0C000C00u | ((unsigned)(nxk[q] - sxk[0]) << 16) | (unsigned)(sxk[q] - sxk[0]);
+                auto rows = [&](auto mode) {
+                    // two rows at a time, so that their LDS reads overlap
+                    // (the second repeats the first where there is none)
+                    for (int ey = r0; ey < nrows; ey += 2 * rstep) {
+                        const int ez = ey + rstep < nrows ? ey + rstep : ey;
+                        const int2 yv = s_row[k & 1][ey], zv = s_row[k & 1][ez];
+                        const unsigned d = resize_dword<decltype(mode)::value>(
+                            wd + __umul24(((unsigned)yv.x & 0xFFFFu) - wy0, ws),
+                            wd + __umul24(((unsigned)yv.x >> 16) - wy0, ws), shb, sel, tap, (unsigned)yv.y, sse);
+                        const unsigned f = resize_dword<decltype(mode)::value>(
+                            wd + __umul24(((unsigned)zv.x & 0xFFFFu) - wy0, ws),
+                            wd + __umul24(((unsigned)zv.x >> 16) - wy0, ws), shb, sel, tap, (unsigned)zv.y, sse);
+                        emit(ey, d);
+                        if (ez != ey) emit(ez, f);
+                    }
+                };
+                if (rmode == 1) rows(ModeTag<1>{});
+                else if (rmode == 0) rows(ModeTag<0>{});
+                else rows(ModeTag<2>{});
+            } else {
+                for (int ey = r0; ey < nrows; ey += rstep) {
+                    const int2 yv = s_row[k & 1][ey];
+                    emit(ey, resize4((const uint8_t*)src, __umul24(((unsigned)yv.x & 0xFFFFu) - wy0, 4 * ws),
+                                     __umul24(((unsigned)yv.x >> 16) - wy0, 4 * ws), sxk, nxk, tap, yv.y, sse));
+                }
+            }
+        }
+        if (k < m) {
+            if (tid < ORB_CH_ROWS) s_row[(k + 1) & 1][tid] = make_int2((int)yt.x, (int)yt.y);
+            __syncthreads();
+        }
+    }
+}
+
+// LDS that the phases use one after another: the horizontal blur sums (phase
+// 2), then the FAST queue and the tile's candidate list (phases 3-5).
 template <int TH>
 union LevelScratch {
-    unsigned win[LW_MAX];
     uint4 hs[TH + 6][LT_W / 4];
     struct {
         unsigned short queue[(TH + 2) * (LT_W + 2)];
@@ -317,6 +550,7 @@ union LevelScratch {
     } f;
 };
 
+// level < 0: the tiles of every level whose tile height is TH.
 template <int TH>
 __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__ jobs,
                                                     const RunTable* __restrict__ rt, int level)
@@ -324,7 +558,6 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
     __shared__ __align__(16) unsigned pxw[(TH + 2 * LT_HALO)][LP_WD];   // level pixels, tile + 4-px halo
     __shared__ unsigned mmw[(TH + 2)][LP_WD];         // FAST strength, tile + 1-px ring
     __shared__ LevelScratch<TH> u;
-    __shared__ int xs0[LP_W], xa[LP_W], ys0[(TH + 2 * LT_HALO)], yb[(TH + 2 * LT_HALO)];
     __shared__ int s_qn, s_nq, s_kn, s_base;
     __shared__ int s_col[LT_W], s_row[TH];      // FAST cell of each tile column / row, edge flags
     const uint8_t* px = (const uint8_t*)pxw;
@@ -334,7 +567,13 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
     // Every wave finds its tile itself (uniform scalar loads), so the first
     // barrier comes only after the tile's memory reads have been issued; the
     // counters cleared here are first used after that barrier.
-    const int blk = xcd_block(blockIdx.x, gridDim.x);
+    int blk = xcd_block(blockIdx.x, gridDim.x);
+    if (level < 0) {
+        const int* starts = rt->all_start[TH == 16 ? 1 : 0];
+        level = 0;
+        while (blk >= starts[level + 1]) level++;
+        blk -= starts[level];
+    }
     const int tpj = rt->tiles_per_job[level];
     const int job = tpj > 0 ? blk / tpj : find_segment(rt->tile_start[level], rt->njobs, blk);
     if (tid == 0) {
@@ -372,224 +611,38 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
         }
     };
 
-    // A resized dword of the tile proper (px row ey, dword c) also goes
-    // straight to the level image.
-    auto level_out = [&](int ey, int c, unsigned d) {
-        const int y = ty0 + ey - LT_HALO, x0 = tx0 + 4 * (c - 1);
-        if (ey >= LT_HALO && ey < LT_HALO + TH && c >= 1 && c <= LT_W / 4 && y < h) {
-            uint8_t* dst = L.lvl + (unsigned)(y * pitch + x0);
-            if (x0 + 3 < w) {
-                gstore4(dst, d);
-            } else {
-                for (int k = 0; k < 4; k++)
-                    if (x0 + k < w) dst[k] = (uint8_t)(d >> (8 * k));
-            }
-        }
-    };
-
-    // ---- 1. pixels with halo, one dword (4 columns) per slot
-    if (level == 0) {
-        const uint8_t* src = J.src;
-        const int sp = J.src_pitch;
-        if (interior) {
-            // The 720 dwords, 3 per thread, read before any wait (indexes past
-            // the end repeat the last dword); aligned when the input sits in
-            // level 0, whose rows are 64-byte aligned.
-            unsigned d[3];
+    // ---- 1. pixels with halo, one dword (4 columns) per slot: 720 (or 432)
+    // dwords, 3 per thread, read before any wait (indexes past the end repeat
+    // the last dword).  A border tile reads reflected rows (REFLECT_101), and
+    // bytewise the dwords that reach past a level edge, as far as the halo is
+    // used (3 pixels).
+    {
+        const uint8_t* src = level == 0 ? J.src : L.lvl;
+        const int sp = level == 0 ? J.src_pitch : pitch;
+        unsigned d[3];
 #pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const int e = min(tid + 256 * k, (TH + 2 * LT_HALO) * LP_WD - 1);
-                const int ey = e / LP_WD, ex = (e - ey * LP_WD) * 4;
-                const unsigned off = (unsigned)((ty0 - LT_HALO + ey) * sp + (tx0 - LT_HALO + ex));
+        for (int k = 0; k < 3; k++) {
+            const int e = min(tid + 256 * k, (TH + 2 * LT_HALO) * LP_WD - 1);
+            const int ey = e / LP_WD, x = tx0 - LT_HALO + (e - ey * LP_WD) * 4;
+            int y = ty0 - LT_HALO + ey;
+            if (!interior) y = reflect101(y, h);
+            const unsigned off = (unsigned)(y * sp + x);
+            if (interior || (x >= 0 && x + 3 < w)) {
                 d[k] = (sp & 3) == 0 ? gload4(src + off) : gload4u(src + off);
-            }
-            cell_tables();
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const int e = tid + 256 * k;
-                if (e < (TH + 2 * LT_HALO) * LP_WD) pxw[e / LP_WD][e % LP_WD] = d[k];
-            }
-        } else {
-            cell_tables();
-            for (int e = tid; e < (TH + 2 * LT_HALO) * LP_WD; e += 256) {
-                const int ey = e / LP_WD, ex = (e - ey * LP_WD) * 4;
-                const int y = reflect101(ty0 - LT_HALO + ey, h);
+            } else {
+                d[k] = 0;
                 const uint8_t* r = src + (size_t)y * sp;
-                unsigned d = 0;
+                if (x < w + LT_HALO) {
 #pragma unroll
-                for (int k = 0; k < 4; k++) d |= (unsigned)r[reflect101(tx0 - LT_HALO + ex + k, w)] << (8 * k);
-                pxw[ey][ex >> 2] = d;
-            }
-        }
-    } else {
-        // cv::resize INTER_LINEAR 8U fixed point from level l-1: the source
-        // index and 11-bit taps of each column and row come from the level's
-        // tables (computed on the host with OpenCV's double/float statements).
-        const LevelJob& P = J.lv[level - 1];
-        const int sw = P.w, sp = P.pitch;
-        // The source rectangle the tile reads (the level's per-tile-column and
-        // per-tile-row tables), in whole aligned dwords (level rows start
-        // 64-byte aligned, so no read leaves its row's pitch).  It is staged
-        // in LDS when it fits, in the same memory round trip as the taps;
-        // otherwise (scale factors near 2 and above) the taps are read from
-        // global memory directly.
-        const uint2 xw = cload8(L.xwin + t % L.tiles_x), yw = cload8(L.ywin + t / L.tiles_x);
-        const int wx0 = (int)xw.x & ~3, wy0 = (int)yw.x;
-        const int nwd = ((int)xw.y >> 2) - (wx0 >> 2) + 1, nwr = (int)yw.y - wy0 + 1;
-        const bool staged = nwd <= 64 && nwd * nwr <= LW_MAX;
-        // All reads are issued before the first wait: one tap table entry per
-        // thread (columns: threads 0..71, rows: 128..167) and the first
-        // LS_K * 256 window dwords, in row-major order (row = e / nwd by a
-        // 20-bit reciprocal, exact for e * nwd < 2^20).
-        // (The row table follows the column table: ytab == xtab + w.)
-        const int ti = tid < 128 ? reflect101(tx0 - LT_HALO + min(tid, LP_W - 1), w)
-                                 : w + reflect101(ty0 - LT_HALO + min(tid - 128, (TH + 2 * LT_HALO) - 1), h);
-        const uint2 tv = gload8((const uint8_t*)(L.xtab + ti));
-        const int nst = staged ? nwd * nwr : 0;
-        const unsigned rcp = ((1u << 20) + (unsigned)nwd - 1u) / (unsigned)nwd;
-        const uint8_t* srow = P.lvl + (size_t)wy0 * sp + wx0;
-        unsigned wv[LS_K];
-        if (nst > 0) {
-            // unconditional reads (indexes past the window repeat its last
-            // dword), so that none of them waits for another
-#pragma unroll
-            for (int k = 0; k < LS_K; k++) {
-                const int e = min(tid + 256 * k, nst - 1);
-                const int r = (int)(__umul24((unsigned)e, rcp) >> 20);
-                wv[k] = gload4(srow + (unsigned)(r * sp + 4 * (e - r * nwd)));
+                    for (int q = 0; q < 4; q++) d[k] |= (unsigned)gload1(r + reflect101(x + q, w)) << (8 * q);
+                }
             }
         }
         cell_tables();
-        if (tid < LP_W) {
-            xs0[tid] = (int)tv.x;
-            xa[tid] = (int)tv.y;
-        } else if (tid >= 128 && tid < 128 + (TH + 2 * LT_HALO)) {
-            ys0[tid - 128] = (int)tv.x;
-            yb[tid - 128] = (int)tv.y;
-        }
 #pragma unroll
-        for (int k = 0; k < LS_K; k++)
-            if (tid + 256 * k < nst) u.win[tid + 256 * k] = wv[k];
-        for (int e = tid + 256 * LS_K; e < nst; e += 256) {
-            const int r = (int)(__umul24((unsigned)e, rcp) >> 20);
-            u.win[e] = gload4(srow + (unsigned)(r * sp + 4 * (e - r * nwd)));
-        }
-        __syncthreads();
-        // Each of 252 threads owns one 4-column group (taps kept in
-        // registers) and rows r0, r0 + 14, r0 + 28 of the tile.
-        if (tid < 14 * LP_WD) {
-            const int c = tid % LP_WD, r0 = tid / LP_WD;
-            const int xoff = staged ? wx0 : 0;
-            int sxk[4], nxk[4], tap[4];
-            unsigned sse[4];                       // SSE2 rounding for the column (xtab bit 30)
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int e = xs0[4 * c + k];
-                const int sx = e & 0x3FFFFFFF;
-                sse[k] = (unsigned)e >> 30;
-                sxk[k] = sx - xoff;
-                nxk[k] = (sx + 1 < sw ? sx + 1 : sx) - xoff;
-                tap[k] = xa[4 * c + k];
-            }
-            // Rounding of the tile's columns (reflected halo included): all
-            // scalar, all SSE2, or per column where the tile reaches the last
-            // columns the SSE2 kernel leaves to the scalar pass.
-            const int maxcol = max(min(tx0 + LT_W + LT_HALO - 1, w - 1), LT_HALO);
-            const int rmode = L.rs_end == 0 ? 0 : (maxcol < L.rs_end ? 1 : 2);
-            // The four pixels' source bytes usually lie within 8 bytes (scale
-            // factors up to ~2.3; reflected halo columns may run backwards, so
-            // the span is taken over all of them): then a source row is three
-            // aligned dword reads realigned by two v_alignbyte, each pixel's
-            // tap pair (p[sx], p[nx]) one v_perm into 16-bit lanes, and S one
-            // v_dot2_u32_u16 with the packed taps (a0 | a1 << 16).
-            int b0 = sxk[0], b1 = nxk[0];
-#pragma unroll
-            for (int k = 1; k < 4; k++) {
-                b0 = min(b0, sxk[k]);
-                b1 = max(b1, nxk[k]);
-            }
-            if (staged && b1 - b0 <= 7) {
-                const unsigned* wd = u.win + (b0 >> 2);
-                const unsigned shb = (unsigned)(b0 & 3);
-                const int ws = nwd;                        // window row stride in dwords
-                unsigned sel[4];
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                    sel[k] = 0x0C000C00u | ((unsigned)(nxk[k] - b0) << 16) | (unsigned)(sxk[k] - b0);
-                auto rows = [&](auto mode) {
-                    constexpr int MODE = decltype(mode)::value;
-                    for (int ey = r0; ey < (TH + 2 * LT_HALO); ey += 14) {
-                        const unsigned sy01 = (unsigned)ys0[ey];
-                        const unsigned* q0 = wd + __umul24((sy01 & 0xFFFFu) - wy0, ws);
-                        const unsigned* q1 = wd + __umul24((sy01 >> 16) - wy0, ws);
-                        const unsigned w00 = __builtin_amdgcn_alignbyte(q0[1], q0[0], shb);
-                        const unsigned w01 = __builtin_amdgcn_alignbyte(q0[2], q0[1], shb);
-                        const unsigned w10 = __builtin_amdgcn_alignbyte(q1[1], q1[0], shb);
-                        const unsigned w11 = __builtin_amdgcn_alignbyte(q1[2], q1[1], shb);
-                        const unsigned ybv = (unsigned)yb[ey];
-                        unsigned d = 0;
-                        if constexpr (MODE == 1) {
-                            // SSE2 rounding with the horizontal taps scaled by
-                            // 16: S16 = 16 S, so S16 & 0xFFFF00 = (S >> 4) << 8
-                            // (S16 < 2^23), and the high word of its product
-                            // with b << 8 is ((S >> 4) * b) >> 16 in one
-                            // v_mul_hi_u32_u24.  t = h0 + h1 + 2 <= 1023 fits
-                            // a 16-bit lane: the >> 2 is done two pixels at a
-                            // time and the four bytes gathered by one v_perm.
-                            const unsigned bs0 = (ybv << 8) & 0xFFFF00u, bs1 = (ybv >> 8) & 0xFFFF00u;
-                            unsigned t[4];
-#pragma unroll
-                            for (int k = 0; k < 4; k++) {
-                                const orb_u16x2 tk = __builtin_bit_cast(orb_u16x2, (unsigned)tap[k] << 4);
-                                const unsigned S0 = __builtin_amdgcn_udot2(
-                                    __builtin_bit_cast(orb_u16x2, __builtin_amdgcn_perm(w01, w00, sel[k])), tk, 0u, false);
-                                const unsigned S1 = __builtin_amdgcn_udot2(
-                                    __builtin_bit_cast(orb_u16x2, __builtin_amdgcn_perm(w11, w10, sel[k])), tk, 0u, false);
-                                t[k] = mulhi_u24(S0 & 0xFFFF00u, bs0) + mulhi_u24(S1 & 0xFFFF00u, bs1) + 2u;
-                            }
-                            const orb_u16x2 two = {2, 2};
-                            const unsigned u01 = __builtin_bit_cast(unsigned, __builtin_bit_cast(orb_u16x2, t[0] | (t[1] << 16)) >> two);
-                            const unsigned u23 = __builtin_bit_cast(unsigned, __builtin_bit_cast(orb_u16x2, t[2] | (t[3] << 16)) >> two);
-                            d = __builtin_amdgcn_perm(u23, u01, 0x06040200u);
-                        } else {
-                            const unsigned bv0 = ybv & 0xFFFFu, bv1 = ybv >> 16;
-#pragma unroll
-                            for (int k = 0; k < 4; k++) {
-                                const orb_u16x2 tk = __builtin_bit_cast(orb_u16x2, (unsigned)tap[k]);
-                                const unsigned S0 = __builtin_amdgcn_udot2(
-                                    __builtin_bit_cast(orb_u16x2, __builtin_amdgcn_perm(w01, w00, sel[k])), tk, 0u, false);
-                                const unsigned S1 = __builtin_amdgcn_udot2(
-                                    __builtin_bit_cast(orb_u16x2, __builtin_amdgcn_perm(w11, w10, sel[k])), tk, 0u, false);
-                                d |= vresize<MODE>(S0, S1, bv0, bv1, sse[k]) << (8 * k);
-                            }
-                        }
-                        pxw[ey][c] = d;
-                        level_out(ey, c, d);
-                    }
-                };
-                if (rmode == 1) rows(ModeTag<1>{});
-                else if (rmode == 0) rows(ModeTag<0>{});
-                else rows(ModeTag<2>{});
-            } else if (staged) {
-                const uint8_t* wb = (const uint8_t*)u.win;
-                const int ws = nwd * 4;
-                for (int ey = r0; ey < (TH + 2 * LT_HALO); ey += 14) {
-                    const unsigned sy01 = (unsigned)ys0[ey];
-                    const unsigned d = resize4(wb, __umul24((sy01 & 0xFFFFu) - wy0, ws),
-                                               __umul24((sy01 >> 16) - wy0, ws), sxk, nxk, tap, yb[ey], sse);
-                    pxw[ey][c] = d;
-                    level_out(ey, c, d);
-                }
-            } else {
-                for (int ey = r0; ey < (TH + 2 * LT_HALO); ey += 14) {
-                    const unsigned sy01 = (unsigned)ys0[ey];
-                    const unsigned d = resize4((const __attribute__((address_space(1))) uint8_t*)P.lvl,
-                                               __umul24(sy01 & 0xFFFFu, sp), __umul24(sy01 >> 16, sp), sxk, nxk, tap,
-                                               yb[ey], sse);
-                    pxw[ey][c] = d;
-                    level_out(ey, c, d);
-                }
-            }
+        for (int k = 0; k < 3; k++) {
+            const int e = tid + 256 * k;
+            if (e < (TH + 2 * LT_HALO) * LP_WD) pxw[e / LP_WD][e % LP_WD] = d[k];
         }
     }
     __syncthreads();
@@ -599,7 +652,7 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
     // pass on the row sums, symmetric taps.
     const int gc = tid & 15;                      // 4-column group of the tile
     // Level 0 copied out when the input is not level 0 itself (levels >= 1
-    // are written by the resize).
+    // are the pyramid kernel's).
     if (level == 0 && J.src != L.lvl) {
         for (int r = tid >> 4; r < TH; r += 16) {
             const int y = ty0 + r, x0 = tx0 + 4 * gc;
@@ -1906,19 +1959,11 @@ __global__ __launch_bounds__(256) void describe_kernel(const ImageJob* __restric
 }
 
 // ============================================================ zero fill
-// Counters and per-cell flags of every job (one workgroup per job).
+// Counters and per-cell flags of every job (one workgroup per job), for runs
+// whose pyramid launch does not clear them.
 __global__ void zero_counters_kernel(const ImageJob* __restrict__ jobs, int njobs)
 {
-    const int j = blockIdx.x;
-    if (j >= njobs) return;
-    const ImageJob& J = jobs[j];
-    if (threadIdx.x < ORB_CNT_SLOTS) gstore4((uint8_t*)(J.counters + threadIdx.x), 0u);
-    // 32 threads per level, the levels side by side
-    for (int l = threadIdx.x >> 5; l < J.nlevels; l += blockDim.x >> 5) {
-        uint8_t* f = J.lv[l].cellflag;
-        const int n = J.lv[l].ncells;
-        for (int i = threadIdx.x & 31; i < n; i += 32) gstore1(f + i, 0);
-    }
+    if ((int)blockIdx.x < njobs) zero_job(jobs[blockIdx.x]);
 }
 
 // ========================================================= Hamming helpers
@@ -2502,20 +2547,42 @@ __global__ __launch_bounds__(256) void save_prev_kernel(const MatchArgs* __restr
 
 // ============================================================= launchers
 // ev (optional): events recorded after each stage -- [0] start, then one per
-// pyramid level (max_levels), octree, describe.
+// pyramid level (max_levels; level 1 with the resize of all levels), octree,
+// describe.  Without events the levels' tiles are one launch.
 extern "C" hipError_t orb_launch_extract(const ImageJob* d_jobs, const RunTable* d_rt, const RunTable* h_rt,
                                          hipStream_t st, hipEvent_t* ev)
 {
     int e = 0;
     if (ev) (void)hipEventRecord(ev[e++], st);
-    zero_counters_kernel<<<h_rt->njobs, 256, 0, st>>>(d_jobs, h_rt->njobs);
-    for (int l = 0; l < h_rt->max_levels; l++) {
-        const int nb = h_rt->tile_start[l][h_rt->njobs];
-        if (nb > 0) {
-            if (h_rt->tile_h[l] == 16) level_kernel<16><<<nb, 256, 0, st>>>(d_jobs, d_rt, l);
-            else level_kernel<32><<<nb, 256, 0, st>>>(d_jobs, d_rt, l);
+    auto pyramid = [&](int zero) {
+        for (int c = 0; c < h_rt->nchains; c++) {
+            const int nb = h_rt->chain_start[c][h_rt->njobs];
+            if (nb <= 0) continue;
+            if (h_rt->chain_variant == 0)
+                pyramid_kernel<0><<<nb, ORB_CH_T, 0, st>>>(d_jobs, d_rt, c, c == 0 ? zero : 0);
+            else
+                pyramid_kernel<1><<<nb, ORB_CH_T, 0, st>>>(d_jobs, d_rt, c, c == 0 ? zero : 0);
         }
-        if (ev) (void)hipEventRecord(ev[e++], st);
+    };
+    auto tiles = [&](int th, int level) {
+        const int nb = level < 0 ? h_rt->all_start[th == 16 ? 1 : 0][h_rt->max_levels]
+                                 : h_rt->tile_start[level][h_rt->njobs];
+        if (nb <= 0) return;
+        if (th == 16) level_kernel<16><<<nb, 256, 0, st>>>(d_jobs, d_rt, level);
+        else level_kernel<32><<<nb, 256, 0, st>>>(d_jobs, d_rt, level);
+    };
+    if (ev || !h_rt->chain_zeroes) zero_counters_kernel<<<h_rt->njobs, 256, 0, st>>>(d_jobs, h_rt->njobs);
+    if (!ev) {
+        pyramid(h_rt->chain_zeroes);
+        tiles(32, -1);
+        tiles(16, -1);
+    } else {
+        // stage by stage: level 0, then the pyramid with level 1, then the others
+        for (int l = 0; l < h_rt->max_levels; l++) {
+            if (l == 1) pyramid(0);
+            tiles(h_rt->tile_h[l], l);
+            (void)hipEventRecord(ev[e++], st);
+        }
     }
     octree_kernel<<<h_rt->njobs * h_rt->max_levels, OCT_T, 0, st>>>(d_jobs, h_rt->max_levels);
     if (ev) (void)hipEventRecord(ev[e++], st);

@@ -14,6 +14,24 @@
 #define ORB_MAX_ROOTS 16
 #define ORB_LIST_CAP 1024      // quadtree list capacity per level (LDS; one node per octree thread)
 #define ORB_TILE_W 64          // level kernel output tile
+#define ORB_MAX_CHAINS (ORB_MAX_LEVELS - 1)
+// Pyramid kernel: tile of a chain's last level (small for runs of few images,
+// large for many), threads, and the most dwords, dwords a row and rows of a
+// window in LDS.  Large tiles in a batch of 128 images of 1241 x 376: 96 x 48
+// and 6144 dwords 151 us, 64 x 64 153, 128 x 32 155, 64 x 32 and 4096 dwords
+// 175, 128 x 64 with 1024 threads 179; 2560 dwords (three chains) 161.
+#define ORB_CH_VARIANTS 2
+#define ORB_CH_W(v) ((v) ? 96 : 32)
+#define ORB_CH_H(v) ((v) ? 48 : 16)
+#define ORB_CH_T 512
+#define ORB_CH_DWORDS 6144
+#define ORB_CH_COLS 96
+#define ORB_CH_ROWS 160
+// At most this many small tiles: the small variant.  Images of 640 x 480, 8
+// levels, small (one launch) against large (two): 4 images (216 small tiles)
+// 15.0 us against 24.3, 8 20.8 against 25.5, 12 (648) 27.6 against 28.7, 16
+// 34.5 against 31.7, 32 55.6 against 39.7.
+#define ORB_CH_FEW 640
 #define ORB_EDGE 19            // EDGE_THRESHOLD, ORBextractor.cc:81
 #define ORB_MIN_BORDER 16      // EDGE_THRESHOLD - 3, ORBextractor.cc:1049
 
@@ -65,20 +83,39 @@ struct LevelJob {
     unsigned long long* ret;         // kept keypoints in output order
     const int2* xtab;                // levels >= 1: per column {sx | sse2 << 30, a0 | a1 << 16} of the
     const int2* ytab;                // resize from level-1; per row {sy, b0 | b1 << 16}
-    const int2* xwin;                // levels >= 1: per tile column / row, the source
-    const int2* ywin;                // columns / rows {first, last} the tile's taps read
     const unsigned short* octx;      // quadtree place at depth ORB_OCT_D of a candidate at (x, y):
     const unsigned short* octy;      // octx[x] ^ octy[y] (x, y relative to the border)
 };
 
+// A run of pyramid levels that one launch computes, base + 1 .. base + m from
+// base, a workgroup per tile of the last.  Per tile column (and row), m + 1
+// entries, of base first: the first and last column a workgroup needs of the
+// level (a, b), the [o0, o1) it writes, and for columns the window's dwords a
+// row and ceil(2^20 / dwords).
+struct ChainWin {
+    int a, b, o0, o1;
+    int nd;
+    unsigned rcp;
+    int pad[2];
+};
+struct ChainJob {
+    int base, m;
+    int tiles_x, tiles_y;
+    int staged;                      // the windows fit in LDS (else m = 1, read from memory)
+    const ChainWin* xr;
+    const ChainWin* yr;
+};
+
 struct ImageJob {
     const uint8_t* src;              // input image (level 0), src_pitch bytes per row; the
-    int src_pitch;                   // level-0 kernel copies it into lv[0].lvl unless it is lv[0].lvl
+    int src_pitch;                   // level kernel copies it into lv[0].lvl unless it is lv[0].lvl
     int nlevels, iniTh, minTh;
     int out_cap;                     // keypoint output capacity
     int* counters;                   // ORB_CNT_SLOTS ints
     OrbKeyPoint* kps;                // out_cap keypoints
     uint8_t* desc;                   // out_cap x 32 bytes
+    int nchains[ORB_CH_VARIANTS];
+    ChainJob ch[ORB_CH_VARIANTS][ORB_MAX_CHAINS];
     LevelJob lv[ORB_MAX_LEVELS];
 };
 
@@ -92,6 +129,12 @@ struct RunTable {
     int desc_start[(ORB_MAX_JOBS + 1) * ORB_MAX_LEVELS];  // describe kernel: first block of (job, level)
     int tiles_per_job[ORB_MAX_LEVELS];  // > 0: every job has this many tiles at the level
     int tile_h[ORB_MAX_LEVELS];         // level kernel tile height at the level (32 or 16)
+    int all_start[2][ORB_MAX_LEVELS + 1];   // one launch for the levels of tile height 32 / 16: first block of each
+    int chain_variant;                  // of the jobs' chains
+    int nchains;                        // pyramid launches
+    int chain_start[ORB_MAX_CHAINS][ORB_MAX_JOBS + 1];   // per pyramid launch: first block of job j
+    int chain_per_job[ORB_MAX_CHAINS];  // > 0: every job has this many blocks
+    int chain_zeroes;                   // the first pyramid launch has a block for every job, and clears its counters
     int desc_per_job;                   // > 0: every job has this many describe blocks
 };
 
