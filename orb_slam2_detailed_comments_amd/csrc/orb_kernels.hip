@@ -26,7 +26,11 @@ __constant__ __align__(16) signed char c_pattern[1024] = {   // BRIEF pairs, x0,
 #include "orb_pattern.inc"
 };
 __constant__ unsigned c_icmask[4 * 16 * 9];   // orientation disc byte masks [alignment][|v|][dword]
-__constant__ int c_gauss[7];   // 7x7 sigma-2 integer taps (sum need not be 256)
+// 7x7 sigma-2 blur as two matrix products: the band matrices of the integer
+// taps (8 bytes of k a lane; the second one's k as level_kernel's first product
+// leaves its rows) and the sums that undo the signed operands' offsets.
+__constant__ __align__(16) uint2 c_band[2][64];
+__constant__ int c_bandsum[2];
 
 // umax16: the orientation disc half-widths of the constructor
 // (ORBextractor.cc:542-570).  Byte k of dword c of a patch row whose first
@@ -47,7 +51,26 @@ extern "C" hipError_t orb_upload_constants(const int* umax16, const int* gauss7)
             }
     hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(c_icmask), m, sizeof(m));
     if (e != hipSuccess) return e;
-    return hipMemcpyToSymbol(HIP_SYMBOL(c_gauss), gauss7, 7 * sizeof(int));
+    uint2 band[2][64];
+    int sum = 0;
+    for (int i = 0; i < 7; i++) sum += gauss7[i];
+    if (sum > 257) return hipErrorInvalidValue;         // a row sum must fit 16 bits
+    for (int lane = 0; lane < 64; lane++) {
+        const int n = lane & 15, g = lane >> 4;
+        unsigned w[2][2] = {};
+        for (int j = 0; j < 8; j++) {
+            // columns: byte k of the window that starts 4 pixels left of the
+            // tile's 16; rows: 4 of each of two 16-row products
+            const int tap[2] = {8 * g + j - n - 1, (j < 4 ? 4 * g + j : 12 + 4 * g + j) - n};
+            for (int d = 0; d < 2; d++)
+                if (tap[d] >= 0 && tap[d] < 7) w[d][j >> 2] |= (unsigned)gauss7[tap[d]] << (8 * (j & 3));
+        }
+        for (int d = 0; d < 2; d++) band[d][lane] = make_uint2(w[d][0], w[d][1]);
+    }
+    e = hipMemcpyToSymbol(HIP_SYMBOL(c_band), band, sizeof(band));
+    if (e != hipSuccess) return e;
+    const int bias[2] = {128 * sum - 32768, sum * (32768 + 128)};
+    return hipMemcpyToSymbol(HIP_SYMBOL(c_bandsum), bias, sizeof(bias));
 }
 
 // ------------------------------------------------------------------ helpers
@@ -170,6 +193,7 @@ __device__ __forceinline__ int lanes_below(unsigned long long mask)
 #define LK_CAP 1536                  // per-tile candidates, both thresholds
 
 typedef unsigned short orb_us2 __attribute__((ext_vector_type(2)));
+typedef int orb_v4i __attribute__((ext_vector_type(4)));
 
 // The largest t + 1 at which the pixel is a FAST-9 corner: the largest minimum
 // over the 16 runs of 9 contiguous ring pixels less the centre, or the centre
@@ -543,25 +567,16 @@ __global__ __launch_bounds__(ORB_CH_T) void pyramid_kernel(const ImageJob* __res
     }
 }
 
-// LDS that the phases use one after another: the horizontal blur sums (phase
-// 2), then the FAST queue and the tile's candidate list (phases 3-5).
-template <int TH>
-union LevelScratch {
-    uint4 hs[TH + 6][LT_W / 4];
-    struct {
-        unsigned short queue[(TH + 2) * (LT_W + 2)];
-        unsigned kloc[LK_CAP];       // tile-local candidate: ly | lx | score | passes
-    } f;
-};
-
 // level < 0: the tiles of every level whose tile height is TH.
 template <int TH>
 __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__ jobs,
                                                     const RunTable* __restrict__ rt, int level)
 {
-    __shared__ __align__(16) unsigned pxw[(TH + 2 * LT_HALO)][LP_WD];   // level pixels, tile + 4-px halo
+    __shared__ __align__(16) unsigned pxw[(TH + 2 * LT_HALO) + 1][LP_WD];   // level pixels, tile + 4-px halo (and what
+                                                                            // the blur's 32-byte windows reach past)
     __shared__ unsigned mmw[(TH + 2)][LP_WD];         // FAST strength, tile + 1-px ring
-    __shared__ LevelScratch<TH> u;
+    __shared__ unsigned short queue[(TH + 2) * (LT_W + 2)];   // FAST candidates
+    __shared__ unsigned kloc[LK_CAP];            // tile-local keypoints: ly | lx | score | passes
     __shared__ int s_qn, s_nq, s_kn, s_base;
     __shared__ int s_col[LT_W], s_row[TH];      // FAST cell of each tile column / row, edge flags
     const uint8_t* px = (const uint8_t*)pxw;
@@ -624,10 +639,16 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
         const uint8_t* src = level == 0 ? J.src : L.lvl;
         const int sp = level == 0 ? J.src_pitch : pitch;
         unsigned d[3];
+        static_assert(256 == 14 * LP_WD + 4, "the next dword is 14 rows and 4 dwords on");
+        int ey = tid / LP_WD, ex = tid - ey * LP_WD;
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            const int e = min(tid + 256 * k, (TH + 2 * LT_HALO) * LP_WD - 1);
-            const int ey = e / LP_WD, x = tx0 - LT_HALO + (e - ey * LP_WD) * 4;
+            if (k) {
+                const int past = ex + 4 >= LP_WD ? 1 : 0;
+                ey = min(ey + 14 + past, TH + 2 * LT_HALO - 1);
+                ex = ex + 4 - past * LP_WD;
+            }
+            const int x = tx0 - LT_HALO + ex * 4;
             int y = ty0 - LT_HALO + ey;
             if (!interior) y = reflect101(y, h);
             const unsigned off = (unsigned)(y * sp + x);
@@ -646,14 +667,12 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
 #pragma unroll
         for (int k = 0; k < 3; k++) {
             const int e = tid + 256 * k;
-            if (e < (TH + 2 * LT_HALO) * LP_WD) pxw[e / LP_WD][e % LP_WD] = d[k];
+            if (e < (TH + 2 * LT_HALO) * LP_WD) (&pxw[0][0])[e] = d[k];
         }
     }
     __syncthreads();
 
-    // ---- 2. the level (copied out) and its 7x7 blur.  Horizontal taps as
-    // two v_dot4_u32_u8 per output on byte quads (v_alignbyte); the vertical
-    // pass on the row sums, symmetric taps.
+    // ---- 2. the level (copied out) and its 7x7 blur
     const int gc = tid & 15;                      // 4-column group of the tile
     // Level 0 copied out when the input is not level 0 itself (levels >= 1
     // are the pyramid kernel's).
@@ -671,75 +690,73 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
             }
         }
     }
-    const unsigned T1 = (unsigned)c_gauss[0] | (c_gauss[1] << 8) | (c_gauss[2] << 16) | ((unsigned)c_gauss[3] << 24);
-    const unsigned T2 = (unsigned)c_gauss[4] | (c_gauss[5] << 8) | (c_gauss[6] << 16);
-    // Two adjacent 4-column groups per task (they share two source dwords).
-    for (int e = tid; e < (TH + 6) * (LT_W / 8); e += 256) {
-        const int rr = e >> 3, c = 2 * (e & 7);  // blur row rr <-> px row rr+1
-        const unsigned* pr = &pxw[rr + 1][c];
-        const unsigned D[4] = {pr[0], pr[1], pr[2], pr[3]};
-#pragma unroll
-        for (int g = 0; g < 2; g++) {
-            const unsigned D0 = D[g], D1 = D[g + 1], D2 = D[g + 2];
-            uint4 o;
-            o.x = __builtin_amdgcn_udot4(__builtin_amdgcn_alignbyte(D1, D0, 1), T1,
-                                         __builtin_amdgcn_udot4(__builtin_amdgcn_alignbyte(D2, D1, 1), T2, 0u, false),
-                                         false);
-            o.y = __builtin_amdgcn_udot4(__builtin_amdgcn_alignbyte(D1, D0, 2), T1,
-                                         __builtin_amdgcn_udot4(__builtin_amdgcn_alignbyte(D2, D1, 2), T2, 0u, false),
-                                         false);
-            o.z = __builtin_amdgcn_udot4(__builtin_amdgcn_alignbyte(D1, D0, 3), T1,
-                                         __builtin_amdgcn_udot4(__builtin_amdgcn_alignbyte(D2, D1, 3), T2, 0u, false),
-                                         false);
-            o.w = __builtin_amdgcn_udot4(D1, T1, __builtin_amdgcn_udot4(D2, T2, 0u, false), false);
-            u.hs[rr][c + g] = o;
-        }
-    }
-    __syncthreads();
+    // The blur: a wavefront takes 16 columns.  Row sums of 16 rows at a time
+    // are pixels (as signed bytes) times the column band; they fit 16 bits,
+    // and a lane then holds 4 rows of one column, which is where the second
+    // product takes its k from: signed high and low bytes times the row band,
+    // laid out so that a lane ends with 4 columns of one row.  Rows and bytes
+    // past the tile's halo meet zero taps.  As two passes of v_dot4 and 24-bit
+    // multiplies through LDS it was 200 vector instructions a wavefront and two
+    // barriers, and the kernel is bound by those: 128 images of 1241 x 376 500 us
+    // so, 460 with the matrix units; 64 of four sizes 280 and 256.
     {
-        // Row sums are <= 255 * 257 and taps < 256: 24-bit multiplies.
-        const unsigned k0 = (unsigned)c_gauss[3], k1 = (unsigned)c_gauss[4], k2 = (unsigned)c_gauss[5],
-                       k3 = (unsigned)c_gauss[6];
-        // rows r .. r + RP - 1 of the tile from 6 + RP row-sum vectors
-        constexpr int RP = TH / 16;
-        static_assert(RP * 16 == TH && 16 * (LT_W / 4) == 256, "RP rows and one column group per thread");
-        const int r = (tid >> 4) * RP, x0 = tx0 + 4 * gc;
+        const int g = lane >> 4, n = lane & 15, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const long colband = __builtin_bit_cast(long, c_band[0][lane]), rowband = __builtin_bit_cast(long, c_band[1][lane]);
+        const int cb = c_bandsum[0], rs = c_bandsum[1];
+        const orb_v4i bias0 = {cb, cb, cb, cb}, bias1 = {rs, rs, rs, rs}, none = {0, 0, 0, 0};
+        unsigned lo[TH / 16 + 1], hi[TH / 16 + 1];
+#pragma unroll
+        for (int t = 0; t <= TH / 16; t++) {
+            uint2 a = *(const uint2*)&pxw[min(16 * t + n + 1, TH + 2 * LT_HALO - 1)][4 * wv + 2 * g];
+            a.x ^= 0x80808080u;
+            a.y ^= 0x80808080u;
+            const orb_v4i sums =                   // row sum - 32768
+                __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, a), colband, bias0, 0, 0, 0);
+            const unsigned p01 = __builtin_amdgcn_perm((unsigned)sums[1], (unsigned)sums[0], 0x05010400u);
+            const unsigned p23 = __builtin_amdgcn_perm((unsigned)sums[3], (unsigned)sums[2], 0x05010400u);
+            lo[t] = __builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u;
+            hi[t] = __builtin_amdgcn_perm(p23, p01, 0x07060302u);
+        }
         // Column rounding: columns < bs_end as OpenCV's SSE2 column kernel
         // (SymmColumnVec_32s8u: the taps as floats k / 2^16, the sum rounded
         // half to even, which for these exact sums is (acc + 0x7FFF + bit 16
         // of acc) >> 16), the others as its scalar one ((acc + 2^15) >> 16).
+        // rb: how many bits of acc's bit 16 count (1 or 0).
+        const int x0 = tx0 + 16 * wv + 4 * g;
         unsigned rb[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) rb[k] = x0 + k < L.bs_end ? 1u : 0u;
-        uint4 q[6 + RP];
 #pragma unroll
-        for (int i = 0; i < 6 + RP; i++) q[i] = u.hs[r + i][gc];
+        for (int t = 0; t < TH / 16; t++) {
+            const orb_v4i high = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                __builtin_bit_cast(long, make_uint2(hi[t], hi[t + 1])), rowband, none, 0, 0, 0);
+            const orb_v4i low = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                __builtin_bit_cast(long, make_uint2(lo[t], lo[t + 1])), rowband, bias1, 0, 0, 0);
+            unsigned v[4];
 #pragma unroll
-        for (int hh = 0; hh < RP; hh++) {
-            const int y = ty0 + r + hh;
-            if (y >= h) continue;
-            unsigned out = 0;
-#define ORB_VBLUR(comp, k)                                                                              \
-            {                                                                                            \
-                const unsigned acc = __umul24(q[hh + 3].comp, k0) +                                      \
-                                     __umul24(q[hh + 2].comp + q[hh + 4].comp, k1) +                     \
-                                     __umul24(q[hh + 1].comp + q[hh + 5].comp, k2) +                     \
-                                     __umul24(q[hh].comp + q[hh + 6].comp, k3);                          \
-                const unsigned v = (acc + (1u << 15) - rb[k] + ((acc >> 16) & rb[k])) >> 16;            \
-                out |= (v > 255u ? 255u : v) << (8 * (k));                                              \
+            for (int k = 0; k < 4; k++) {
+                const unsigned acc = ((unsigned)high[k] << 8) + (unsigned)low[k];
+                v[k] = acc + __builtin_amdgcn_ubfe(acc, 16, rb[k]) + (0x8000u - rb[k]);
             }
-            ORB_VBLUR(x, 0) ORB_VBLUR(y, 1) ORB_VBLUR(z, 2) ORB_VBLUR(w, 3)
-#undef ORB_VBLUR
+            // >> 16, clamped to 255 two at a time, and the four bytes gathered
+            const orb_us2 top = {255, 255};
+            const unsigned v01 = __builtin_bit_cast(unsigned, __builtin_elementwise_min(
+                __builtin_bit_cast(orb_us2, __builtin_amdgcn_perm(v[1], v[0], 0x07060302u)), top));
+            const unsigned v23 = __builtin_bit_cast(unsigned, __builtin_elementwise_min(
+                __builtin_bit_cast(orb_us2, __builtin_amdgcn_perm(v[3], v[2], 0x07060302u)), top));
+            const unsigned out = __builtin_amdgcn_perm(v23, v01, 0x06040200u);
+            const int y = ty0 + 16 * t + n;
             uint8_t* db = L.blur + (unsigned)(y * pitch + x0);
-            if (x0 + 3 < w) {
-                gstore4(db, out);
-            } else {
-                for (int k = 0; k < 4; k++)
-                    if (x0 + k < w) db[k] = (uint8_t)(out >> (8 * k));
+            if (y < h) {
+                if (x0 + 3 < w) {
+                    gstore4(db, out);
+                } else {
+                    for (int k = 0; k < 4; k++)
+                        if (x0 + k < w) db[k] = (uint8_t)(out >> (8 * k));
+                }
             }
         }
     }
-    __syncthreads();                              // hs is reused below
 
     // ---- 3. FAST strength on the tile plus a 1-px ring, detection areas
     // only.  The cardinal pre-test runs on 12-pixel groups (two pixels per
@@ -830,7 +847,7 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
             // queue entry: m-row << 8 | byte column in mmw (tile col + 4)
             const unsigned ebase = ((unsigned)my << 8) | (unsigned)(12 * g);
             for (unsigned m = cand; m; m &= m - 1)
-                u.f.queue[pos++] = (unsigned short)(ebase + (unsigned)__builtin_ctz(m));
+                queue[pos++] = (unsigned short)(ebase + (unsigned)__builtin_ctz(m));
         }
     }
     __syncthreads();
@@ -846,7 +863,7 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
         for (int h = 0; h < 2; h++) {
             const int q = q0 + 256 * h + tid;
             if (q < qn) {
-                e[h] = u.f.queue[q];
+                e[h] = queue[q];
                 const int my = e[h] >> 8, col = e[h] & 255;
                 const int sv = fast_strength(px + (my + 3) * LP_W + col, LP_W);
                 mm[my * LP_W + col] = (uint8_t)sv;
@@ -861,7 +878,7 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
                 int base = 0;
                 if (lane == 0) base = atomicAdd(&s_nq, __popcll(bal));
                 base = __builtin_amdgcn_readfirstlane(base);     // every lane is active here
-                if (keep[h]) u.f.queue[base + lanes_below(bal)] = (unsigned short)e[h];
+                if (keep[h]) queue[base + lanes_below(bal)] = (unsigned short)e[h];
             }
         }
     }
@@ -879,7 +896,7 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
         bool keepA = false, keepB = false;
         unsigned loc = 0u;
         if (q < nq) {
-            const int e = u.f.queue[q];
+            const int e = queue[q];
             const int ly = (e >> 8) - 1, lx = (e & 255) - 4;
             const uint8_t* mrow = mm + (ly + 1) * LP_W + (lx + 4);
             const int mc = mrow[0];
@@ -908,7 +925,7 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
             if (lane == 0) base = atomicAdd(&s_kn, __popcll(bal));
             base = __builtin_amdgcn_readfirstlane(base);     // every lane is active here
             const int pos = base + lanes_below(bal);
-            if (keep && pos < LK_CAP) u.f.kloc[pos] = loc | (keepA ? 1u << 19 : 0u) | (keepB ? 1u << 20 : 0u);
+            if (keep && pos < LK_CAP) kloc[pos] = loc | (keepA ? 1u << 19 : 0u) | (keepB ? 1u << 20 : 0u);
         }
     }
     __syncthreads();
@@ -925,7 +942,7 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
     const int base = s_base;
     for (int i = tid; i < min(kn, LK_CAP); i += 256) {
         if (base + i >= L.key_cap) break;
-        const unsigned loc = u.f.kloc[i];
+        const unsigned loc = kloc[i];
         const int x = tx0 + (int)(loc & 63u), y = ty0 + (int)((loc >> 6) & 31u);
         const int mc = (int)((loc >> 11) & 255u);
         const int cj = s_col[loc & 63u] & 0xFFFF, ci = s_row[(loc >> 6) & 31u] & 0xFFFF;
