@@ -114,14 +114,14 @@ struct LevelPlan {
     int nIni;
     float hX;
     int root_x[ORB_MAX_ROOTS + 1];
-    int key_cap, list_cap;
-    size_t key_off, ret_off, cell_off;
+    int key_cap, seg_cap, list_cap;
+    size_t key_off, seg_off, ret_off, cell_off;
 };
 
 struct Plan {
     int W = 0, H = 0;
     LevelPlan lv[ORB_MAX_LEVELS];
-    size_t img_bytes = 0, nkeys = 0, nret = 0, ncells = 0;
+    size_t img_bytes = 0, nkeys = 0, nseg = 0, nret = 0, ncells = 0;
     int out_cap = 0;
 };
 
@@ -328,7 +328,7 @@ struct orb_extractor {
         p = Plan();
         p.W = W;
         p.H = H;
-        size_t img = 0, nk = 0, nr = 0, ncell = 0;
+        size_t img = 0, nk = 0, ns = 0, nr = 0, ncell = 0;
         int out = 0;
         for (int l = 0; l < nlevels; l++) {
             LevelPlan& L = p.lv[l];
@@ -361,20 +361,34 @@ struct orb_extractor {
             L.hX = (float)(L.maxBorderX - minBorderX) / L.nIni;
             for (int i = 0; i <= L.nIni; i++) L.root_x[i] = (int)(L.hX * (float)i);
             // Strict 3x3 non-max suppression keeps at most one pixel per 2x2
-            // block of a cell; candidates of both thresholds are stored.
-            L.key_cap = 2 * L.ncells * ((L.wCell + 1) / 2) * ((L.hCell + 1) / 2);
+            // block of a cell and threshold.  The quadtree keeps one threshold
+            // a cell; the lists hold both, of every tile that appends to them:
+            // a tile of 64 columns meets at most 62 / wCell + 2 cells' columns,
+            // half of which, each rounded up, hold candidates; rows likewise.
+            // (For either tile height, so that a change of heights moves no
+            // buffer.)
+            L.key_cap = L.ncells * ((L.wCell + 1) / 2) * ((L.hCell + 1) / 2);
+            L.seg_cap = 0;
+            for (int th = 16; th <= 32; th += 16) {
+                const int per_tile = 2 * ((ORB_TILE_W + (ORB_TILE_W - 2) / L.wCell + 2) / 2) * ((th + (th - 2) / L.hCell + 2) / 2);
+                const int tiles = L.tiles_x * ((L.h + th - 1) / th);
+                L.seg_cap = std::max(L.seg_cap, (tiles + ORB_SEGS - 1) / ORB_SEGS * per_tile);
+            }
             L.cell_off = ncell;
             ncell += (size_t)L.ncells;
             L.list_cap = std::max(quota[l] + 3, 4 * L.nIni);
             if (L.list_cap > ORB_LIST_CAP) return ORB_E_ARG;
             L.key_off = nk;
             nk += (size_t)L.key_cap;
+            L.seg_off = ns;
+            ns += (size_t)ORB_SEGS * L.seg_cap;
             L.ret_off = nr;
             nr += (size_t)L.list_cap;
             out += L.list_cap;
         }
         p.img_bytes = img;
         p.nkeys = nk;
+        p.nseg = ns;
         p.nret = nr;
         p.ncells = ncell;
         p.out_cap = out;
@@ -398,7 +412,7 @@ struct orb_extractor {
         };
         const size_t o_stage = take((size_t)W * H);   // host frames land here (one linear copy)
         const size_t o_lvl = take(p.img_bytes), o_blur = take(p.img_bytes), o_cell = take(p.ncells);
-        const size_t o_keys = take(p.nkeys * 8), o_keys2 = take(p.nkeys * 8), o_node = take(p.nkeys * 4);
+        const size_t o_keys = take(p.nseg * 8), o_segs = take((size_t)nlevels * ORB_SEGS * ORB_SEG_STRIDE * 4), o_keys2 = take(p.nkeys * 8), o_node = take(p.nkeys * 4);
         const size_t o_ret = take(p.nret * 8);
         const size_t o_ctr = take(ORB_CNT_SLOTS * 4);
         const size_t o_kps = take((size_t)p.out_cap * sizeof(OrbKeyPoint));
@@ -471,7 +485,7 @@ struct orb_extractor {
             L.hX = P.hX;
             L.scale = scale[l];
             for (int i = 0; i <= P.nIni; i++) L.root_x[i] = P.root_x[i];
-            L.key_cap = P.key_cap;
+            L.seg_cap = P.seg_cap;
             L.ncells = P.ncells;
             L.list_cap = P.list_cap;
             L.rs_end = rounding ? sse2_resize_end(P.w) : 0;
@@ -479,7 +493,8 @@ struct orb_extractor {
             L.lvl = (uint8_t*)(d_mem + o_lvl + P.img_off);
             L.blur = (uint8_t*)(d_mem + o_blur + P.img_off);
             L.cellflag = (uint8_t*)(d_mem + o_cell + P.cell_off);
-            L.keys = (unsigned long long*)(d_mem + o_keys) + P.key_off;
+            L.segs = (int*)(d_mem + o_segs) + (size_t)l * ORB_SEGS * ORB_SEG_STRIDE;
+            L.keys = (unsigned long long*)(d_mem + o_keys) + P.seg_off;
             L.keys2 = (unsigned long long*)(d_mem + o_keys2) + P.key_off;
             L.node = (int*)(d_mem + o_node) + P.key_off;
             L.ret = (unsigned long long*)(d_mem + o_ret) + P.ret_off;

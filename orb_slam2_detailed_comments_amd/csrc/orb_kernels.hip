@@ -399,6 +399,8 @@ __device__ __forceinline__ unsigned resize_dword(const unsigned* q0, const unsig
 __device__ __forceinline__ void zero_job(const ImageJob& J)
 {
     if (threadIdx.x < ORB_CNT_SLOTS) gstore4((uint8_t*)(J.counters + threadIdx.x), 0u);
+    for (int i = threadIdx.x; i < J.nlevels * ORB_SEGS; i += blockDim.x)
+        gstore4((uint8_t*)(J.lv[i / ORB_SEGS].segs + i % ORB_SEGS * ORB_SEG_STRIDE), 0u);
     // 32 threads per level, the levels side by side
     for (int l = threadIdx.x >> 5; l < J.nlevels; l += blockDim.x >> 5) {
         uint8_t* f = J.lv[l].cellflag;
@@ -930,18 +932,19 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
     }
     __syncthreads();
 
-    // ---- 5. append the tile's candidates to the level list as
+    // ---- 5. append the tile's candidates to one of the level's lists as
     // (score << 32 | cell row, cell col, y, x in cell) | passes
     const int kn = s_kn;
     if (kn == 0) return;
     if (tid == 0) {
-        s_base = atomicAdd(&J.counters[ORB_CNT_KEYS + level], kn);
-        if (kn > LK_CAP || s_base + kn > L.key_cap) atomicOr(&J.counters[ORB_CNT_ERR], ORB_ERR_KEYS);
+        s_base = atomicAdd(L.segs + t % ORB_SEGS * ORB_SEG_STRIDE, kn);
+        if (kn > LK_CAP || s_base + kn > L.seg_cap) atomicOr(&J.counters[ORB_CNT_ERR], ORB_ERR_KEYS);
     }
     __syncthreads();
     const int base = s_base;
+    unsigned long long* keys = L.keys + (size_t)(t % ORB_SEGS) * L.seg_cap;
     for (int i = tid; i < min(kn, LK_CAP); i += 256) {
-        if (base + i >= L.key_cap) break;
+        if (base + i >= L.seg_cap) break;
         const unsigned loc = kloc[i];
         const int x = tx0 + (int)(loc & 63u), y = ty0 + (int)((loc >> 6) & 31u);
         const int mc = (int)((loc >> 11) & 255u);
@@ -951,7 +954,7 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
         const unsigned ok = ((unsigned)ci << 20) | ((unsigned)cj << 12) | (yl << 6) | xl;
         unsigned long long key = ((unsigned long long)(unsigned)(mc - 1) << 32) | ok;
         key |= (unsigned long long)((loc >> 19) & 3u) << 40;         // ORB_KEY_INI, ORB_KEY_MIN
-        gstore8(L.keys + base + i, key);
+        gstore8(keys + base + i, key);
     }
 }
 
@@ -969,6 +972,7 @@ __global__ __launch_bounds__(256) void level_kernel(const ImageJob* __restrict__
 // order, membership and retained keys are exactly the list's.  Ties in the phase-2 sort are broken by creation order
 // (newer = larger), the oracle's fixed stand-in for the heap address.
 #define OCT_T 1024
+static_assert(OCT_T == 64 * ORB_SEGS, "a wavefront per candidate list");
 #define OCT_REG 4                    // general form: candidates per thread held in registers
 #define OCT_D ORB_OCT_D
 #define OCT_KEYS 8192                // fast form: candidates held in LDS (the others in global memory)
@@ -1120,7 +1124,9 @@ __device__ __forceinline__ void child_rect(int rx, int ry, int q, int* crx, int*
 __device__ __forceinline__ bool octree_fast(OctFast& S, const LevelJob& L, int level, int* ctr)
 {
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int K0 = min(ctr[ORB_CNT_KEYS + level], L.key_cap);
+    // this wavefront's candidate list
+    const int K0 = min(L.segs[wv * ORB_SEG_STRIDE], L.seg_cap);
+    const unsigned long long* list = L.keys + (size_t)wv * L.seg_cap;
     const int N = L.quota, n = L.nIni, nCols = L.nCols, ncells = L.ncells;
     const int wC = L.wCell, hC = L.hCell;
     const int nwords = OCT_WORDS(n);
@@ -1139,7 +1145,7 @@ __device__ __forceinline__ bool octree_fast(OctFast& S, const LevelJob& L, int l
     // set alone).
     unsigned long long key[4];
 #pragma unroll
-    for (int m = 0; m < 4; m++) key[m] = gload8u64(L.keys + min(tid + OCT_T * m, max(K0 - 1, 0)));
+    for (int m = 0; m < 4; m++) key[m] = gload8u64(list + min(lane + 64 * m, max(K0 - 1, 0)));
     const bool lds_flags = ncells <= OCT_FLAGS;
     if (lds_flags)
         for (int i = tid; i < ncells; i += OCT_T) S.flag[i] = gload1(L.cellflag + i);
@@ -1147,7 +1153,7 @@ __device__ __forceinline__ bool octree_fast(OctFast& S, const LevelJob& L, int l
     if (tid <= OCT_D) S.na[tid] = S.nm[tid] = 0;
     if (tid == 0) S.nkeys = S.deep = 0;
     __syncthreads();
-    for (int c0 = 0; c0 < K0; c0 += 4 * OCT_T) {
+    for (int c0 = 0; c0 < K0; c0 += 4 * 64) {
         unsigned o[4];
         unsigned long long k[4];
         int cnt = 0;
@@ -1160,12 +1166,12 @@ __device__ __forceinline__ bool octree_fast(OctFast& S, const LevelJob& L, int l
             o[m] = (unsigned)(L.octx[__umul24(j, wC) + xl] ^ L.octy[__umul24(i, hC) + yl]);
             const unsigned c = __umul24(i, nCols) + j;
             const int f = lds_flags ? S.flag[c] : gload1(L.cellflag + c);
-            v[m] = c0 + tid + OCT_T * m < K0 && (k[m] & (f ? ORB_KEY_INI : ORB_KEY_MIN));
+            v[m] = c0 + lane + 64 * m < K0 && (k[m] & (f ? ORB_KEY_INI : ORB_KEY_MIN));
             cnt += v[m] ? 1 : 0;
         }
-        if (c0 + 4 * OCT_T < K0) {
+        if (c0 + 4 * 64 < K0) {
 #pragma unroll
-            for (int m = 0; m < 4; m++) key[m] = gload8u64(L.keys + min(c0 + 4 * OCT_T + tid + OCT_T * m, K0 - 1));
+            for (int m = 0; m < 4; m++) key[m] = gload8u64(list + min(c0 + 4 * 64 + lane + 64 * m, K0 - 1));
         }
         const int inc = wave_scan(cnt);
         int base = 0;
@@ -1406,8 +1412,12 @@ __device__ __forceinline__ bool octree_fast(OctFast& S, const LevelJob& L, int l
 // The general form: any candidate set, pass by pass.
 __device__ __forceinline__ void octree_general(OctGeneral& S, const LevelJob& L, int level, int* ctr)
 {
-    const int tid = threadIdx.x;
-    const int K0 = min(ctr[ORB_CNT_KEYS + level], L.key_cap);
+    const int tid = threadIdx.x, lane = tid & 63;
+    // this wavefront's candidate list, and the longest
+    const int K0 = min(L.segs[(tid >> 6) * ORB_SEG_STRIDE], L.seg_cap);
+    const unsigned long long* list = L.keys + (size_t)(tid >> 6) * L.seg_cap;
+    int longest = 0;
+    for (int s = 0; s < ORB_SEGS; s++) longest = max(longest, min(L.segs[s * ORB_SEG_STRIDE], L.seg_cap));
     const int N = L.quota;
     const int wC = L.wCell, hC = L.hCell;
     int* node = L.node;
@@ -1420,11 +1430,11 @@ __device__ __forceinline__ void octree_general(OctGeneral& S, const LevelJob& L,
     // candidates' order does not matter: the level kernels append them in
     // no fixed order, and every later step depends only on the set.)
     int K = 0;
-    for (int c0 = 0; c0 < K0; c0 += OCT_T * OCT_REG) {
+    for (int c0 = 0; c0 < longest; c0 += 64 * OCT_REG) {
         unsigned long long key[OCT_REG];
         unsigned char flag[OCT_REG];
 #pragma unroll
-        for (int m = 0; m < OCT_REG; m++) key[m] = gload8u64(L.keys + min(c0 + tid + OCT_T * m, K0 - 1));
+        for (int m = 0; m < OCT_REG; m++) key[m] = c0 + lane + 64 * m < K0 ? gload8u64(list + c0 + lane + 64 * m) : 0ull;
 #pragma unroll
         for (int m = 0; m < OCT_REG; m++) {
             const unsigned ok = (unsigned)key[m];
@@ -1434,7 +1444,7 @@ __device__ __forceinline__ void octree_general(OctGeneral& S, const LevelJob& L,
         bool v[OCT_REG];
 #pragma unroll
         for (int m = 0; m < OCT_REG; m++) {
-            v[m] = c0 + tid + OCT_T * m < K0 && (key[m] & (flag[m] ? ORB_KEY_INI : ORB_KEY_MIN));
+            v[m] = c0 + lane + 64 * m < K0 && (key[m] & (flag[m] ? ORB_KEY_INI : ORB_KEY_MIN));
             cnt += v[m] ? 1 : 0;
         }
         int pos = block_scan(cnt, S.scan, half, &total);

@@ -448,13 +448,17 @@ int orb_extractor_debug_candidates(orb_extractor* ex, int level, int* xyr, int c
     if (!ex || !ex->d_mem || !n || level < 0 || level >= ex->nlevels) return ORB_E_ARG;
     HIP_TRY(hipSetDevice(ex->ctx->device));
     HIP_TRY(hipStreamSynchronize(ex->ctx->stream));
-    int c[ORB_CNT_SLOTS];
-    HIP_TRY(hipMemcpy(c, ex->hjob.counters, sizeof(c), hipMemcpyDeviceToHost));
+    int c[ORB_SEGS * ORB_SEG_STRIDE];
     const LevelJob& L = ex->hjob.lv[level];
-    int k = std::min(c[ORB_CNT_KEYS + level], L.key_cap);
-    std::vector<unsigned long long> all(k);
+    HIP_TRY(hipMemcpy(c, L.segs, sizeof(c), hipMemcpyDeviceToHost));
+    std::vector<unsigned long long> all;
     std::vector<uint8_t> flags(L.ncells);
-    if (k) HIP_TRY(hipMemcpy(all.data(), L.keys, (size_t)k * 8, hipMemcpyDeviceToHost));
+    for (int s = 0; s < ORB_SEGS; s++) {
+        const int ks = std::min(c[s * ORB_SEG_STRIDE], L.seg_cap);
+        if (!ks) continue;
+        all.resize(all.size() + ks);
+        HIP_TRY(hipMemcpy(all.data() + all.size() - ks, L.keys + (size_t)s * L.seg_cap, (size_t)ks * 8, hipMemcpyDeviceToHost));
+    }
     HIP_TRY(hipMemcpy(flags.data(), L.cellflag, L.ncells, hipMemcpyDeviceToHost));
     std::vector<unsigned long long> keys;
     for (unsigned long long key : all) {
@@ -462,7 +466,7 @@ int orb_extractor_debug_candidates(orb_extractor* ex, int level, int* xyr, int c
         const bool flagged = flags[((ok >> 20) & 255) * L.nCols + ((ok >> 12) & 255)] != 0;
         if (key & (flagged ? ORB_KEY_INI : ORB_KEY_MIN)) keys.push_back(key & ORB_KEY_RANK);
     }
-    k = (int)keys.size();
+    const int k = (int)keys.size();
     *n = k;
     if (k > capacity) return ORB_E_CAPACITY;
     std::sort(keys.begin(), keys.end(), [](unsigned long long a, unsigned long long b) {

@@ -147,7 +147,7 @@ struct orb_server {
             delete e;
             return -1;
         }
-        const size_t need = p.img_bytes * 2 + p.ncells + p.nkeys * 20 + p.nret * 8 + (size_t)p.out_cap * 96 + 65536;
+        const size_t need = p.img_bytes * 2 + p.ncells + p.nseg * 8 + p.nkeys * 12 + p.nret * 8 + (size_t)p.out_cap * 96 + 65536;
         bool any = false;
         for (const Slot& sl : slots) any |= sl.w == c.w && sl.h == c.h && sl.nfeatures == c.nfeatures;
         if (used + need > budget) {
