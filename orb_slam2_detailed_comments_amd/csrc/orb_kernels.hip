@@ -25,7 +25,7 @@
 __constant__ __align__(16) signed char c_pattern[1024] = {   // BRIEF pairs, x0,y0,x1,y1
 #include "orb_pattern.inc"
 };
-__constant__ unsigned c_icmask[4 * 16 * 9];   // orientation disc byte masks [alignment][|v|][dword]
+__constant__ __align__(16) uint4 c_icmask[4 * 16 * 3];   // orientation disc byte masks [alignment][|v|][16 bytes]
 // 7x7 sigma-2 blur as two matrix products: the band matrices of the integer
 // taps (8 bytes of k a lane; the second one's k as level_kernel's first product
 // leaves its rows) and the sums that undo the signed operands' offsets.
@@ -38,16 +38,16 @@ __constant__ int c_bandsum[2];
 // mask byte is 0xFF iff |u| <= umax[|v|].
 extern "C" hipError_t orb_upload_constants(const int* umax16, const int* gauss7)
 {
-    unsigned m[4 * 16 * 9];
+    unsigned m[4 * 16 * 12];
     for (int al = 0; al < 4; al++)
         for (int av = 0; av < 16; av++)
-            for (int c = 0; c < 9; c++) {
+            for (int c = 0; c < 12; c++) {
                 unsigned w = 0;
                 for (int k = 0; k < 4; k++) {
                     const int u = 4 * c + k - 15 - al;
                     if ((u < 0 ? -u : u) <= umax16[av]) w |= 0xFFu << (8 * k);
                 }
-                m[(al * 16 + av) * 9 + c] = w;
+                m[(al * 16 + av) * 12 + c] = w;
             }
     hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(c_icmask), m, sizeof(m));
     if (e != hipSuccess) return e;
@@ -1808,9 +1808,10 @@ __device__ __forceinline__ void sincos_canonical_dev(double x, double* s, double
 
 // A 16-lane group per kept keypoint, four per wavefront; a workgroup serves
 // 16 keypoints of one (image, level), so the level's geometry and output
-// offset are uniform across it.  Lane j of a group holds patch rows j, j+16
-// (and j+32), each loaded with constant column offsets, and BRIEF pairs
-// 16j .. 16j+15 (descriptor bytes 2j, 2j+1).
+// offset are uniform across it.  The lanes of a group share the rows of its
+// patches; lane j takes BRIEF pairs 16j .. 16j+15 (descriptor bytes 2j, 2j+1).
+// Bound: latency of the patch reads (185 MB from memory in a batch of 128 images
+// of 1241 x 376), with 5 wavefronts a SIMD and half the vector issue slots used.
 #define DESC_G 16
 static_assert(256 / DESC_G == ORB_DESC_KPB, "describe blocks are counted on the host");
 __global__ __launch_bounds__(256) void describe_kernel(const ImageJob* __restrict__ jobs,
@@ -1818,6 +1819,7 @@ __global__ __launch_bounds__(256) void describe_kernel(const ImageJob* __restric
 {
     __shared__ uint2 s_brief[ORB_DESC_KPB][37 * 5];   // per group: 37 rows x 40 bytes
     __shared__ uint4 s_pat[64];
+    __shared__ uint4 s_mask[4 * 16 * 3];
     const int sub = threadIdx.x & (DESC_G - 1), grp = threadIdx.x / DESC_G;
     const int nseg = rt->njobs * rt->max_levels;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -1842,6 +1844,7 @@ __global__ __launch_bounds__(256) void describe_kernel(const ImageJob* __restric
     {
         const int t = threadIdx.x;
         ((unsigned*)s_pat)[(((t >> 2) & 3) * 16 + (t >> 4)) * 4 + (t & 3)] = ((const unsigned*)c_pattern)[t];
+        if (t < 4 * 16 * 3) s_mask[t] = c_icmask[t];
     }
     __syncthreads();
     if (level >= J.nlevels || idx >= (int)gload4((const uint8_t*)(ctr + ORB_CNT_RET + level))) return;   // the whole group leaves
@@ -1862,25 +1865,23 @@ __global__ __launch_bounds__(256) void describe_kernel(const ImageJob* __restric
     // and unused.
     const int xa0 = (cx - 15) & ~3;               // 31 px + <= 3 of alignment: 9 dwords a row
     const int xb0 = (cx - 18) & ~3;               // 37 px + <= 3 of alignment: 10 dwords a row
-    // A row is read as two 16-byte loads and the rest.
-    unsigned pa[2][9], pb[3][10];
-    // Disc rows: lane j holds v = -j and v = +j, which share one disc mask.
+    // Neighbouring lanes read neighbouring pieces of a row, so that a load meets
+    // 64 / 3 or 64 / 5 rows' cache lines and not 64: the orientation patch in 93
+    // pieces of 16 bytes (3 a row, the last of one dword in use), the blur window
+    // in 185 of 8 bytes (5 a row), which is also its layout in LDS.  (A lane per
+    // row was 68 M cache accesses on 128 images of 1241 x 376, this is 39 M: 169
+    // us and 154; 64 images of four sizes 46 and 44.)
+    uint4 pa[6];
+    uint2 pb[12];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const uint8_t* rp = L.lvl + (size_t)(cy + (h ? sub : -sub)) * pitch + xa0;
-        const uint4 q0 = gload16(rp), q1 = gload16(rp + 16);
-        pa[h][0] = q0.x, pa[h][1] = q0.y, pa[h][2] = q0.z, pa[h][3] = q0.w;
-        pa[h][4] = q1.x, pa[h][5] = q1.y, pa[h][6] = q1.z, pa[h][7] = q1.w;
-        pa[h][8] = gload4(rp + 32);
+    for (int k = 0; k < 6; k++) {
+        const int i = min(sub + 16 * k, 92), r = (i * 171) >> 9;          // i / 3
+        pa[k] = gload16(L.lvl + (unsigned)((cy - 15 + r) * pitch + xa0 + 16 * (i - 3 * r)));
     }
 #pragma unroll
-    for (int h = 0; h < 3; h++) {
-        const uint8_t* rp = L.blur + (size_t)(cy - 18 + min(sub + 16 * h, 36)) * pitch + xb0;
-        const uint4 q0 = gload16(rp), q1 = gload16(rp + 16);
-        const uint2 q2 = gload8(rp + 32);
-        pb[h][0] = q0.x, pb[h][1] = q0.y, pb[h][2] = q0.z, pb[h][3] = q0.w;
-        pb[h][4] = q1.x, pb[h][5] = q1.y, pb[h][6] = q1.z, pb[h][7] = q1.w;
-        pb[h][8] = q2.x, pb[h][9] = q2.y;
+    for (int k = 0; k < 12; k++) {
+        const int i = min(sub + 16 * k, 184), r = (i * 205) >> 10;        // i / 5
+        pb[k] = gload8(L.blur + (unsigned)((cy - 18 + r) * pitch + xb0 + 8 * (i - 5 * r)));
     }
 
     // IC_Angle (ORBextractor.cc:94-141): m10 = sum u*I, m01 = sum v*I over
@@ -1889,26 +1890,30 @@ __global__ __launch_bounds__(256) void describe_kernel(const ImageJob* __restric
     // v_dot4_u32_u8 for the masked sum and for sum (u+20)*I.
     const int al = (cx - 15) & 3;                 // u of byte k of dword c: 4c + k - 15 - al
     const unsigned w0 = (unsigned)(5 - al) * 0x01010101u + 0x03020100u;   // bytes u+20 of dword 0
-    int m10 = 0, m01 = 0;
-    const unsigned* mk = c_icmask + (al * 16 + sub) * 9;
-    unsigned mask[9];
+    int m01 = 0;
+    unsigned s1 = 0, su = 0;
 #pragma unroll
-    for (int c = 0; c < 9; c++) mask[c] = mk[c];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int v = h ? sub : -sub;
-        unsigned s1 = 0, su = 0;
-#pragma unroll
-        for (int c = 0; c < 9; c++) {
-            const unsigned md = pa[h][c] & mask[c];
-            s1 = __builtin_amdgcn_udot4(md, 0x01010101u, s1, false);
-            su = __builtin_amdgcn_udot4(md, w0 + (unsigned)(4 * c) * 0x01010101u, su, false);
-        }
-        if (h == 0 || sub > 0) {                  // row v = 0 once
-            m01 += v * (int)s1;
-            m10 += (int)su - 20 * (int)s1;
+    for (int k = 0; k < 6; k++) {
+        const int i = min(sub + 16 * k, 92), r = (i * 171) >> 9, c = i - 3 * r, v = r - 15;
+        uint4 d = pa[k];
+        const uint4 m = s_mask[(al * 16 + max(v, -v)) * 3 + c];
+        d.x &= m.x, d.y &= m.y, d.z &= m.z, d.w &= m.w;
+        unsigned row = __builtin_amdgcn_udot4(d.x, 0x01010101u, 0u, false);
+        row = __builtin_amdgcn_udot4(d.y, 0x01010101u, row, false);
+        row = __builtin_amdgcn_udot4(d.z, 0x01010101u, row, false);
+        row = __builtin_amdgcn_udot4(d.w, 0x01010101u, row, false);
+        const unsigned w = w0 + __builtin_amdgcn_perm(0u, (unsigned)(16 * c), 0u);   // 16 c in each byte
+        unsigned us = __builtin_amdgcn_udot4(d.x, w, 0u, false);
+        us = __builtin_amdgcn_udot4(d.y, w + 0x04040404u, us, false);
+        us = __builtin_amdgcn_udot4(d.z, w + 0x08080808u, us, false);
+        us = __builtin_amdgcn_udot4(d.w, w + 0x0C0C0C0Cu, us, false);
+        if (k < 5 || sub < 13) {                  // 93 pieces
+            m01 += v * (int)row;
+            s1 += row;
+            su += us;
         }
     }
+    int m10 = (int)su - 20 * (int)s1;
     m10 = (int)row16_sum((unsigned)m10);
     m01 = (int)row16_sum((unsigned)m01);
     const float angle_deg = fast_atan2_dev((float)m01, (float)m10);
@@ -1923,13 +1928,8 @@ __global__ __launch_bounds__(256) void describe_kernel(const ImageJob* __restric
     // under the orientation and rotation arithmetic above.
     uint2* win = s_brief[grp];
 #pragma unroll
-    for (int h = 0; h < 3; h++) {
-        const int r = sub + 16 * h;
-        if (r < 37) {
-#pragma unroll
-            for (int c = 0; c < 5; c++) win[r * 5 + c] = make_uint2(pb[h][2 * c], pb[h][2 * c + 1]);
-        }
-    }
+    for (int k = 0; k < 12; k++)
+        if (k < 11 || sub < 9) win[sub + 16 * k] = pb[k];     // 185 pieces
 
     // Rotated BRIEF (ORBextractor.cc:153-204) on the blurred level, sampled
     // from the staged window (row stride 40 bytes, centre at row 18).
