@@ -470,6 +470,7 @@ struct orb_extractor {
             L.h = P.h;
             L.pitch = P.pitch;
             L.tiles_x = P.tiles_x;
+            L.txrcp = (unsigned)((((uint64_t)1 << 31) + P.tiles_x - 1) / P.tiles_x);
             L.tiles_y = P.tiles_y;
             L.nCols = P.nCols;
             L.nRows = P.nRows;
@@ -727,7 +728,10 @@ struct orb_extractor {
             bool eq = n > 0;
             for (int j = 0; j < n; j++)
                 eq = eq && rt.tile_start[l][j + 1] - rt.tile_start[l][j] == rt.tile_start[l][1] - rt.tile_start[l][0];
-            rt.tiles_per_job[l] = eq ? rt.tile_start[l][1] - rt.tile_start[l][0] : 0;
+            const int per = eq ? rt.tile_start[l][1] - rt.tile_start[l][0] : 0;
+            // (the reciprocal is exact while blocks * tiles < 2^31)
+            rt.tiles_per_job[l] = (int64_t)n * per * per < ((int64_t)1 << 31) ? per : 0;
+            rt.tiles_rcp[l] = per > 0 ? (unsigned)((((uint64_t)1 << 31) + per - 1) / per) : 0;
         }
         for (int g = 0; g < 2; g++) {
             int all = 0;

@@ -68,6 +68,7 @@ struct OrbKeyPoint {
 struct LevelJob {
     int w, h, pitch;                 // level size and row pitch (bytes)
     int tiles_x, tiles_y;            // level kernel tiles
+    unsigned txrcp;                  // ceil(2^31 / tiles_x): t / tiles_x = umulhi(2 t, txrcp)
     int nCols, nRows, wCell, hCell;  // FAST cell grid (ORBextractor.cc:1065-1071)
     unsigned wrcp, hrcp;             // ceil(2^32 / wCell), ceil(2^32 / hCell): x / cell = umulhi(x, rcp)
     int maxBorderX, maxBorderY;
@@ -135,7 +136,8 @@ struct RunTable {
     int max_levels;
     int tile_start[ORB_MAX_LEVELS][ORB_MAX_JOBS + 1];   // per level: first tile block of job j
     int desc_start[(ORB_MAX_JOBS + 1) * ORB_MAX_LEVELS];  // describe kernel: first block of (job, level)
-    int tiles_per_job[ORB_MAX_LEVELS];  // > 0: every job has this many tiles at the level
+    int tiles_per_job[ORB_MAX_LEVELS];  // > 0: every job has this many tiles at the level,
+    unsigned tiles_rcp[ORB_MAX_LEVELS]; // and block / tiles = umulhi(2 block, ceil(2^31 / tiles))
     int tile_h[ORB_MAX_LEVELS];         // level kernel tile height at the level (32 or 16)
     int all_start[2][ORB_MAX_LEVELS + 1];   // one launch for the levels of tile height 32 / 16: first block of each
     int chain_variant;                  // of the jobs' chains
