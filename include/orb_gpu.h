@@ -256,7 +256,9 @@ int orb_batch_stereo_results(orb_batch* b, int pair, float* uRight, float* depth
  * every slot's keypoints and descriptors (slot s at keypoints + s *
  * capacity, descriptors + s * capacity * 32, counts[s] of them) and, for
  * stereo pairs, every pair's uRight / depth (pair p at uRight + p * capacity;
- * either may be NULL), with one wait for the counts and one for the data. */
+ * either may be NULL).  The device writes everything into pinned memory at
+ * once, counts first, then groups of slots, and each group is copied out as
+ * soon as it is there. */
 int orb_batch_upload_images(orb_batch* b, int n, const int* slots, const uint8_t* const* images,
                             const size_t* strides);
 int orb_batch_read_all(orb_batch* b, orb_keypoint* keypoints, uint8_t* descriptors, int capacity, int* counts,

@@ -390,9 +390,9 @@ __device__ __forceinline__ unsigned resize_dword(const unsigned* q0, const unsig
 // the host, by tile column and row).  At scale factor 1.2 all seven levels
 // are one launch, with 1.4 times the pixels computed.  Bound: latency (one
 // LDS round trip and barrier per level) in a single call, VALU in a batch.
-// One image of 640 x 480 14.9 us and every level's tiles after it 12.2, where a
-// launch per level that resized its own tile took 82; 128 images of 1241 x 376
-// 151 + 566 us (725).
+// One image of 640 x 480 14.9 us, and every level's tiles after it 12.2 (9 with
+// the tiles' later changes), where a launch per level that resized its own tile
+// took 82; 128 images of 1241 x 376 148 + 566 us (725; 420 for the 566 now).
 // The source index and 11-bit taps of each column and row come from the
 // level's tables (computed on the host with OpenCV's double/float
 // statements).
