@@ -229,6 +229,20 @@ struct CtxRef {
     orb_context* operator->() const { return p; }
 };
 
+// Pinned landing buffer of a call's results, written by the device: counters,
+// then the arrays of an extractor's results, cap entries each.
+struct Landing {
+    char* h = nullptr;
+    int cap = 0;
+    Landing() = default;
+    Landing(const Landing&) = delete;
+    Landing& operator=(const Landing&) = delete;
+    ~Landing()
+    {
+        if (h) (void)hipHostFree(h);
+    }
+};
+
 struct orb_extractor {
     CtxRef ctx;
     int nfeatures = 0, nlevels = 0, iniTh = 0, minTh = 0;
@@ -251,10 +265,7 @@ struct orb_extractor {
     ImageJob* d_job = nullptr;
     RunTable* h_rt = nullptr;
     RunTable* d_rt = nullptr;
-    // pinned landing buffer of a call's results, written by the device:
-    // counters, then six arrays of res_cap entries (res_at)
-    char* h_res = nullptr;
-    int res_cap = 0;
+    Landing land;
     // stereo state (this extractor as the left view)
     float* d_uR = nullptr;
     float* d_depth = nullptr;
@@ -836,26 +847,26 @@ struct orb_extractor {
 
     // Adds the results to a copy list into the pinned buffer: the counters,
     // and as many entries of each wanted array as the device counted.
-    int list_results(const Outputs& o, CopyList& l)
+    int list_results(const Outputs& o, CopyList& l, Landing& to) const
     {
         static_assert(2 * (1 + 2) + 2 <= ORB_COPY_LIST && 1 + kOutArrays <= ORB_COPY_LIST, "a stereo or an RGB-D frame");
-        if (hjob.out_cap > res_cap) {
+        if (hjob.out_cap > to.cap) {
             const size_t cap = (size_t)(hjob.out_cap + 63) / 64 * 64;
-            if (h_res) (void)hipHostFree(h_res);          // its last copies have ended
-            h_res = nullptr;
-            res_cap = 0;
-            if (hipHostMalloc((void**)&h_res, res_at((int)cap, kOutArrays), hipHostMallocCoherent) != hipSuccess) {
-                h_res = nullptr;
+            if (to.h) (void)hipHostFree(to.h);            // its last copies have ended
+            to.h = nullptr;
+            to.cap = 0;
+            if (hipHostMalloc((void**)&to.h, res_at((int)cap, kOutArrays), hipHostMallocCoherent) != hipSuccess) {
+                to.h = nullptr;
                 return ORB_E_OOM;
             }
-            res_cap = (int)cap;
+            to.cap = (int)cap;
         }
         OutArray a[kOutArrays];
         out_arrays(o, a);
-        l.op[l.n++] = CopyOp{(const unsigned*)hjob.counters, (unsigned*)h_res, nullptr, ORB_CNT_SLOTS, 0};
+        l.op[l.n++] = CopyOp{(const unsigned*)hjob.counters, (unsigned*)to.h, nullptr, ORB_CNT_SLOTS, 0};
         for (int i = 0; i < kOutArrays; i++)
             if (a[i].to)
-                l.op[l.n++] = CopyOp{(const unsigned*)a[i].from, (unsigned*)(h_res + res_at(res_cap, i)),
+                l.op[l.n++] = CopyOp{(const unsigned*)a[i].from, (unsigned*)(to.h + res_at(to.cap, i)),
                                      hjob.counters + ORB_CNT_NOUT, hjob.out_cap * a[i].words, a[i].words};
         return ORB_OK;
     }
@@ -869,9 +880,9 @@ struct orb_extractor {
         return at;
     }
     // After the copy list has run: the results into the caller's arrays.
-    int take_results(const Outputs& o, int cap, int* n) const
+    int take_results(const Outputs& o, int cap, int* n, const Landing& at) const
     {
-        const int* c = (const int*)h_res;
+        const int* c = (const int*)at.h;
         if (c[ORB_CNT_ERR]) return ORB_E_OVERFLOW;
         const int cnt = c[ORB_CNT_NOUT];
         *n = cnt;
@@ -879,19 +890,20 @@ struct orb_extractor {
         OutArray a[kOutArrays];
         out_arrays(o, a);
         for (int i = 0; i < kOutArrays; i++)
-            if (a[i].to && cnt > 0) std::memcpy(a[i].to, h_res + res_at(res_cap, i), (size_t)cnt * a[i].words * 4);
+            if (a[i].to && cnt > 0) std::memcpy(a[i].to, at.h + res_at(at.cap, i), (size_t)cnt * a[i].words * 4);
         return ORB_OK;
     }
 
-    int read_results(const Outputs& o, int cap, int* n)
+    int read_results(const Outputs& o, int cap, int* n) { return read_results(o, cap, n, land); }
+    int read_results(const Outputs& o, int cap, int* n, Landing& to) const
     {
         CopyList l;
         l.n = 0;
-        const int rc = list_results(o, l);
+        const int rc = list_results(o, l, to);
         if (rc) return rc;
         HIP_TRY(orb_launch_copy_list(&l, ORB_COPY_BLOCKS, ctx->stream));
         HIP_TRY(hipStreamSynchronize(ctx->stream));
-        return take_results(o, cap, n);
+        return take_results(o, cap, n, to);
     }
     int read_results(orb_keypoint* kps, int cap, uint8_t* desc, int* n)
     {
@@ -963,7 +975,6 @@ struct orb_extractor {
         if (d_job) (void)hipFree(d_job);
         if (d_rt) (void)hipFree(d_rt);
         delete h_rt;
-        if (h_res) (void)hipHostFree(h_res);
         if (d_kin) (void)hipFree(d_kin);
         if (d_din) (void)hipFree(d_din);
         if (d_pair_jobs) (void)hipFree(d_pair_jobs);

@@ -6,6 +6,8 @@
 // level.  Those values are computed here with the same float statements as the
 // reference and packed into ImageJob descriptors; the pixel and keypoint work
 // runs in the gfx950 kernels of orb_kernels.hip.
+#include <mutex>
+
 #include "orb_internal.h"
 
 // ====================================================================== C ABI
@@ -409,14 +411,14 @@ int orb_stereo_frame(orb_extractor* left, orb_extractor* right, const uint8_t* i
     orr.desc = dr;
     CopyList l;
     l.n = 0;
-    rc = left->list_results(ol, l);
-    if (!rc) rc = right->list_results(orr, l);
+    rc = left->list_results(ol, l, left->land);
+    if (!rc) rc = right->list_results(orr, l, right->land);
     if (rc) return rc;
     HIP_TRY(orb_launch_copy_list(&l, ORB_COPY_BLOCKS, st));
     HIP_TRY(hipStreamSynchronize(st));
-    rc = left->take_results(ol, capacity, nl);
+    rc = left->take_results(ol, capacity, nl, left->land);
     if (rc) return rc;
-    return right->take_results(orr, capacity, nr);
+    return right->take_results(orr, capacity, nr, right->land);
 }
 
 int orb_extractor_debug_image(orb_extractor* ex, int level, int kind, uint8_t* dst, size_t dst_stride)
@@ -632,6 +634,11 @@ struct orb_batch {
         graph = nullptr;
         drop_branches();
     }
+
+    // orb_batch_results: one landing buffer for every slot (allocating one a
+    // slot costs 250 us each)
+    Landing slot_land;
+    std::mutex slot_mu;
 
     // orb_batch_read_all: the results' layout in pinned memory that the device
     // writes, with the counters first and the slots in groups, so that the
@@ -1326,7 +1333,11 @@ int orb_batch_results(orb_batch* b, int slot, orb_keypoint* keypoints, int capac
 {
     if (!b || slot < 0 || slot >= (int)b->ex.size() || !n) return ORB_E_ARG;
     HIP_TRY(hipSetDevice(b->ctx->device));
-    return b->ex[slot]->read_results(keypoints, capacity, descriptors, n);
+    orb_extractor::Outputs o;
+    o.kps = keypoints;
+    o.desc = descriptors;
+    std::lock_guard<std::mutex> g(b->slot_mu);
+    return b->ex[slot]->read_results(o, capacity, n, b->slot_land);
 }
 
 int orb_batch_stereo_results(orb_batch* b, int pair, float* uRight, float* depth, int capacity, int* n)
