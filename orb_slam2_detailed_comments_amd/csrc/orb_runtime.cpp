@@ -640,14 +640,26 @@ struct orb_batch {
     Landing slot_land;
     std::mutex slot_mu;
 
+    // Offsets of every output in a results buffer.  Each buffer has its own, as
+    // they are made at different times; an offset, and the copy list made with
+    // it, holds for these left slots only (uRight and depth are theirs).
+    struct OutLayout {
+        std::vector<size_t> ctr, kps, desc, ur, dep;
+        std::vector<int> lefts;
+        size_t bytes = 0;
+    };
+
     // orb_batch_read_all: the results' layout in pinned memory that the device
     // writes, with the counters first and the slots in groups, so that the
     // host copies one group out while the device writes the next
     char* h_all = nullptr;
+    size_t all_cap = 0;
+    OutLayout all_at;
     CopyOp* d_all_ops = nullptr;
+    size_t all_ops_cap = 0;
     std::vector<int> all_start;             // first operation of each group (0: the counters)
     std::vector<hipEvent_t> all_ev;         // recorded after each group
-    int all_pairs = -1;                     // pair count the layout was built for
+    bool all_ready = false;                 // the layout and the list are those of the slots and pairs
 
     // Pinned transfers (orb_batch_pinned_images / _upload_pinned /
     // _read_async).  Inputs: every slot's image at its device pitch in one
@@ -664,9 +676,8 @@ struct orb_batch {
     char* h_out = nullptr;
     char* d_out = nullptr;
     CopyOp* d_out_ops = nullptr;
-    size_t out_bytes = 0;
+    OutLayout out_at;
     int n_out_ops = 0, out_pairs = -1;      // pair count the output layout was built for
-    std::vector<size_t> out_ctr, out_kps, out_desc, out_ur, out_dep;
     hipEvent_t out_ev = nullptr;            // recorded after the device-to-host copy
     bool out_ready = false;                 // a read has been enqueued since the layout was built
 
@@ -713,7 +724,7 @@ struct orb_batch {
     int refresh_pinned()
     {
         drop_pinned_out();
-        drop_read_all();
+        all_ready = false;
         return d_in_ops ? write_in_ops() : ORB_OK;
     }
 
@@ -725,64 +736,57 @@ struct orb_batch {
         h_out = nullptr;
         d_out = nullptr;
         d_out_ops = nullptr;
-        out_bytes = 0;
         n_out_ops = 0;
         out_pairs = -1;
         out_ready = false;
     }
 
-    // Offsets of every output in a results buffer.
-    void layout_out()
+    OutLayout layout_out() const
     {
         const int n = (int)ex.size(), np = (int)pl.size();
-        out_ctr.assign(n, 0);
-        out_kps.assign(n, 0);
-        out_desc.assign(n, 0);
-        out_ur.assign(np, 0);
-        out_dep.assign(np, 0);
-        size_t o = 0;
+        OutLayout at;
+        at.lefts = pl;
+        auto take = [&](size_t bytes) {
+            const size_t o = at.bytes;
+            at.bytes += up256(bytes);
+            return o;
+        };
         for (int s = 0; s < n; s++) {
-            const ImageJob& J = ex[s]->hjob;
-            const size_t cap = (size_t)J.out_cap;
-            out_ctr[s] = o;
-            o += up256(ORB_CNT_SLOTS * 4);
-            out_kps[s] = o;
-            o += up256(cap * sizeof(OrbKeyPoint));
-            out_desc[s] = o;
-            o += up256(cap * 32);
+            const size_t cap = (size_t)ex[s]->hjob.out_cap;
+            at.ctr.push_back(take(ORB_CNT_SLOTS * 4));
+            at.kps.push_back(take(cap * sizeof(OrbKeyPoint)));
+            at.desc.push_back(take(cap * 32));
         }
         for (int p = 0; p < np; p++) {
             const size_t cap = (size_t)ex[pl[p]]->hjob.out_cap;
-            out_ur[p] = o;
-            o += up256(cap * 4);
-            out_dep[p] = o;
-            o += up256(cap * 4);
+            at.ur.push_back(take(cap * 4));
+            at.dep.push_back(take(cap * 4));
         }
-        out_bytes = o;
+        return at;
     }
 
     // The copy list of the slots' counters into such a buffer at dst, and of
     // the other outputs of slots s0 .. s1 - 1 and pairs p0 .. p1 - 1.
-    void list_counters(char* dst, std::vector<CopyOp>& ops) const
+    void list_counters(char* dst, const OutLayout& at, std::vector<CopyOp>& ops) const
     {
         for (size_t s = 0; s < ex.size(); s++)
-            ops.push_back(CopyOp{(const unsigned*)ex[s]->hjob.counters, (unsigned*)(dst + out_ctr[s]), nullptr,
+            ops.push_back(CopyOp{(const unsigned*)ex[s]->hjob.counters, (unsigned*)(dst + at.ctr[s]), nullptr,
                                  ORB_CNT_SLOTS, 0});
     }
-    void list_outputs(char* dst, int s0, int s1, int p0, int p1, std::vector<CopyOp>& ops) const
+    void list_outputs(char* dst, const OutLayout& at, int s0, int s1, int p0, int p1, std::vector<CopyOp>& ops) const
     {
         for (int s = s0; s < s1; s++) {
             const ImageJob& J = ex[s]->hjob;
             const int* cnt = J.counters + ORB_CNT_NOUT;
-            ops.push_back(CopyOp{(const unsigned*)J.kps, (unsigned*)(dst + out_kps[s]), cnt,
+            ops.push_back(CopyOp{(const unsigned*)J.kps, (unsigned*)(dst + at.kps[s]), cnt,
                                  J.out_cap * (int)(sizeof(OrbKeyPoint) / 4), (int)(sizeof(OrbKeyPoint) / 4)});
-            ops.push_back(CopyOp{(const unsigned*)J.desc, (unsigned*)(dst + out_desc[s]), cnt, J.out_cap * 8, 8});
+            ops.push_back(CopyOp{(const unsigned*)J.desc, (unsigned*)(dst + at.desc[s]), cnt, J.out_cap * 8, 8});
         }
         for (int p = p0; p < p1; p++) {
             const orb_extractor* L = ex[pl[p]];
             const int* cnt = L->hjob.counters + ORB_CNT_NOUT;
-            ops.push_back(CopyOp{(const unsigned*)L->d_uR, (unsigned*)(dst + out_ur[p]), cnt, L->hjob.out_cap, 1});
-            ops.push_back(CopyOp{(const unsigned*)L->d_depth, (unsigned*)(dst + out_dep[p]), cnt, L->hjob.out_cap, 1});
+            ops.push_back(CopyOp{(const unsigned*)L->d_uR, (unsigned*)(dst + at.ur[p]), cnt, L->hjob.out_cap, 1});
+            ops.push_back(CopyOp{(const unsigned*)L->d_depth, (unsigned*)(dst + at.dep[p]), cnt, L->hjob.out_cap, 1});
         }
     }
 
@@ -791,26 +795,37 @@ struct orb_batch {
     int all_groups() const { return std::max(1, std::min(8, (int)ex.size() / 8)); }
     int setup_read_all()
     {
-        if (h_all && all_pairs == (int)pl.size()) return ORB_OK;
-        drop_read_all();
-        layout_out();
-        if (hipHostMalloc((void**)&h_all, out_bytes, hipHostMallocCoherent) != hipSuccess) {
+        if (all_ready && all_at.lefts == pl) return ORB_OK;
+        all_ready = false;
+        all_at = layout_out();
+        if (all_at.bytes > all_cap) {
+            if (h_all) (void)hipHostFree(h_all);          // its last copies have ended
             h_all = nullptr;
-            return ORB_E_OOM;
+            all_cap = 0;
+            if (hipHostMalloc((void**)&h_all, all_at.bytes, hipHostMallocCoherent) != hipSuccess) {
+                h_all = nullptr;
+                return ORB_E_OOM;
+            }
+            all_cap = all_at.bytes;
         }
         const int n = (int)ex.size(), np = (int)pl.size(), ng = all_groups();
         std::vector<CopyOp> ops;
         all_start.assign(1, 0);
-        list_counters(h_all, ops);
+        list_counters(h_all, all_at, ops);
         for (int g = 0; g < ng; g++) {
             all_start.push_back((int)ops.size());
-            list_outputs(h_all, n * g / ng, n * (g + 1) / ng, np * g / ng, np * (g + 1) / ng, ops);
+            list_outputs(h_all, all_at, n * g / ng, n * (g + 1) / ng, np * g / ng, np * (g + 1) / ng, ops);
         }
         all_start.push_back((int)ops.size());
-        if (hipMalloc(&d_all_ops, ops.size() * sizeof(CopyOp)) != hipSuccess) {
+        if (ops.size() > all_ops_cap) {
+            if (d_all_ops) (void)hipFree(d_all_ops);
             d_all_ops = nullptr;
-            drop_read_all();
-            return ORB_E_OOM;
+            all_ops_cap = 0;
+            if (hipMalloc(&d_all_ops, ops.size() * sizeof(CopyOp)) != hipSuccess) {
+                d_all_ops = nullptr;
+                return ORB_E_OOM;
+            }
+            all_ops_cap = ops.size();
         }
         HIP_TRY(hipMemcpy(d_all_ops, ops.data(), ops.size() * sizeof(CopyOp), hipMemcpyHostToDevice));
         while ((int)all_ev.size() < ng + 1) {
@@ -818,32 +833,23 @@ struct orb_batch {
             HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem));
             all_ev.push_back(e);
         }
-        all_pairs = np;
+        all_ready = true;
         return ORB_OK;
     }
-    void drop_read_all()
-    {
-        if (h_all) (void)hipHostFree(h_all);
-        if (d_all_ops) (void)hipFree(d_all_ops);
-        h_all = nullptr;
-        d_all_ops = nullptr;
-        all_pairs = -1;
-    }
-
     int setup_pinned_out()
     {
         if (h_out && out_pairs == (int)pl.size()) return ORB_OK;
         drop_pinned_out();
-        layout_out();
+        out_at = layout_out();
         const int n = (int)ex.size(), np = (int)pl.size();
-        if (hipHostMalloc((void**)&h_out, out_bytes) != hipSuccess) {
+        if (hipHostMalloc((void**)&h_out, out_at.bytes) != hipSuccess) {
             h_out = nullptr;
             return ORB_E_OOM;
         }
-        if (hipMalloc((void**)&d_out, out_bytes) != hipSuccess) return ORB_E_OOM;
+        if (hipMalloc((void**)&d_out, out_at.bytes) != hipSuccess) return ORB_E_OOM;
         std::vector<CopyOp> ops;
-        list_counters(d_out, ops);
-        list_outputs(d_out, 0, n, 0, np, ops);
+        list_counters(d_out, out_at, ops);
+        list_outputs(d_out, out_at, 0, n, 0, np, ops);
         n_out_ops = (int)ops.size();
         if (hipMalloc(&d_out_ops, ops.size() * sizeof(CopyOp)) != hipSuccess) return ORB_E_OOM;
         HIP_TRY(hipMemcpy(d_out_ops, ops.data(), ops.size() * sizeof(CopyOp), hipMemcpyHostToDevice));
@@ -857,7 +863,7 @@ struct orb_batch {
     {
         if (!h_out || !out_ready) return ORB_E_ARG;
         HIP_TRY(hipEventSynchronize(out_ev));
-        const int* c = (const int*)(h_out + out_ctr[slot]);
+        const int* c = (const int*)(h_out + out_at.ctr[slot]);
         if (c[ORB_CNT_ERR]) return ORB_E_OVERFLOW;
         *n = c[ORB_CNT_NOUT];
         return ORB_OK;
@@ -865,7 +871,8 @@ struct orb_batch {
 
     ~orb_batch()
     {
-        drop_read_all();
+        if (h_all) (void)hipHostFree(h_all);
+        if (d_all_ops) (void)hipFree(d_all_ops);
         for (hipEvent_t e : all_ev) (void)hipEventDestroy(e);
         if (h_in) (void)hipHostFree(h_in);
         if (d_in) (void)hipFree(d_in);
@@ -993,7 +1000,7 @@ int orb_batch_read_all(orb_batch* b, orb_keypoint* keypoints, uint8_t* descripto
     const int bad = [&] {
         HIP_TRY(hipEventSynchronize(b->all_ev[0]));
         for (int s = 0; s < n; s++) {
-            const int* c = (const int*)(b->h_all + b->out_ctr[s]);
+            const int* c = (const int*)(b->h_all + b->all_at.ctr[s]);
             if (c[ORB_CNT_ERR]) return ORB_E_OVERFLOW;
             counts[s] = c[ORB_CNT_NOUT];
             if (counts[s] > capacity) return ORB_E_CAPACITY;
@@ -1009,14 +1016,14 @@ int orb_batch_read_all(orb_batch* b, orb_keypoint* keypoints, uint8_t* descripto
         for (int s = n * g / ng; s < n * (g + 1) / ng; s++) {
             const size_t c = (size_t)counts[s];
             if (!c) continue;
-            std::memcpy(keypoints + (size_t)s * capacity, b->h_all + b->out_kps[s], c * sizeof(orb_keypoint));
-            std::memcpy(descriptors + (size_t)s * capacity * 32, b->h_all + b->out_desc[s], c * 32);
+            std::memcpy(keypoints + (size_t)s * capacity, b->h_all + b->all_at.kps[s], c * sizeof(orb_keypoint));
+            std::memcpy(descriptors + (size_t)s * capacity * 32, b->h_all + b->all_at.desc[s], c * 32);
         }
         for (int p = np * g / ng; p < np * (g + 1) / ng; p++) {
             const size_t c = (size_t)counts[b->pl[p]];
             if (!c) continue;
-            if (uRight) std::memcpy(uRight + (size_t)p * capacity, b->h_all + b->out_ur[p], c * 4);
-            if (depth) std::memcpy(depth + (size_t)p * capacity, b->h_all + b->out_dep[p], c * 4);
+            if (uRight) std::memcpy(uRight + (size_t)p * capacity, b->h_all + b->all_at.ur[p], c * 4);
+            if (depth) std::memcpy(depth + (size_t)p * capacity, b->h_all + b->all_at.dep[p], c * 4);
         }
     }
     return ORB_OK;
@@ -1053,7 +1060,7 @@ int orb_batch_read_async(orb_batch* b)
     if (rc) return rc;
     hipStream_t st = b->ctx->stream;
     HIP_TRY(orb_launch_copy_ops(b->d_out_ops, b->n_out_ops, 8, st));
-    HIP_TRY(hipMemcpyAsync(b->h_out, b->d_out, b->out_bytes, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(b->h_out, b->d_out, b->out_at.bytes, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipEventRecord(b->out_ev, st));
     b->out_ready = true;
     return ORB_OK;
@@ -1066,8 +1073,8 @@ int orb_batch_pinned_results(orb_batch* b, int slot, const orb_keypoint** keypoi
     HIP_TRY(hipSetDevice(b->ctx->device));
     const int rc = b->pinned_count(slot, n);
     if (rc) return rc;
-    if (keypoints) *keypoints = (const orb_keypoint*)(b->h_out + b->out_kps[slot]);
-    if (descriptors) *descriptors = (const uint8_t*)(b->h_out + b->out_desc[slot]);
+    if (keypoints) *keypoints = (const orb_keypoint*)(b->h_out + b->out_at.kps[slot]);
+    if (descriptors) *descriptors = (const uint8_t*)(b->h_out + b->out_at.desc[slot]);
     return ORB_OK;
 }
 
@@ -1077,8 +1084,8 @@ int orb_batch_pinned_stereo(orb_batch* b, int pair, const float** uRight, const 
     HIP_TRY(hipSetDevice(b->ctx->device));
     const int rc = b->pinned_count(b->pl[pair], n);
     if (rc) return rc;
-    if (uRight) *uRight = (const float*)(b->h_out + b->out_ur[pair]);
-    if (depth) *depth = (const float*)(b->h_out + b->out_dep[pair]);
+    if (uRight) *uRight = (const float*)(b->h_out + b->out_at.ur[pair]);
+    if (depth) *depth = (const float*)(b->h_out + b->out_at.dep[pair]);
     return ORB_OK;
 }
 
@@ -1111,6 +1118,7 @@ int orb_batch_set_stereo(orb_batch* b, int npairs, const int* left_slots, const 
     HIP_TRY(hipStreamSynchronize(b->ctx->stream));
     b->drop_graph();
     b->drop_pinned_out();
+    b->all_ready = false;
     if (b->d_sargs) (void)hipFree(b->d_sargs);
     b->d_sargs = nullptr;
     b->pl.clear();
