@@ -386,9 +386,12 @@ int orb_vocabulary_bow_time(orb_vocabulary* v, int n_images, const uint8_t* desc
  * results are identical either way.  No reference counterpart: a tuning and
  * test aid.  orb_context_last_rounds returns the rounds the last windowed
  * search on this context ran and sets *sequential (may be NULL) to 1 if it
- * fell back to the in-order pass for some pair or frame. */
+ * fell back to the in-order pass for some pair or frame;
+ * orb_context_last_restarts how often it started over because its candidate
+ * lists did not fit (an equal call after it fits). */
 int orb_context_set_round_limit(orb_context* ctx, int rounds);
 int orb_context_last_rounds(const orb_context* ctx, int* sequential);
+int orb_context_last_restarts(const orb_context* ctx);
 
 /* ---------------------------------------------------------------- windowed matching
  * ORBmatcher::SearchForInitialization (src/ORBmatcher.cc:573-717) over the

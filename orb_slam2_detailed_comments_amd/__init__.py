@@ -47,6 +47,7 @@ SIGNATURES = {
     "orb_extractor_set_tile_heights": (_I, [_P, _I, _P]),
     "orb_context_set_round_limit": (_I, [_P, _I]),
     "orb_context_last_rounds": (_I, [_P, _P]),
+    "orb_context_last_restarts": (_I, [_P]),
     "orb_batch_set_tile_heights": (_I, [_P, _I, _P]),
     "orb_batch_autotune_tiles": (_I, [_P, _I, _P, _P, _P]),
     "orb_batch_read_all": (_I, [_P, _P, _P, _I, _P, _P, _P]),
@@ -209,6 +210,12 @@ class Context:
         r = lib().orb_context_last_rounds(self.h, ctypes.byref(seq))
         _check("orb_context_last_rounds", min(r, 0))
         return r, bool(seq.value)
+
+    def last_restarts(self):
+        """How often the last windowed search started over with longer candidate lists."""
+        r = lib().orb_context_last_restarts(self.h)
+        _check("orb_context_last_restarts", min(r, 0))
+        return r
 
     def close(self):
         if getattr(self, "h", None) and _lib is not None:

@@ -138,7 +138,7 @@ struct orb_context {
     // windowed searches: rounds before the sequential pass, and what the
     // last search used
     int round_limit = 48;
-    int last_rounds = 0, last_sequential = 0;
+    int last_rounds = 0, last_sequential = 0, last_restarts = 0;
     // brute-force matcher scratch
     uint8_t* d_q = nullptr;
     uint8_t* d_t = nullptr;

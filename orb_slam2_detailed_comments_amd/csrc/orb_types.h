@@ -234,6 +234,16 @@ struct BowJob {
     int off, n;
 };
 
+// Where a frame's (or pair's) candidate lists go in the call's buffer: a region
+// of its own, and past that the end of the buffer, which the frames share.
+// Counters are of entries asked for, on the device.
+struct ListRoom {
+    unsigned long long* asked;         // of this frame
+    unsigned long long* asked_shared;  // of the shared part (beyond shared_cap: lists are missing)
+    unsigned long long start, cap;     // the region
+    unsigned long long shared_start, shared_cap;
+};
+
 // One frame pair of ORBmatcher::SearchForInitialization: F1 / F2 keypoints
 // (mvKeysUn) and descriptors, the grid bounds (mnMinX .. mnMaxY), the search
 // positions (vbPrevMatched), parameters, scratch and
@@ -256,10 +266,9 @@ struct WinPair {
     const float* uright;    // SearchByProjection's frames: mvuRight and occupancy
     const uint8_t* occupied;   // (occupied keypoints are left out); null: octave 0 only
     int* cnt;               // n1: candidates per query
-    unsigned* off;          // n1: where each query's list starts
-    int2* cand;             // (i2, distance) lists
-    unsigned long long* total;   // list entries asked for (beyond cand_cap: lists are missing)
-    unsigned long long cand_cap;
+    unsigned long long* off;     // n1: where each query's list starts in cand
+    int2* cand;             // (i2, distance) lists of the whole call
+    ListRoom room;
     int* m12;               // n1: vnMatches12
     float2* prev_out;       // n1: vbPrevMatched afterwards
     int* nmatch;            // nmatches
@@ -301,10 +310,9 @@ struct ProjFrame {
     const uint8_t* qdesc;
     int nq;
     int* cnt;                   // candidates per query
-    unsigned* off;              // where each query's list starts
+    unsigned long long* off;    // where each query's list starts in cand
     unsigned* cand;             // i2 | distance << 12 | octave << 21, GetFeaturesInArea order
-    unsigned long long* total;  // as WinPair's
-    unsigned long long cand_cap;
+    ListRoom room;
     int* out[2];                // outcome per query by round parity: keypoint or -1
     int* claim[3];              // per keypoint: first claiming query (with observations), by round mod 3
     int* changed;               // [ORB_PROJ_MAXIT]: bit 0 round k changed some outcome, bit 2 not run

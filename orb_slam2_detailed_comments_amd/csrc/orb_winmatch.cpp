@@ -3,7 +3,8 @@
 // orb_winmatch.hip).  A call copies its inputs to the device once, launches
 // the grid, the candidate lists, four rounds and the finish, copies every
 // result back and waits once; it goes on only if some pair has not settled,
-// or if the lists did not fit their buffer (which then grows).  Device and
+// or if the lists did not fit their buffer (which then grows, so that an equal
+// call fits).  Device and
 // pinned buffers are the context's, grown on demand and kept between calls.
 #include <chrono>
 #include <cstring>
@@ -13,6 +14,7 @@
 
 using namespace orb_detail;
 
+extern "C" int orb_win_queries_per_block(void);
 extern "C" hipError_t orb_launch_win_lists(const WinPair* d_pairs, int npairs, int max_n1, hipStream_t st);
 extern "C" hipError_t orb_launch_win_rounds(const WinPair* d_pairs, int npairs, int max_n1, int k0, int k1,
                                             hipStream_t st);
@@ -38,28 +40,46 @@ struct Block {
     }
 };
 
-// Room per query for candidate lists when a call starts (entries); a call
-// whose windows hold more grows its lists to what they asked for, and the
-// buffer stays that large for the next.
-constexpr size_t kListStart = 64;
+// The candidate lists' places in the context's buffer.  A pair's (or frame's)
+// queries have a region of kListRegion entries each (a window holds no more
+// than the frame's keypoints); workgroups past their region's end take from the
+// rest of the buffer, which all share.  The regions follow from the call alone,
+// so what an equal call takes from the rest is known up to the workgroups that
+// straddle the regions' ends: a call that did not fit makes the buffer that
+// large, and a quarter more for the next frames.
+// A local-map search of 4000 keypoints, th 5 (75 entries a query): 288 us; 334
+// with even shares of a buffer as large as the asked total, which the asked
+// list outgrew by the shares' rounding, so that every call ran twice.
+constexpr size_t kListRegion = 64;
 
-// The lists' regions in a buffer of `have` entries: a pair's (or frame's)
-// nq[i] queries get kListStart entries each, or an even share of the buffer
-// if that is more, or what the pair asked for.  base[i] and cap[i] in
-// entries; returns the total.
-size_t list_regions(const std::vector<size_t>& nq, size_t have, const unsigned long long* asked,
-                    std::vector<size_t>& base, std::vector<unsigned long long>& cap)
-{
-    size_t all = 0, total = 0;
-    for (const size_t n : nq) all += n;
-    const size_t per = std::max(kListStart, all ? have / all : 0);
-    for (size_t i = 0; i < nq.size(); i++) {
-        cap[i] = asked ? std::max<unsigned long long>(nq[i] * kListStart, asked[i]) : nq[i] * per;
-        base[i] = total;
-        total += (size_t)cap[i];
+struct Lists {
+    std::vector<size_t> nq, nk;             // queries, keypoints a window can hold
+    size_t regions = 0;                     // entries of all regions
+
+    void add(int n_queries, int n_keys)
+    {
+        nq.push_back((size_t)n_queries);
+        nk.push_back((size_t)n_keys);
+        regions += region(nq.size() - 1);
     }
-    return total;
-}
+    size_t region(size_t i) const { return nq[i] * std::min(kListRegion, nk[i]); }
+
+    // Entries an equal call needs, from what this one asked for; a workgroup
+    // has per_block queries.
+    size_t need(const unsigned long long* asked, size_t per_block) const
+    {
+        size_t shared = 0;
+        for (size_t i = 0; i < nq.size(); i++)
+            if (asked[i] > region(i)) shared += (size_t)asked[i] - region(i) + per_block * nk[i];
+        return regions + shared + shared / 4;
+    }
+
+    // Room i in a buffer of `have` entries; counters: a frame's each, then the shared one.
+    ListRoom room(size_t i, size_t start, size_t have, unsigned long long* counters) const
+    {
+        return ListRoom{counters + i, counters + nq.size(), start, region(i), regions, have - regions};
+    }
+};
 
 // steps > 0: after the call's own run, `steps` more runs of the device work
 // with the inputs resident in HBM, their
@@ -90,9 +110,9 @@ int sfi_impl(orb_context* ctx, int n_pairs, const orb_keypoint* kp1, const uint8
     const size_t i_kp2 = B.add_in(n2 * sizeof(OrbKeyPoint)), i_d2 = B.add_in(n2 * 32);
     const size_t i_pairs = B.add_in(P * sizeof(WinPair));
     const size_t o_m12 = B.add_out(n1 * 4), o_prev = B.add_out(n1 * 8), o_nm = B.add_out(P * 4);
-    const size_t o_tot = B.add_out(P * 8), o_chg = B.add_out(P * ORB_WIN_MAXIT * 4);
+    const size_t o_tot = B.add_out((P + 1) * 8), o_chg = B.add_out(P * ORB_WIN_MAXIT * 4);
     const size_t s_rec = B.add_scratch(n2 * 16), s_cells = B.add_scratch(P * (64 * 48 + 1) * 4);
-    const size_t s_cnt = B.add_scratch(n1 * 4), s_off = B.add_scratch(n1 * 4);
+    const size_t s_cnt = B.add_scratch(n1 * 4), s_off = B.add_scratch(n1 * 8);
     // round state: outcomes by parity, claims and claim counts by round mod 3
     const size_t s_out = B.add_scratch(2 * n1 * 4), s_claim = B.add_scratch(3 * n2 * ORB_WIN_SLOTS * 4);
     const size_t s_ccnt = B.add_scratch(3 * n2 * 4);
@@ -111,8 +131,7 @@ int sfi_impl(orb_context* ctx, int n_pairs, const orb_keypoint* kp1, const uint8
         std::memcpy(h_in + i_d2, desc2, n2 * 32);
     }
     WinPair* pairs = (WinPair*)(h_in + i_pairs);
-    std::vector<size_t> nq(P), base(P);
-    std::vector<unsigned long long> cap(P);
+    Lists lists;
     for (int p = 0; p < n_pairs; p++) {
         WinPair& w = pairs[p];
         std::memset(&w, 0, sizeof(w));
@@ -133,8 +152,7 @@ int sfi_impl(orb_context* ctx, int n_pairs, const orb_keypoint* kp1, const uint8
         w.rec = (float4*)(d_s + s_rec) + off2[p];
         w.cell_start = (int*)(d_s + s_cells) + (size_t)p * (64 * 48 + 1);
         w.cnt = (int*)(d_s + s_cnt) + off1[p];
-        w.off = (unsigned*)(d_s + s_off) + off1[p];
-        w.total = (unsigned long long*)(d_out + o_tot) + p;
+        w.off = (unsigned long long*)(d_s + s_off) + off1[p];
         w.m12 = (int*)(d_out + o_m12) + off1[p];
         w.prev_out = (float2*)(d_out + o_prev) + off1[p];
         w.nmatch = (int*)(d_out + o_nm) + p;
@@ -144,22 +162,23 @@ int sfi_impl(orb_context* ctx, int n_pairs, const orb_keypoint* kp1, const uint8
             w.ccnt[b] = (int*)(d_s + s_ccnt) + b * n2 + off2[p];
         }
         w.changed = (int*)(d_out + o_chg) + (size_t)p * ORB_WIN_MAXIT;
-        nq[p] = (size_t)w.n1;
+        lists.add(w.n1, w.n2);
     }
     const unsigned long long* tot = (const unsigned long long*)(h_out + o_tot);
     const int* chg = (const int*)(h_out + o_chg);
-    // the lists' regions into the pairs, and all pairs to the device
-    auto place_lists = [&](const unsigned long long* asked) -> int {
-        const size_t n = list_regions(nq, ctx->wcand_cap / sizeof(int2), asked, base, cap);
+    // a buffer of at least n entries, and the lists' places in it
+    auto place_lists = [&](size_t n) -> int {
         const int rg = ctx->grow(&ctx->d_wcand, &ctx->wcand_cap, std::max<size_t>(n, 1) * sizeof(int2));
         if (rg) return rg;
+        size_t start = 0;
         for (int p = 0; p < n_pairs; p++) {
-            pairs[p].cand = (int2*)ctx->d_wcand + base[p];
-            pairs[p].cand_cap = cap[p];
+            pairs[p].cand = (int2*)ctx->d_wcand;
+            pairs[p].room = lists.room(p, start, ctx->wcand_cap / sizeof(int2), (unsigned long long*)(d_out + o_tot));
+            start += lists.region(p);
         }
         return ORB_OK;
     };
-    rc = place_lists(nullptr);
+    rc = place_lists(lists.regions);
     if (rc) return rc;
     HIP_TRY(hipMemcpyAsync(d_in, h_in, B.in, hipMemcpyHostToDevice, st));
     const WinPair* d_pairs = (const WinPair*)(d_in + i_pairs);
@@ -167,6 +186,7 @@ int sfi_impl(orb_context* ctx, int n_pairs, const orb_keypoint* kp1, const uint8
         const int limit = std::min(ctx->round_limit, ORB_WIN_MAXIT);
         int k = 0;
         bool settled = false;
+        ctx->last_restarts = 0;
         HIP_TRY(orb_launch_win_lists(d_pairs, n_pairs, max_n1, st));
         // Rounds in chunks of 4, each followed by the finish of the pairs
         // that have settled; pairs still changing at the limit get the
@@ -178,10 +198,9 @@ int sfi_impl(orb_context* ctx, int n_pairs, const orb_keypoint* kp1, const uint8
             HIP_TRY(orb_launch_win_finish(d_pairs, n_pairs, 0, st));
             HIP_TRY(hipMemcpyAsync(h_out, d_out, B.out, hipMemcpyDeviceToHost, st));
             HIP_TRY(hipStreamSynchronize(st));
-            bool fits = true;
-            for (int p = 0; p < n_pairs; p++) fits = fits && tot[p] <= cap[p];
-            if (!fits) {                           // longer lists, from the start
-                const int rl = place_lists(tot);
+            if (tot[P] > pairs[0].room.shared_cap) {   // longer lists, from the start
+                ctx->last_restarts++;
+                const int rl = place_lists(lists.need(tot, orb_win_queries_per_block()));
                 if (rl) return rl;
                 HIP_TRY(hipMemcpyAsync(d_in + i_pairs, pairs, P * sizeof(WinPair), hipMemcpyHostToDevice, st));
                 HIP_TRY(orb_launch_win_lists(d_pairs, n_pairs, max_n1, st));
@@ -254,6 +273,7 @@ int orb_search_for_initialization_time(orb_context* ctx, int n_pairs, const orb_
 extern "C" hipError_t orb_launch_proj_prep(ProjFrame* d_frames, int nframes, int max_nq, int rule, const float* d_pts,
                                            const int* d_pt_off, const float* d_scale, int nlevels, const float* d_cam,
                                            int mono, float th, hipStream_t st);
+extern "C" int orb_proj_queries_per_block(void);
 extern "C" hipError_t orb_launch_proj_lists(const WinPair* d_grid, const ProjFrame* d_frames, int nframes, int max_nq,
                                             hipStream_t st);
 extern "C" hipError_t orb_launch_proj_rounds(ProjFrame* d_frames, int nframes, int max_nq, int k0, int k1,
@@ -310,10 +330,10 @@ int proj_search(orb_context* ctx, int rule, int n_frames, const orb_keypoint* kp
                  i_ptoff = B.add_in((F + 1) * 4), i_scale = B.add_in(ORB_MAX_LEVELS * 4), i_cam = B.add_in(F * 7 * 4),
                  i_grid = B.add_in(F * sizeof(WinPair)), i_frames = B.add_in(F * sizeof(ProjFrame));
     const size_t o_ptm = B.add_out(np * 4), o_keyp = B.add_out(nk * 4), o_nm = B.add_out(F * 4),
-                 o_tot = B.add_out(F * 8), o_chg = B.add_out(F * ORB_PROJ_MAXIT * 4);
+                 o_tot = B.add_out((F + 1) * 8), o_chg = B.add_out(F * ORB_PROJ_MAXIT * 4);
     const size_t s_rec = B.add_scratch(nk * 16), s_cells = B.add_scratch(F * (64 * 48 + 1) * 4),
                  s_q = B.add_scratch(np * sizeof(ProjQuery)), s_cnt = B.add_scratch(np * 4),
-                 s_off = B.add_scratch(np * 4), s_out = B.add_scratch(2 * np * 4), s_claim = B.add_scratch(3 * nk * 4);
+                 s_off = B.add_scratch(np * 8), s_out = B.add_scratch(2 * np * 4), s_claim = B.add_scratch(3 * nk * 4);
     int rc = ctx->grow(&ctx->d_win, &ctx->win_cap, B.in + B.out + B.scratch);
     if (!rc) rc = ctx->grow_pinned(&ctx->h_win, &ctx->hwin_cap, B.in + B.out);
     if (rc) return rc;
@@ -334,8 +354,7 @@ int proj_search(orb_context* ctx, int rule, int n_frames, const orb_keypoint* kp
     if (rule == 2) std::memcpy(h_in + i_cam, cam, F * 7 * 4);
     WinPair* grid = (WinPair*)(h_in + i_grid);
     ProjFrame* frames = (ProjFrame*)(h_in + i_frames);
-    std::vector<size_t> nq(F), base(F);
-    std::vector<unsigned long long> cap(F);
+    Lists rooms;
     for (int f = 0; f < n_frames; f++) {
         const int k0 = key_off[f], q0 = pt_off[f];
         WinPair& w = grid[f];
@@ -350,7 +369,6 @@ int proj_search(orb_context* ctx, int rule, int n_frames, const orb_keypoint* kp
         w.maxY = bounds[4 * f + 3];
         w.rec = (float4*)(d_s + s_rec) + k0;
         w.cell_start = (int*)(d_s + s_cells) + (size_t)f * (64 * 48 + 1);
-        w.total = (unsigned long long*)(d_out + o_tot) + f;
         ProjFrame& P = frames[f];
         std::memset(&P, 0, sizeof(P));
         P.kp = w.kp2;
@@ -366,8 +384,7 @@ int proj_search(orb_context* ctx, int rule, int n_frames, const orb_keypoint* kp
         P.qdesc = (const uint8_t*)(d_in + i_pdesc) + (size_t)q0 * 32;
         P.nq = pt_off[f + 1] - q0;
         P.cnt = (int*)(d_s + s_cnt) + q0;
-        P.off = (unsigned*)(d_s + s_off) + q0;
-        P.total = w.total;
+        P.off = (unsigned long long*)(d_s + s_off) + q0;
         for (int b = 0; b < 2; b++) P.out[b] = (int*)(d_s + s_out) + b * np + q0;
         for (int b = 0; b < 3; b++) P.claim[b] = (int*)(d_s + s_claim) + b * nk + k0;
         P.changed = (int*)(d_out + o_chg) + (size_t)f * ORB_PROJ_MAXIT;
@@ -377,21 +394,23 @@ int proj_search(orb_context* ctx, int rule, int n_frames, const orb_keypoint* kp
         P.pt_match = (int*)(d_out + o_ptm) + q0;
         P.key_point = (int*)(d_out + o_keyp) + k0;
         P.nmatch = (int*)(d_out + o_nm) + f;
-        nq[f] = (size_t)P.nq;
+        rooms.add(P.nq, P.n);
     }
     const unsigned long long* tot = (const unsigned long long*)(h_out + o_tot);
     const int* chg = (const int*)(h_out + o_chg);
-    auto place_lists = [&](const unsigned long long* asked) -> int {
-        const size_t n = list_regions(nq, ctx->wcand_cap / sizeof(unsigned), asked, base, cap);
+    auto place_lists = [&](size_t n) -> int {
         const int rg = ctx->grow(&ctx->d_wcand, &ctx->wcand_cap, std::max<size_t>(n, 1) * sizeof(unsigned));
         if (rg) return rg;
+        size_t start = 0;
         for (int f = 0; f < n_frames; f++) {
-            frames[f].cand = (unsigned*)ctx->d_wcand + base[f];
-            frames[f].cand_cap = cap[f];
+            frames[f].cand = (unsigned*)ctx->d_wcand;
+            frames[f].room = grid[f].room =
+                rooms.room(f, start, ctx->wcand_cap / sizeof(unsigned), (unsigned long long*)(d_out + o_tot));
+            start += rooms.region(f);
         }
         return ORB_OK;
     };
-    rc = place_lists(nullptr);
+    rc = place_lists(rooms.regions);
     if (rc) return rc;
     HIP_TRY(hipMemcpyAsync(d_in, h_in, B.in, hipMemcpyHostToDevice, st));
     const WinPair* d_grid = (const WinPair*)(d_in + i_grid);
@@ -407,6 +426,7 @@ int proj_search(orb_context* ctx, int rule, int n_frames, const orb_keypoint* kp
         const int limit = std::min(ctx->round_limit, ORB_PROJ_MAXIT);
         int k = 0;
         bool settled = false;
+        ctx->last_restarts = 0;
         int rl = lists();
         if (rl) return rl;
         // claim-resolution rounds until every frame has a round that changed
@@ -419,10 +439,9 @@ int proj_search(orb_context* ctx, int rule, int n_frames, const orb_keypoint* kp
             HIP_TRY(orb_launch_proj_finish(d_frames, n_frames, 0, st));
             HIP_TRY(hipMemcpyAsync(h_out, d_out, B.out, hipMemcpyDeviceToHost, st));
             HIP_TRY(hipStreamSynchronize(st));
-            bool fits = true;
-            for (int f = 0; f < n_frames; f++) fits = fits && tot[f] <= cap[f];
-            if (!fits) {                           // longer lists, from the start
-                rl = place_lists(tot);
+            if (tot[F] > frames[0].room.shared_cap) {  // longer lists, from the start
+                ctx->last_restarts++;
+                rl = place_lists(rooms.need(tot, orb_proj_queries_per_block()));
                 if (rl) return rl;
                 HIP_TRY(hipMemcpyAsync(d_in + i_frames, frames, F * sizeof(ProjFrame), hipMemcpyHostToDevice, st));
                 rl = lists();
@@ -480,6 +499,8 @@ int orb_context_last_rounds(const orb_context* ctx, int* sequential)
     if (sequential) *sequential = ctx->last_sequential;
     return ctx->last_rounds;
 }
+
+int orb_context_last_restarts(const orb_context* ctx) { return ctx ? ctx->last_restarts : ORB_E_ARG; }
 
 int orb_search_by_projection(orb_context* ctx, int n_frames, const orb_keypoint* kp, const uint8_t* desc,
                              const float* uright, const uint8_t* occupied, const int32_t* key_off,

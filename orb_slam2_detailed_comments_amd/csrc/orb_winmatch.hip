@@ -113,26 +113,36 @@ __device__ __forceinline__ int grid_enumerate(const int* __restrict__ cell_start
 // Room for n list entries of each group of a workgroup of 256 (n is the same
 // for a group's G lanes, 0 where there is no query): *off receives the
 // group's first entry; false where the lists do not fit.  One atomic per
-// workgroup.
+// workgroup, and another where the frame's region is full: the frames' regions
+// keep them off one counter (25 ns an append, one after another, 1800
+// workgroups in 16 frames of 1800 queries).
 template <int G>
-__device__ __forceinline__ bool take_entries(int n, unsigned long long* total, unsigned long long cap, unsigned* off)
+__device__ __forceinline__ bool take_entries(int n, const ListRoom& R, unsigned long long* off)
 {
     __shared__ int s_n[256 / G];
     __shared__ unsigned long long s_base;
+    __shared__ int s_fits;
     const int g = threadIdx.x / G;
     if ((threadIdx.x & (G - 1)) == 0) s_n[g] = n;
     __syncthreads();
     if (threadIdx.x == 0) {
         int all = 0;
         for (int i = 0; i < 256 / G; i++) all += s_n[i];
-        s_base = all > 0 ? atomicAdd(total, (unsigned long long)all) : 0;
+        const unsigned long long want = (unsigned)all;
+        const unsigned long long o = want ? atomicAdd(R.asked, want) : 0;
+        s_base = R.start + o;
+        s_fits = 1;
+        if (o + want > R.cap) {
+            const unsigned long long os = atomicAdd(R.asked_shared, want);
+            s_base = R.shared_start + os;
+            s_fits = os + want <= R.shared_cap;
+        }
     }
     __syncthreads();
     unsigned long long o = s_base;
     for (int i = 0; i < g; i++) o += (unsigned)s_n[i];
-    const bool fits = o + (unsigned)n <= cap;
-    *off = fits ? (unsigned)o : 0u;
-    return fits;
+    *off = s_fits ? o : 0;
+    return s_fits != 0;
 }
 
 // Cell of keypoint (x, y) (PosInGrid: round() of the float offset times the
@@ -212,7 +222,8 @@ __global__ __launch_bounds__(1024) void win_grid_kernel(const WinPair* __restric
         for (int i = tid; i < n; i += 1024) P.ccnt[0][i] = P.ccnt[1][i] = 0;
         for (int k = tid; k < ORB_WIN_MAXIT; k += 1024) P.changed[k] = k == 0 ? 1 : 4;   // bit 2: not run
     }
-    if (tid == 0) *P.total = 0;
+    if (tid == 0) *P.room.asked = 0;
+    if (tid == 0 && blockIdx.x == 0) *P.room.asked_shared = 0;
     float4 rec[WIN_PER];
     int cell[WIN_PER], at[WIN_PER];
 #pragma unroll
@@ -302,8 +313,8 @@ __global__ __launch_bounds__(256) void win_fill_kernel(const WinPair* __restrict
         if (grid_window(P.minX, P.maxX, P.minY, P.maxY, x, y, r, &cx0, &cx1, &cy0, &cy1))
             n = grid_count<WIN_G>(P.cell_start, cx0, cx1, cy0, cy1);
     }
-    unsigned off;
-    const bool fits = take_entries<WIN_G>(n, P.total, P.cand_cap, &off);
+    unsigned long long off;
+    const bool fits = take_entries<WIN_G>(n, P.room, &off);
     if (q >= P.n1) return;
     int cnt = 0;
     if (n > 0 && fits) {
@@ -486,6 +497,8 @@ __global__ __launch_bounds__(64) void win_greedy_kernel(const WinPair* __restric
     if (lane == 0) *P.nmatch = s_n;
 }
 
+extern "C" int orb_win_queries_per_block(void) { return 256 / WIN_G; }
+
 extern "C" hipError_t orb_launch_win_lists(const WinPair* d_pairs, int npairs, int max_n1, hipStream_t st)
 {
     if (npairs <= 0) return hipSuccess;
@@ -619,8 +632,8 @@ __global__ __launch_bounds__(256) void proj_fill_kernel(const ProjFrame* __restr
     if ((Q.flags & ORB_PQ_VALID) &&
         grid_window(P.minX, P.maxX, P.minY, P.maxY, Q.x, Q.y, Q.r, &cx0, &cx1, &cy0, &cy1))
         n = grid_count<16>(P.cell_start, cx0, cx1, cy0, cy1);
-    unsigned off;
-    const bool fits = take_entries<16>(n, P.total, P.cand_cap, &off);
+    unsigned long long off;
+    const bool fits = take_entries<16>(n, P.room, &off);
     if (q >= P.nq) return;
     int cnt = 0;
     if (n > 0 && fits) {
@@ -789,7 +802,7 @@ __global__ __launch_bounds__(1024) void proj_finish_kernel(const ProjFrame* __re
     __shared__ int s_count[2];
     const ProjFrame& P = frames[blockIdx.x];
     const int kc = proj_settled_round(P.changed);
-    if (kc == 0 || *P.total > P.cand_cap) return;      // more rounds, or longer lists, to come
+    if (kc == 0 || *P.room.asked_shared > P.room.shared_cap) return;   // more rounds, or longer lists, to come
     const int* out = P.out[kc & 1];
     for (int i = threadIdx.x; i < P.n; i += 1024) owner[i] = -1;
     if (threadIdx.x < WIN_HISTO) hist[threadIdx.x] = 0;
@@ -847,8 +860,10 @@ extern "C" hipError_t orb_launch_proj_prep(ProjFrame* d_frames, int nframes, int
     return hipGetLastError();
 }
 
+extern "C" int orb_proj_queries_per_block(void) { return 256 / 16; }
+
 // d_grid: one WinPair per frame carrying the grid fields (kp2, n2, bounds,
-// uright, occupied, rec, cell_start) and the list total.
+// uright, occupied, rec, cell_start) and the lists' room.
 extern "C" hipError_t orb_launch_proj_lists(const WinPair* d_grid, const ProjFrame* d_frames, int nframes, int max_nq,
                                             hipStream_t st)
 {
@@ -969,7 +984,7 @@ __global__ __launch_bounds__(1024) void win_finish_kernel(const WinPair* __restr
     __shared__ int s_n;
     const WinPair& P = pairs[blockIdx.x];
     const int ks = win_settled_round(P.changed);
-    if (ks == 0 || *P.total > P.cand_cap) return;  // more rounds, the sequential pass or longer lists to come
+    if (ks == 0 || *P.room.asked_shared > P.room.shared_cap) return;   // more rounds, the sequential pass or longer lists to come
     const int* out = P.out[ks & 1];
     const int n1 = P.n1, t = threadIdx.x;
     constexpr int PER = WIN_PER;                   // queries t, t + 1024, ... of a thread, read together
