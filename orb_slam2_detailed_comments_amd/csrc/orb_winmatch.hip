@@ -50,13 +50,15 @@ __device__ __forceinline__ bool grid_window(float minX, float maxX, float minY, 
 }
 
 // Keypoints in the window's cells, by a group of G lanes (all of them call).
+// A negative radius (negative threshold or window) can put the last row before
+// the first: such columns hold none, as in the reference's loops.
 template <int G>
 __device__ __forceinline__ int grid_count(const int* __restrict__ cell_start, int cx0, int cx1, int cy0, int cy1)
 {
     const int sub = threadIdx.x & (G - 1);
     int n = 0;
     for (int ix = cx0 + sub; ix <= cx1; ix += G)
-        n += cell_start[ix * WIN_ROWS + cy1 + 1] - cell_start[ix * WIN_ROWS + cy0];
+        n += max(cell_start[ix * WIN_ROWS + cy1 + 1] - cell_start[ix * WIN_ROWS + cy0], 0);
 #pragma unroll
     for (int o = 1; o < G; o <<= 1) n += __shfl_xor(n, o, G);
     return n;
@@ -78,7 +80,7 @@ __device__ __forceinline__ int grid_enumerate(const int* __restrict__ cell_start
         int a = 0, len = 0;
         if (ix <= cx1) {
             a = cell_start[ix * WIN_ROWS + cy0];
-            len = cell_start[ix * WIN_ROWS + cy1 + 1] - a;
+            len = max(cell_start[ix * WIN_ROWS + cy1 + 1] - a, 0);
         }
         int inc = len;                             // inclusive scan of the run lengths
 #pragma unroll
