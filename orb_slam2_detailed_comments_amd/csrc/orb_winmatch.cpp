@@ -235,9 +235,11 @@ int sfi_impl(orb_context* ctx, int n_pairs, const orb_keypoint* kp1, const uint8
         }
         *ms = (float)(std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count() / steps);
     }
-    if (N1) {
-        std::memcpy(matches12, h_out + o_m12, n1 * 4);
-        std::memcpy(prev_matched, h_out + o_prev, n1 * 8);
+    // (rows before the first pair's are not the call's to write)
+    const size_t r1 = (size_t)off1[0];
+    if (n1 > r1) {
+        std::memcpy(matches12 + r1, h_out + o_m12 + r1 * 4, (n1 - r1) * 4);
+        std::memcpy(prev_matched + 2 * r1, h_out + o_prev + r1 * 8, (n1 - r1) * 8);
     }
     std::memcpy(nmatches, h_out + o_nm, P * 4);
     return ORB_OK;
@@ -476,8 +478,10 @@ int proj_search(orb_context* ctx, int rule, int n_frames, const orb_keypoint* kp
         }
         *ms = (float)(std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count() / steps);
     }
-    if (Q) std::memcpy(pt_match, h_out + o_ptm, np * 4);
-    if (N) std::memcpy(key_point, h_out + o_keyp, nk * 4);
+    // (rows before the first frame's are not the call's to write)
+    const size_t k0 = (size_t)key_off[0], q0 = (size_t)pt_off[0];
+    if (np > q0) std::memcpy(pt_match + q0, h_out + o_ptm + q0 * 4, (np - q0) * 4);
+    if (nk > k0) std::memcpy(key_point + k0, h_out + o_keyp + k0 * 4, (nk - k0) * 4);
     std::memcpy(nmatches, h_out + o_nm, F * 4);
     return ORB_OK;
 }
