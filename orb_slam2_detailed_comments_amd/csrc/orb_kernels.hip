@@ -2791,14 +2791,13 @@ __global__ __launch_bounds__(256) void knn_mfma_kernel(const uint8_t* __restrict
     __shared__ int2 s_key[3][NG][64];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hb = lane >> 5, i32 = lane & 31;
-    // XCD x (workgroups b with b % 8 == x) takes chunks x, x + 8, ..., all
-    // query blocks of a chunk one after another, so the chunk's rows come
-    // from memory once and from that XCD's L2 after that (2000 x 1M search
-    // 220 -> 197 us against chunks spread over the XCDs).
-    const int nqb = (nq + 32 * NG - 1) / (32 * NG);
-    const int slot = blockIdx.x / ORB_NUM_XCD;
-    const int chunk = slot / nqb * ORB_NUM_XCD + blockIdx.x % ORB_NUM_XCD;
-    const int qbase = slot % nqb * 32 * NG;
+    // XCD x (workgroups b with b % 8 == x; a row of the grid is a multiple of
+    // 8 of them) takes chunks x, x + 8, ..., a grid row's chunks' query blocks
+    // one after another, so a chunk's rows come from memory once and from that
+    // XCD's L2 after that (2000 x 1M search 220 -> 197 us against chunks spread
+    // over the XCDs).
+    const int chunk = (int)(blockIdx.y * ORB_NUM_XCD + blockIdx.x % ORB_NUM_XCD);
+    const int qbase = (int)(blockIdx.x / ORB_NUM_XCD) * 32 * NG;
     if (chunk >= nchunks) return;
 
     // Query operands: lane (query i32, half hb) holds words 4 hb + c.
@@ -2970,6 +2969,22 @@ extern "C" int orb_knn_chunk_rows(int nq, long long nm, int method, size_t max_e
     return rows;
 }
 
+// The MFMA search's grid: query blocks (8 workgroups each, a chunk apiece) by
+// groups of 8 chunks.  HIP wants fewer than 2^32 threads along x and 65536
+// workgroups along y: at most 2^27 queries, and 2^31 rows are 2^15 groups of
+// KNN_CHUNK rows (smaller chunks are for grids below 1024 workgroups).
+// Returns 0, or -1 where the grid does not fit.
+extern "C" int orb_knn_grid(int nq, long long nm, int chunk_rows, unsigned* x, unsigned* y)
+{
+    const long long chunks = (nm + chunk_rows - 1) / chunk_rows;
+    const long long gx = ORB_NUM_XCD * (((long long)nq + 32 * KNN_NG - 1) / (32 * KNN_NG));
+    const long long gy = (chunks + ORB_NUM_XCD - 1) / ORB_NUM_XCD;
+    if (gx * 256 >= (1ll << 32) || gy > 65535) return -1;
+    *x = (unsigned)gx;
+    *y = (unsigned)gy;
+    return 0;
+}
+
 extern "C" hipError_t orb_launch_knn2(const uint8_t* q, int nq, const uint8_t* m, long long nm, int method,
                                       float ratio, uint2* part, int chunk_rows, int* idx2, int* dist2,
                                       uint8_t* accept, hipStream_t st, hipEvent_t* ev)
@@ -2978,10 +2993,10 @@ extern "C" hipError_t orb_launch_knn2(const uint8_t* q, int nq, const uint8_t* m
     if (nq <= 0) return hipSuccess;
     if (ev) (void)hipEventRecord(ev[0], st);
     if (nchunks > 0) {
+        unsigned gx = 0, gy = 0;
+        if (method == 1 && orb_knn_grid(nq, nm, chunk_rows, &gx, &gy)) return hipErrorInvalidValue;
         if (method == 1)
-            knn_mfma_kernel<KNN_NG><<<(nchunks + ORB_NUM_XCD - 1) / ORB_NUM_XCD * ORB_NUM_XCD *
-                                          ((nq + 32 * KNN_NG - 1) / (32 * KNN_NG)),
-                                      256, 0, st>>>(q, nq, m, nm, part, nchunks, chunk_rows);
+            knn_mfma_kernel<KNN_NG><<<dim3(gx, gy), 256, 0, st>>>(q, nq, m, nm, part, nchunks, chunk_rows);
         else
             knn_popc_kernel<<<dim3(nchunks, (nq + 255) / 256), 256, 0, st>>>(q, nq, m, nm, part, nchunks, chunk_rows);
     }
