@@ -1405,7 +1405,8 @@ __device__ __forceinline__ bool octree_fast(OctFast& S, const LevelJob& L, int l
             const int pos = (int)(at & 0xFFFFu) +
                             (at >> 31 ? __popc(((at >> 16) & 15u) >> (quadrant(place, depth + 1) + 1)) : 0);
             put(k, place | ((unsigned)pos << 16));
-            if (more) atomicAdd((int*)&S.cc[pos] + quadrant(place, depth + 2), 1);
+            // (past depth OCT_D every node holds one key, and its count alone matters)
+            if (more) atomicAdd((int*)&S.cc[pos] + quadrant(place, min(depth + 2, OCT_D)), 1);
         }
         __syncthreads();
     }
