@@ -159,9 +159,11 @@ struct orb_context {
     size_t win_cap = 0;
     void* d_wcand = nullptr;
     size_t wcand_cap = 0;
-    // pinned staging of the windowed searches' inputs and outputs
+    // pinned staging of the windowed searches' inputs and outputs, and the
+    // events of its two halves' copies
     void* h_win = nullptr;
     size_t hwin_cap = 0;
+    hipEvent_t win_ev[2] = {nullptr, nullptr};
     // map-point scratch: observation descriptors, offsets, chosen rows
     uint8_t* d_mp = nullptr;
     int* d_mpo = nullptr;

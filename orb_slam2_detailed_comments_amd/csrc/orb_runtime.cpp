@@ -57,6 +57,8 @@ void orb_context_release_ref(orb_context* ctx)
     for (void* q : mp)
         if (q) (void)hipFree(q);
     if (ctx->h_win) (void)hipHostFree(ctx->h_win);
+    for (hipEvent_t e : ctx->win_ev)
+        if (e) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }

@@ -48,8 +48,8 @@ int reserve_pinned(orb_context* ctx, void** p, size_t* cap, size_t bytes)
 }
 
 // A call's device block: what is copied in, what is copied out, then scratch.
-// Inputs are packed in pinned memory at their device offsets, so that one
-// copy takes them; so are the outputs.
+// The outputs are packed in pinned memory at their device offsets, so that one
+// copy takes them; so are the inputs (Upload).
 struct Block {
     size_t in = 0, out = 0, scratch = 0;
     size_t add_in(size_t bytes) { return add(in, bytes); }
@@ -60,6 +60,65 @@ struct Block {
         const size_t o = end;
         end += up(bytes);
         return o;
+    }
+};
+
+// A call's inputs on their way to the device: arrays of the caller's at the
+// offsets below `tables`, then what the host keeps for the call (jobs, offsets,
+// parameters) up to `in`.  Up to kWindow bytes of arrays are packed in front of
+// the tables in pinned memory, and one copy takes both.  More of them go through
+// the window's halves in turn, one being filled while the other is copied, and
+// the tables follow: so the pinned buffer does not grow with them, whose first
+// allocation costs 0.3 ms a megabyte.
+// Last-frame searches of 256 frames (61 MB): first call of a context 27 ms with
+// everything pinned and 8.6 so, later ones 4.37 and 3.4; 64 frames (15 MB) 7.9
+// and 5.3, later 0.87 and 0.84.  Windows of 4 MB: 32 frames (7.6 MB) 525 us, 497
+// in one copy; of 2 MB: 16 frames (3.8 MB) 326 us, 286 in one copy.
+constexpr size_t kWindow = (size_t)8 << 20;
+
+struct Upload {
+    orb_context* ctx;
+    char* d;
+    char* h = nullptr;
+    size_t tables, in, window;
+    int half = 0;
+    bool busy[2] = {false, false};
+
+    Upload(orb_context* c, size_t tables_at, size_t in_bytes)
+        : ctx(c), d((char*)c->d_win), tables(tables_at), in(in_bytes), window(std::min(tables_at, kWindow))
+    {
+    }
+    size_t pinned_bytes() const { return window + (in - tables); }
+    bool whole() const { return window == tables; }
+    template <class T>
+    T* table(size_t at) const
+    {
+        return (T*)(h + window + (at - tables));
+    }
+    int put(size_t at, const void* src, size_t bytes)
+    {
+        if (whole()) {
+            std::memcpy(h + at, src, bytes);
+            return ORB_OK;
+        }
+        for (size_t o = 0; o < bytes; o += kWindow / 2, half ^= 1) {
+            const size_t n = std::min(bytes - o, kWindow / 2);
+            char* to = h + half * (kWindow / 2);
+            hipEvent_t& ev = ctx->win_ev[half];
+            if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+            if (busy[half]) HIP_TRY(hipEventSynchronize(ev));
+            std::memcpy(to, (const char*)src + o, n);
+            HIP_TRY(hipMemcpyAsync(d + at + o, to, n, hipMemcpyHostToDevice, ctx->stream));
+            HIP_TRY(hipEventRecord(ev, ctx->stream));
+            busy[half] = true;
+        }
+        return ORB_OK;
+    }
+    int finish() const
+    {
+        const size_t from = whole() ? 0 : tables;
+        HIP_TRY(hipMemcpyAsync(d + from, whole() ? h : h + window, in - from, hipMemcpyHostToDevice, ctx->stream));
+        return ORB_OK;
     }
 };
 
@@ -140,20 +199,24 @@ int sfi_impl(orb_context* ctx, int n_pairs, const orb_keypoint* kp1, const uint8
     const size_t s_out = B.add_scratch(2 * n1 * 4), s_claim = B.add_scratch(3 * n2 * ORB_WIN_SLOTS * 4);
     const size_t s_ccnt = B.add_scratch(3 * n2 * 4);
     int rc = reserve(ctx, &ctx->d_win, &ctx->win_cap, B.in + B.out + B.scratch);
-    if (!rc) rc = reserve_pinned(ctx, &ctx->h_win, &ctx->hwin_cap, B.in + B.out);
+    if (rc) return rc;
+    Upload up_in(ctx, i_pairs, B.in);
+    rc = reserve_pinned(ctx, &ctx->h_win, &ctx->hwin_cap, up_in.pinned_bytes() + B.out);
     if (rc) return rc;
     char *d_in = (char*)ctx->d_win, *d_out = d_in + B.in, *d_s = d_out + B.out;
-    char *h_in = (char*)ctx->h_win, *h_out = h_in + B.in;
+    char* h_out = (char*)ctx->h_win + up_in.pinned_bytes();
+    up_in.h = (char*)ctx->h_win;
     if (N1) {
-        std::memcpy(h_in + i_kp1, kp1, n1 * sizeof(OrbKeyPoint));
-        std::memcpy(h_in + i_d1, desc1, n1 * 32);
-        std::memcpy(h_in + i_prev, prev_matched, n1 * 8);
+        rc = up_in.put(i_kp1, kp1, n1 * sizeof(OrbKeyPoint));
+        if (!rc) rc = up_in.put(i_d1, desc1, n1 * 32);
+        if (!rc) rc = up_in.put(i_prev, prev_matched, n1 * 8);
     }
     if (N2) {
-        std::memcpy(h_in + i_kp2, kp2, n2 * sizeof(OrbKeyPoint));
-        std::memcpy(h_in + i_d2, desc2, n2 * 32);
+        if (!rc) rc = up_in.put(i_kp2, kp2, n2 * sizeof(OrbKeyPoint));
+        if (!rc) rc = up_in.put(i_d2, desc2, n2 * 32);
     }
-    WinPair* pairs = (WinPair*)(h_in + i_pairs);
+    if (rc) return rc;
+    WinPair* pairs = up_in.table<WinPair>(i_pairs);
     Lists lists;
     for (int p = 0; p < n_pairs; p++) {
         WinPair& w = pairs[p];
@@ -202,8 +265,8 @@ int sfi_impl(orb_context* ctx, int n_pairs, const orb_keypoint* kp1, const uint8
         return ORB_OK;
     };
     rc = place_lists(lists.regions);
+    if (!rc) rc = up_in.finish();
     if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(d_in, h_in, B.in, hipMemcpyHostToDevice, st));
     const WinPair* d_pairs = (const WinPair*)(d_in + i_pairs);
     auto run_device = [&]() -> int {
         const int limit = std::min(ctx->round_limit, ORB_WIN_MAXIT);
@@ -360,25 +423,29 @@ int proj_search(orb_context* ctx, int rule, int n_frames, const orb_keypoint* kp
                  s_q = B.add_scratch(np * sizeof(ProjQuery)), s_cnt = B.add_scratch(np * 4),
                  s_off = B.add_scratch(np * 8), s_out = B.add_scratch(2 * np * 4), s_claim = B.add_scratch(3 * nk * 4);
     int rc = reserve(ctx, &ctx->d_win, &ctx->win_cap, B.in + B.out + B.scratch);
-    if (!rc) rc = reserve_pinned(ctx, &ctx->h_win, &ctx->hwin_cap, B.in + B.out);
+    if (rc) return rc;
+    Upload up_in(ctx, i_ptoff, B.in);
+    rc = reserve_pinned(ctx, &ctx->h_win, &ctx->hwin_cap, up_in.pinned_bytes() + B.out);
     if (rc) return rc;
     char *d_in = (char*)ctx->d_win, *d_out = d_in + B.in, *d_s = d_out + B.out;
-    char *h_in = (char*)ctx->h_win, *h_out = h_in + B.in;
+    char* h_out = (char*)ctx->h_win + up_in.pinned_bytes();
+    up_in.h = (char*)ctx->h_win;
     if (N) {
-        std::memcpy(h_in + i_kp, kp, nk * sizeof(OrbKeyPoint));
-        std::memcpy(h_in + i_desc, desc, nk * 32);
-        std::memcpy(h_in + i_ur, uright, nk * 4);
-        std::memcpy(h_in + i_occ, occupied, nk);
+        rc = up_in.put(i_kp, kp, nk * sizeof(OrbKeyPoint));
+        if (!rc) rc = up_in.put(i_desc, desc, nk * 32);
+        if (!rc) rc = up_in.put(i_ur, uright, nk * 4);
+        if (!rc) rc = up_in.put(i_occ, occupied, nk);
     }
     if (Q) {
-        std::memcpy(h_in + i_pts, pts, np * 24);
-        std::memcpy(h_in + i_pdesc, pdesc, np * 32);
+        if (!rc) rc = up_in.put(i_pts, pts, np * 24);
+        if (!rc) rc = up_in.put(i_pdesc, pdesc, np * 32);
     }
-    std::memcpy(h_in + i_ptoff, pt_off, (F + 1) * 4);
-    std::memcpy(h_in + i_scale, scale, (size_t)nlevels * 4);
-    if (rule == 2) std::memcpy(h_in + i_cam, cam, F * 7 * 4);
-    WinPair* grid = (WinPair*)(h_in + i_grid);
-    ProjFrame* frames = (ProjFrame*)(h_in + i_frames);
+    if (rc) return rc;
+    std::memcpy(up_in.table<char>(i_ptoff), pt_off, (F + 1) * 4);
+    std::memcpy(up_in.table<char>(i_scale), scale, (size_t)nlevels * 4);
+    if (rule == 2) std::memcpy(up_in.table<char>(i_cam), cam, F * 7 * 4);
+    WinPair* grid = up_in.table<WinPair>(i_grid);
+    ProjFrame* frames = up_in.table<ProjFrame>(i_frames);
     Lists rooms;
     for (int f = 0; f < n_frames; f++) {
         const int k0 = key_off[f], q0 = pt_off[f];
@@ -436,8 +503,8 @@ int proj_search(orb_context* ctx, int rule, int n_frames, const orb_keypoint* kp
         return ORB_OK;
     };
     rc = place_lists(rooms.regions);
+    if (!rc) rc = up_in.finish();
     if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(d_in, h_in, B.in, hipMemcpyHostToDevice, st));
     const WinPair* d_grid = (const WinPair*)(d_in + i_grid);
     ProjFrame* d_frames = (ProjFrame*)(d_in + i_frames);
     auto lists = [&]() -> int {
