@@ -86,7 +86,6 @@ inline void disc_umax(int umax[16])
     }
 }
 
-// Border index of REFLECT_101 (the level kernel's halo rule).
 // First level column that OpenCV's SSE2 VResizeLinearVec_32s8u leaves to
 // the scalar pass: it covers 16 columns at a time while x <= w - 16, then 4
 // at a time while x < w - 4 (imgwarp.cpp, OpenCV 2.4/3.x).
@@ -96,13 +95,6 @@ inline int sse2_resize_end(int w)
     while (x <= w - 16) x += 16;
     while (x < w - 4) x += 4;
     return x;
-}
-
-inline int reflect101(int i, int n)
-{
-    if (i < 0) i = -i;
-    if (i >= n) i = 2 * n - 2 - i;
-    return i < 0 ? 0 : (i >= n ? n - 1 : i);
 }
 
 struct LevelPlan {
@@ -553,7 +545,6 @@ struct orb_extractor {
                     tab[t].x = std::min(std::max(sy, 0), sh - 1) | (std::min(std::max(sy + 1, 0), sh - 1) << 16);
                     tab[t].y = (int)std::nearbyint((1.f - fy) * 2048.f) | ((int)std::nearbyint(fy * 2048.f) << 16);
                 }
-                const size_t ty = t - h;
             }
         }
         // Quadtree place at depth ORB_OCT_D, split into its x and y parts: the

@@ -1879,10 +1879,9 @@ __global__ __launch_bounds__(256) void describe_kernel(const ImageJob* __restric
     // any use: the 31x31 orientation patch of the level and the 37x37 window
     // of the blurred level that every rotated BRIEF sample falls in (pattern
     // radius <= 18.39 px).  Keypoints lie >= 19 px inside the level (x <= w-20,
-    // y <= h-20), so every dword lies in rows that have a successor and ends
-    // at most 2 bytes past the row's last pixel: inside the level's buffer.
-    // Blur window rows past the patch (37..47) are clamped to its last row
-    // and unused.
+    // y <= h-20), so the pieces end at most 13 (level) and 2 (blur) bytes past
+    // a row's last pixel, and every row read has successors: inside the level's
+    // buffer.
     const int xa0 = (cx - 15) & ~3;               // 31 px + <= 3 of alignment: 9 dwords a row
     const int xb0 = (cx - 18) & ~3;               // 37 px + <= 3 of alignment: 10 dwords a row
     // Neighbouring lanes read neighbouring pieces of a row, so that a load meets
@@ -2765,15 +2764,15 @@ __device__ __forceinline__ knn_v8i expand_query(unsigned w)
 // Workgroup: 4 wavefronts, the same 32 * NG queries, one map chunk; wavefront
 // w takes the 32-row tiles w, w + 4, ...  Bound: the MFMA pipe (a kernel of
 // the same instructions on registers alone reaches 7.5 of the 10 POP/s).
-// 2000 queries x 1M rows: search and merge 170 us (6.2 POP/s) where int8
-// MFMAs with every key kept took 404 us; 64 x 1M 15 us (171).
+// 2000 queries x 1M rows: search 184 us (5.6 POP/s), a call among others 178
+// where int8 MFMAs with every key kept took 402; 64 x 1M 14 us (171).
 //
 // v_mfma_scale_f32_32x32x64_f8f6f4 on FP4 operands does 65536 multiply-adds
 // in 32 cycles, twice the int8 rate, and a descriptor word expands into one
 // operand lane with 5 VALU ops.  sum m (1 - 2q) = Hamming - |q|; the C input
 // adds 256 and the row / 8192, so every accumulator is a non-negative
-// multiple of 2^-13 of at most 22 bits, exact in float, and its bits order
-// as an integer:
+// multiple of 2^-13 below 513, of at most 23 bits (an empty query against a
+// full row), exact in float, and its bits order as an integer:
 //   key = Hamming - |q| + 256 + row / 8192.
 // |q| is constant per query, so keys order (distance, row).
 //
@@ -2903,7 +2902,7 @@ __global__ __launch_bounds__(256) void knn_mfma_kernel(const uint8_t* __restrict
 // its lanes stride over the chunks, then 16 of them take a row each of the
 // best row's group (knn_mfma_kernel keeps one key per group of 16).  knn_popc_kernel's keys are
 // the two smallest already, and then the group holds none nearer.  Bound:
-// latency; 8 us for 2000 queries x 123 chunks, where one thread per query
+// latency; 4 us for 2000 queries x 123 chunks, where one thread per query
 // took 47 us, a chain of scattered reads.
 __global__ __launch_bounds__(256) void knn_merge_kernel(const uint2* __restrict__ part, int nq, int nchunks,
                                                         int chunk_rows, const uint8_t* __restrict__ q,
@@ -2957,9 +2956,9 @@ __global__ __launch_bounds__(256) void knn_merge_kernel(const uint2* __restrict_
 // Rows per map chunk: KNN_CHUNK, halved while the grid has fewer than 1024
 // workgroups (the GPU holds that many), down to 512 rows, as long as the
 // partial keys (one entry per query and chunk) stay within max_entries.
-// Search of 500 x 100k: 13 us at 512 rows, 169 us before at 8192 (26
-// workgroups); 2000 x 1M: 197 us at 8192 rows, 201 at 4096, 211 at 2048, and
-// the merge grows with the chunks.
+// Search + merge in us at 8192, 4096, 2048 and 512 rows: 500 x 100k 23 + 6, 15
+// + 6, 12 + 6, 13 + 7; 2000 x 1M 186 + 7, 187 + 8, 197 + 10, 258 + 21; 64 x 1M
+// 24 + 6, 15 + 7, 13 + 9, 14 + 18 (the merge grows with the chunks).
 extern "C" int orb_knn_chunk_rows(int nq, long long nm, int method, size_t max_entries)
 {
     const long long tiles = method == 1 ? (nq + 32 * KNN_NG - 1) / (32 * KNN_NG) : (nq + 255) / 256;

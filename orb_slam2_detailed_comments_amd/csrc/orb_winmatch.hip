@@ -299,7 +299,7 @@ __device__ __forceinline__ int row_distance(const uint4 a0, const uint4 a1, cons
 // Each level-0 query takes room for all its window's keypoints and stores the
 // (i2, distance) of those inside the circle, in the reference's order.
 // Bound: latency (a few dependent loads per query).  2000 queries, window 100:
-// 9.5 us; counting, scanning and filling in turn, a wavefront per query that
+// 9.8 us; counting, scanning and filling in turn, a wavefront per query that
 // walked its window column by column, took 44 us.
 #define WIN_G 32
 __global__ __launch_bounds__(256) void win_fill_kernel(const WinPair* __restrict__ pairs)
@@ -340,13 +340,6 @@ __global__ __launch_bounds__(256) void win_fill_kernel(const WinPair* __restrict
     }
 }
 
-// One wavefront per pair.  Query by query, in index order: lanes take the
-// list positions lane, lane+64, ... (ascending), skip candidates already
-// held at a distance <= theirs, and keep (first minimum as distance << 12 |
-// position, second smallest distance); a butterfly merge gives the
-// reference's sequential best / second.  Lane 0 applies TH_LOW, the ratio
-// and the steal of a matched target; the rotation histogram counts every
-// match event, as rotHist's sizes do.
 // The first round k >= 1 that ran, changed no outcome and read complete
 // claims (round k - 1 did not overflow its slots): its outcomes are the
 // in-order pass's.  0 if there is none.
@@ -369,6 +362,13 @@ __device__ __forceinline__ int proj_settled_round(const int* chg)
     return b ? __ffsll((long long)b) - 1 : 0;
 }
 
+// One wavefront per pair.  Query by query, in index order: lanes take the
+// list positions lane, lane+64, ... (ascending), skip candidates already
+// held at a distance <= theirs, and keep (first minimum as distance << 12 |
+// position, second smallest distance); a butterfly merge gives the
+// reference's sequential best / second.  Lane 0 applies TH_LOW, the ratio
+// and the steal of a matched target; the rotation histogram counts every
+// match event, as rotHist's sizes do.
 __global__ __launch_bounds__(64) void win_greedy_kernel(const WinPair* __restrict__ pairs, int skip_settled)
 {
     __shared__ int vmd[WIN_CAP];
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(256) void proj_prep_last_kernel(ProjFrame* __restri
 // GetFeaturesInArea's level rule and circle and the mvuRight check (:111-118:
 // the right-image u within the radius), in the reference's order.
 // Bound: latency (a few dependent loads per query).  16 frames x 1800 points,
-// th 15: 27 us (counting, scanning and filling in turn 91 us); 1 frame, th 3:
+// th 15: 28 us (counting, scanning and filling in turn 91 us); 1 frame, th 3:
 // 9 us (26).
 __global__ __launch_bounds__(256) void proj_fill_kernel(const ProjFrame* __restrict__ frames)
 {
