@@ -82,11 +82,19 @@ struct Upload {
     char* h = nullptr;
     size_t tables, in, window;
     int half = 0;
-    bool busy[2] = {false, false};
+    bool busy[2] = {false, false}, sent = false;
 
     Upload(orb_context* c, size_t tables_at, size_t in_bytes)
         : ctx(c), d((char*)c->d_win), tables(tables_at), in(in_bytes), window(std::min(tables_at, kWindow))
     {
+    }
+    Upload(const Upload&) = delete;
+    Upload& operator=(const Upload&) = delete;
+    // A call that ends before its tables are sent (no room for the lists) leaves
+    // no copy from the window under way: the next call refills or frees it.
+    ~Upload()
+    {
+        if (!sent && (busy[0] || busy[1])) (void)hipStreamSynchronize(ctx->stream);
     }
     size_t pinned_bytes() const { return window + (in - tables); }
     bool whole() const { return window == tables; }
@@ -114,10 +122,11 @@ struct Upload {
         }
         return ORB_OK;
     }
-    int finish() const
+    int finish()
     {
         const size_t from = whole() ? 0 : tables;
         HIP_TRY(hipMemcpyAsync(d + from, whole() ? h : h + window, in - from, hipMemcpyHostToDevice, ctx->stream));
+        sent = true;
         return ORB_OK;
     }
 };
